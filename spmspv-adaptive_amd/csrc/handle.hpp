@@ -173,8 +173,9 @@ struct spmspv_handle_s {
 
 constexpr long long kSigPending = -0x5A5A5A5A5A5ALL;
 // host-coherent signal words: 1 selector word, 3 result count, 16.. a BFS
-// level's frontier size and choice (16) and its selector features (17..24)
-constexpr int kSigWords = 32, kSigBfs = 16;
+// level's frontier size and choice (16) and its selector features (17..24),
+// 26.. a multi-source BFS level's frontier size and degree sum
+constexpr int kSigWords = 32, kSigBfs = 16, kSigMs = 26;
 
 namespace spmspv {
 int set_error(spmspv_handle_t h, int code, const std::string& msg);
