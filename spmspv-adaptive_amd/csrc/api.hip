@@ -658,7 +658,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
           xin = h->dense_x();
         }
         if ((rc = ensure_row_tiles(h))) return rc;
-        launch_row_merge(s, masked, hits, h->csr_row, h->csr_col, h->csr_val, xin, nullptr, m, h->nnz,
+        launch_row_merge(s, masked, hits, h->csr_row, h->csr_col, h->csr_val, xin, m, h->nnz,
                          h->row_split, h->n_row_tiles, h->row_vt, yout, h->bitmap, h->row_carry_val,
                          h->row_carry_row, h->row_carry_hit, h->time_main ? h->evk0 : nullptr,
                          h->time_main ? h->evk1 : nullptr, h->gate);

@@ -5,16 +5,24 @@
 //
 // A level runs the boolean form of the slot chosen for it (row and column
 // indices only: no matrix value is read and no FP32 arithmetic is done):
-//   K0/K2  top-down: frontier vertices scan their columns and claim
+//   K0/K2  top-down: frontier vertices scan their columns and mark
 //          unvisited rows (naive team per vertex / merge-path balanced);
 //   K1/K3  top-down gather of all neighbours' row keys, in-house radix sort
-//          of the keys alone, then each distinct row claimed;
-//   K4     bottom-up: each unvisited row (one lane) scans its neighbours
-//          and stops at the first frontier member;
-//   K5/K7  merge-path row tiles OR-ing the frontier bits of each row's
-//          columns into a hit bit, then claim (on booleans the masked and
-//          unmasked row kernels coincide);
-//   K6     naive row scan without early exit, hit bits, then claim.
+//          of the keys alone, then each distinct row marked;
+//   K4/K5/K7  bottom-up: each unvisited row scans its neighbours and stops at
+//          the first frontier member (on booleans the masked and unmasked
+//          load-balanced row products coincide, and a row's result is known
+//          at its first hit: the merge-path scan of every nonzero that K5/K7
+//          ran before took 420 us at a large level of R-MAT s22, this 60 to
+//          120 us; at a level of one or two vertices, where no row stops
+//          early, 660 us against 390);
+//   K6     naive row scan without early exit.
+// Every slot marks the rows it reaches in the next frontier's bit array;
+// one collect pass then takes the unvisited ones among them, writes their
+// levels and lists them, with one list append per workgroup round: device
+// atomics on one address take 16 ns each, and an append per wave in every
+// slot kernel had made those kernels wait for the counter. R-MAT s22, one
+// source: 1,440 -> 490 us.
 // Levels are int32 and unique, so any order of claims gives the same
 // levels. The selector for level L+1 runs in the same stream right after
 // level L (features of the new frontier + MLP, one launch), and a last
@@ -39,7 +47,7 @@ struct BfsState {
   unsigned* fbits[2] = {nullptr, nullptr};  // frontier bit arrays
   int* front[2] = {nullptr, nullptr};       // frontier lists
   int* cnt = nullptr;                       // [0],[1] sizes, [2] level, [3] bottom-up queue size
-  int* queue = nullptr;                     // m: rows the bottom-up head left undecided
+  int2* queue = nullptr;                    // bottom-up: (row, chunk) items the head left undecided
   unsigned long long* reached = nullptr;    // [0] vertices, [1] degree sum
   void* alloc = nullptr;
   hipStream_t own_stream = nullptr;
@@ -52,36 +60,21 @@ struct BfsState {
 namespace {
 
 constexpr int kBfsGrid = 2048;
-constexpr int kBuBatch = 8;  // neighbours each row tests in the bottom-up head pass
-constexpr int kBuTeam = 8;   // lanes per queued row in the bottom-up tail pass
+constexpr int kBfsNT = 256;
+constexpr int kBuBatch = 8;    // neighbours each row tests in the bottom-up head pass
+constexpr int kBuTeam = 16;    // lanes per queued item in the bottom-up tail pass
+constexpr int kBuChunk = 256;  // neighbours per queued item
+constexpr int kBuUnroll = 4;   // neighbours a lane has in flight
+constexpr int kBuRows = 8;     // most rows per thread and queue append
 
-__device__ __forceinline__ int wave_append(int* counter, bool pred) {
-  const uint64_t b = __ballot(pred);
-  if (!b) return -1;
-  const int leader = __builtin_ctzll(b);
-  int base = 0;
-  if (lane() == leader) base = atomicAdd(counter, __popcll(b));
-  base = __shfl(base, leader, kWave);
-  const uint64_t lt = lane() == 0 ? 0ull : (~0ull >> (kWave - lane()));
-  return pred ? base + __popcll(b & lt) : -1;
-}
-
-__device__ __forceinline__ bool try_claim(unsigned* visited, int v) {
+// Marks row v in the next frontier unless it is visited or marked already
+// (visited is constant while a slot's kernels run).
+__device__ __forceinline__ void mark_row(const unsigned* __restrict__ visited, unsigned* nbits, int v) {
   const unsigned bit = 1u << (v & 31);
-  if (__hip_atomic_load(visited + (v >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit)
-    return false;
-  return !(atomicOr(visited + (v >> 5), bit) & bit);
-}
-
-// Called by every lane of a wave (convergent): appends the claimed vertices.
-__device__ __forceinline__ void record(int v, bool claimed, int level, int* levels, int* nf,
-                                       int* ncnt, unsigned* nbits) {
-  const int pos = wave_append(ncnt, claimed);
-  if (claimed) {
-    levels[v] = level;
-    nf[pos] = v;
-    atomicOr(nbits + (v >> 5), 1u << (v & 31));
-  }
+  if (visited[v >> 5] & bit) return;
+  unsigned* w = nbits + (v >> 5);
+  if (__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit) return;
+  atomicOr(w, bit);
 }
 
 __global__ void k_bfs_init(int* levels, int n, unsigned* visited, unsigned* fb0, unsigned* fb1,
@@ -106,14 +99,14 @@ __global__ void k_bfs_init(int* levels, int n, unsigned* visited, unsigned* fb0,
   }
 }
 
-// Opens a level: empties the next frontier, advances the level number and
-// the device epoch that the level's look-back kernels use (their launch
-// arguments are frozen inside a captured graph).
 // The next level's frontier size and selector choice, tagged with the level
 // counter, into one host-coherent word (sig[0]), its selector features into
 // sig[1..8] first: the host polls one word per level instead of waiting for
-// the stream and three copies.
-__global__ void k_bfs_signal(const int* __restrict__ cnt, int nxt, const Ctl* __restrict__ ctl, long long* sig) {
+// the stream and three copies. Then opens that level: the counts of the
+// frontier it will fill and of its queue at 0, the level number and the
+// device epoch that its look-back kernels use (their launch arguments are
+// frozen inside a captured graph) advanced.
+__global__ void k_bfs_signal(int* cnt, int nxt, Ctl* ctl, long long* sig) {
   // the feature words are acknowledged (each writer waits for its store)
   // before the level word goes out; the host reads nothing else, so no L2
   // write-back is needed
@@ -126,54 +119,28 @@ __global__ void k_bfs_signal(const int* __restrict__ cnt, int nxt, const Ctl* __
     const long long w = ((long long)(cnt[2] & 0xffffff) << 40) | ((long long)(ctl->kernel_choice & 0xff) << 32) |
                         (long long)(unsigned)cnt[nxt];
     __hip_atomic_store(sig, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
-}
-
-__global__ void k_bfs_begin(int* cnt, int nxt, unsigned* nbits, int words, Ctl* ctl) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    cnt[nxt] = 0;
+    cnt[nxt ^ 1] = 0;
     cnt[2] += 1;
     cnt[3] = 0;
     ctl->epoch += 16;
   }
-  for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < words; w += gridDim.x * blockDim.x)
-    nbits[w] = 0u;
 }
 
-// K0: top-down, a team of 2^lg lanes per frontier vertex; loops are
-// wave-uniform so that wave_append stays convergent.
-__global__ __launch_bounds__(256) void k_td_naive(const int* __restrict__ colptr,
-                                                  const int* __restrict__ crow,
-                                                  const int* __restrict__ f, int* cnt, int cur,
-                                                  int lg, unsigned* visited, int* levels, int* nf,
-                                                  unsigned* nbits) {
+// K0: top-down, a team of 2^lg lanes per frontier vertex.
+__global__ __launch_bounds__(kBfsNT) void k_td_naive(const int* __restrict__ colptr,
+                                                     const int* __restrict__ crow,
+                                                     const int* __restrict__ f, const int* __restrict__ cnt,
+                                                     int cur, int lg, const unsigned* __restrict__ visited,
+                                                     unsigned* nbits) {
   const int fsz = cnt[cur];
-  const int level = cnt[2];
-  int* ncnt = cnt + (cur ^ 1);
-  const int team = 1 << lg, tpw = kWave >> lg;
+  const int team = 1 << lg;
   const int tl = threadIdx.x & (team - 1);
-  const int tin = (threadIdx.x & (kWave - 1)) >> lg;
-  const long long gw = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const long long nw = ((long long)gridDim.x * blockDim.x) >> 6;
-  for (long long base = gw * tpw; base < fsz; base += nw * tpw) {
-    const long long e = base + tin;
-    int b = 0, len = 0;
-    if (e < fsz) {
-      const int u = f[e];
-      b = colptr[u];
-      len = colptr[u + 1] - b;
-    }
-    const int mx = wave_max(len);
-    for (int k0 = 0; k0 < mx; k0 += team) {
-      const int k = k0 + tl;
-      bool cl = false;
-      int v = 0;
-      if (k < len) {
-        v = crow[b + k];
-        cl = try_claim(visited, v);
-      }
-      record(v, cl, level, levels, nf, ncnt, nbits);
-    }
+  const long long t0 = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> lg;
+  const long long nt = ((long long)gridDim.x * blockDim.x) >> lg;
+  for (long long i = t0; i < fsz; i += nt) {
+    const int u = f[i];
+    const int b = colptr[u], e = colptr[u + 1];
+    for (int k = b + tl; k < e; k += team) mark_row(visited, nbits, crow[k]);
   }
 }
 
@@ -184,15 +151,13 @@ __global__ __launch_bounds__(NT) void k_td_lb(const int* __restrict__ ptr,
                                               const int* __restrict__ xbeg,
                                               const int* __restrict__ split,
                                               const int* __restrict__ crow, const Ctl* ctl,
-                                              int* cnt, int cur, unsigned* visited, int* levels,
-                                              int* nf, unsigned* nbits) {
+                                              const int* __restrict__ cnt, int cur,
+                                              const unsigned* __restrict__ visited, unsigned* nbits) {
   constexpr int T = NT * VT;
   __shared__ int s_ptr[T + 2];
   __shared__ int s_beg[T + 2];
   __shared__ int s_seg[T];
   const int xnnz = cnt[cur];
-  const int level = cnt[2];
-  int* ncnt = cnt + (cur ^ 1);
   const long long ntiles = ctl->n_tiles;
   const long long W = (long long)xnnz + ctl->bin_len;
   for (long long t = blockIdx.x; t < ntiles; t += gridDim.x) {
@@ -222,180 +187,224 @@ __global__ __launch_bounds__(NT) void k_td_lb(const int* __restrict__ ptr,
       }
     }
     __syncthreads();
+    // all of a thread's rows are loaded before the first is tested
     const int np = (int)(b1 - b0);
-    for (int q0 = 0; q0 < np; q0 += NT) {
-      const int q = q0 + threadIdx.x;
-      bool cl = false;
-      int v = 0;
+    int v[VT];
+#pragma unroll
+    for (int j = 0; j < VT; ++j) {
+      const int q = j * NT + threadIdx.x;
+      v[j] = -1;
       if (q < np) {
         const int sg = s_seg[q];
-        v = crow[s_beg[sg] + (int)(b0 + q - s_ptr[sg])];
-        cl = try_claim(visited, v);
+        v[j] = crow[s_beg[sg] + (int)(b0 + q - s_ptr[sg])];
       }
-      record(v, cl, level, levels, nf, ncnt, nbits);
     }
+#pragma unroll
+    for (int j = 0; j < VT; ++j)
+      if (v[j] >= 0) mark_row(visited, nbits, v[j]);
     __syncthreads();
   }
 }
 
-// After the sort slots: claims the unique neighbour keys.
-// Claims the distinct rows of a sorted key list of *n_dev items (repeats
-// are skipped without a test-and-set).
-__global__ void k_claim_sorted(const unsigned* __restrict__ keys, const long long* __restrict__ n_dev,
-                               int* cnt, int cur, unsigned* visited, int* levels, int* nf, unsigned* nbits) {
+// After the sort slots: marks the distinct rows of a sorted key list of
+// *n_dev items (repeats are skipped without a test).
+__global__ void k_mark_sorted(const unsigned* __restrict__ keys, const long long* __restrict__ n_dev,
+                              const unsigned* __restrict__ visited, unsigned* nbits) {
   const long long k = *n_dev;
-  const int level = cnt[2];
-  int* ncnt = cnt + (cur ^ 1);
-  for (long long i0 = (long long)blockIdx.x * blockDim.x; i0 < k; i0 += (long long)gridDim.x * blockDim.x) {
-    const long long i = i0 + threadIdx.x;
-    bool cl = false;
-    int v = 0;
-    if (i < k) {
-      v = (int)keys[i];
-      if (i == 0 || keys[i - 1] != (unsigned)v) cl = try_claim(visited, v);
-    }
-    record(v, cl, level, levels, nf, ncnt, nbits);
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < k;
+       i += (long long)gridDim.x * blockDim.x) {
+    const unsigned v = keys[i];
+    if (i == 0 || keys[i - 1] != v) mark_row(visited, nbits, (int)v);
   }
 }
 
-// K4 as the bottom-up step of a direction-optimising BFS, in two passes.
-// Head: one lane per unvisited row tests its first B neighbours (the column
-// loads, then the frontier-bit loads, each issued together) and claims the
-// row at a hit; a row with no hit among more than B neighbours goes to a
-// queue. Tail: a team of kBuTeam lanes per queued row tests the rest, kBuTeam
-// neighbours per step, and stops at the first hit. A team per row for every
-// row keeps a whole wave on a row until each of its lanes is done (64 ms for
-// a small-frontier level of R-MAT s22 with one wave per row), and one lane
-// per row for every row leaves a wave waiting on its longest row (86 ms);
-// in R-MAT rows the hubs come first (low ids), so once the frontier holds
-// them most rows stop in the head.
+// Bottom-up step of a direction-optimising BFS, in two passes. Head: one
+// lane per unvisited row tests its first B neighbours (the column loads, then
+// the frontier-bit loads, each issued together); a wave owns 64 rows and
+// stores their two bit words without atomics. A row with no hit among more
+// than B neighbours is queued in chunks of kBuChunk neighbours, with one
+// append per workgroup and `rows` (<= kBuRows) rows per thread. Tail: a team
+// of kBuTeam lanes per queued chunk, kBuTeam * kBuUnroll neighbours per step,
+// stops at the first hit (its own, or one that another chunk of the row
+// has marked when it starts). A team per row for every row keeps a whole wave
+// on a row until each of its lanes is done (64 ms for a small-frontier level
+// of R-MAT s22 with one wave per row), and one lane per row for every row
+// leaves a wave waiting on its longest row (86 ms); in R-MAT rows the hubs
+// come first (low ids), so once the frontier holds them most rows stop in the
+// head.
 template <int B>
-__global__ __launch_bounds__(256) void k_bu_head(const int* __restrict__ row_ptr,
-                                                 const int* __restrict__ col, int m,
-                                                 const unsigned* __restrict__ fbits, int* cnt, int cur,
-                                                 unsigned* visited, int* levels, int* nf, unsigned* nbits,
-                                                 int* queue) {
-  const int level = cnt[2];
-  int* ncnt = cnt + (cur ^ 1);
-  for (long long base = (long long)blockIdx.x * blockDim.x; base < m;
-       base += (long long)gridDim.x * blockDim.x) {
-    const long long r = base + threadIdx.x;
-    bool active = r < m;
-    if (active) active = !((visited[r >> 5] >> (r & 31)) & 1u);
-    int b = 0, e = 0;
-    if (active) {
-      b = row_ptr[r];
-      e = row_ptr[r + 1];
+__global__ __launch_bounds__(kBfsNT) void k_bu_head(const int* __restrict__ row_ptr,
+                                                    const int* __restrict__ col, int m, int rows,
+                                                    const unsigned* __restrict__ fbits,
+                                                    const unsigned* __restrict__ visited, unsigned* nbits,
+                                                    int2* queue, int* qcount) {
+  __shared__ int s_i[kBfsNT / kWave];
+  __shared__ int s_base;
+  const long long step = (long long)kBfsNT * rows;
+  for (long long b0 = (long long)blockIdx.x * step; b0 < m; b0 += (long long)gridDim.x * step) {
+    int nc[kBuRows];
+    int mine = 0;
+#pragma unroll
+    for (int k = 0; k < kBuRows; ++k) {
+      nc[k] = 0;
+      if (k >= rows) continue;
+      const long long r = b0 + (long long)k * kBfsNT + threadIdx.x;
+      int b = 0, e = 0;
+      if (r < m && !((visited[r >> 5] >> (r & 31)) & 1u)) {
+        b = row_ptr[r];
+        e = row_ptr[r + 1];
+      }
+      bool found = false;
+      if (b < e) {
+        int u[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) u[j] = col[min(b + j, e - 1)];
+        unsigned w[B];
+#pragma unroll
+        for (int j = 0; j < B; ++j) w[j] = fbits[(unsigned)u[j] >> 5];
+#pragma unroll
+        for (int j = 0; j < B; ++j) found = found || ((w[j] >> (u[j] & 31)) & 1u);
+        if (!found && e - b > B) nc[k] = (e - b - B + kBuChunk - 1) / kBuChunk;
+        mine += nc[k];
+      }
+      const uint64_t bal = __ballot(found);
+      const unsigned half = lane() < 32 ? (unsigned)bal : (unsigned)(bal >> 32);
+      if ((lane() & 31) == 0 && half) nbits[r >> 5] = half;
     }
-    const bool go = active && b < e;
-    int u[B];
+    int tot;
+    int pos = block_excl_sum<kBfsNT, int>(mine, s_i, &tot);
+    if (tot == 0) continue;  // the same in every thread
+    if (threadIdx.x == 0) s_base = atomicAdd(qcount, tot);
+    __syncthreads();
+    pos += s_base;
+    __syncthreads();
 #pragma unroll
-    for (int j = 0; j < B; ++j) u[j] = col[go ? min(b + j, e - 1) : 0];
-    unsigned w[B];
-#pragma unroll
-    for (int j = 0; j < B; ++j) w[j] = fbits[(unsigned)u[j] >> 5];
-    bool found = false;
-#pragma unroll
-    for (int j = 0; j < B; ++j) found = found || (go && b + j < e && ((w[j] >> (u[j] & 31)) & 1u));
-    const bool cl = go && found;
-    if (cl) atomicOr(visited + (r >> 5), 1u << (r & 31));
-    record((int)r, cl, level, levels, nf, ncnt, nbits);
-    const bool more = go && !found && e - b > B;
-    const int q = wave_append(cnt + 3, more);
-    if (more) queue[q] = (int)r;
+    for (int k = 0; k < kBuRows; ++k) {
+      const int r = (int)(b0 + (long long)k * kBfsNT + threadIdx.x);
+      for (int q = 0; q < nc[k]; ++q) queue[pos++] = make_int2(r, q);
+    }
   }
 }
 
-template <int B, int TEAM>
-__global__ __launch_bounds__(256) void k_bu_tail(const int* __restrict__ row_ptr,
-                                                 const int* __restrict__ col,
-                                                 const unsigned* __restrict__ fbits, int* cnt, int cur,
-                                                 unsigned* visited, int* levels, int* nf, unsigned* nbits,
-                                                 const int* __restrict__ queue) {
-  const int level = cnt[2];
-  int* ncnt = cnt + (cur ^ 1);
-  const int nq = cnt[3];
-  constexpr int TPW = kWave / TEAM;
-  const int tl = threadIdx.x & (TEAM - 1);
-  const int tin = (threadIdx.x & (kWave - 1)) / TEAM;
-  const long long gw = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const long long nw = ((long long)gridDim.x * blockDim.x) >> 6;
-  for (long long q0 = gw * TPW; q0 < nq; q0 += nw * TPW) {
-    const long long qi = q0 + tin;
+template <int B>
+__global__ __launch_bounds__(kBfsNT) void k_bu_tail(const int* __restrict__ row_ptr,
+                                                    const int* __restrict__ col,
+                                                    const unsigned* __restrict__ fbits, unsigned* nbits,
+                                                    const int2* __restrict__ queue,
+                                                    const int* __restrict__ qcount) {
+  const int nq = *qcount;
+  const int tl = threadIdx.x & (kBuTeam - 1);
+  const long long team = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / kBuTeam;
+  const long long nteams = (long long)gridDim.x * blockDim.x / kBuTeam;
+  const long long wbase = team - (team % (kWave / kBuTeam));
+  for (long long t0 = wbase; t0 < nq; t0 += nteams) {
+    const long long t = t0 + (team - wbase);
     int r = 0, b = 0, e = 0;
-    if (qi < nq) {
-      r = queue[qi];
-      b = row_ptr[r] + B;
-      e = row_ptr[r + 1];
+    bool open = false;
+    if (t < nq) {
+      const int2 it = queue[t];
+      r = it.x;
+      b = row_ptr[r] + B + it.y * kBuChunk;
+      e = min(b + kBuChunk, row_ptr[r + 1]);
+      const unsigned w = __hip_atomic_load(nbits + (r >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      open = !((w >> (r & 31)) & 1u);
     }
-    bool found = false;
-    // wave-uniform loop: every team of the wave steps until all are done
-    for (int k0 = b; __ballot(!found && k0 < e) != 0ull; k0 += TEAM) {
-      const int k = k0 + tl;
-      const bool ok = !found && k < e;
-      const int v = col[ok ? k : 0];
-      int h = ok ? (int)((fbits[(unsigned)v >> 5] >> (v & 31)) & 1u) : 0;
+    int found = 0;
+    // wave-uniform trips: until every team's chunk ends or has a hit
+    for (int k0 = b; __ballot(open && !found && k0 < e) != 0ull; k0 += kBuTeam * kBuUnroll) {
+      int u[kBuUnroll];
 #pragma unroll
-      for (int o = TEAM >> 1; o > 0; o >>= 1) h |= __shfl_xor(h, o, kWave);
-      found = found || h;
+      for (int j = 0; j < kBuUnroll; ++j) {
+        const int k = k0 + j * kBuTeam + tl;
+        u[j] = open && !found && k < e ? col[k] : -1;
+      }
+#pragma unroll
+      for (int j = 0; j < kBuUnroll; ++j)
+        if (u[j] >= 0) found |= (int)((fbits[(unsigned)u[j] >> 5] >> (u[j] & 31)) & 1u);
+#pragma unroll
+      for (int o = kBuTeam >> 1; o > 0; o >>= 1) found |= __shfl_xor(found, o, kWave);
     }
-    const bool cl = qi < nq && found && tl == 0;
-    if (cl) atomicOr(visited + (r >> 5), 1u << (r & 31));
-    record(r, cl, level, levels, nf, ncnt, nbits);
+    if (found && tl == 0) atomicOr(nbits + (r >> 5), 1u << (r & 31));
   }
 }
 
-// Claims rows whose hit bit a row kernel set (hits & ~visited); clears hits.
-__global__ void k_claim_bits(unsigned* hits, int m, int* cnt, int cur, unsigned* visited,
-                             int* levels, int* nf, unsigned* nbits) {
+// Ends a level: of the marked rows the unvisited ones (they stay marked: the
+// next frontier's bits) become visited, get their level and are listed; the
+// consumed frontier's bits are cleared for the level after the next. A thread
+// takes a word of 32 rows; where a wave's words hold many rows, its lanes
+// take the rows of two words at a time, so that levels and list entries
+// leave as adjacent words.
+__global__ __launch_bounds__(kBfsNT) void k_bfs_collect(unsigned* nbits, unsigned* cbits, int n, int* cnt, int cur,
+                                                        unsigned* visited, int* __restrict__ levels,
+                                                        int* __restrict__ nf) {
+  __shared__ int s_i[kBfsNT / kWave];
+  __shared__ int s_base;
   const int level = cnt[2];
-  int* ncnt = cnt + (cur ^ 1);
-  const int words = (m + 31) >> 5;
-  for (long long w0 = (long long)blockIdx.x * blockDim.x; w0 < words; w0 += (long long)gridDim.x * blockDim.x) {
-    const long long w = w0 + threadIdx.x;
+  const int words = (n + 31) >> 5;
+  for (int w0 = blockIdx.x * kBfsNT; w0 < words; w0 += gridDim.x * kBfsNT) {
+    const int w = w0 + threadIdx.x;
     unsigned nw = 0;
     if (w < words) {
-      const unsigned h = hits[w];
+      cbits[w] = 0u;
+      const unsigned h = nbits[w];
       if (h) {
-        hits[w] = 0u;
-        nw = h & ~visited[w];
-        if (nw) {
-          visited[w] |= nw;  // one thread per word: no race
-          nbits[w] |= nw;
-        }
+        const unsigned vis = visited[w];
+        nw = h & ~vis;
+        if (nw != h) nbits[w] = nw;
+        if (nw) visited[w] = vis | nw;
       }
     }
     const int c = __popc(nw);
-    const int inc = wave_incl_sum(c);
-    const int tot = __shfl(inc, kWave - 1, kWave);
-    int base = 0;
-    if (lane() == kWave - 1 && tot) base = atomicAdd(ncnt, tot);
-    base = __shfl(base, kWave - 1, kWave);
-    int pos = base + inc - c;
-    while (nw) {
-      const int bit = __ffs(nw) - 1;
-      nw &= nw - 1;
-      const int v = (int)(w << 5) + bit;
-      levels[v] = level;
-      nf[pos++] = v;
+    int tot;
+    int pos = block_excl_sum<kBfsNT, int>(c, s_i, &tot);
+    if (tot == 0) continue;  // the same in every thread
+    if (threadIdx.x == 0) s_base = atomicAdd(cnt + (cur ^ 1), tot);
+    __syncthreads();
+    pos += s_base;
+    __syncthreads();
+    if (wave_sum(c) > 2 * kWave) {
+      const int wb = w0 + (threadIdx.x & ~(kWave - 1));
+      const int bit = lane() & 31;
+#pragma unroll 4
+      for (int k = 0; k < kWave / 2; ++k) {
+        const int src = 2 * k + (lane() >> 5);
+        const unsigned word = __shfl(nw, src, kWave);
+        const int p = __shfl(pos, src, kWave);
+        if ((word >> bit) & 1u) {
+          const int v = ((wb + src) << 5) + bit;
+          levels[v] = level;
+          nf[p + __popc(word & ((1u << bit) - 1u))] = v;
+        }
+      }
+    } else {
+      while (nw) {
+        const int v = (w << 5) + __ffs(nw) - 1;
+        nw &= nw - 1;
+        levels[v] = level;
+        nf[pos++] = v;
+      }
     }
   }
 }
 
 // Graph500 edge count: sum of degrees over reached vertices.
-__global__ void k_reached(const int* __restrict__ levels, const int* __restrict__ colptr, int n,
-                          unsigned long long* out) {
-  unsigned long long c = 0, d = 0;
-  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
+template <int NT>
+__global__ __launch_bounds__(NT) void k_reached(const int* __restrict__ levels, const int* __restrict__ colptr,
+                                                int n, unsigned long long* out) {
+  __shared__ long long s_l[NT / kWave];
+  long long c = 0, d = 0;
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
+    const int len = colptr[v + 1] - colptr[v];
     if (levels[v] >= 0) {
       ++c;
-      d += (unsigned long long)(colptr[v + 1] - colptr[v]);
+      d += len;
     }
-  c = wave_sum(c);
-  d = wave_sum(d);
-  if (lane() == 0) {
-    atomicAdd(out, c);
-    atomicAdd(out + 1, d);
+  }
+  c = block_sum<NT, long long>(c, s_l);
+  d = block_sum<NT, long long>(d, s_l);
+  if (threadIdx.x == 0) {
+    atomicAdd(out, (unsigned long long)c);
+    atomicAdd(out + 1, (unsigned long long)d);
   }
 }
 
@@ -405,9 +414,9 @@ int lg2(int t) {
   return l;
 }
 
-// Enqueues one level on stream s: begin, the slot's kernels on frontier
-// `cur`, the selector on the new frontier, and the readback of
-// (new frontier size, next slot) into pinned host memory.
+// Enqueues one level on stream s: the slot's kernels on frontier `cur`, the
+// collect pass, the selector on the new frontier, and the word with
+// (new frontier size, next slot) for the host.
 void enqueue_level(spmspv_handle_t h, hipStream_t s, int slot, int cur, int* levels,
                    const SelectorArgs& sel) {
   BfsState* b = h->bfs;
@@ -416,21 +425,19 @@ void enqueue_level(spmspv_handle_t h, hipStream_t s, int slot, int cur, int* lev
   int* f = b->front[cur];
   int* nf = b->front[nxt];
   unsigned* nbits = b->fbits[nxt];
-  hipLaunchKernelGGL(k_bfs_begin, dim3(std::min(1024, (words + 255) / 256)), dim3(256), 0, s, b->cnt,
-                     nxt, nbits, words, h->ctl);
   switch (slot) {
     case SPMSPV_K_COL_NAIVE_ATOMIC:
-      hipLaunchKernelGGL(k_td_naive, dim3(kBfsGrid), dim3(256), 0, s, h->csc_colptr, h->csc_row, f,
-                         b->cnt, cur, lg2(h->team_col), b->visited, levels, nf, nbits);
+      hipLaunchKernelGGL(k_td_naive, dim3(kBfsGrid), dim3(kBfsNT), 0, s, h->csc_colptr, h->csc_row, f,
+                         b->cnt, cur, lg2(h->team_col), b->visited, nbits);
       break;
     case SPMSPV_K_COL_LB_ATOMIC:
       hipLaunchKernelGGL((k_td_lb<kLbNT, kLbVT>), dim3(kBfsGrid), dim3(kLbNT), 0, s, h->ptr, h->xbeg,
-                         h->split, h->csc_row, h->ctl, b->cnt, cur, b->visited, levels, nf, nbits);
+                         h->split, h->csc_row, h->ctl, b->cnt, cur, b->visited, nbits);
       break;
     case SPMSPV_K_COL_NAIVE_SORT:
     case SPMSPV_K_COL_LB_SORT: {
       // boolean: the neighbours' row keys alone, sorted, then each distinct
-      // row claimed
+      // row marked
       int* bk = reinterpret_cast<int*>(h->sb.keyA);
       if (slot == SPMSPV_K_COL_NAIVE_SORT)
         launch_naive_col(s, 2, h->csc_colptr, h->csc_row, nullptr, f, nullptr, h->ptr, h->n, 0,
@@ -442,31 +449,29 @@ void enqueue_level(spmspv_handle_t h, hipStream_t s, int slot, int cur, int* lev
       kb.valA = kb.valB = nullptr;
       const int fb = launch_radix_sort(s, kb, h->m, &h->ctl->bin_len, h->ctl, -1, h->nnz, false, Ep{0, 1},
                                        Gate{}, h->small_sort_cap);
-      hipLaunchKernelGGL(k_claim_sorted, dim3(kBfsGrid), dim3(256), 0, s, fb ? kb.keyB : kb.keyA,
-                         &h->ctl->bin_len, b->cnt, cur, b->visited, levels, nf, nbits);
+      hipLaunchKernelGGL(k_mark_sorted, dim3(kBfsGrid), dim3(kBfsNT), 0, s, fb ? kb.keyB : kb.keyA,
+                         &h->ctl->bin_len, b->visited, nbits);
       break;
     }
-    case SPMSPV_K_ROW_NAIVE:
+    case SPMSPV_K_SPMV_NAIVE:
+      launch_row_naive(s, true, true, h->csr_row, h->csr_col, nullptr, nullptr, b->fbits[cur],
+                       h->m, h->team_row, nullptr, nbits);
+      break;
+    default:  // 4, 5, 7: bottom-up
       if (h->nnz > 0) {
-        hipLaunchKernelGGL((k_bu_head<kBuBatch>), dim3(kBfsGrid), dim3(256), 0, s, h->csr_row, h->csr_col,
-                           h->m, b->fbits[cur], b->cnt, cur, b->visited, levels, nf, nbits, b->queue);
-        hipLaunchKernelGGL((k_bu_tail<kBuBatch, kBuTeam>), dim3(kBfsGrid), dim3(256), 0, s, h->csr_row,
-                           h->csr_col, b->fbits[cur], b->cnt, cur, b->visited, levels, nf, nbits, b->queue);
+        // rows per thread and queue append: as many as leave every CU its workgroups
+        const int rows = std::max(1, std::min(kBuRows, h->m / (kBfsNT * 1024)));
+        const long long blocks = ((long long)h->m + (long long)kBfsNT * rows - 1) / (kBfsNT * rows);
+        hipLaunchKernelGGL((k_bu_head<kBuBatch>), dim3((unsigned)std::min<long long>(kBfsGrid, blocks)),
+                           dim3(kBfsNT), 0, s, h->csr_row, h->csr_col, h->m, rows, b->fbits[cur], b->visited,
+                           nbits, b->queue, b->cnt + 3);
+        hipLaunchKernelGGL((k_bu_tail<kBuBatch>), dim3(kBfsGrid), dim3(kBfsNT), 0, s, h->csr_row, h->csr_col,
+                           b->fbits[cur], nbits, b->queue, b->cnt + 3);
       }
       break;
-    default: {  // 5, 6, 7: boolean row kernels (hit bits only), then claim
-      if (slot == SPMSPV_K_SPMV_NAIVE)
-        launch_row_naive(s, true, true, h->csr_row, h->csr_col, nullptr, nullptr, b->fbits[cur],
-                         h->m, h->team_row, nullptr, h->bitmap);
-      else
-        launch_row_merge(s, true, true, h->csr_row, h->csr_col, nullptr, nullptr, b->fbits[cur],
-                         h->m, h->nnz, h->row_split, h->n_row_tiles, h->row_vt, nullptr, h->bitmap,
-                         h->row_carry_val, h->row_carry_row, h->row_carry_hit);
-      hipLaunchKernelGGL(k_claim_bits, dim3(std::min(kBfsGrid, (words + 255) / 256)), dim3(256), 0, s,
-                         h->bitmap, h->m, b->cnt, cur, b->visited, levels, nf, nbits);
-      break;
-    }
   }
+  hipLaunchKernelGGL(k_bfs_collect, dim3(std::min(kBfsGrid, (words + kBfsNT - 1) / kBfsNT)), dim3(kBfsNT), 0, s,
+                     nbits, b->fbits[cur], h->n, b->cnt, cur, b->visited, levels, nf);
   launch_prep(s, h->csc_colptr, nf, h->n, 0, b->cnt + nxt, h->ptr, h->xbeg, h->split, h->scan_state,
               h->tile_mm, h->ctl, &sel, Ep{0, 0}, h->prep_samp);
   hipLaunchKernelGGL(k_bfs_signal, dim3(1), dim3(64), 0, s, b->cnt, nxt, h->ctl, h->sig_dev + kSigBfs);
@@ -489,7 +494,8 @@ int bfs_alloc(spmspv_handle_t h) {
   };
   const size_t o_vis = take(words * 4), o_fb0 = take(words * 4), o_fb1 = take(words * 4);
   const size_t o_f0 = take(n * 4 + 4), o_f1 = take(n * 4 + 4), o_cnt = take(64), o_r = take(64);
-  const size_t o_q = take(m * 4 + 4);
+  // at most one item per row and one more per kBuChunk of its neighbours
+  const size_t o_q = take((m + (size_t)h->nnz / kBuChunk + 64) * sizeof(int2));
   if (hipMalloc(&b->alloc, off) != hipSuccess) {
     delete b;
     return set_error(h, SPMSPV_OUT_OF_MEMORY, "bfs buffers");
@@ -502,7 +508,7 @@ int bfs_alloc(spmspv_handle_t h) {
   b->front[1] = reinterpret_cast<int*>(p + o_f1);
   b->cnt = reinterpret_cast<int*>(p + o_cnt);
   b->reached = reinterpret_cast<unsigned long long*>(p + o_r);
-  b->queue = reinterpret_cast<int*>(p + o_q);
+  b->queue = reinterpret_cast<int2*>(p + o_q);
   if (!h->stream) {
     if (hipStreamCreateWithFlags(&b->own_stream, hipStreamNonBlocking) != hipSuccess) {
       (void)hipFree(b->alloc);
@@ -554,7 +560,7 @@ static int bfs_run(spmspv_handle_t h, int src, int* d_levels, int policy, int us
   if (!h->csr_row) return set_error(h, SPMSPV_MAT_FORMAT_ERR, "bfs needs CSR input");
   int rc;
   if ((rc = ensure_arena(h)) || (rc = need_csc(h))) return rc;
-  if ((rc = ensure_row_tiles(h)) || (rc = ensure_mat_features(h)) || (rc = bfs_alloc(h))) return rc;
+  if ((rc = ensure_mat_features(h)) || (rc = bfs_alloc(h))) return rc;
   BfsState* b = h->bfs;
   hipStream_t s = h->stream ? h->stream : b->own_stream;
   const int smode = policy >= 0 ? 2 : h->sel_mode, sfixed = policy >= 0 ? policy : h->sel_fixed;
@@ -658,7 +664,8 @@ static int bfs_run(spmspv_handle_t h, int src, int* d_levels, int policy, int us
   h->stream = saved;
   if (out_of_sequence) return set_error(h, SPMSPV_DEVICE_ERROR, "bfs: a level's word arrived out of sequence");
   if (e != hipSuccess) return set_error(h, SPMSPV_DEVICE_ERROR, std::string("bfs: ") + hipGetErrorString(e));
-  hipLaunchKernelGGL(k_reached, dim3(std::min(1024, (h->n + 255) / 256)), dim3(256), 0, s, d_levels,
+  // 256 workgroups: two atomics each on one pair of words
+  hipLaunchKernelGGL(k_reached<1024>, dim3(std::min(256, (h->n + 1023) / 1024)), dim3(1024), 0, s, d_levels,
                      h->csc_colptr, h->n, b->reached);
   unsigned long long red[2] = {0, 0};
   e = hipMemcpyAsync(red, b->reached, sizeof(red), hipMemcpyDeviceToHost, s);

@@ -315,13 +315,11 @@ int resident_blocks(const void* kernel, int block);
 void launch_row_split(hipStream_t s, const int* row_ptr, int m, int nnz, int* split, int ntiles,
                       int tile);
 // vt in {5, 7, 11}: merged items per thread (tile = 256 * vt).
-// x == nullptr: the boolean form, x given by its bit array xbits alone:
-// hit bits into ybits, no values read (val may be null), y not written (may
-// be null). Otherwise, with masked or hits, x must be
-// the support-encoded vector (launch_encode_x / launch_scatter with
-// encode); without either it is plain dense x.
+// With masked or hits, x must be the support-encoded vector
+// (launch_encode_x / launch_scatter with encode); without either it is plain
+// dense x.
 void launch_row_merge(hipStream_t s, bool masked, bool hits, const int* row_ptr, const int* col,
-                      const float* val, const float* x, const unsigned* xbits, int m, int nnz,
+                      const float* val, const float* x, int m, int nnz,
                       const int* split, int ntiles, int vt, float* y, unsigned* ybits,
                       float* carry_val, int* carry_row, int* carry_hit,
                       hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr, Gate g = {});

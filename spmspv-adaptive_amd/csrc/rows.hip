@@ -92,7 +92,7 @@ __device__ __forceinline__ void seg_scan_row(bool f, float v, int h, float* cin,
   *tail_h = th;
 }
 
-constexpr int kXPlain = 0, kXEnc = 1, kXBits = 2;
+constexpr int kXPlain = 0, kXEnc = 1;
 
 // One merge-path tile: rows i0..i1-1 end in it, nonzeros j0..j0+nj-1.
 struct RowTile {
@@ -125,10 +125,7 @@ __device__ __forceinline__ RowTile row_tile(const int* __restrict__ split, int t
 //   kXPlain: x values (support not needed: SpMV with dense output),
 //   kXEnc  : the support-encoded x (+0.0 outside the support, a nonzero bit
 //            pattern inside it, an explicit zero stored as -0.0), so one
-//            gather yields both the value and the support bit,
-//   kXBits : only x's bit array (boolean semiring of the BFS levels): no
-//            values are read (val may be null), a row's result is its hit
-//            bit alone and y is not written (may be null).
+//            gather yields both the value and the support bit.
 // Loads use a per-tile base pointer with 32-bit offsets and are
 // unconditional (clamped) so that a stage's loads issue back to back.
 // Rows that cross tiles leave their tail in carry_*[t] (row i1), which
@@ -138,7 +135,7 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
                                                   const int* __restrict__ col,
                                                   const float* __restrict__ val,
                                                   const float* __restrict__ x,
-                                                  const unsigned* __restrict__ xbits, int m, int nnz,
+                                                  int m, int nnz,
                                                   const int* __restrict__ split, int ntiles,
                                                   float* __restrict__ y, unsigned* ybits,
                                                   float* __restrict__ carry_val,
@@ -165,8 +162,7 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
 
   int cN[VT];  // stage 2: columns / values loading
   float vN[VT];
-  float vG[VT], xG[VT];  // stage 1: values, gathered x (or bit words), rows
-  int cG[VT];
+  float vG[VT], xG[VT];  // stage 1: values, gathered x, rows
   int rs[VT], re[VT];
 
   auto load_cv = [&](int tt) {
@@ -180,16 +176,13 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
       unsigned k = tid + i * NT;
       k = k < lim ? k : lim;
       cN[i] = __builtin_nontemporal_load(ct + k);
-      if (XIN != kXBits) vN[i] = __builtin_nontemporal_load(val + jb + k);
+      vN[i] = __builtin_nontemporal_load(val + jb + k);
     }
   };
   auto gather = [&](int tt) {
     const RowTile g = row_tile(split, tt, T, W);
 #pragma unroll
-    for (int i = 0; i < VT; ++i) {
-      if (XIN == kXBits) xG[i] = __builtin_bit_cast(float, xbits[(unsigned)cN[i] >> 5]);
-      else xG[i] = x[(unsigned)cN[i]];
-    }
+    for (int i = 0; i < VT; ++i) xG[i] = x[(unsigned)cN[i]];
     const unsigned lim = (unsigned)(m - 1 - g.i0);
     const int* __restrict__ rt = row_ptr + g.i0;
 #pragma unroll
@@ -203,10 +196,7 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
     // registers keep their roles from tile to tile and the loop needs no
     // copy of a register whose load is in flight (a copy waits for it)
 #pragma unroll
-    for (int i = 0; i < VT; ++i) {
-      if (XIN != kXBits) asm volatile("v_mov_b32 %0, %1" : "=v"(vG[i]) : "v"(vN[i]));
-      else asm volatile("v_mov_b32 %0, %1" : "=v"(cG[i]) : "v"(cN[i]));
-    }
+    for (int i = 0; i < VT; ++i) asm volatile("v_mov_b32 %0, %1" : "=v"(vG[i]) : "v"(vN[i]));
   };
 
   // Stages run unconditionally (past the last tile they reload it, from
@@ -223,16 +213,9 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
 #pragma unroll
     for (int i = 0; i < VT; ++i) {
       const unsigned k = tid + i * NT;
-      bool in;
-      float p;
-      if (XIN == kXBits) {
-        in = (__builtin_bit_cast(unsigned, xG[i]) >> (cG[i] & 31)) & 1u;
-        p = 0.f;
-      } else {
-        in = __builtin_bit_cast(unsigned, xG[i]) != 0u;
-        p = vG[i] * xG[i];
-        if (MASKED) p = in ? p : 0.f;
-      }
+      const bool in = __builtin_bit_cast(unsigned, xG[i]) != 0u;
+      float p = vG[i] * xG[i];
+      if (MASKED) p = in ? p : 0.f;
       if (k < (unsigned)g.nj) {
         s_p[k] = p;
         if (HITS) s_ph[k] = (unsigned char)in;
@@ -249,7 +232,7 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
           if (re[i] > rs[i] && re[i] > g.j0) {
             s_end[re[i] - 1 - g.j0] = g.i0 + (int)k;
           } else {
-            if (XIN != kXBits) yt[k] = 0.f;
+            yt[k] = 0.f;
             if (HITS) s_yh[k] = 0;
           }
         }
@@ -293,7 +276,7 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
             first_hit = hit;
             had_end = true;
           } else {
-            if (XIN != kXBits) y[(unsigned)r] = sum;
+            y[(unsigned)r] = sum;
             if (HITS) s_yh[r - g.i0] = (unsigned char)hit;
           }
           sum = 0.f;
@@ -305,7 +288,7 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
     int hin, tail_h;
     seg_scan_row<NT>(had_end, sum, hit, &cin, &hin, &tail_v, &tail_h, s_f, s_sv, s_sh);
     if (had_end) {
-      if (XIN != kXBits) y[(unsigned)first_row] = cin + first_sum;
+      y[(unsigned)first_row] = cin + first_sum;
       if (HITS) s_yh[first_row - g.i0] = (unsigned char)(hin | first_hit);
     }
     if (tid == 0) {
@@ -345,7 +328,7 @@ __global__ void k_row_fixup(const float* __restrict__ carry_val, const int* __re
     float s;
     if (!carry_run<int>(carry_val, carry_row, HITS ? carry_hit : nullptr, t, ntiles, r, s, h))
       continue;
-    if (y) y[r] += s;  // null: hit bits only (boolean rows)
+    y[r] += s;
     if (HITS && h) atomicOr(ybits + (r >> 5), 1u << (r & 31));
   }
 }
@@ -369,13 +352,13 @@ int resident_blocks(const void* kernel, int block) {
 }
 
 void launch_row_merge(hipStream_t s, bool masked, bool hits, const int* row_ptr, const int* col,
-                      const float* val, const float* x, const unsigned* xbits, int m, int nnz,
+                      const float* val, const float* x, int m, int nnz,
                       const int* split, int ntiles, int vt, float* y, unsigned* ybits,
                       float* carry_val, int* carry_row, int* carry_hit, hipEvent_t ev_begin,
                       hipEvent_t ev_end, Gate g) {
   if (m <= 0 || ntiles <= 0) return;
   if (nnz == 0) {  // every row is empty; no hits
-    if (y) launch_fill_f32(s, y, m, 0.f, g);
+    launch_fill_f32(s, y, m, 0.f, g);
     return;
   }
   // one resident wave of workgroups, each walking many tiles
@@ -384,12 +367,11 @@ void launch_row_merge(hipStream_t s, bool masked, bool hits, const int* row_ptr,
     const void* fn = (const void*)k_row_merge<kRowNT, V, XI, MK, HT>;                           \
     hipLaunchKernelGGL((k_row_merge<kRowNT, V, XI, MK, HT>),                                    \
                        dim3(std::min(ntiles, resident_blocks(fn, kRowNT))), dim3(kRowNT), 0, s, \
-                       row_ptr, col, val, x, xbits, m, nnz, split, ntiles, y, ybits, carry_val, \
+                       row_ptr, col, val, x, m, nnz, split, ntiles, y, ybits, carry_val, \
                        carry_row, carry_hit, g);                                                \
   }
 #define SPMSPV_ROW_MERGE_VT(V)                                   \
-  if (!x) SPMSPV_ROW_MERGE(V, kXBits, true, true)                \
-  else if (masked && hits) SPMSPV_ROW_MERGE(V, kXEnc, true, true) \
+  if (masked && hits) SPMSPV_ROW_MERGE(V, kXEnc, true, true) \
   else if (masked) SPMSPV_ROW_MERGE(V, kXEnc, true, false)       \
   else if (hits) SPMSPV_ROW_MERGE(V, kXEnc, false, true)         \
   else SPMSPV_ROW_MERGE(V, kXPlain, false, false)

@@ -45,3 +45,18 @@ def test_bfs_multi_hub_degrees(gpu, hubs, nsrc):
         for i, s in enumerate(srcs):
             ref, _ = oracle.bfs(n, cp, ri, int(s))
             np.testing.assert_array_equal(got[:, i], ref, err_msg=f"source {s}")
+
+
+@pytest.mark.parametrize("graphs", [0, 1])
+@pytest.mark.parametrize("policy", [0, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("n,hubs", [(5003, (7, 8, 9, 263, 264, 265)), (40961, (255, 256, 257, 520, 30000))])
+def test_bfs_hub_degrees(gpu, n, hubs, policy, graphs):
+    A = hub_graph(n, hubs, len(hubs))
+    M = sa.Matrix(n, n, A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    cp, ri, _ = oracle.csr_to_csc(n, n, A.indptr, A.indices, A.data)
+    lev = sa.DeviceArray(n, np.int32)
+    for src in (0, len(hubs) - 1, n - 1):
+        st = M.A.bfs(src, lev, policy=policy, use_graphs=graphs)
+        ref, _ = oracle.bfs(n, cp, ri, src)
+        np.testing.assert_array_equal(lev.to_host(), ref)
+        assert int(st[3]) == int((ref >= 0).sum())
