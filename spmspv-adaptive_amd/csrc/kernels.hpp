@@ -197,6 +197,12 @@ struct SortBufs {
   float* carry_val;
   int* carry_idx;
 };
+// Items of a sort: keys and up to two payload words (null: absent).
+struct SortSet {
+  unsigned* k = nullptr;
+  unsigned* v = nullptr;
+  unsigned* w = nullptr;
+};
 // n_hint: item count when the host knows it (exact grids), else -1 and the
 // grids cover n_cap. ep: first of the 5 epochs the sort + reduce use.
 // small_cap (<= kSmallSortCap): largest item count that takes the
@@ -204,6 +210,14 @@ struct SortBufs {
 void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* ykey, float* yval,
                         long long binlen_hint, long long n_cap, Ep ep, Gate g = {},
                         int small_cap = kSmallSortCap);
+// Sorts in[*n_dev] by key < range, stable, its passes writing out0 and out1 in
+// turn (`in` may be out1, and is not written otherwise); returns which of the
+// two holds the result. With ep.dev >= 0 (captured graphs) the passes use
+// device epochs ep.dev + pass, otherwise ep.v + pass (4 at most). b gives the
+// digit counts' buffers.
+int launch_radix_sets(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out0, const SortSet& out1,
+                      int range, const long long* n_dev, Ctl* ctl, long long n_hint, long long n_cap,
+                      bool skip_small, Ep ep, Gate g = {}, int small_cap = kSmallSortCap);
 // Sorts (keyA, valA)[*n_dev] by key < range; returns 0 if the result is in
 // A, 1 if in B. With valA and valB null it sorts the keys alone.
 int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long long* n_dev, Ctl* ctl,

@@ -26,10 +26,24 @@ namespace spmspv {
 // cnt (this wave's 256 counters) holds the per-digit counts of the wave's
 // chunk and rank[j] the stable rank of item j among equal digits inside
 // the chunk.
+// A digit is `bits` (<= 8) wide, one ballot per bit.
+__device__ __forceinline__ uint64_t digit_peers(unsigned d, bool valid, int bits) {
+  uint64_t peers = __ballot(valid);
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    if (b >= bits) break;
+    const bool bit = (d >> b) & 1u;
+    const uint64_t bb = __ballot(bit);
+    peers &= bit ? bb : ~bb;
+  }
+  return peers;
+}
+
 template <int IPT>
 __device__ __forceinline__ void wave_rank(const unsigned (&key)[IPT], const bool (&valid)[IPT],
                                           int shift, unsigned* cnt, int (&rank)[IPT],
-                                          unsigned (&dig)[IPT], int nj = IPT) {
+                                          unsigned (&dig)[IPT], int nj = IPT, int bits = 8) {
+  const unsigned mask = (1u << bits) - 1u;
   for (int k = lane(); k < 256; k += kWave) cnt[k] = 0u;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -41,14 +55,8 @@ __device__ __forceinline__ void wave_rank(const unsigned (&key)[IPT], const bool
       dig[j] = 0u;
       continue;
     }
-    const unsigned d = valid[j] ? ((key[j] >> shift) & 255u) : 0u;
-    uint64_t peers = __ballot(valid[j]);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t bb = __ballot(bit);
-      peers &= bit ? bb : ~bb;
-    }
+    const unsigned d = valid[j] ? ((key[j] >> shift) & mask) : 0u;
+    const uint64_t peers = digit_peers(d, valid[j], bits);
     unsigned base = 0;
     if (valid[j]) base = cnt[d];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -217,20 +225,25 @@ __device__ __forceinline__ void load_tile_keys(const unsigned* __restrict__ kin,
 
 template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__ kin,
-                                                    const long long* __restrict__ n_dev, int shift,
+                                                    const long long* __restrict__ n_dev, int shift, int bits,
                                                     unsigned* __restrict__ cnt, int small_cap,
                                                     Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
   static_assert(NT == 256, "one thread per digit");
+  const unsigned mask = (1u << bits) - 1u;
   __shared__ unsigned s_cnt[NW * 256];
   const long long n = *n_dev;
   if (n <= small_cap) return;
   const unsigned ntiles = (unsigned)((n + TILE - 1) / TILE);
   const int w = threadIdx.x / kWave;
   // tiles are independent: any grid covers them. Only counts are needed
-  // here (no ranks): plain LDS atomics into a private histogram per wave
+  // here (no ranks): LDS atomics into a private histogram per wave. Lanes that
+  // add to one LDS word take turns, so where many lanes hold the first lane's
+  // digit (power-law column indices), those lanes add once between them (52 ->
+  // 20 us for 15.9 M such keys; the same grouping of every digit by ballots
+  // costs 7.4 -> 10.7 us for 1.4 M even ones)
   for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
     unsigned key[IPT];
     bool valid[IPT];
@@ -240,29 +253,37 @@ __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < IPT; ++j)
-      if (valid[j]) atomicAdd(&s_cnt[w * 256 + ((key[j] >> shift) & 255u)], 1u);
+    {
+      const unsigned d = (key[j] >> shift) & mask;
+      const uint64_t same = __ballot(valid[j] && d == (unsigned)__builtin_amdgcn_readfirstlane((int)d));
+      const bool many = __popcll(same) > 4;
+      const bool in_same = (same >> lane()) & 1ull;
+      if (many && same && __builtin_ctzll(same) == lane())
+        atomicAdd(&s_cnt[w * 256 + d], (unsigned)__popcll(same));
+      if (valid[j] && !(many && in_same)) atomicAdd(&s_cnt[w * 256 + d], 1u);
+    }
     __syncthreads();
     unsigned tot = 0;
 #pragma unroll
     for (int q = 0; q < NW; ++q) tot += s_cnt[q * 256 + threadIdx.x];
-    cnt[(size_t)threadIdx.x * ntiles + t] = tot;
+    if (threadIdx.x <= mask) cnt[(size_t)threadIdx.x * ntiles + t] = tot;
     __syncthreads();
   }
 }
 
-// In-place exclusive scan of cnt[0 .. 256 * ntiles) (ntiles from n and the
+// In-place exclusive scan of cnt[0 .. 2^bits * ntiles) (ntiles from n and the
 // sort tile), ordered tiles of NT * IPT entries with decoupled look-back.
 template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
                                                    const long long* __restrict__ n_dev, int sort_tile,
-                                                   int small_cap, unsigned long long* state, Ctl* ctl,
+                                                   int bits, int small_cap, unsigned long long* state, Ctl* ctl,
                                                    Ep epa, Gate g) {
   if (gate_shut(g)) return;
   __shared__ unsigned long long s_pre;
   __shared__ unsigned s_t[NT / kWave];
   const long long n = *n_dev;
   if (n <= small_cap) return;
-  const long long E = 256 * ((n + sort_tile - 1) / sort_tile);
+  const long long E = ((n + sort_tile - 1) / sort_tile) << bits;
   const unsigned nb = (unsigned)((E + NT * IPT - 1) / (NT * IPT));
   const unsigned t = blockIdx.x;
   if (t >= nb) return;
@@ -289,73 +310,69 @@ __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
   }
 }
 
-template <int NT, int IPT>
-__global__ __launch_bounds__(NT) void k_sort_scatter(const unsigned* __restrict__ kin,
-                                                     const float* __restrict__ vin,
-                                                     unsigned* __restrict__ kout,
-                                                     float* __restrict__ vout,
-                                                     const long long* __restrict__ n_dev, int shift,
-                                                     const unsigned* __restrict__ pos0,
+// PAY: payload words per item (0: keys only).
+template <int NT, int IPT, int PAY>
+__global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, const long long* __restrict__ n_dev,
+                                                     int shift, int bits, const unsigned* __restrict__ pos0,
                                                      int small_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
   static_assert(NT == 256, "one thread per digit");
   __shared__ unsigned s_k[TILE];
-  __shared__ float s_v[TILE];
+  __shared__ unsigned s_v[PAY > 0 ? TILE : 1];
+  __shared__ unsigned s_w[PAY > 1 ? TILE : 1];
   __shared__ unsigned s_cnt[NW * 256];
   __shared__ unsigned s_dstart[256];
   __shared__ unsigned s_gbase[256];
   __shared__ unsigned s_t[NW];
+  const unsigned mask = (1u << bits) - 1u;
   const long long n = *n_dev;
   if (n <= small_cap) return;
   const unsigned ntiles = (unsigned)((n + TILE - 1) / TILE);
   const int w = threadIdx.x / kWave;
-  const int d = threadIdx.x;
+  const unsigned d = threadIdx.x;
   // tiles are independent: any grid covers them
   for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const long long base = (long long)t * TILE;
     // this tile's global start of digit d, from the scan (issued with the keys)
-    const unsigned gb = pos0[(size_t)d * ntiles + t];
-    unsigned key[IPT];
-    float val[IPT];
+    const unsigned gb = pos0[(size_t)(d & mask) * ntiles + t];
+    unsigned key[IPT], pv[IPT], pw[IPT];
     bool valid[IPT];
     int rank[IPT];
     unsigned dig[IPT];
-    load_tile_keys<NT, IPT>(kin, n, base, key, valid);
-      if (vin) {  // null: keys only
+    load_tile_keys<NT, IPT>(in.k, n, base, key, valid);
 #pragma unroll
-      for (int j = 0; j < IPT; ++j) {
-        const long long gi = base + (long long)w * kWave * IPT + j * kWave + lane();
-        val[j] = vin[valid[j] ? gi : n - 1];
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < IPT; ++j) val[j] = 0.f;
+    for (int j = 0; j < IPT; ++j) {
+      const long long gi = base + (long long)w * kWave * IPT + j * kWave + lane();
+      if (PAY > 0) pv[j] = in.v[valid[j] ? gi : n - 1];
+      if (PAY > 1) pw[j] = in.w[valid[j] ? gi : n - 1];
     }
-    wave_rank<IPT>(key, valid, shift, s_cnt + w * 256, rank, dig);
+    wave_rank<IPT>(key, valid, shift, s_cnt + w * 256, rank, dig, IPT, bits);
     __syncthreads();
     const unsigned tot = digit_wave_offsets<NW>(s_cnt);
     unsigned dtot;
     s_dstart[d] = block_excl_sum<NT, unsigned>(tot, s_t, &dtot);
     s_gbase[d] = gb;
     __syncthreads();
-  #pragma unroll
+#pragma unroll
     for (int j = 0; j < IPT; ++j) {
       if (valid[j]) {
         const unsigned p = s_dstart[dig[j]] + s_cnt[w * 256 + dig[j]] + rank[j];
         s_k[p] = key[j];
-        s_v[p] = val[j];
+        if (PAY > 0) s_v[p] = pv[j];
+        if (PAY > 1) s_w[p] = pw[j];
       }
     }
     __syncthreads();
     const int cnt = (int)min((long long)TILE, n - base);
     for (int i = threadIdx.x; i < cnt; i += NT) {
       const unsigned k = s_k[i];
-      const unsigned dd = (k >> shift) & 255u;
-      const unsigned g = s_gbase[dd] + (i - s_dstart[dd]);
-      kout[g] = k;
-      if (vout) vout[g] = s_v[i];
+      const unsigned dd = (k >> shift) & mask;
+      const unsigned q = s_gbase[dd] + (i - s_dstart[dd]);
+      out.k[q] = k;
+      if (PAY > 0) out.v[q] = s_v[i];
+      if (PAY > 1) out.w[q] = s_w[i];
     }
     __syncthreads();
   }
@@ -363,18 +380,17 @@ __global__ __launch_bounds__(NT) void k_sort_scatter(const unsigned* __restrict_
 
 // --------------------------------------------------- single-workgroup path
 // n <= TILE: all passes in LDS. mode 0: reduce and write (ykey, yval,
-// ctl->ynnz). mode 1: write the sorted pairs to (kout, vout).
-template <int NT, int IPT>
-__global__ __launch_bounds__(NT) void k_sort_small(const unsigned* __restrict__ kin,
-                                                   const float* __restrict__ vin,
-                                                   const long long* __restrict__ n_dev, int passes,
-                                                   int mode, Ctl* ctl, int* ykey, float* yval,
-                                                   unsigned* kout, float* vout, int cap, Gate g) {
+// ctl->ynnz). mode 1: write the sorted items to `out`.
+template <int NT, int IPT, int PAY>
+__global__ __launch_bounds__(NT) void k_sort_small(SortSet in, const long long* __restrict__ n_dev, int passes,
+                                                   int mode, Ctl* ctl, int* ykey, float* yval, SortSet out,
+                                                   int cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
   __shared__ unsigned s_k[TILE];
   __shared__ float s_v[TILE];
+  __shared__ unsigned s_w[PAY > 1 ? TILE : 1];
   __shared__ unsigned s_cnt[NW * 256];
   __shared__ unsigned s_dstart[256];
   __shared__ unsigned s_t[NW];
@@ -386,7 +402,7 @@ __global__ __launch_bounds__(NT) void k_sort_small(const unsigned* __restrict__ 
   const int w = threadIdx.x / kWave;
   // items per thread for this n (<= IPT): every wave ranks its share
   const int ie = (int)((n + NT - 1) / NT);
-  unsigned key[IPT];
+  unsigned key[IPT], pw[IPT];
   float val[IPT];
   bool valid[IPT];
   int rank[IPT];
@@ -395,8 +411,9 @@ __global__ __launch_bounds__(NT) void k_sort_small(const unsigned* __restrict__ 
   for (int j = 0; j < IPT; ++j) {
     const int gi = w * kWave * ie + j * kWave + lane();
     valid[j] = j < ie && gi < n;
-    key[j] = valid[j] ? kin[gi] : 0u;
-    val[j] = valid[j] && vin ? vin[gi] : 0.f;  // vin null: keys only
+    key[j] = valid[j] ? in.k[gi] : 0u;
+    val[j] = PAY > 0 && valid[j] ? __uint_as_float(in.v[gi]) : 0.f;
+    if (PAY > 1) pw[j] = valid[j] ? in.w[gi] : 0u;
   }
   for (int p = 0; p < passes; ++p) {
     wave_rank<IPT>(key, valid, 8 * p, s_cnt + w * 256, rank, dig, ie);
@@ -412,6 +429,7 @@ __global__ __launch_bounds__(NT) void k_sort_small(const unsigned* __restrict__ 
         const unsigned pos = s_dstart[dig[j]] + s_cnt[w * 256 + dig[j]] + rank[j];
         s_k[pos] = key[j];
         s_v[pos] = val[j];
+        if (PAY > 1) s_w[pos] = pw[j];
       }
     }
     __syncthreads();
@@ -422,6 +440,7 @@ __global__ __launch_bounds__(NT) void k_sort_small(const unsigned* __restrict__ 
         if (valid[j]) {
           key[j] = s_k[gi];
           val[j] = s_v[gi];
+          if (PAY > 1) pw[j] = s_w[gi];
         }
       }
       __syncthreads();
@@ -430,8 +449,9 @@ __global__ __launch_bounds__(NT) void k_sort_small(const unsigned* __restrict__ 
   const int cnt = (int)n;
   if (mode == 1) {
     for (int i = threadIdx.x; i < cnt; i += NT) {
-      kout[i] = s_k[i];
-      if (vout) vout[i] = s_v[i];
+      out.k[i] = s_k[i];
+      if (PAY > 0) out.v[i] = __float_as_uint(s_v[i]);
+      if (PAY > 1) out.w[i] = s_w[i];
     }
     return;
   }
@@ -520,11 +540,12 @@ __global__ void k_carry_fixup(const float* __restrict__ carry_val, const int* __
   }
 }
 
-static int key_passes(int range) {
+static int key_bits(int range) {
   int bits = 1;
   while (bits < 32 && (1u << bits) < (unsigned)range) ++bits;
-  return (bits + 7) / 8;
+  return bits;
 }
+static int key_passes(int range) { return (key_bits(range) + 7) / 8; }
 
 // Grid for a launch over n items in tiles of `tile`: exact when the host
 // knows n (n_hint >= 0), else the bound n_cap.
@@ -536,52 +557,63 @@ static int tiles_grid(long long n_hint, long long n_cap, int tile) {
 // One counted pass (count, scan, scatter) over *n_dev items; tiles beyond
 // the device-side count exit at once. small_cap: passes do nothing when
 // n <= small_cap (the single-workgroup path handled them).
-static void launch_digit_pass(hipStream_t s, const SortBufs& b, const unsigned* kin, const float* vin,
-                              unsigned* kout, float* vout, int shift, const long long* n_dev, Ctl* ctl,
-                              long long n_hint, long long n_cap, int small_cap, Ep e, Gate g) {
+static void launch_digit_pass(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out, int shift,
+                              int bits, const long long* n_dev, Ctl* ctl, long long n_hint, long long n_cap,
+                              int small_cap, Ep e, Gate g) {
   const int tiles = tiles_grid(n_hint, n_cap, kSortTile);
   const int pgrid = std::min(tiles, 2048);  // count / scatter loop over their tiles
-  const int sgrid = (int)std::max<long long>(1, (256LL * tiles + kDScanTile - 1) / kDScanTile);
-  hipLaunchKernelGGL((k_digit_count<kSortNT, kSortIPT>), dim3(pgrid), dim3(kSortNT), 0, s, kin, n_dev,
-                     shift, b.dcount, small_cap, g);
+  const int sgrid = (int)std::max<long long>(1, (((long long)tiles << bits) + kDScanTile - 1) / kDScanTile);
+  hipLaunchKernelGGL((k_digit_count<kSortNT, kSortIPT>), dim3(pgrid), dim3(kSortNT), 0, s, in.k, n_dev,
+                     shift, bits, b.dcount, small_cap, g);
   hipLaunchKernelGGL((k_digit_scan<kDScanNT, kDScanIPT>), dim3(sgrid), dim3(kDScanNT), 0, s, b.dcount,
-                     n_dev, kSortTile, small_cap, b.dstate, ctl, e, g);
-  hipLaunchKernelGGL((k_sort_scatter<kSortNT, kSortIPT>), dim3(pgrid), dim3(kSortNT), 0, s, kin, vin, kout,
-                     vout, n_dev, shift, b.dcount, small_cap, g);
+                     n_dev, kSortTile, bits, small_cap, b.dstate, ctl, e, g);
+#define SPMSPV_SCATTER(PAY)                                                                                  \
+  hipLaunchKernelGGL((k_sort_scatter<kSortNT, kSortIPT, PAY>), dim3(pgrid), dim3(kSortNT), 0, s, in, out, n_dev, \
+                     shift, bits, b.dcount, small_cap, g)
+  if (in.w) SPMSPV_SCATTER(2);
+  else if (in.v) SPMSPV_SCATTER(1);
+  else SPMSPV_SCATTER(0);
+#undef SPMSPV_SCATTER
 }
 
-// Sorts (keyA, valA)[*n_dev] by key < range; returns 0 when the result is
-// in A, 1 when in B. ep.dev >= 0 (captured graphs) uses device epochs
-// ep.dev + pass; otherwise ep.v + pass.
-int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long long* n_dev, Ctl* ctl,
-                      long long n_hint, long long n_cap, bool skip_small, Ep ep, Gate g, int small_cap) {
-  const int passes = key_passes(range);
-  const int final_b = passes & 1;
+// The digits of a key of key_bits(range) bits are as equal as they can be:
+// 20 bits are 7 + 7 + 6, not 8 + 8 + 4 (fewer ballots per item and counts per
+// tile, longer runs of equal digits to store).
+int launch_radix_sets(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out0, const SortSet& out1,
+                      int range, const long long* n_dev, Ctl* ctl, long long n_hint, long long n_cap,
+                      bool skip_small, Ep ep, Gate g, int small_cap) {
+  const int total = key_bits(range), passes = key_passes(range), per = (total + passes - 1) / passes;
+  const int last = (passes & 1) ? 0 : 1;
+  const SortSet outs[2] = {out0, out1};
   const bool small_known = n_hint >= 0 && n_hint <= small_cap;
   const bool big_known = n_hint > small_cap;
   if (!big_known && !skip_small) {
-    hipLaunchKernelGGL((k_sort_small<kSortNT, kSortIPT>), dim3(1), dim3(kSortNT), 0, s, b.keyA,
-                       b.valA, n_dev, passes, 1, ctl, nullptr, nullptr, final_b ? b.keyB : b.keyA,
-                       final_b ? b.valB : b.valA, small_cap, g);
+#define SPMSPV_SMALL(PAY)                                                                                \
+  hipLaunchKernelGGL((k_sort_small<kSortNT, kSortIPT, PAY>), dim3(1), dim3(kSortNT), 0, s, in, n_dev, passes, 1, \
+                     ctl, nullptr, nullptr, outs[last], small_cap, g)
+    if (in.w) SPMSPV_SMALL(2);
+    else if (in.v) SPMSPV_SMALL(1);
+    else SPMSPV_SMALL(0);
+#undef SPMSPV_SMALL
   }
-  if (small_known) return final_b;
+  if (small_known) return last;
   for (int p = 0; p < passes; ++p) {
-    const unsigned* kin = (p & 1) ? b.keyB : b.keyA;
-    const float* vin = (p & 1) ? b.valB : b.valA;
-    unsigned* kout = (p & 1) ? b.keyA : b.keyB;
-    float* vout = (p & 1) ? b.valA : b.valB;
     const Ep e{ep.v + (unsigned)p, ep.dev < 0 ? -1 : ep.dev + p};
-    launch_digit_pass(s, b, kin, vin, kout, vout, 8 * p, n_dev, ctl, n_hint, n_cap, small_cap, e, g);
+    const int shift = p * per, bits = std::min(per, total - shift);
+    launch_digit_pass(s, b, p == 0 ? in : outs[(p - 1) & 1], outs[p & 1], shift, bits, n_dev, ctl, n_hint, n_cap,
+                      small_cap, e, g);
   }
-  return final_b;
+  return last;
 }
 
-// One stable partition pass of (keyA, valA) into (keyB, valB) on the 8-bit
-// digit (key >> shift) & 255. Afterwards b.dcount[d * ntiles] (ntiles =
-// ceil(n / kSortTile)) is the start of digit d in the output.
-void launch_partition_pass(hipStream_t s, const SortBufs& b, int shift, const long long* n_dev, Ctl* ctl,
-                           long long n_hint, long long n_cap, Ep ep) {
-  launch_digit_pass(s, b, b.keyA, b.valA, b.keyB, b.valB, shift, n_dev, ctl, n_hint, n_cap, -1, ep, Gate{});
+static SortSet set_a(const SortBufs& b) { return {b.keyA, reinterpret_cast<unsigned*>(b.valA), nullptr}; }
+static SortSet set_b(const SortBufs& b) { return {b.keyB, reinterpret_cast<unsigned*>(b.valB), nullptr}; }
+
+int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long long* n_dev, Ctl* ctl,
+                      long long n_hint, long long n_cap, bool skip_small, Ep ep, Gate g, int small_cap) {
+  const int last = launch_radix_sets(s, b, set_a(b), set_b(b), set_a(b), range, n_dev, ctl, n_hint, n_cap, skip_small,
+                                     ep, g, small_cap);
+  return last == 0 ? 1 : 0;
 }
 
 void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* ykey, float* yval,
@@ -591,8 +623,8 @@ void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* 
   const bool small_known = binlen_hint >= 0 && binlen_hint <= small_cap;
   const bool big_known = binlen_hint > small_cap;
   if (!big_known) {
-    hipLaunchKernelGGL((k_sort_small<kSortNT, kSortIPT>), dim3(1), dim3(kSortNT), 0, s, b.keyA,
-                       b.valA, n_dev, passes, 0, ctl, ykey, yval, nullptr, nullptr, small_cap, g);
+    hipLaunchKernelGGL((k_sort_small<kSortNT, kSortIPT, 1>), dim3(1), dim3(kSortNT), 0, s, set_a(b), n_dev, passes, 0,
+                       ctl, ykey, yval, SortSet{}, small_cap, g);
   }
   if (small_known) return;
   const int fb = launch_radix_sort(s, b, m, n_dev, ctl, binlen_hint, n_cap, true, ep, g, small_cap);
