@@ -194,6 +194,21 @@ __device__ __forceinline__ T block_min(T v, T* lds) {
   return r;
 }
 
+// Largest i in [lo, hi) with a[i] <= v, by the whole block (a ascending,
+// a[lo] <= v < a[hi]): every round tests NT places at once. lds: NT/64 ints.
+template <int NT>
+__device__ __forceinline__ int block_last_le(const int* __restrict__ a, int lo, int hi, int v, int* lds) {
+  while (hi - lo > 1) {
+    const long long len = hi - lo;
+    auto probe = [&](int i) { return lo + (int)(len * (i + 1) / (NT + 1)); };
+    const int below = block_sum<NT, int>(a[probe(threadIdx.x)] <= v ? 1 : 0, lds);
+    const int nlo = below > 0 ? probe(below - 1) : lo, nhi = below < NT ? probe(below) : hi;
+    lo = nlo;
+    hi = nhi;
+  }
+  return lo;
+}
+
 // ---------------------------------------------------------------- tickets
 // Persistent-tile helpers. Every workgroup loops: t = next_tile(); if t >=
 // ntiles break. The ticket order guarantees that when a workgroup holds tile

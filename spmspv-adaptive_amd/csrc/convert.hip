@@ -1,8 +1,12 @@
 // Matrix preparation and matrix features on gfx950:
 //  * CSR -> CSC transpose (ToCSC, spmspv.h:383-419, which called
-//    cusparseScsr2csc): expand row ids, stable radix sort of (col, nnz id)
-//    with the in-house sort, gather rows/values, and column pointers from
-//    the sorted column ids. Stability keeps rows ascending in each column.
+//    cusparseScsr2csc): expand row ids, stable radix sort of (col, row, value)
+//    with the in-house sort, its last pass writing the CSC's arrays, and
+//    column pointers from the sorted column ids. Stability keeps rows
+//    ascending in each column. Bound by the passes' traffic (24 bytes per
+//    nonzero and pass); sorting nonzero ids instead moves 16 but then gathers
+//    rows and values at random (513 us of 1,130 at R-MAT s19, 15.9 M nonzeros,
+//    400 us in all now).
 //  * Row-degree features (computeMatFeture_serial, spmspv.h:2274-2334, and
 //    the int-mean stdRow of extractMatFeatureParallel, spmspv.h:920-976):
 //    one grid-stride pass with per-workgroup partials, a degree histogram,
@@ -16,32 +20,79 @@
 namespace spmspv {
 
 
-__global__ void k_expand_rows(const int* __restrict__ row_ptr, int m, int* __restrict__ rowid) {
-  for (long long r = (long long)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; r < m;
-       r += (long long)gridDim.x * (blockDim.x / kWave)) {
-    const int b = row_ptr[r], e = row_ptr[r + 1];
-    for (int j = b + lane(); j < e; j += kWave) rowid[j] = (int)r;
+// Row of every nonzero, a tile of NT * IPT nonzeros per workgroup: the row of
+// the tile's first nonzero by search, the starts of the rows that begin in
+// the tile marked in LDS, then a running maximum (a wave per row left most
+// lanes idle on short rows and one wave on each long row: 83 us at 15.9 M
+// nonzeros, 37 us so). IPT is odd: a thread's consecutive LDS words.
+template <int NT, int IPT>
+__global__ __launch_bounds__(NT) void k_expand_rows(const int* __restrict__ row_ptr, int m, int nnz,
+                                                    int* __restrict__ rowid) {
+  constexpr int TILE = NT * IPT, NW = NT / kWave, RPT = 4;
+  __shared__ int s_row[TILE];
+  __shared__ int s_i[NW];
+  const int base = blockIdx.x * TILE;
+  const int cnt = min(TILE, nnz - base), end = base + cnt;
+#pragma unroll
+  for (int k = 0; k < IPT; ++k) s_row[k * NT + threadIdx.x] = 0;
+  const int r0 = block_last_le<NT>(row_ptr, 0, m, base, s_i);
+  if (threadIdx.x == 0) s_row[0] = r0;
+  // NT * RPT rows per round: where rows are short or empty a tile holds
+  // several times its nonzeros in rows
+  for (int rb = r0 + 1;;) {
+    int b[RPT], e[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int r = min(rb + k * NT + (int)threadIdx.x, m - 1);
+      b[k] = row_ptr[r];
+      e[k] = row_ptr[r + 1];
+    }
+    bool has = false;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      const int r = rb + k * NT + (int)threadIdx.x;
+      if (r < m && b[k] < end && e[k] > b[k]) {
+        s_row[b[k] - base] = r;
+        has = true;
+      }
+    }
+    // does the next round's first row start in this tile as well?
+    const bool more = rb + RPT * NT < m && e[RPT - 1] < end;
+    if (!__syncthreads_or(threadIdx.x == NT - 1 && more)) break;
+    rb += RPT * NT;
+    // past a round of empty rows, to the next row that has a nonzero
+    if (!__syncthreads_or(has)) rb = block_last_le<NT>(row_ptr, rb, m, row_ptr[rb], s_i);
   }
+  __syncthreads();
+  int mx = 0;
+#pragma unroll
+  for (int k = 0; k < IPT; ++k) mx = max(mx, s_row[threadIdx.x * IPT + k]);
+  int inc = mx;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int v = __shfl_up(inc, o, kWave);
+    if (lane() >= o) inc = max(inc, v);
+  }
+  if (lane() == kWave - 1) s_i[threadIdx.x / kWave] = inc;
+  int run = __shfl_up(inc, 1, kWave);
+  if (lane() == 0) run = 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NW; ++k)
+    if (k < (int)threadIdx.x / kWave) run = max(run, s_i[k]);
+#pragma unroll
+  for (int k = 0; k < IPT; ++k) {
+    run = max(run, s_row[threadIdx.x * IPT + k]);
+    s_row[threadIdx.x * IPT + k] = run;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < cnt; i += NT) rowid[base + i] = s_row[i];
 }
 
-__global__ void k_keys_from_cols(const int* __restrict__ col, int nnz, unsigned* __restrict__ key,
-                                 unsigned* __restrict__ idx) {
-  for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < nnz;
-       j += (long long)gridDim.x * blockDim.x) {
-    key[j] = (unsigned)col[j];
-    idx[j] = (unsigned)j;
-  }
-}
-
-__global__ void k_gather_csc(const unsigned* __restrict__ skey, const unsigned* __restrict__ sidx,
-                             const int* __restrict__ rowid, const float* __restrict__ val, int nnz,
-                             int n, int* __restrict__ crow, float* __restrict__ cval,
-                             int* __restrict__ colptr) {
+// colptr from the sorted column of every nonzero.
+__global__ void k_col_bounds(const unsigned* __restrict__ skey, int nnz, int n, int* __restrict__ colptr) {
   for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < nnz;
        p += (long long)gridDim.x * blockDim.x) {
-    const unsigned j = sidx[p];
-    crow[p] = rowid[j];
-    cval[p] = val[j];
     const int c = (int)skey[p];
     const int cprev = p == 0 ? -1 : (int)skey[p - 1];
     for (int q = cprev + 1; q <= c; ++q) colptr[q] = (int)p;  // columns (cprev, c] start at p
@@ -52,6 +103,13 @@ __global__ void k_gather_csc(const unsigned* __restrict__ skey, const unsigned* 
 
 __global__ void k_set_ll(long long* p, long long v) { *p = v; }
 
+void launch_expand_rows(hipStream_t s, const int* row_ptr, int m, int nnz, int* rowid) {
+  constexpr int NT = 256, IPT = 9;
+  if (nnz > 0)
+    hipLaunchKernelGGL((k_expand_rows<NT, IPT>), dim3((nnz - 1) / (NT * IPT) + 1), dim3(NT), 0, s, row_ptr, m, nnz,
+                       rowid);
+}
+
 hipError_t launch_csr_to_csc_sorted(hipStream_t s, const int* row_ptr, const int* col, const float* val,
                               int m, int n, int nnz, int* colptr, int* crow, float* cval,
                               const SortBufs& b, long long* n_dev, Ctl* ctl, Ep ep) {
@@ -60,20 +118,19 @@ hipError_t launch_csr_to_csc_sorted(hipStream_t s, const int* row_ptr, const int
     return hipGetLastError();
   }
   const int g = (int)std::min<long long>(8192, ((long long)nnz + 255) / 256);
-  // row id of every nonzero, parked in crow until the gather below
-  hipLaunchKernelGGL(k_expand_rows, dim3(std::min(8192, (m + 3) / 4 + 1)), dim3(256), 0, s, row_ptr,
-                     m, crow);
-  hipLaunchKernelGGL(k_keys_from_cols, dim3(g), dim3(256), 0, s, col, nnz, b.keyA,
-                     reinterpret_cast<unsigned*>(b.valA));
+  // the passes write two sets of arrays in turn, the last one the set with
+  // the CSC's own; the row ids start in the set that the first one reads
+  const SortSet csc{b.keyB, reinterpret_cast<unsigned*>(crow), reinterpret_cast<unsigned*>(cval)};
+  const SortSet tmp{b.keyA, reinterpret_cast<unsigned*>(b.valA), reinterpret_cast<unsigned*>(b.valB)};
+  const bool odd = radix_passes(n) & 1;
+  unsigned* rowid = odd ? tmp.v : csc.v;
+  launch_expand_rows(s, row_ptr, m, nnz, reinterpret_cast<int*>(rowid));
   hipLaunchKernelGGL(k_set_ll, dim3(1), dim3(1), 0, s, n_dev, (long long)nnz);
-  const int fb = launch_radix_sort(s, b, n, n_dev, ctl, nnz, nnz, false, ep);
-  const unsigned* sk = fb ? b.keyB : b.keyA;
-  const unsigned* si = reinterpret_cast<const unsigned*>(fb ? b.valB : b.valA);
-  // gather into the free key buffer, then move the rows into crow
-  int* rows_out = reinterpret_cast<int*>(fb ? b.keyA : b.keyB);
-  hipLaunchKernelGGL(k_gather_csc, dim3(g), dim3(256), 0, s, sk, si, crow, val, nnz, n, rows_out,
-                     cval, colptr);
-  return hipMemcpyAsync(crow, rows_out, sizeof(int) * (size_t)nnz, hipMemcpyDeviceToDevice, s);
+  const SortSet in{const_cast<unsigned*>(reinterpret_cast<const unsigned*>(col)), rowid,
+                   const_cast<unsigned*>(reinterpret_cast<const unsigned*>(val))};
+  launch_radix_sets(s, b, in, odd ? csc : tmp, odd ? tmp : csc, n, n_dev, ctl, nnz, nnz, false, ep);
+  hipLaunchKernelGGL(k_col_bounds, dim3(g), dim3(256), 0, s, csc.k, nnz, n, colptr);
+  return hipGetLastError();
 }
 
 // ------------------------------------------------------- mat features

@@ -218,6 +218,7 @@ void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* 
 int launch_radix_sets(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out0, const SortSet& out1,
                       int range, const long long* n_dev, Ctl* ctl, long long n_hint, long long n_cap,
                       bool skip_small, Ep ep, Gate g = {}, int small_cap = kSmallSortCap);
+int radix_passes(int range);  // of a sort by keys < range
 // Sorts (keyA, valA)[*n_dev] by key < range; returns 0 if the result is in
 // A, 1 if in B. With valA and valB null it sorts the keys alone.
 int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long long* n_dev, Ctl* ctl,
@@ -344,6 +345,8 @@ void launch_row_naive(hipStream_t s, bool masked, bool hits, const int* row_ptr,
                       float* y, unsigned* ybits);
 
 // --- CSC construction ----------------------------------------------------
+// rowid[j] = row of nonzero j
+void launch_expand_rows(hipStream_t s, const int* row_ptr, int m, int nnz, int* rowid);
 hipError_t launch_csr_to_csc_sorted(hipStream_t s, const int* row_ptr, const int* col, const float* val,
                               int m, int n, int nnz, int* colptr, int* crow, float* cval,
                               const SortBufs& b, long long* n_dev, Ctl* ctl, Ep ep);

@@ -546,6 +546,7 @@ static int key_bits(int range) {
   return bits;
 }
 static int key_passes(int range) { return (key_bits(range) + 7) / 8; }
+int radix_passes(int range) { return key_passes(range); }
 
 // Grid for a launch over n items in tiles of `tile`: exact when the host
 // knows n (n_hint >= 0), else the bound n_cap.
