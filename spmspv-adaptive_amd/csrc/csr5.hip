@@ -27,6 +27,7 @@
 #include <algorithm>
 
 #include "handle.hpp"
+#include "ranking.hpp"
 
 namespace spmspv {
 
@@ -141,9 +142,9 @@ __global__ void k_row_markers(const int* __restrict__ row_ptr, int m, int T, int
   }
 }
 
+// The copy of a matrix whose columns keep their order.
 __global__ void k_csr5_transpose(const int* __restrict__ col, const float* __restrict__ val, int nnz,
-                                 int T, int S, long long total, const int* __restrict__ cperm,
-                                 const int* __restrict__ item, int* __restrict__ ccol,
+                                 int T, int S, long long total, int* __restrict__ ccol,
                                  float* __restrict__ cval) {
   for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < total;
        q += (long long)gridDim.x * blockDim.x) {
@@ -156,11 +157,8 @@ __global__ void k_csr5_transpose(const int* __restrict__ col, const float* __res
     const int l = r >> 2, i = g * 4 + (r & 3);
     const long long src = t * T + (long long)l * S + i;
     const bool ok = src < nnz;
-    // with an item order, position src of the copy holds CSR item item[src]
-    const long long j = ok ? (item ? (long long)item[src] : src) : 0;
-    const int c = ok ? col[j] : 0;
-    ccol[q] = ok ? (cperm ? cperm[c] : c) : 0;
-    cval[q] = ok ? val[j] : 0.f;
+    ccol[q] = ok ? col[src] : 0;
+    cval[q] = ok ? val[src] : 0.f;
   }
 }
 
@@ -454,33 +452,7 @@ __global__ void k_col_keys_from_count(const unsigned* __restrict__ cnt, int n, l
   }
 }
 __global__ void k_set_count(long long* p, long long v) { *p = v; }
-// sort 1 of the item order: key = new column of item j, value = j
-__global__ void k_item_keys_col(const int* __restrict__ col, int nnz, const int* __restrict__ cperm,
-                                unsigned* __restrict__ keys, float* __restrict__ vals) {
-  for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < nnz;
-       j += (long long)gridDim.x * blockDim.x) {
-    keys[j] = (unsigned)cperm[col[j]];
-    vals[j] = __int_as_float((int)j);
-  }
-}
-// sort 2: key = row of the item (binary search in row_ptr), value = item,
-// written into (keys, vals_out) from the order of sort 1 (in place allowed)
-__global__ void k_item_keys_row(const float* vals_in, int nnz, const int* __restrict__ row_ptr, int m,
-                                unsigned* keys, float* vals_out) {
-  for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < nnz;
-       q += (long long)gridDim.x * blockDim.x) {
-    const float v = vals_in[q];
-    const int j = __float_as_int(v);
-    int lo = 0, hi = m;  // last row r with row_ptr[r] <= j
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (row_ptr[mid] <= j) lo = mid;
-      else hi = mid;
-    }
-    keys[q] = (unsigned)lo;
-    vals_out[q] = v;
-  }
-}
+__global__ void k_set_int(int* p, int v) { *p = v; }
 __global__ void k_invert_order(const float* __restrict__ vals, int n, int* __restrict__ cperm) {
   for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < n;
        q += (long long)gridDim.x * blockDim.x)
@@ -509,24 +481,230 @@ bool launch_column_order(hipStream_t s, const ColumnOrderArgs& a, const int* col
   return hipGetLastError() == hipSuccess;
 }
 
-// The items of every row ordered by their new column (two stable sorts: by
-// new column, then by row); returns the order (CSR item of every position)
-// in the sort buffers, valid until they are reused, or null.
-static const int* launch_item_order(hipStream_t s, const ColumnOrderArgs& a, const int* row_ptr,
-                                    const int* col, int nnz, int m, int n, const int* cperm) {
-  if (nnz <= 0 || nnz > a.sb_cap || m <= 0) return nullptr;
-  const int grid = std::max(1, std::min(8192, (nnz + 255) / 256));
-  hipLaunchKernelGGL(k_item_keys_col, dim3(grid), dim3(256), 0, s, col, nnz, cperm, a.sb.keyA, a.sb.valA);
-  hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, s, a.n_dev, (long long)nnz);
-  const Ep e1{a.ep.v + 4u, -1};
-  const int f1 = launch_radix_sort(s, a.sb, n, a.n_dev, a.ctl, nnz, nnz, false, e1);
-  // sort 2 reads its keys from wherever sort 1 left the items, into A
-  hipLaunchKernelGGL(k_item_keys_row, dim3(grid), dim3(256), 0, s, f1 ? a.sb.valB : a.sb.valA, nnz, row_ptr,
-                     m, a.sb.keyA, a.sb.valA);
-  const Ep e2{a.ep.v + 8u, -1};
-  const int f2 = launch_radix_sort(s, a.sb, m, a.n_dev, a.ctl, nnz, nnz, false, e2);
-  if (hipGetLastError() != hipSuccess) return nullptr;
-  return reinterpret_cast<const int*>(f2 ? a.sb.valB : a.sb.valA);
+// ---- items of every row in the order of their new columns --------------------
+// Rows of up to kOrderWin nonzeros: one workgroup takes the rows that start in
+// its window of kOrderWin CSR positions, which are consecutive positions and at
+// most kOrderCap of them, sorts them in LDS by (row, new column) and writes
+// them to their places in the tiles. A longer row (it can only be the last one
+// of a window) is left to a sort of all such rows' items through memory.
+// Two stable sorts of every item through memory, by new column, then by row,
+// took 1,740 us at R-MAT s19 (15.9 M nonzeros), this 480 us: 330 in LDS, which
+// the ranking's ballots and LDS round trips bound, 150 for the 15 % of the
+// items in long rows. Two workgroups of 512 threads share a CU's LDS (10 bytes
+// per item and the counters) and overlap each other's barriers; one of 1,024
+// with twice the window took 435 us in LDS, four of 256 (two thirds of the
+// window, more long rows) 20 us more in all.
+constexpr int kOrderNT = 512, kOrderIPT = 12, kOrderCap = kOrderNT * kOrderIPT, kOrderWin = kOrderCap / 2;
+
+// where CSR position p lies in the copy (the layout in k_csr5_transpose)
+__device__ __forceinline__ long long csr5_place(long long p, int T, int S) {
+  const long long t = p / T;
+  const int o = (int)(p - t * T);
+  const int l = o / S, i = o - l * S;
+  return t * T + (i >> 2) * (4 * kWave) + l * 4 + (i & 3);
+}
+
+// Rows of more than kOrderWin nonzeros: their number (high word of *count) and
+// nonzeros (low word), and each one's row and first item among them.
+__global__ void k_long_rows(const int* __restrict__ row_ptr, int m, unsigned long long* count,
+                            int* __restrict__ long_row, int* __restrict__ long_off) {
+  for (long long r0 = (long long)blockIdx.x * blockDim.x; r0 < m; r0 += (long long)gridDim.x * blockDim.x) {
+    const long long r = r0 + threadIdx.x;
+    const int len = r < m ? row_ptr[r + 1] - row_ptr[r] : 0;
+    const unsigned long long mine = len > kOrderWin ? (1ull << 32) + (unsigned)len : 0ull;
+    if (!__ballot(mine != 0ull)) continue;
+    // one atomic per wave: rows and nonzeros of the wave at once
+    const unsigned long long inc = wave_incl_sum(mine);
+    unsigned long long base = 0;
+    if (lane() == kWave - 1) base = atomicAdd(count, inc);
+    base = __shfl(base, kWave - 1, kWave) + inc - mine;
+    if (mine) {
+      long_row[base >> 32] = (int)r;
+      long_off[base >> 32] = (int)(unsigned)base;
+    }
+  }
+}
+
+// their items: key = new column, v = index of the row among them, w = value
+__global__ void k_long_items(const int* __restrict__ row_ptr, const int* __restrict__ col,
+                             const float* __restrict__ val, const int* __restrict__ cperm,
+                             const int* __restrict__ long_row, const int* __restrict__ long_off, int items,
+                             SortSet s) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < items; i += gridDim.x * blockDim.x) {
+    const int li = (int)s.v[i];
+    const int j = row_ptr[long_row[li]] + (i - long_off[li]);
+    s.k[i] = (unsigned)cperm[col[j]];
+    s.w[i] = __float_as_uint(val[j]);
+  }
+}
+
+// sorted (key = row index, v = new column, w = value) to their places
+__global__ void k_long_place(const int* __restrict__ row_ptr, const int* __restrict__ long_row,
+                             const int* __restrict__ long_off, int items, SortSet s, int T, int S,
+                             int* __restrict__ ccol, float* __restrict__ cval) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < items; i += gridDim.x * blockDim.x) {
+    const int li = (int)s.k[i];
+    const long long q = csr5_place((long long)row_ptr[long_row[li]] + (i - long_off[li]), T, S);
+    ccol[q] = (int)s.v[i];
+    cval[q] = __uint_as_float(s.w[i]);
+  }
+}
+
+template <int NT, int IPT>
+__global__ __launch_bounds__(NT) void k_order_rows(const int* __restrict__ row_ptr, const int* __restrict__ col,
+                                                   const float* __restrict__ val, const int* __restrict__ cperm,
+                                                   const int* __restrict__ rows_ne, const int* __restrict__ ne_before,
+                                                   int m, int nnz, int nbits, int T, int S, long long total,
+                                                   int* __restrict__ ccol, float* __restrict__ cval) {
+  constexpr int CAP = NT * IPT, WIN = CAP / 2, NW = NT / kWave;
+  __shared__ unsigned s_k[CAP];
+  __shared__ float s_v[CAP];
+  __shared__ unsigned short s_r[CAP];
+  __shared__ unsigned s_cnt[NW * 256];
+  __shared__ unsigned s_dstart[256];
+  __shared__ unsigned s_t[NW];
+  __shared__ int s_i[NW];
+  if (blockIdx.x == gridDim.x - 1) {  // positions past the data, to the end of the last tile
+    for (long long p = nnz + (long long)threadIdx.x; p < total; p += NT) {
+      const long long q = csr5_place(p, T, S);
+      ccol[q] = 0;
+      cval[q] = 0.f;
+    }
+  }
+  const long long w0 = (long long)blockIdx.x * WIN;
+  const int w1 = (int)min(w0 + WIN, (long long)nnz);
+  // the rows that start in [w0, w1): r0 .. rl, CSR positions [j0, j1)
+  int r0 = block_last_le<NT>(row_ptr, 0, m, (int)w0, s_i);
+  if (row_ptr[r0] < w0) ++r0;
+  const int j0 = row_ptr[r0];
+  if (j0 >= w1) return;
+  const int rl = block_last_le<NT>(row_ptr, r0, m, w1 - 1, s_i);
+  const int bl = row_ptr[rl], el = row_ptr[rl + 1];
+  const bool is_long = el - bl > WIN;
+  const int cnt = (is_long ? bl : el) - j0;
+  if (cnt <= 0) return;
+  // items per thread (<= IPT): every wave gets its share
+  const int ie = (cnt + NT - 1) / NT;
+  for (int i = threadIdx.x; i < cnt; i += NT) s_r[i] = 0;
+  __syncthreads();
+  const int n1 = ne_before[rl] + (is_long ? 0 : 1);
+  for (int i = ne_before[r0] + (int)threadIdx.x; i < n1; i += NT) s_r[row_ptr[rows_ne[i]] - j0] = 1;
+  __syncthreads();
+  // row of every item, counted among the window's rows with nonzeros (only
+  // these are walked: there may be any number of empty rows between them)
+  int nrows;
+  {
+    const int i0 = threadIdx.x * ie;
+    int heads = 0;
+    for (int k = 0; k < ie; ++k) heads += i0 + k < cnt ? s_r[i0 + k] : 0;
+    int run = block_excl_sum<NT, int>(heads, s_i, &nrows) - 1;
+    for (int k = 0; k < ie; ++k) {
+      if (i0 + k < cnt) {
+        run += s_r[i0 + k];
+        s_r[i0 + k] = (unsigned short)run;
+      }
+    }
+  }
+  __syncthreads();
+  const int w = threadIdx.x / kWave;
+  const int p0 = w * kWave * ie + lane();
+  unsigned key[IPT], row[IPT], dig[IPT];
+  float v[IPT];
+  bool valid[IPT];
+  int rank[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const int p = p0 + j * kWave;
+    valid[j] = j < ie && p < cnt;
+    key[j] = valid[j] ? (unsigned)col[j0 + p] : 0u;
+    v[j] = valid[j] ? val[j0 + p] : 0.f;
+    row[j] = valid[j] ? s_r[p] : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) key[j] = valid[j] ? (unsigned)cperm[key[j]] : 0u;
+  // stable LDS radix sort by (row, new column), digits of equal width
+  const int bits = nbits + (nrows > 1 ? 32 - __builtin_clz(nrows - 1) : 0);
+  const int passes = max(1, (bits + 7) / 8), per = (bits + passes - 1) / passes;
+  for (int ps = 0; ps < passes; ++ps) {
+    const int shift = ps * per, db = min(per, bits - shift);
+    const unsigned mask = (1u << db) - 1u;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+      dig[j] = valid[j] ? (unsigned)((((unsigned long long)row[j] << nbits) | key[j]) >> shift) & mask : 0u;
+    wave_rank_digits<IPT>(dig, valid, s_cnt + w * 256, rank, ie, db);
+    __syncthreads();
+    unsigned tot = 0;
+    if (threadIdx.x < 256) tot = digit_wave_offsets<NW>(s_cnt);
+    unsigned dtot;
+    const unsigned dex = block_excl_sum<NT, unsigned>(tot, s_t, &dtot);
+    if (threadIdx.x < 256) s_dstart[threadIdx.x] = dex;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+      if (valid[j]) {
+        const unsigned q = s_dstart[dig[j]] + s_cnt[w * 256 + dig[j]] + rank[j];
+        s_k[q] = key[j];
+        s_v[q] = v[j];
+        s_r[q] = (unsigned short)row[j];
+      }
+    }
+    __syncthreads();
+    if (ps + 1 < passes) {
+#pragma unroll
+      for (int j = 0; j < IPT; ++j) {
+        const int p = p0 + j * kWave;
+        if (valid[j]) {
+          key[j] = s_k[p];
+          v[j] = s_v[p];
+          row[j] = s_r[p];
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (int i = threadIdx.x; i < cnt; i += NT) {
+    const long long q = csr5_place((long long)j0 + i, T, S);
+    ccol[q] = (int)s_k[i];
+    cval[q] = s_v[i];
+  }
+}
+
+// Every row's items in the order of their new columns, at their places in
+// ccol / cval. nlong rows of more than kOrderWin nonzeros hold `items` of them.
+static void launch_order_rows(hipStream_t s, const ColumnOrderArgs& a, const int* row_ptr, const int* col,
+                              const float* val, int m, int n, int nnz, int T, int S, long long total,
+                              const int* cperm, const int* rows_ne, const int* ne_before, int nlong, int items,
+                              const int* long_row, const int* long_off, int* ccol, float* cval) {
+  int nbits = 1;
+  while (nbits < 31 && (1 << nbits) < n) ++nbits;
+  if (nlong > 0) {
+    // two sorts, by new column, then by row; all passes write two sets of
+    // arrays in turn, the last one the set that is not the copy's own arrays
+    const int grid = std::max(1, std::min(8192, (items + 255) / 256));
+    const SortSet tmp{a.sb.keyA, reinterpret_cast<unsigned*>(a.sb.valA), reinterpret_cast<unsigned*>(a.sb.valB)};
+    const SortSet own{a.sb.keyB, reinterpret_cast<unsigned*>(ccol), reinterpret_cast<unsigned*>(cval)};
+    const int p1 = radix_passes(n), p2 = nlong > 1 ? radix_passes(nlong) : 0;
+    const SortSet sets[2] = {(p1 + p2) & 1 ? tmp : own, (p1 + p2) & 1 ? own : tmp};
+    // the first pass reads sets[1] and writes sets[0]
+    launch_expand_rows(s, long_off, nlong, items, reinterpret_cast<int*>(sets[1].v));
+    hipLaunchKernelGGL(k_long_items, dim3(grid), dim3(256), 0, s, row_ptr, col, val, cperm, long_row, long_off, items,
+                       sets[1]);
+    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, s, a.n_dev, (long long)items);
+    const Ep e1{a.ep.v + 4u, -1}, e2{a.ep.v + 8u, -1};
+    const int f1 = launch_radix_sets(s, a.sb, sets[1], sets[0], sets[1], n, a.n_dev, a.ctl, items, items, false, e1,
+                                     Gate{}, 0);
+    const auto by_row = [](const SortSet& q) { return SortSet{q.v, q.k, q.w}; };
+    SortSet done = by_row(sets[f1]);
+    if (nlong > 1) {
+      const SortSet o0 = sets[f1 ^ 1], o1 = done;
+      const int f2 = launch_radix_sets(s, a.sb, done, o0, o1, nlong, a.n_dev, a.ctl, items, items, false, e2, Gate{}, 0);
+      done = f2 ? o1 : o0;
+    }
+    hipLaunchKernelGGL(k_long_place, dim3(grid), dim3(256), 0, s, row_ptr, long_row, long_off, items, done, T, S, ccol,
+                       cval);
+  }
+  hipLaunchKernelGGL((k_order_rows<kOrderNT, kOrderIPT>), dim3((nnz - 1) / kOrderWin + 1), dim3(kOrderNT), 0, s,
+                     row_ptr, col, val, cperm, rows_ne, ne_before, m, nnz, nbits, T, S, total, ccol, cval);
 }
 
 int csr5_sigma_of(int sigma, int m, long long nnz) {
@@ -558,6 +736,8 @@ size_t csr5_bytes(int m, int n, long long nnz, int S) {
   b += up(sizeof(int) * (size_t)(m / kScanPart + 2));                    // part sums
   b += up(sizeof(float) * (size_t)(ntiles + 1)) * 3;                     // carries
   b += up(sizeof(int) * (size_t)std::max(n, 1));                         // column order
+  b += up(sizeof(unsigned long long));                                   // rows over kOrderWin: counts,
+  b += up(sizeof(int) * (size_t)(nnz / kOrderWin + 2)) * 2;              // rows, first items
   return b;
 }
 
@@ -600,10 +780,17 @@ hipError_t csr5_build(hipStream_t s, const int* row_ptr, const int* col, const f
   int* cperm = reinterpret_cast<int*>(p);
   p += up(sizeof(int) * (size_t)std::max(n, 1));
   c.n = n;
-  const int* item = nullptr;
-  if (order && launch_column_order(s, *order, col, nnz, n, cperm)) {
+  unsigned long long* long_count = reinterpret_cast<unsigned long long*>(p);
+  p += up(sizeof(unsigned long long));
+  int* long_row = reinterpret_cast<int*>(p);
+  p += up(sizeof(int) * (size_t)(nnz / kOrderWin + 2));
+  int* long_off = reinterpret_cast<int*>(p);
+  // the order needs the sort buffers to hold a key per column
+  if (order && nnz <= order->sb_cap && launch_column_order(s, *order, col, nnz, n, cperm)) {
     c.cperm = cperm;
-    item = launch_item_order(s, *order, row_ptr, col, nnz, m, n, cperm);
+    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(1), 0, s, reinterpret_cast<long long*>(long_count), 0ll);
+    hipLaunchKernelGGL(k_long_rows, dim3(std::max(1, std::min(2048, (m + 255) / 256))), dim3(256), 0, s, row_ptr, m,
+                       long_count, long_row, long_off);
   }
 
   const int parts = (m + kScanPart - 1) / kScanPart;
@@ -614,7 +801,10 @@ hipError_t csr5_build(hipStream_t s, const int* row_ptr, const int* col, const f
                        c.rows_empty);
   }
   launch_fill_i32(s, reinterpret_cast<int*>(c.flags), (long long)(ntiles + 1) * kWave, 0);
+  h_pin[2] = h_pin[3] = 0;
   hipError_t e = hipMemcpyAsync(h_pin, sums + parts, sizeof(int), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && c.cperm)
+    e = hipMemcpyAsync(h_pin + 2, long_count, sizeof(*long_count), hipMemcpyDeviceToHost, s);
   if (e != hipSuccess) return e;
   if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
   c.n_ne = parts > 0 ? h_pin[0] : 0;
@@ -625,8 +815,18 @@ hipError_t csr5_build(hipStream_t s, const int* row_ptr, const int* col, const f
     hipLaunchKernelGGL(k_row_markers, dim3(std::min(8192, (m + 255) / 256)), dim3(256), 0, s, row_ptr,
                        m, T, S, c.flags);
     const long long total = (long long)ntiles * T;
-    hipLaunchKernelGGL(k_csr5_transpose, dim3((unsigned)std::min<long long>(8192, (total + 255) / 256)),
-                       dim3(256), 0, s, col, val, nnz, T, S, total, c.cperm, item, c.ccol, c.cval);
+    if (c.cperm) {
+      const int items = h_pin[2], nlong = h_pin[3];  // low and high word of the count
+      if (nlong > 0) {
+        // the rows' first items are searched as a row pointer is
+        hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, long_off + nlong, items);
+      }
+      launch_order_rows(s, *order, row_ptr, col, val, m, n, nnz, T, S, total, cperm, c.rows_ne, rank, nlong, items,
+                        long_row, long_off, c.ccol, c.cval);
+    } else {
+      hipLaunchKernelGGL(k_csr5_transpose, dim3((unsigned)std::min<long long>(8192, (total + 255) / 256)),
+                         dim3(256), 0, s, col, val, nnz, T, S, total, c.ccol, c.cval);
+    }
   }
   *out = c;
   return hipGetLastError();

@@ -30,6 +30,7 @@ SHAPES = {
     "sparse-rows": ([1 if r % 300 == 7 else 0 for r in range(200000)], 3000),
     "short-rows": ([r % 3 for r in range(30011)], 70000),
     "windows": ([6143, 6144, 6145, 1, 6144, 6144, 0, 12287, 2, 20000, 6145], 30000),
+    "half-windows": ([3071, 3072, 3073, 1, 3072, 3072, 0, 6143, 2, 6144, 3073], 30000),
     "long-and-short": ([9000] + [r % 5 for r in range(9001)] + [15000, 1, 0, 7000], 66000),
 }
 
