@@ -19,6 +19,15 @@
 // (only vertices that received a push can cross the threshold: every
 // other vertex above it was in S and is now at 0). At the end p += r.
 // With every residual at most eps (1 - d) / n, sum|p - p*| <= eps * d.
+//
+// y's keys are sorted and distinct, so the vertices that cross the threshold
+// come out in order: one kernel pushes, lists them and takes their residuals
+// for the next iteration (k_pr_push). It reads y's count on the device, so the
+// host waits once per iteration, for the next set's size. An iteration is
+// launches and short kernels: with separate take, push, compaction and count
+// kernels (6 to 20 us each, the push waiting on one atomic per vertex) and a
+// second wait for y's count, R-MAT s18 at eps 1e-4 took 7,400 us, 85
+// iterations, 5,300 us so.
 #include <chrono>
 
 #include "handle.hpp"
@@ -30,60 +39,152 @@ struct PrState {
   float* w = nullptr;         // n: column weight sums
   float* r = nullptr;         // n: residuals
   int* fk[2] = {nullptr, nullptr};  // n: active keys (sorted)
-  float* fv[2] = {nullptr, nullptr};  // n: scratch values of the compaction
-  float* xv = nullptr;        // n: x values of the active set
+  float* fv[2] = {nullptr, nullptr};  // n: x values of the active set
   int* yk = nullptr;          // m
   float* yv = nullptr;        // m
-  unsigned* bits = nullptr;   // ceil(n/32)+2: vertices crossing the threshold
 };
 
 namespace {
 
-__global__ void k_col_weights(const int* __restrict__ colptr, const float* __restrict__ cval, int n,
-                              float* __restrict__ w) {
-  // one wave per column, lanes stride its entries (hub columns stay wide)
-  const int wid = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-  const int nw = gridDim.x * blockDim.x / kWave;
-  for (int c = wid; c < n; c += nw) {
+constexpr int kPrNT = 256, kPrIPT = 8, kPrTile = kPrNT * kPrIPT;  // k_pr_push
+static_assert(kPrTile >= kPrepTile, "the look-back words are laid out for k_prep's tiles");
+constexpr int kLongCol = 1024;
+
+// Weight sums of the columns of at most kLongCol entries, a team of 16 lanes
+// per column.
+__global__ __launch_bounds__(256) void k_col_weights(const int* __restrict__ colptr, const float* __restrict__ cval,
+                                                     int n, float* __restrict__ w) {
+  constexpr int TEAM = 16;
+  const int tl = threadIdx.x & (TEAM - 1);
+  const long long nt = (long long)gridDim.x * blockDim.x / TEAM;
+  for (long long c = ((long long)blockIdx.x * blockDim.x + threadIdx.x) / TEAM; c < n; c += nt) {
     const int b = colptr[c], e = colptr[c + 1];
+    if (e - b > kLongCol) continue;
     float s = 0.f;
-    for (int i = b + lane(); i < e; i += kWave) s += cval[i];
-    s = wave_sum(s);
-    if (lane() == 0) w[c] = s;
+    for (int i = b + tl; i < e; i += 4 * TEAM) {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = i + k * TEAM < e ? cval[i + k * TEAM] : 0.f;
+      s += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+#pragma unroll
+    for (int o = TEAM / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, TEAM);
+    if (tl == 0) w[c] = s;
   }
 }
 
-__global__ void k_pr_init(int n, float r0, float* __restrict__ p, float* __restrict__ r,
-                          int* __restrict__ fk) {
+// The longer ones, a workgroup per column (one wave per hub column took 480 us
+// at R-MAT s18). Each workgroup looks through its own stride of columns, so
+// that hubs beside each other spread over the workgroups; the number of
+// workgroups is prime, since R-MAT's hubs also share their low bits.
+template <int NT>
+__global__ __launch_bounds__(NT) void k_long_col_weights(const int* __restrict__ colptr,
+                                                         const float* __restrict__ cval, int n,
+                                                         float* __restrict__ w) {
+  __shared__ int s_cols[NT];
+  __shared__ int s_i[NT / kWave];
+  __shared__ float s_f[NT / kWave];
+  for (long long k0 = 0; k0 * gridDim.x + blockIdx.x < n; k0 += NT) {
+    const long long c = (k0 + threadIdx.x) * gridDim.x + blockIdx.x;
+    const int is_long = c < n && colptr[c + 1] - colptr[c] > kLongCol ? 1 : 0;
+    int tot;
+    const int pos = block_excl_sum<NT, int>(is_long, s_i, &tot);
+    if (is_long) s_cols[pos] = (int)c;
+    __syncthreads();
+    for (int q = 0; q < tot; ++q) {
+      const int col = s_cols[q], b = colptr[col], e = colptr[col + 1];
+      float s = 0.f;
+      for (int i = b + (int)threadIdx.x; i < e; i += 4 * NT) {
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = i + k * NT < e ? cval[i + k * NT] : 0.f;
+        s += (v[0] + v[1]) + (v[2] + v[3]);
+      }
+      s = block_sum<NT, float>(s, s_f);
+      if (threadIdx.x == 0) w[col] = s;
+    }
+    __syncthreads();
+  }
+}
+
+__device__ __forceinline__ float share(float r, float w) { return w > 0.f ? r / w : 0.f; }
+
+// p, r, and the first active set (every vertex) with its residuals taken.
+__global__ void k_pr_init(int n, float r0, const float* __restrict__ w, float* __restrict__ p,
+                          float* __restrict__ r, int* __restrict__ fk, float* __restrict__ fv) {
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
-    p[v] = 0.f;
-    r[v] = r0;
+    p[v] = r0;
+    r[v] = 0.f;
     fk[v] = v;
+    fv[v] = share(r0, w[v]);
   }
 }
 
-__global__ void k_pr_take(const int* __restrict__ fk, int cnt, const float* __restrict__ w,
-                          float* __restrict__ p, float* __restrict__ r, float* __restrict__ xv) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x) {
-    const int u = fk[i];
-    const float ru = r[u];
-    p[u] += ru;
-    r[u] = 0.f;
-    const float wu = w[u];
-    xv[i] = wu > 0.f ? ru / wu : 0.f;
-  }
-}
-
-__global__ void k_pr_push(const int* __restrict__ yk, const float* __restrict__ yv,
-                          const Ctl* __restrict__ ctl, float d, float thr, float* __restrict__ r,
-                          unsigned* __restrict__ bits) {
+// r[v] += d * y_v; the vertices over the threshold, in y's (ascending) order,
+// are the next active set: listed with their x value, their residual taken.
+// Tiles of kPrTile entries of y with decoupled look-back; the last one sends
+// the set's size to the host, which only queues further work on this stream.
+__global__ __launch_bounds__(kPrNT) void k_pr_push(const int* __restrict__ yk, const float* __restrict__ yv,
+                                                   Ctl* ctl, float d, float thr, const float* __restrict__ w,
+                                                   float* __restrict__ p, float* __restrict__ r,
+                                                   int* __restrict__ fk, float* __restrict__ fv,
+                                                   unsigned long long* state, Ep ep, long long* sig) {
+  __shared__ unsigned long long s_pre;
+  __shared__ int s_w[kPrNT / kWave];
   const int cnt = ctl->ynnz;  // y's keys are distinct: one writer per r[v]
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += gridDim.x * blockDim.x) {
-    const int v = yk[i];
-    const float nr = r[v] + d * yv[i];
-    r[v] = nr;
-    if (nr > thr) atomicOr(&bits[v >> 5], 1u << (v & 31));
+  const unsigned ntiles = (unsigned)((cnt + kPrTile - 1) / kPrTile);
+  const unsigned t = blockIdx.x;
+  if (t >= ntiles) {
+    if (ntiles == 0 && t == 0 && threadIdx.x == 0) *sig = 0;
+    return;
   }
+  const int wv = threadIdx.x / kWave;
+  const int i0 = (int)t * kPrTile + wv * kWave * kPrIPT + lane();
+  int v[kPrIPT];
+  float nr[kPrIPT], wt[kPrIPT];
+  // entries past the end repeat the last one and are not stored
+#pragma unroll
+  for (int j = 0; j < kPrIPT; ++j) {
+    const int i = min(i0 + j * kWave, cnt - 1);
+    v[j] = yk[i];
+    nr[j] = yv[i];
+  }
+#pragma unroll
+  for (int j = 0; j < kPrIPT; ++j) {
+    nr[j] = r[v[j]] + d * nr[j];
+    wt[j] = w[v[j]];
+  }
+  const uint64_t lt = lane() == 0 ? 0ull : (~0ull >> (kWave - lane()));
+  int rank[kPrIPT], mine = 0;
+  bool over[kPrIPT];
+#pragma unroll
+  for (int j = 0; j < kPrIPT; ++j) {
+    const bool in = i0 + j * kWave < cnt;
+    over[j] = in && nr[j] > thr;
+    const uint64_t bal = __ballot(over[j]);
+    rank[j] = mine + __popcll(bal & lt);
+    mine += __popcll(bal);
+    if (in) r[v[j]] = over[j] ? 0.f : nr[j];
+    if (over[j]) p[v[j]] += nr[j];
+  }
+  if (lane() == 0) s_w[wv] = mine;
+  __syncthreads();
+  int before = 0, tot = 0;
+#pragma unroll
+  for (int k = 0; k < kPrNT / kWave; ++k) {
+    before += k < wv ? s_w[k] : 0;
+    tot += s_w[k];
+  }
+  const long long pre = (long long)tile_prefix(state, t, ep_of(ctl, ep), (unsigned long long)tot, &s_pre);
+#pragma unroll
+  for (int j = 0; j < kPrIPT; ++j) {
+    if (over[j]) {
+      const long long o = pre + before + rank[j];
+      fk[o] = v[j];
+      fv[o] = share(nr[j], wt[j]);
+    }
+  }
+  if (t == ntiles - 1 && threadIdx.x == 0) *sig = pre + tot;
 }
 
 __global__ void k_pr_finish(int n, float* __restrict__ p, const float* __restrict__ r) {
@@ -101,7 +202,7 @@ namespace spmspv {
 int pr_alloc(spmspv_handle_t h) {
   if (h->pr) return SPMSPV_SUCCESS;
   auto* st = new PrState();
-  const size_t n = h->n, m = h->m, words = (n + 31) / 32 + 2;
+  const size_t n = h->n, m = h->m;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -109,8 +210,8 @@ int pr_alloc(spmspv_handle_t h) {
     return o;
   };
   const size_t ow = take(n * 4), orr = take(n * 4), of0 = take(n * 4), of1 = take(n * 4);
-  const size_t ov0 = take(n * 4), ov1 = take(n * 4), oxv = take(n * 4);
-  const size_t oyk = take(m * 4), oyv = take(m * 4), ob = take(words * 4);
+  const size_t ov0 = take(n * 4), ov1 = take(n * 4);
+  const size_t oyk = take(m * 4), oyv = take(m * 4);
   if (hipMalloc(&st->alloc, off) != hipSuccess) {
     delete st;
     return set_error(h, SPMSPV_OUT_OF_MEMORY, "pagerank buffers");
@@ -122,16 +223,8 @@ int pr_alloc(spmspv_handle_t h) {
   st->fk[1] = reinterpret_cast<int*>(p + of1);
   st->fv[0] = reinterpret_cast<float*>(p + ov0);
   st->fv[1] = reinterpret_cast<float*>(p + ov1);
-  st->xv = reinterpret_cast<float*>(p + oxv);
   st->yk = reinterpret_cast<int*>(p + oyk);
   st->yv = reinterpret_cast<float*>(p + oyv);
-  st->bits = reinterpret_cast<unsigned*>(p + ob);
-  launch_fill_i32(h->stream, reinterpret_cast<int*>(st->bits), (long long)words, 0);
-  if (hipStreamSynchronize(h->stream) != hipSuccess) {
-    (void)hipFree(st->alloc);
-    delete st;
-    return set_error(h, SPMSPV_DEVICE_ERROR, "pagerank init");
-  }
   h->pr = st;
   return SPMSPV_SUCCESS;
 }
@@ -173,31 +266,30 @@ int spmspv_pagerank(spmspv_handle_t h, float damping, float eps, int max_iter, i
     }
   } restore{h, saved_mode, saved_fixed};
   const auto t0 = std::chrono::steady_clock::now();
-  hipLaunchKernelGGL(k_col_weights, dim3(grid_of((long long)n * kWave)), dim3(256), 0, s, h->csc_colptr,
-                     h->csc_val, n, st->w);
+  hipLaunchKernelGGL(k_col_weights, dim3(grid_of((long long)n * 16)), dim3(256), 0, s, h->csc_colptr, h->csc_val, n,
+                     st->w);
+  if (h->nnz > kLongCol)
+    hipLaunchKernelGGL(k_long_col_weights<512>, dim3(509), dim3(512), 0, s, h->csc_colptr, h->csc_val, n, st->w);
   const float r0 = (1.f - damping) / (float)n;
   const float thr = eps * r0;
-  hipLaunchKernelGGL(k_pr_init, dim3(grid_of(n)), dim3(256), 0, s, n, r0, d_rank, st->r, st->fk[0]);
+  hipLaunchKernelGGL(k_pr_init, dim3(grid_of(n)), dim3(256), 0, s, n, r0, st->w, d_rank, st->r, st->fk[0], st->fv[0]);
   HIP_TRY(h, hipGetLastError());
   int cur = 0, cnt = n, it = 0;
   double pushes = 0.0;
   while (cnt > 0 && it < max_iter) {
     if (sizes) sizes[it] = cnt;
     pushes += cnt;
-    hipLaunchKernelGGL(k_pr_take, dim3(grid_of(cnt)), dim3(256), 0, s, st->fk[cur], cnt, st->w, d_rank,
-                       st->r, st->xv);
+    if ((rc = spmspv_set_sparse_x(h, st->fk[cur], st->fv[cur], cnt))) return rc;
+    int used = -1;
+    if ((rc = spmspv_run_auto(h, 1.f, nullptr, st->yk, st->yv, nullptr, &used))) return rc;
+    __atomic_store_n(h->sig + 3, kSigPending, __ATOMIC_RELEASE);
+    hipLaunchKernelGGL(k_pr_push, dim3((unsigned)((h->m + kPrTile - 1) / kPrTile)), dim3(kPrNT), 0, s, st->yk, st->yv,
+                       h->ctl, damping, thr, st->w, d_rank, st->r, st->fk[cur ^ 1], st->fv[cur ^ 1], h->scan_state,
+                       next_ep(h, 1), h->sig_dev + 3);
     HIP_TRY(h, hipGetLastError());
-    if ((rc = spmspv_set_sparse_x(h, st->fk[cur], st->xv, cnt))) return rc;
-    int ynnz = 0, used = -1;
-    if ((rc = spmspv_run_auto(h, 1.f, nullptr, st->yk, st->yv, &ynnz, &used))) return rc;
-    // the residual update and the threshold test, then the crossing
-    // vertices as the next sorted active set (the compaction clears the bits)
-    hipLaunchKernelGGL(k_pr_push, dim3(grid_of(ynnz)), dim3(256), 0, s, st->yk, st->yv, h->ctl, damping,
-                       thr, st->r, st->bits);
-    launch_compact(s, st->bits, nullptr, n, st->r, 0, st->fk[cur ^ 1], st->fv[cur ^ 1], h->scan_state,
-                   h->ctl, next_ep(h, 1));
-    HIP_TRY(h, hipGetLastError());
-    if ((rc = readback_ynnz(h, &cnt))) return rc;
+    long long next = 0;
+    if ((rc = wait_signal(h, 3, &next))) return rc;
+    cnt = (int)next;
     cur ^= 1;
     ++it;
   }
