@@ -97,9 +97,11 @@ static size_t carve(spmspv_handle_t h, char* base) {
   int* split = c.take<int>(lb_tiles);
   int* tls = c.take<int>(lb_tiles);
   int* tmm = c.take<int>(2 * prep_tiles);
-  const size_t bucket_tiles = m / 8192 + 258;
-  unsigned long long* ss =
-      c.take<unsigned long long>(std::max(std::max(prep_tiles, cmp_tiles), bucket_tiles));
+  // look-back words of one launch: scan tiles, compaction tiles, or the
+  // small-x path's workgroups (at least 8,192 rows each, or 512 of them)
+  const size_t fused_groups = m / 8192 + 514;
+  const size_t look_words = std::max(std::max(prep_tiles, cmp_tiles), fused_groups);
+  unsigned long long* ss = c.take<unsigned long long>(look_words);
   float* acc = c.take<float>(m);
   unsigned* bm = c.take<unsigned>(mwords + 2);
   unsigned char* mk = c.take<unsigned char>(mwords * 32 + 64);
@@ -141,7 +143,7 @@ static size_t carve(spmspv_handle_t h, char* base) {
     h->prep_samp = psamp;
     h->bin_ws = bws;
     h->bin_base_bits = -1;
-    h->scan_words = std::max(std::max(prep_tiles, cmp_tiles), bucket_tiles);
+    h->scan_words = look_words;
     h->sort_words = dscan_tiles;
     h->red_words = red_tiles;
     h->ctl = ctl;
@@ -476,7 +478,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
   } gate_restore{h};
   if (kid >= SPMSPV_K_COL_NAIVE_ATOMIC && kid <= SPMSPV_K_COL_LB_SORT && !h->gate.word && !y_dense &&
       h->small_x_path && h->fuse_cap > 0 && h->vec_type != SPMSPV_VEC_DENSE && h->sparse_valid &&
-      h->xnnz <= kFuseKeys &&
+      h->xnnz <= kFuseKeys && m <= kFuseRowsMax &&
       h->binlen_host <= h->fuse_cap) {  // (binlen_host -1: not known yet)
     if ((rc = need_csc(h))) return rc;
     if (h->count_to_host) mark_sig3();
@@ -485,7 +487,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
     const SelectorArgs fixed{nullptr, nullptr, 2, kid, wait ? h->sig_dev + 1 : nullptr, 0};
     launch_col_fused(s, h->csc_colptr, h->csc_row, h->csc_val, h->x_key, h->x_val, h->n, h->xnnz, m, h->ptr,
                      h->xbeg, h->split, h->ctl, fixed, y_key ? y_key : h->yk_tmp, y_val ? y_val : h->yv_tmp,
-                     h->count_to_host ? h->sig_dev + 3 : nullptr, h->fuse_cap);
+                     h->count_to_host ? h->sig_dev + 3 : nullptr, h->fuse_cap, h->scan_state, next_ep(h, 1));
     h->launches++;
     if ((rc = check_launch(h, "small-x column path"))) return rc;
     h->prep_valid = true;
@@ -1396,12 +1398,13 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   // this size class fitted, nothing is queued behind it
   // (a selector pinned to a row slot keeps it: the path computes a column slot's result)
   const bool fused = h->small_x_path && h->fuse_cap > 0 && !d_y_dense && h->xnnz <= kFuseKeys &&
+                     h->m <= kFuseRowsMax &&
                      !(h->sel_mode == 2 && (h->sel_fixed < 0 || h->sel_fixed > SPMSPV_K_COL_LB_SORT));
   const bool spec = h->speculate && guess >= 0 && speculable(h, guess) && !(fused && h->spec_fused[cls]);
   if (fused) {
     launch_col_fused(h->stream, h->csc_colptr, h->csc_row, h->csc_val, h->x_key, h->x_val, h->n, h->xnnz, h->m,
                      h->ptr, h->xbeg, h->split, h->ctl, sel, d_y_key ? d_y_key : h->yk_tmp,
-                     d_y_val ? d_y_val : h->yv_tmp, nullptr, h->fuse_cap);
+                     d_y_val ? d_y_val : h->yv_tmp, nullptr, h->fuse_cap, h->scan_state, next_ep(h, 1));
     h->launches++;
     if ((rc = check_launch(h, "small-x column path"))) return rc;
     h->prep_valid = true;

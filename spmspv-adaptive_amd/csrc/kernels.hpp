@@ -165,22 +165,23 @@ void launch_set_bits(hipStream_t s, const int* key, int nnz, const int* nnz_dev,
                      unsigned* bits);
 void launch_clear_keys(hipStream_t s, const int* key, int nnz, float* dense, unsigned* bits);
 
-// Single-launch small-x column path: x of at most kFuseKeys keys whose
-// products (bin_len) fit kFuseCap run scan, gather, LDS sort, reduce and
-// the sorted output in one workgroup (k_col_fused, sort.hip). It also
+// Single-launch small-x column path (smallx.hip): x of at most kFuseKeys keys
+// whose products (bin_len) fit kFuseCap, on at most kFuseRowsMax rows. It also
 // writes the column scan (ptr, xbeg, split, ctl) like launch_prep, so a
 // call that does not fit goes on with the usual launches (gated on
 // ctl->kernel_choice, which gets kSelDone when the launch finished the
 // call). In auto mode (sel.mode != 2) a call that fits is reported as
 // kFusedSlot, the sort-based slot whose result it computes. Returns false
-// (nothing launched) when xnnz > kFuseKeys.
+// (nothing launched) when xnnz or m is larger.
 constexpr int kFuseNT = 1024, kFuseKeys = 4096, kFuseCap = kFuseNT * 11;
+constexpr int kFuseRowsMax = 1 << 26;  // 512 workgroups of kFuseRows: two rounds of one per CU
 constexpr int kFusedSlot = 1;  // SPMSPV_K_COL_NAIVE_SORT
 // cap (<= kFuseCap): largest bin_len that takes the single launch (the
-// autotuner may lower it).
+// autotuner may lower it). state: a look-back word per workgroup.
 bool launch_col_fused(hipStream_t s, const int* colptr, const int* crow, const float* cval, const int* xkey,
                       const float* xval, int ncols, int xnnz, int m, int* ptr, int* xbeg, int* split, Ctl* ctl,
-                      const SelectorArgs& sel, int* ykey, float* yval, long long* count_sig, int cap);
+                      const SelectorArgs& sel, int* ykey, float* yval, long long* count_sig, int cap,
+                      unsigned long long* state, Ep ep);
 
 // --- sort path -----------------------------------------------------------
 // Sorts (bkey, bval)[bin_len] by key (< m) with an LSD radix sort

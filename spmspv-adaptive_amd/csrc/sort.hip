@@ -64,9 +64,7 @@ __device__ __forceinline__ V block_seg_excl(bool f, V v, int* s_f, V* s_v, V* la
 // (called by all threads with the tile's head count) returns the number of
 // heads of all earlier tiles. Segment ends whose head lies in an earlier
 // tile go to carry_val/carry_idx[tile] for the fix-up kernel.
-// With COHERENT the outputs go out as device-coherent stores (visible to
-// every XCD and to copies once acknowledged, no L2 write-back needed).
-template <int NT, int IPT, typename PrefixFn, bool COHERENT = false>
+template <int NT, int IPT, typename PrefixFn>
 __device__ __forceinline__ long long tile_reduce(const unsigned* s_k, const float* s_v, int cnt,
                                                  unsigned prev_key, bool global_start,
                                                  PrefixFn get_prefix, int* ykey, float* yval,
@@ -103,20 +101,14 @@ __device__ __forceinline__ long long tile_reduce(const unsigned* s_k, const floa
     if (head[j]) {
       ++hc;
       acc = s_v[i];
-      if (COHERENT)
-        __hip_atomic_store(ykey + gpre + hc - 1, (int)s_k[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      else
-        ykey[gpre + hc - 1] = (int)s_k[i];
+      ykey[gpre + hc - 1] = (int)s_k[i];
     } else {
       acc += s_v[i];
     }
     const bool end = (i == cnt - 1) || (s_k[i + 1] != s_k[i]);
     if (end) {
       if (hc > 0) {
-        if (COHERENT)
-          __hip_atomic_store(yval + gpre + hc - 1, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else
-          yval[gpre + hc - 1] = acc;
+        yval[gpre + hc - 1] = acc;
       } else {
         carry_val[tile] = acc;
         carry_idx[tile] = (int)(gpre - 1);
@@ -570,270 +562,6 @@ void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* 
   const int fgrid = std::min(2048, std::max(1, tiles_grid(binlen_hint, n_cap, kRedTile) / 256 + 1));
   hipLaunchKernelGGL(k_carry_fixup, dim3(fgrid), dim3(256), 0, s, b.carry_val, b.carry_idx, n_dev,
                      kRedTile, small_cap, yval, g);
-}
-
-// ------------------------------------------------ single-launch small x
-// A column SpMSpV whose x has at most kFuseKeys keys and whose products fit
-// one workgroup's LDS runs in one launch of one workgroup: the column
-// scan of x (as k_prep's single tile, including the merge-path splits, so a
-// call that does not fit continues with the usual launches), then, when
-// bin_len <= kFuseCap and sparse outputs are given, the gather of every
-// product (row, a*x) in x order, a stable LDS radix sort by row, the
-// in-order reduce and the sorted output with its count. The result is the
-// sort-based slots' (the same products, the same order). In auto mode a
-// call that fits skips the network (a size rule in front of it: no slot
-// reads less than the products of x); one that does not fit runs the
-// selector as k_prep does. When it finishes the call it sets the done flag
-// in ctl->kernel_choice (which shuts every gated launch queued behind it),
-// writes the count to ctl->ynnz, then to *count_sig and the selector word
-// (flagged kSelDone, count in the bin_len field) once the outputs are
-// complete.
-// One workgroup of 1,024 threads (four waves per SIMD, so that each wave's
-// LDS and memory waits overlap three others'); KPT keys and IPT products per
-// thread.
-template <int NT, int KPT, int IPT>
-__global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr, const int* __restrict__ crow,
-                                                  const float* __restrict__ cval, const int* __restrict__ xkey,
-                                                  const float* __restrict__ xval, int ncols, int xnnz, int passes,
-                                                  int* __restrict__ ptr, int* __restrict__ xbeg,
-                                                  int* __restrict__ split, Ctl* ctl, SelectorArgs sel,
-                                                  int* __restrict__ ykey, float* __restrict__ yval,
-                                                  long long* count_sig, int cap) {
-  static_assert(NT >= 256 && NT % 256 == 0, "a thread per radix digit");
-  constexpr int NW = NT / kWave, CAP = NT * IPT, KEYS = NT * KPT;
-  constexpr int kRawBytes = CAP * 8 > kNWeights * 4 ? CAP * 8 : kNWeights * 4;
-  // the sort's keys and values, or the selector's weights (never both);
-  // before the sort, the keys' space holds the product -> x entry map
-  __shared__ __align__(16) unsigned char s_raw[kRawBytes];
-  __shared__ int s_ptr[KEYS + 1];
-  __shared__ int s_beg[KEYS];
-  __shared__ unsigned s_cnt[NW * 256];
-  __shared__ unsigned s_dstart[256];
-  __shared__ unsigned s_t[NW];
-  __shared__ long long s_l[NW];
-  __shared__ int s_i[NW];
-  __shared__ int s_f[NW];
-  __shared__ float s_fv[NW];
-  __shared__ MatFeat s_mf;
-  unsigned* s_k = reinterpret_cast<unsigned*>(s_raw);
-  float* s_v = reinterpret_cast<float*>(s_raw + CAP * 4);
-  float* s_w = reinterpret_cast<float*>(s_raw);
-  int* s_seg = reinterpret_cast<int*>(s_raw);
-  // the selector's weights and matrix features, loaded beside the column
-  // scan (stored to LDS only when the products do not fit, after the scan:
-  // their LDS space is the sort's)
-  constexpr int kWPT = (kNWeights + NT - 1) / NT;
-  constexpr int kMF = sizeof(MatFeat) / sizeof(double);
-  float wr[kWPT];
-  double mfr = 0.0;
-  if (sel.mode != 2 && sel.mat) {
-    if (sel.weights) {
-#pragma unroll
-      for (int i = 0; i < kWPT; ++i) {
-        const int idx = threadIdx.x + i * NT;
-        wr[i] = idx < kNWeights ? sel.weights[idx] : 0.f;
-      }
-    }
-    if (threadIdx.x < kMF) mfr = reinterpret_cast<const double*>(sel.mat)[threadIdx.x];
-  }
-  // ---- column scan of x
-  const int base = threadIdx.x * KPT;
-  int c[KPT], beg[KPT], len[KPT];
-#pragma unroll
-  for (int j = 0; j < KPT; ++j) c[j] = xnnz > 0 ? xkey[base + j < xnnz ? base + j : xnnz - 1] : 0;
-#pragma unroll
-  for (int j = 0; j < KPT; ++j) {
-    const int ok = (base + j < xnnz && (unsigned)c[j] < (unsigned)ncols) ? 1 : 0;
-    const int ci = c[j] & -ok;
-    beg[j] = colptr[ci];
-    len[j] = colptr[ci + ok];
-    c[j] = ok;
-  }
-  long long tsum = 0;
-  int mx = 0, mn = INT_MAX;
-#pragma unroll
-  for (int j = 0; j < KPT; ++j) {
-    len[j] = c[j] ? len[j] - beg[j] : 0;
-    beg[j] = c[j] ? beg[j] : 0;
-    if (c[j]) {
-      mx = max(mx, len[j]);
-      mn = min(mn, len[j]);
-    }
-    tsum += len[j];
-  }
-  mx = block_max<NT, int>(mx, s_i);
-  mn = block_min<NT, int>(mn, s_i);
-  long long bl;
-  long long run = block_excl_sum<NT, long long>(tsum, s_l, &bl);
-#pragma unroll
-  for (int j = 0; j < KPT; ++j) {
-    const int i = base + j;
-    if (i < xnnz) {
-      ptr[i] = (int)run;
-      xbeg[i] = beg[j];
-      s_ptr[i] = (int)run;
-      s_beg[i] = beg[j];
-      if (split) {
-        const long long Mi = i + run;
-        const long long Mn = Mi + len[j] + 1;
-        for (long long d = (Mi / kLbTile + 1) * kLbTile; d <= Mn; d += kLbTile) split[d / kLbTile] = i + 1;
-      }
-      run += len[j];
-    }
-  }
-  if (threadIdx.x == 0) {
-    ptr[xnnz] = (int)bl;
-    s_ptr[xnnz] = (int)bl;
-    ctl->bin_len = bl;
-    ctl->max_len = xnnz > 0 ? mx : 0;
-    ctl->min_len = mn;
-    ctl->xnnz = xnnz;
-    const long long nt = ((long long)xnnz + bl + kLbTile - 1) / kLbTile;
-    ctl->n_tiles = nt;
-    if (split) {
-      split[0] = 0;
-      split[nt] = xnnz;
-    }
-  }
-  const bool fuse = bl <= CAP && bl <= cap && ykey != nullptr && yval != nullptr;
-  if (!fuse) {
-    if (sel.mode == 2 || !sel.mat) {
-      // a fixed slot (or no selector): the gated launches behind run
-      if (threadIdx.x == 0) {
-        if (sel.mode == 2) ctl->kernel_choice = sel.fixed;
-        if (sel.stash) *sel.stash = sel_word(bl, sel.mode == 2 ? sel.fixed : -1);
-      }
-      return;
-    }
-    // the selector, as the last tile of k_prep runs it
-    {
-      if (sel.weights) {
-#pragma unroll
-        for (int i = 0; i < kWPT; ++i) {
-          const int idx = threadIdx.x + i * NT;
-          if (idx < kNWeights) s_w[wlds_index(idx)] = wr[i];
-        }
-      }
-      if (threadIdx.x < kMF) reinterpret_cast<double*>(&s_mf)[threadIdx.x] = mfr;
-      __syncthreads();
-      SelectorArgs sl = sel;
-      if (sel.weights) sl.weights = s_w;
-      sl.mat = &s_mf;
-      select_in_wave(ctl, sl, (double)xnnz, (double)bl, (double)(xnnz > 0 ? mx : 0));
-    }
-    if (sel.stash && threadIdx.x == 0) *sel.stash = sel_word(bl, ctl->kernel_choice);
-    return;
-  }
-  __syncthreads();  // s_ptr / s_beg complete
-  // products per thread for this call (<= IPT): every wave gets its share,
-  // so that the ranking's per-slot round trips run on all the waves at once
-  // instead of IPT of them in a row on the first few
-  const int ie = (int)((bl + NT - 1) / NT);
-  // ---- product -> x entry map, merge-path style: thread t fills products
-  // t*ie .. t*ie+ie-1 from one search and a forward walk (x entries with
-  // empty columns are stepped over)
-  {
-    const int p0 = threadIdx.x * ie;
-    if (p0 < bl) {
-      int lo = 0, hi = xnnz;  // s_ptr[lo] <= p0 < s_ptr[hi]
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (s_ptr[mid] <= p0) lo = mid;
-        else hi = mid;
-      }
-      int e = lo, nxt = s_ptr[lo + 1];
-#pragma unroll
-      for (int k = 0; k < IPT; ++k) {
-        const int p = p0 + k;
-        if (k < ie && p < bl) {
-          while (nxt <= p) nxt = s_ptr[++e + 1];
-          s_seg[p] = e;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  // ---- products into registers, in x order (wave-major items as wave_rank takes them)
-  const int w = threadIdx.x / kWave;
-  unsigned key[IPT];
-  float val[IPT];
-  bool valid[IPT];
-  int rank[IPT];
-  unsigned dig[IPT];
-  int pos[IPT];
-  float xv[IPT];
-#pragma unroll
-  for (int j = 0; j < IPT; ++j) {
-    const int p = w * kWave * ie + j * kWave + lane();
-    valid[j] = j < ie && p < bl;
-    const int e = valid[j] ? s_seg[p] : 0;
-    pos[j] = valid[j] ? s_beg[e] + (p - s_ptr[e]) : 0;
-    xv[j] = valid[j] ? xval[e] : 0.f;
-  }
-#pragma unroll
-  for (int j = 0; j < IPT; ++j) {
-    key[j] = valid[j] ? (unsigned)crow[pos[j]] : 0u;
-    val[j] = valid[j] ? cval[pos[j]] * xv[j] : 0.f;
-  }
-  __syncthreads();  // every map entry read before the sort reuses the space
-  // ---- LDS radix sort (stable), as k_sort_small; the digit offsets by
-  // threads 0..255 (one per digit)
-  for (int pss = 0; pss < passes; ++pss) {
-    wave_rank<IPT>(key, valid, 8 * pss, s_cnt + w * 256, rank, dig, ie);
-    __syncthreads();
-    unsigned tot = 0;
-    if (threadIdx.x < 256) tot = digit_wave_offsets<NW>(s_cnt);
-    unsigned dtot;
-    const unsigned dex = block_excl_sum<NT, unsigned>(tot, s_t, &dtot);
-    if (threadIdx.x < 256) s_dstart[threadIdx.x] = dex;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {
-      if (valid[j]) {
-        const unsigned q = s_dstart[dig[j]] + s_cnt[w * 256 + dig[j]] + rank[j];
-        s_k[q] = key[j];
-        s_v[q] = val[j];
-      }
-    }
-    __syncthreads();
-    if (pss + 1 < passes) {
-#pragma unroll
-      for (int j = 0; j < IPT; ++j) {
-        const int gi = w * kWave * ie + j * kWave + lane();
-        if (valid[j]) {
-          key[j] = s_k[gi];
-          val[j] = s_v[gi];
-        }
-      }
-      __syncthreads();
-    }
-  }
-  auto no_prefix = [](int) -> long long { return 0; };
-  const long long tot = tile_reduce<NT, IPT, decltype(no_prefix), true>(s_k, s_v, (int)bl, 0u, true, no_prefix, ykey, yval, nullptr,
-                                             nullptr, 0, s_i, s_f, s_fv, ie);
-  // ---- publish: outputs complete, then the count and the done flag
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int choice = sel.mode == 2 ? sel.fixed : kFusedSlot;
-    ctl->ynnz = (int)tot;
-    ctl->sort_small = 1;
-    ctl->kernel_choice = choice | kSelDone;
-    // the outputs are device-coherent and acknowledged (the wait above, in
-    // every thread, before the barrier): no L2 write-back before the words
-    if (count_sig) *count_sig = tot;
-    if (sel.stash) *sel.stash = sel_word(tot, choice | kSelDone);
-  }
-}
-
-bool launch_col_fused(hipStream_t s, const int* colptr, const int* crow, const float* cval, const int* xkey,
-                      const float* xval, int ncols, int xnnz, int m, int* ptr, int* xbeg, int* split, Ctl* ctl,
-                      const SelectorArgs& sel, int* ykey, float* yval, long long* count_sig, int cap) {
-  if (xnnz > kFuseKeys) return false;
-  hipLaunchKernelGGL((k_col_fused<kFuseNT, kFuseKeys / kFuseNT, kFuseCap / kFuseNT>), dim3(1), dim3(kFuseNT), 0, s,
-                     colptr, crow, cval, xkey, xval, ncols, xnnz, key_passes(m), ptr, xbeg, split, ctl, sel, ykey,
-                     yval, count_sig, cap);
-  return true;
 }
 
 }  // namespace spmspv
