@@ -434,6 +434,19 @@ int run_prep(spmspv_handle_t h, bool with_split, const SelectorArgs* sel) {
   return SPMSPV_SUCCESS;
 }
 
+bool needs_scan(int kid) {
+  return kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_ATOMIC ||
+         kid == SPMSPV_K_COL_LB_SORT || kid == SPMSPV_K_COL_BUCKET;
+}
+
+// A column slot on the current x takes the single-launch small-x path (with
+// binlen_host known: and finishes in it).
+bool takes_small_path(spmspv_handle_t h, int kid) {
+  return kid >= SPMSPV_K_COL_NAIVE_ATOMIC && kid <= SPMSPV_K_COL_LB_SORT && h->small_x_path && h->fuse_cap > 0 &&
+         h->vec_type != SPMSPV_VEC_DENSE && h->sparse_valid && h->xnnz <= kFuseKeys && h->m <= kFuseRowsMax &&
+         h->binlen_host <= h->fuse_cap;  // (binlen_host -1: not known yet)
+}
+
 static long long lb_tiles_hint(spmspv_handle_t h) {
   // tiles of the merged (x entries + products) sequence; bin_len <= nnz
   const long long bl = h->binlen_host >= 0 ? h->binlen_host : -1;
@@ -476,10 +489,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       if (on) h->gate = Gate{};
     }
   } gate_restore{h};
-  if (kid >= SPMSPV_K_COL_NAIVE_ATOMIC && kid <= SPMSPV_K_COL_LB_SORT && !h->gate.word && !y_dense &&
-      h->small_x_path && h->fuse_cap > 0 && h->vec_type != SPMSPV_VEC_DENSE && h->sparse_valid &&
-      h->xnnz <= kFuseKeys && m <= kFuseRowsMax &&
-      h->binlen_host <= h->fuse_cap) {  // (binlen_host -1: not known yet)
+  if (!h->gate.word && !y_dense && takes_small_path(h, kid)) {
     if ((rc = need_csc(h))) return rc;
     if (h->count_to_host) mark_sig3();
     const bool wait = h->count_to_host;
@@ -500,8 +510,9 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
         return SPMSPV_SUCCESS;
       }
       h->binlen_host = sel_word_binlen(word);
+    } else if (h->binlen_host >= 0) {
+      return SPMSPV_SUCCESS;  // the products are known to fit: that launch finishes the call
     } else {
-      h->binlen_host = -1;
       h->gate = Gate{&h->ctl->kernel_choice, kid};
       gate_restore.on = true;
     }
@@ -758,7 +769,7 @@ int spmspv_destroy(spmspv_handle_t h) {
   if (h->arena) (void)hipFree(h->arena);
   if (h->csc_alloc) (void)hipFree(h->csc_alloc);
   if (h->flush_buf) (void)hipFree(h->flush_buf);
-  if (h->batch_stash) (void)hipFree(h->batch_stash);
+  batch_release(h);
   if (h->csr5_mem) (void)hipFree(h->csr5_mem);
   if (h->h_pin) (void)hipHostFree(h->h_pin);
   if (h->sig) (void)hipHostFree(h->sig);
@@ -867,8 +878,8 @@ int spmspv_alloc_pre_buffer(spmspv_handle_t h) {
   int rc = ensure_arena(h);
   if (rc) return rc;
   // Everything a later call could allocate is reserved here: the CSR5 copy
-  // at its largest width, the BFS, multi-source BFS and PageRank buffers and a batch stash of
-  // kBatchReserve vectors.
+  // at its largest width, the BFS, multi-source BFS and PageRank buffers and a batch
+  // workspace of the usual size.
   if (h->csr_row) {
     size_t most = 0;
     for (int S = 1; S <= 32; ++S) most = std::max(most, csr5_bytes(h->m, h->n, h->nnz, S));
@@ -883,14 +894,7 @@ int spmspv_alloc_pre_buffer(spmspv_handle_t h) {
     }
   }
   if (h->m == h->n && ((rc = bfs_alloc(h)) || (rc = pr_alloc(h)) || (rc = ms_alloc(h)))) return rc;
-  if (h->batch_cap < spmspv_handle_s::kBatchReserve) {
-    HIP_TRY(h, hipStreamSynchronize(h->stream));
-    if (h->batch_stash) HIP_TRY(h, hipFree(h->batch_stash));
-    h->batch_stash = nullptr;
-    h->batch_cap = 0;
-    HIP_TRY(h, hipMalloc(&h->batch_stash, sizeof(long long) * spmspv_handle_s::kBatchReserve));
-    h->batch_cap = spmspv_handle_s::kBatchReserve;
-  }
+  if ((rc = batch_alloc(h))) return rc;
   if (h->csr_row && (rc = ensure_row_tiles(h))) return rc;
   if ((h->csr_row || h->csc_colptr) && (rc = ensure_mat_features(h))) return rc;
   HIP_TRY(h, hipStreamSynchronize(h->stream));
@@ -1359,12 +1363,6 @@ int spmspv_features(spmspv_handle_t h, float out[SPMSPV_NUM_FEATURES]) {
 // need nothing from the host about x are guessed: the atomic and sort column
 // slots (the sort then sizes its grids from the device-side bin_len), the
 // bucket slot and the load-balanced row slots.
-// slots whose launches read the column scan of x (ptr / xbeg / split)
-static bool needs_scan(int kid) {
-  return kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_ATOMIC ||
-         kid == SPMSPV_K_COL_LB_SORT || kid == SPMSPV_K_COL_BUCKET;
-}
-
 static bool speculable(spmspv_handle_t h, int kid) {
   if (kid == SPMSPV_K_COL_NAIVE_ATOMIC || kid == SPMSPV_K_COL_LB_ATOMIC ||
       kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_SORT)

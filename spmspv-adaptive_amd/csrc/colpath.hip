@@ -610,6 +610,160 @@ void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, i
                      ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp);
 }
 
+// ---------------------------------------------------------------- batch
+// Selector inputs and choice of every vector of a batch, a workgroup per tile
+// of kPrepTile keys: the workgroup of a vector that finishes last adds up the
+// vector's tiles (exact bin_len, longest column; sampled inputs for a large
+// x, as everywhere) and runs the selector. One launch per vector took 12 us
+// for each of them.
+template <int NT, int IPT>
+__global__ __launch_bounds__(NT) void k_batch_select(const int* __restrict__ colptr, const int* __restrict__ xkey,
+                                                     int ncols, const int* __restrict__ tile_vec,
+                                                     const BatchVec* __restrict__ vec, long long* tsum, int* tmax,
+                                                     unsigned* arrive, Ctl* ctls, SelectorArgs sel, long long* stash) {
+  __shared__ __align__(16) float s_w[kNWeights];
+  __shared__ MatFeat s_mf;
+  __shared__ Ctl s_ctl;
+  __shared__ long long s_l[NT / kWave];
+  __shared__ int s_i[NT / kWave];
+  __shared__ unsigned s_last;
+  const int t = blockIdx.x, v = tile_vec[t];
+  const BatchVec bv = vec[v];
+  const int* __restrict__ keys = xkey + bv.key0;
+  const int base = (t - bv.tile0) * (NT * IPT);
+  int c[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const int i = base + j * NT + (int)threadIdx.x;
+    c[j] = i < bv.xnnz ? keys[i] : -1;
+  }
+  long long sum = 0;
+  int mx = 0;
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const int ok = (unsigned)c[j] < (unsigned)ncols ? 1 : 0;
+    const int ci = c[j] & -ok;
+    const int len = colptr[ci + ok] - colptr[ci];
+    sum += len;
+    mx = max(mx, len);
+  }
+  sum = block_sum<NT, long long>(sum, s_l);
+  mx = block_max<NT, int>(mx, s_i);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(&tsum[t], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&tmax[t], mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // in place before the count
+    const unsigned before = __hip_atomic_fetch_add(&arrive[v], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = before == (unsigned)bv.ntiles - 1 ? 1u : 0u;
+    if (s_last) __hip_atomic_store(&arrive[v], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  if (!s_last) return;
+  if (sel.weights)
+    for (int i = threadIdx.x; i < kNWeights; i += NT) s_w[wlds_index(i)] = sel.weights[i];
+  constexpr int kMF = sizeof(MatFeat) / sizeof(double);
+  if (threadIdx.x < kMF)
+    reinterpret_cast<double*>(&s_mf)[threadIdx.x] = reinterpret_cast<const double*>(sel.mat)[threadIdx.x];
+  sum = 0;
+  mx = 0;
+  for (int u = threadIdx.x; u < bv.ntiles; u += NT) {
+    sum += __hip_atomic_load(&tsum[bv.tile0 + u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mx = max(mx, __hip_atomic_load(&tmax[bv.tile0 + u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+  sum = block_sum<NT, long long>(sum, s_l);
+  mx = block_max<NT, int>(mx, s_i);
+  long long fbl = sum;
+  int fmx = mx;
+  if (bv.xnnz > kSampleMin) sample_x<NT>(colptr, keys, ncols, bv.xnnz, s_l, s_i, &fbl, &fmx);
+  if (threadIdx.x == 0) {
+    Ctl* ctl = ctls + v;
+    ctl->bin_len = sum;
+    ctl->max_len = mx;
+    ctl->xnnz = bv.xnnz;
+    ctl->n_tiles = (bv.xnnz + sum + kLbTile - 1) / kLbTile;
+  }
+  SelectorArgs sl = sel;
+  if (sel.weights) sl.weights = s_w;
+  sl.mat = &s_mf;
+  select_in_wave(&s_ctl, sl, (double)bv.xnnz, (double)fbl, (double)fmx);
+  if (threadIdx.x == 0) stash[v] = sel_word(sum, s_ctl.kernel_choice);
+}
+
+// Column scan and merge-path splits of the listed tiles (as k_prep): a tile
+// starts at the sum of the tiles before it, which k_batch_select left.
+template <int NT, int IPT>
+__global__ __launch_bounds__(NT) void k_batch_scan(const int* __restrict__ colptr, const int* __restrict__ xkey,
+                                                   int ncols, const int* __restrict__ list,
+                                                   const int* __restrict__ tile_vec, const BatchVec* __restrict__ vec,
+                                                   const long long* __restrict__ tsum, int key_base,
+                                                   int* __restrict__ ptr_all, int* __restrict__ xbeg_all,
+                                                   int* __restrict__ split_all) {
+  __shared__ long long s_l[NT / kWave];
+  const int t = list[blockIdx.x], v = tile_vec[t];
+  const BatchVec bv = vec[v];
+  const int* __restrict__ keys = xkey + bv.key0;
+  int* __restrict__ ptr = ptr_all + (bv.key0 - key_base) + v;
+  int* __restrict__ xbeg = xbeg_all + (bv.key0 - key_base);
+  int* __restrict__ split = split_all + bv.split0;
+  const int base = (t - bv.tile0) * (NT * IPT) + (int)threadIdx.x * IPT;
+  int c[IPT], beg[IPT], len[IPT];
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) c[j] = base + j < bv.xnnz ? keys[base + j] : -1;
+  long long before = 0;
+  for (int u = bv.tile0 + (int)threadIdx.x; u < t; u += NT) before += tsum[u];
+  long long mine = 0;
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const int ok = (unsigned)c[j] < (unsigned)ncols ? 1 : 0;
+    const int ci = c[j] & -ok;
+    beg[j] = colptr[ci];
+    len[j] = colptr[ci + ok];
+    c[j] = ok;
+  }
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    len[j] = c[j] ? len[j] - beg[j] : 0;
+    beg[j] = c[j] ? beg[j] : 0;
+    mine += len[j];
+  }
+  const long long pre = block_sum<NT, long long>(before, s_l);
+  long long tot;
+  long long run = pre + block_excl_sum<NT, long long>(mine, s_l, &tot);
+#pragma unroll
+  for (int j = 0; j < IPT; ++j) {
+    const int i = base + j;
+    if (i < bv.xnnz) {
+      ptr[i] = (int)run;
+      xbeg[i] = beg[j];
+      const long long Mi = i + run;
+      const long long Mn = Mi + len[j] + 1;
+      for (long long d = (Mi / kLbTile + 1) * kLbTile; d <= Mn; d += kLbTile) split[d / kLbTile] = i + 1;
+      run += len[j];
+    }
+  }
+  if (t == bv.tile0 + bv.ntiles - 1 && threadIdx.x == 0) {
+    const long long bl = pre + tot;
+    ptr[bv.xnnz] = (int)bl;
+    split[0] = 0;
+    split[(bv.xnnz + bl + kLbTile - 1) / kLbTile] = bv.xnnz;
+  }
+}
+
+void launch_batch_select(hipStream_t s, const int* colptr, const int* xkey, int ncols, int ntiles, const int* tile_vec,
+                         const BatchVec* vec, long long* tsum, int* tmax, unsigned* arrive, Ctl* ctls,
+                         const SelectorArgs& sel, long long* stash) {
+  hipLaunchKernelGGL((k_batch_select<kPrepNT, kPrepIPT>), dim3(ntiles), dim3(kPrepNT), 0, s, colptr, xkey, ncols,
+                     tile_vec, vec, tsum, tmax, arrive, ctls, sel, stash);
+}
+
+void launch_batch_scan(hipStream_t s, const int* colptr, const int* xkey, int ncols, int nlist, const int* list,
+                       const int* tile_vec, const BatchVec* vec, const long long* tsum, int key_base, int* ptr,
+                       int* xbeg, int* split) {
+  if (nlist > 0)
+    hipLaunchKernelGGL((k_batch_scan<kPrepNT, kPrepIPT>), dim3(nlist), dim3(kPrepNT), 0, s, colptr, xkey, ncols, list,
+                       tile_vec, vec, tsum, key_base, ptr, xbeg, split);
+}
+
 // ------------------------------------------------------------- naive col
 // mode 0: atomics into acc + hit bitmap; mode 1: bins at ptr[e] + offset;
 // mode 2: row keys only at ptr[e] + offset (boolean: no value is read).

@@ -14,6 +14,7 @@
 struct BfsState;
 struct PrState;
 struct MsState;
+struct BatchState;
 
 struct spmspv_handle_s {
   int m = 0, n = 0, nnz = 0;
@@ -140,7 +141,7 @@ struct spmspv_handle_s {
   size_t csr5_bytes = 0;
   bool csr5_ready = false;
   spmspv::Csr5 csr5{};
-  long long* batch_stash = nullptr;  // selector word (sel_word) per vector of a batch
+  BatchState* batch = nullptr;       // workspace of run_batched
   // speculative dispatch (spmspv_run_auto): the gate launches carry while
   // the selector's choice is still on its way, and per x-size class
   // (log2 of xnnz) the last choice + 1 (0: none yet)
@@ -154,9 +155,6 @@ struct spmspv_handle_s {
   int fuse_cap = spmspv::kFuseCap;             // largest bin_len of that path (autotuned)
   int small_sort_cap = spmspv::kSmallSortCap;  // largest single-workgroup sort (autotuned)
   long long spec_hits = 0, spec_misses = 0;
-  int batch_cap = 0;
-  // batch stash reserved by alloc_pre_buffer; a larger batch grows it
-  static constexpr int kBatchReserve = 4096;
 
   float* dense_x() { return x_dense_user ? x_dense_user : x_dense_int; }
   unsigned* bits() { return bits_user ? bits_user : bits_int; }
@@ -195,9 +193,16 @@ void pr_release(spmspv_handle_t h);
 // Allocates / frees the multi-source BFS buffers (square matrices).
 int ms_alloc(spmspv_handle_t h);
 void ms_release(spmspv_handle_t h);
+// Allocates (for kBatchVecs vectors of at least kBatchKeys keys in all; a
+// larger batch grows it) / frees the workspace of run_batched.
+int batch_alloc(spmspv_handle_t h);
+void batch_release(spmspv_handle_t h);
 // Drops the captured BFS level graphs (they hold matrix and arena pointers).
 void bfs_drop_graphs(spmspv_handle_t h);
 int run_prep(spmspv_handle_t h, bool with_split, const SelectorArgs* sel);
+bool takes_small_path(spmspv_handle_t h, int kid);
+// slots whose launches read the column scan of x (ptr / xbeg / split)
+bool needs_scan(int kid);
 int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_val, bool want_nnz);
 int readback_ynnz(spmspv_handle_t h, int* y_nnz);
 // Waits for the device to write signal word idx (polls, then blocks on the

@@ -110,6 +110,25 @@ __host__ __device__ inline bool sel_word_estimated(long long w) {
 void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, int xnnz,
                  const int* xnnz_dev, int* ptr, int* xbeg, int* split, unsigned long long* state,
                  int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp = nullptr);
+// The vectors of a batch: one launch selects for all of them, one scans all
+// that need it. Vector v has keys xkey[key0 .. key0 + xnnz), tiles
+// [tile0, tile0 + ntiles) of kPrepTile keys (at least one) and, once its
+// slot is known, splits from split0.
+struct BatchVec {
+  int key0, xnnz, tile0, ntiles;
+  long long split0;
+};
+// Per vector: ctls[v].{bin_len, max_len, xnnz, n_tiles} and the selector word
+// (exact bin_len and choice) in stash[v]. tile_vec[t]: vector of tile t;
+// tsum / tmax: per tile; arrive[v]: 0 before and after.
+void launch_batch_select(hipStream_t s, const int* colptr, const int* xkey, int ncols, int ntiles, const int* tile_vec,
+                         const BatchVec* vec, long long* tsum, int* tmax, unsigned* arrive, Ctl* ctls,
+                         const SelectorArgs& sel, long long* stash);
+// ptr (at key0 - key_base + v), xbeg (at key0 - key_base) and split (at split0) as
+// launch_prep, for the tiles listed: list[i] = tile.
+void launch_batch_scan(hipStream_t s, const int* colptr, const int* xkey, int ncols, int nlist, const int* list,
+                       const int* tile_vec, const BatchVec* vec, const long long* tsum, int key_base, int* ptr,
+                       int* xbeg, int* split);
 // Features-only selector: ctl->{bin_len, max_len, min_len, xnnz} of x and,
 // with sel.mat set, the selector's choice (and the selector word in
 // sel.stash). part: 5 * kSelMaxGrid partials. No column scan. With enc set
