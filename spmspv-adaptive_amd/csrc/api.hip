@@ -514,6 +514,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       return SPMSPV_SUCCESS;  // the products are known to fit: that launch finishes the call
     } else {
       h->gate = Gate{&h->ctl->kernel_choice, kid};
+      h->spec_cap = h->nnz;
       gate_restore.on = true;
     }
   }
@@ -541,7 +542,15 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
     case SPMSPV_K_COL_LB_SORT: {
       if ((rc = need_csc(h)) || (rc = need_sparse_x(h))) return rc;
       const bool lb = kid == SPMSPV_K_COL_LB_SORT;
-      if (!h->prep_valid && (rc = run_prep(h, true, nullptr))) return rc;
+      // the scan sends bin_len to the host, which waits for it with the gather
+      // queued behind the scan (a copy and a stream wait after the gather
+      // left the device idle for a round trip)
+      const bool sent = !h->prep_valid && !h->gate.word;
+      if (!h->prep_valid) {
+        const SelectorArgs word{nullptr, nullptr, 0, 0, h->sig_dev + 1};
+        if (sent) __atomic_store_n(h->sig + 1, kSigPending, __ATOMIC_RELEASE);
+        if ((rc = run_prep(h, true, sent ? &word : nullptr))) return rc;
+      }
       int* bk = reinterpret_cast<int*>(h->sb.keyA);
       float* bv = h->sb.valA;
       if (lb)
@@ -555,11 +564,20 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       // queued before the selector's word arrives (speculation): every grid
       // is sized from the device-side count instead of the host's bin_len
       long long hint = -1;
+      if (sent) {
+        long long w = 0;
+        if ((rc = wait_signal(h, 1, &w))) return rc;
+        h->binlen_host = sel_word_binlen(w);
+      }
       if (!h->gate.word) {
         if ((rc = ensure_binlen_host(h))) return rc;
         hint = h->binlen_host;
       }
-      launch_sort_reduce(s, h->sb, m, h->ctl, ok, ov, hint, h->nnz, next_ep(h, 5), h->gate, h->small_sort_cap);
+      // a launch that covers nnz products costs its empty workgroups (7 us of
+      // 23 in the reduce at R-MAT s22, 1 %)
+      const long long most = h->gate.word ? h->spec_cap : h->nnz;
+      launch_sort_reduce(s, h->sb, m, h->ctl, ok, ov, hint, most, next_ep(h, 5), h->gate, h->small_sort_cap,
+                         hint > h->small_sort_cap && !y_dense ? count_sig() : nullptr);
       h->launches += 6;
       if (y_dense) {
         launch_fill_f32(s, y_dense, m, 0.f, h->gate);
@@ -1437,6 +1455,8 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
       ~Ungate() { h->gate = Gate{}; }
     } ungate{h};
     h->gate = Gate{&h->ctl->kernel_choice, guess};
+    h->spec_cap = h->nnz;
+    if (h->spec_binlen[cls] > 0) h->spec_cap = std::min<long long>(h->nnz, 4 * h->spec_binlen[cls] + 65536);
     h->count_to_host = y_nnz != nullptr;
     rc = run_kernel(h, guess, d_y_dense, d_y_key, d_y_val, y_nnz != nullptr);
     h->count_to_host = false;
@@ -1466,7 +1486,9 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   h->binlen_host = sel_word_estimated(word) ? -1 : sel_word_binlen(word);
   h->spec_last[cls] = (signed char)(kid + 1);
   if (kernel_used) *kernel_used = kid;
-  if (spec && kid == guess) {
+  if (h->binlen_host >= 0) h->spec_binlen[cls] = h->binlen_host;
+  const bool sorts = kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_SORT;
+  if (spec && kid == guess && !(sorts && h->binlen_host > h->spec_cap)) {
     h->spec_hits++;
     // the gated tile kernel ran, and with it the clearing of the idle buffer
     if (clear_pending >= 0) h->enc5_clean[clear_pending] = true;
@@ -1478,6 +1500,12 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
     return SPMSPV_SUCCESS;
   }
   if (spec) h->spec_misses++;
+  if (spec && kid == guess && y_nnz) {
+    // more products than the queued sort covers: its launches left the result
+    // alone, but the count of an earlier one is on its way to the host word
+    long long v = 0;
+    if ((rc = wait_signal(h, 3, &v))) return rc;
+  }
   return spmspv_run(h, kid, alpha, d_y_dense, d_y_key, d_y_val, y_nnz);
 }
 

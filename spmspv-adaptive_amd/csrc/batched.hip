@@ -13,7 +13,6 @@
 // launch, a scan and a count copy per vector (12, 10 and 4 us), 2,190 us so.
 // No reference counterpart (the reference runs one vector per call).
 #include <algorithm>
-#include <cstring>
 #include <vector>
 
 #include "handle.hpp"
@@ -21,21 +20,20 @@
 using namespace spmspv;
 
 // Workspace: the vectors' descriptors, control blocks, selector words and
-// tiles (sized by vectors and keys), and the scans' splits (known after the
-// selection). Grown when a batch needs more, freed with the handle.
+// tiles (sized by vectors and keys), with the scans' splits (known after the
+// selection) behind them where they fit, else in `split`. Grown when a batch
+// needs more, freed with the handle.
 struct BatchState {
   char* mem = nullptr;
   size_t bytes = 0;
   int* split = nullptr;
   size_t splits = 0;
-  char* host = nullptr;  // pinned: what is uploaded, and the words read back
-  size_t host_bytes = 0;
 };
 
 namespace {
 
 constexpr int kBatchVecs = 4096;
-constexpr size_t kBatchKeys = 1 << 22, kBatchSplits = 1 << 18;
+constexpr size_t kBatchKeys = 1 << 21, kBatchSplits = 1 << 18;
 
 __global__ void k_batch_counts(const Ctl* __restrict__ ctls, int nvec, int* __restrict__ ynnz) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -72,7 +70,7 @@ struct Layout {
 
 size_t tiles_of(size_t keys) { return std::max<size_t>(1, (keys + kPrepTile - 1) / kPrepTile); }
 
-int grow(spmspv_handle_t h, size_t bytes, size_t splits, size_t host_bytes) {
+int grow(spmspv_handle_t h, size_t bytes, size_t splits) {
   if (!h->batch) h->batch = new BatchState();
   BatchState* b = h->batch;
   if (b->bytes < bytes) {
@@ -91,36 +89,21 @@ int grow(spmspv_handle_t h, size_t bytes, size_t splits, size_t host_bytes) {
     HIP_TRY(h, hipMalloc((void**)&b->split, splits * sizeof(int)));
     b->splits = splits;
   }
-  if (b->host_bytes < host_bytes) {
-    HIP_TRY(h, hipStreamSynchronize(h->stream));
-    if (b->host) HIP_TRY(h, hipHostFree(b->host));
-    b->host = nullptr;
-    b->host_bytes = 0;
-    HIP_TRY(h, hipHostMalloc((void**)&b->host, host_bytes, hipHostMallocDefault));
-    b->host_bytes = host_bytes;
-  }
   return SPMSPV_SUCCESS;
-}
-
-// pinned bytes for a batch: offsets in, descriptors and tile lists out, words in
-size_t host_bytes_of(size_t nvec, size_t tiles) {
-  return up256((nvec + 1) * sizeof(int)) + up256((nvec + 1) * sizeof(long long)) + up256(nvec * sizeof(BatchVec)) +
-         up256(nvec * sizeof(long long)) + 2 * up256(tiles * sizeof(int));
 }
 
 }  // namespace
 
 namespace spmspv {
 int batch_alloc(spmspv_handle_t h) {
-  const size_t keys = std::max<size_t>(kBatchKeys, h->n), tiles = keys / kPrepTile + kBatchVecs + 1;
-  return grow(h, Layout(kBatchVecs, keys, tiles).bytes, kBatchSplits, host_bytes_of(kBatchVecs, tiles));
+  const size_t tiles = kBatchKeys / kPrepTile + kBatchVecs + 1;
+  return grow(h, Layout(kBatchVecs, kBatchKeys, tiles).bytes + kBatchSplits * sizeof(int), 0);
 }
 
 void batch_release(spmspv_handle_t h) {
   if (!h || !h->batch) return;
   if (h->batch->mem) (void)hipFree(h->batch->mem);
   if (h->batch->split) (void)hipFree(h->batch->split);
-  if (h->batch->host) (void)hipHostFree(h->batch->host);
   delete h->batch;
   h->batch = nullptr;
 }
@@ -138,18 +121,11 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
   int rc;
   if ((rc = ensure_arena(h)) || (rc = need_csc(h)) || (rc = ensure_mat_features(h))) return rc;
   hipStream_t s = h->stream;
-  if ((rc = grow(h, 0, 0, host_bytes_of(nvec, 1)))) return rc;
   std::vector<int> vptr(nvec + 1);
   std::vector<long long> yoff(nvec + 1);
-  {
-    char* in = h->batch->host;
-    char* in2 = in + up256((nvec + 1) * sizeof(int));
-    HIP_TRY(h, hipMemcpyAsync(in, d_vptr, sizeof(int) * (nvec + 1), hipMemcpyDeviceToHost, s));
-    HIP_TRY(h, hipMemcpyAsync(in2, d_yoff, sizeof(long long) * (nvec + 1), hipMemcpyDeviceToHost, s));
-    HIP_TRY(h, hipStreamSynchronize(s));
-    std::memcpy(vptr.data(), in, sizeof(int) * (nvec + 1));
-    std::memcpy(yoff.data(), in2, sizeof(long long) * (nvec + 1));
-  }
+  HIP_TRY(h, hipMemcpyAsync(vptr.data(), d_vptr, sizeof(int) * (nvec + 1), hipMemcpyDeviceToHost, s));
+  HIP_TRY(h, hipMemcpyAsync(yoff.data(), d_yoff, sizeof(long long) * (nvec + 1), hipMemcpyDeviceToHost, s));
+  HIP_TRY(h, hipStreamSynchronize(s));
   size_t tiles = 0;
   for (int v = 0; v < nvec; ++v) {
     const int xn = vptr[v + 1] - vptr[v];
@@ -163,7 +139,7 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
   }
   const size_t keys = (size_t)(vptr[nvec] - vptr[0]);
   const Layout at((size_t)nvec, keys, tiles);
-  if ((rc = grow(h, at.bytes, 0, host_bytes_of(nvec, tiles)))) return rc;
+  if ((rc = grow(h, at.bytes, 0))) return rc;
   BatchState* b = h->batch;
   auto* ctls = reinterpret_cast<Ctl*>(b->mem + at.ctls);
   auto* stash = reinterpret_cast<long long*>(b->mem + at.stash);
@@ -173,25 +149,20 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
   auto* tsum = reinterpret_cast<long long*>(b->mem + at.tsum);
   auto* ptr = reinterpret_cast<int*>(b->mem + at.ptr);
   auto* xbeg = reinterpret_cast<int*>(b->mem + at.xbeg);
-  char* hp = b->host;
-  auto* h_vec = reinterpret_cast<BatchVec*>(hp);
-  hp += up256(nvec * sizeof(BatchVec));
-  auto* st = reinterpret_cast<long long*>(hp);
-  hp += up256(nvec * sizeof(long long));
-  auto* h_tile_vec = reinterpret_cast<int*>(hp);
-  hp += up256(tiles * sizeof(int));
-  auto* h_list = reinterpret_cast<int*>(hp);
+  std::vector<BatchVec> h_vec(nvec);
+  std::vector<long long> st(nvec);
+  std::vector<int> h_tile_vec(tiles), h_list(tiles);
   // 1. selection (the arrival counts and control blocks start at zero)
   int tile = 0;
   for (int v = 0; v < nvec; ++v) {
     const int xn = vptr[v + 1] - vptr[v];
     const int nt = (int)tiles_of((size_t)xn);
     h_vec[v] = BatchVec{vptr[v], xn, tile, nt, 0};
-    std::fill(h_tile_vec + tile, h_tile_vec + tile + nt, v);
+    std::fill_n(h_tile_vec.begin() + tile, nt, v);
     tile += nt;
   }
-  HIP_TRY(h, hipMemcpyAsync(d_vec, h_vec, nvec * sizeof(BatchVec), hipMemcpyHostToDevice, s));
-  HIP_TRY(h, hipMemcpyAsync(d_tile_vec, h_tile_vec, tiles * sizeof(int), hipMemcpyHostToDevice, s));
+  HIP_TRY(h, hipMemcpyAsync(d_vec, h_vec.data(), nvec * sizeof(BatchVec), hipMemcpyHostToDevice, s));
+  HIP_TRY(h, hipMemcpyAsync(d_tile_vec, h_tile_vec.data(), tiles * sizeof(int), hipMemcpyHostToDevice, s));
   const SelectorArgs sel{h->have_weights ? h->weights_dev : nullptr, h->mat, h->sel_mode, h->sel_fixed,
                          nullptr, 0, -1, 0.f, h->bucket_lo, h->bucket_hi};
   launch_fill_i32(s, reinterpret_cast<int*>(b->mem), (long long)(at.zeroed / 4), 0);
@@ -200,7 +171,7 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
                       sel, stash);
   h->launches++;
   HIP_TRY(h, hipGetLastError());
-  HIP_TRY(h, hipMemcpyAsync(st, stash, sizeof(long long) * nvec, hipMemcpyDeviceToHost, s));
+  HIP_TRY(h, hipMemcpyAsync(st.data(), stash, sizeof(long long) * nvec, hipMemcpyDeviceToHost, s));
   HIP_TRY(h, hipStreamSynchronize(s));
   for (int v = 0; v < nvec; ++v) {
     const long long need = std::min<long long>(h->m, sel_word_binlen(st[v]));
@@ -235,12 +206,16 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
       for (int t = 0; t < h_vec[v].ntiles; ++t) h_list[nlist++] = h_vec[v].tile0 + t;
     }
   }
-  if ((rc = grow(h, 0, (size_t)splits, 0))) return rc;
+  int* split = reinterpret_cast<int*>(b->mem + at.bytes);
+  if (at.bytes + (size_t)splits * sizeof(int) > b->bytes) {
+    if ((rc = grow(h, 0, (size_t)splits))) return rc;
+    split = b->split;
+  }
   if (nlist > 0) {
-    HIP_TRY(h, hipMemcpyAsync(d_vec, h_vec, nvec * sizeof(BatchVec), hipMemcpyHostToDevice, s));
-    HIP_TRY(h, hipMemcpyAsync(d_list, h_list, nlist * sizeof(int), hipMemcpyHostToDevice, s));
+    HIP_TRY(h, hipMemcpyAsync(d_vec, h_vec.data(), nvec * sizeof(BatchVec), hipMemcpyHostToDevice, s));
+    HIP_TRY(h, hipMemcpyAsync(d_list, h_list.data(), nlist * sizeof(int), hipMemcpyHostToDevice, s));
     launch_batch_scan(s, h->csc_colptr, d_vkey, h->n, nlist, d_list, d_tile_vec, d_vec, tsum, vptr[0], ptr, xbeg,
-                      b->split);
+                      split);
     h->launches++;
     HIP_TRY(h, hipGetLastError());
   }
@@ -265,7 +240,7 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
       h->ctl = ctls + v;
       h->ptr = ptr + (vptr[v] - vptr[0]) + v;
       h->xbeg = xbeg + (vptr[v] - vptr[0]);
-      h->split = b->split + h_vec[v].split0;
+      h->split = split + h_vec[v].split0;
       h->prep_valid = scanned[v] != 0;
       if ((rc = run_kernel(h, kid, nullptr, d_ykey + yoff[v], d_yval + yoff[v], true))) return rc;
     }

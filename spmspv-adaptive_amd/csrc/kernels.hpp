@@ -224,12 +224,14 @@ struct SortSet {
   unsigned* w = nullptr;
 };
 // n_hint: item count when the host knows it (exact grids), else -1 and the
-// grids cover n_cap. ep: first of the 5 epochs the sort + reduce use.
+// grids cover n_cap; with more items than n_cap nothing is sorted. ep: first of the 5 epochs the sort + reduce use.
 // small_cap (<= kSmallSortCap): largest item count that takes the
-// single-workgroup path (the autotuner may lower it).
+// single-workgroup path (the autotuner may lower it). sig (only with
+// binlen_hint > small_cap): the result count goes there once the results are
+// visible.
 void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* ykey, float* yval,
                         long long binlen_hint, long long n_cap, Ep ep, Gate g = {},
-                        int small_cap = kSmallSortCap);
+                        int small_cap = kSmallSortCap, long long* sig = nullptr);
 // Sorts in[*n_dev] by key < range, stable, its passes writing out0 and out1 in
 // turn (`in` may be out1, and is not written otherwise); returns which of the
 // two holds the result. With ep.dev >= 0 (captured graphs) the passes use

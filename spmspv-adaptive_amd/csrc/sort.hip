@@ -151,7 +151,7 @@ template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__ kin,
                                                     const long long* __restrict__ n_dev, int shift, int bits,
                                                     unsigned* __restrict__ cnt, int small_cap,
-                                                    Gate g) {
+                                                    long long n_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__
   const unsigned mask = (1u << bits) - 1u;
   __shared__ unsigned s_cnt[NW * 256];
   const long long n = *n_dev;
-  if (n <= small_cap) return;
+  if (n <= small_cap || n > n_cap) return;
   const unsigned ntiles = (unsigned)((n + TILE - 1) / TILE);
   const int w = threadIdx.x / kWave;
   // tiles are independent: any grid covers them. Only counts are needed
@@ -200,13 +200,14 @@ __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__
 template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
                                                    const long long* __restrict__ n_dev, int sort_tile,
-                                                   int bits, int small_cap, unsigned long long* state, Ctl* ctl,
+                                                   int bits, int small_cap, long long n_cap,
+                                                   unsigned long long* state, Ctl* ctl,
                                                    Ep epa, Gate g) {
   if (gate_shut(g)) return;
   __shared__ unsigned long long s_pre;
   __shared__ unsigned s_t[NT / kWave];
   const long long n = *n_dev;
-  if (n <= small_cap) return;
+  if (n <= small_cap || n > n_cap) return;
   const long long E = ((n + sort_tile - 1) / sort_tile) << bits;
   const unsigned nb = (unsigned)((E + NT * IPT - 1) / (NT * IPT));
   const unsigned t = blockIdx.x;
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
 template <int NT, int IPT, int PAY>
 __global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, const long long* __restrict__ n_dev,
                                                      int shift, int bits, const unsigned* __restrict__ pos0,
-                                                     int small_cap, Gate g) {
+                                                     int small_cap, long long n_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, co
   __shared__ unsigned s_t[NW];
   const unsigned mask = (1u << bits) - 1u;
   const long long n = *n_dev;
-  if (n <= small_cap) return;
+  if (n <= small_cap || n > n_cap) return;
   const unsigned ntiles = (unsigned)((n + TILE - 1) / TILE);
   const int w = threadIdx.x / kWave;
   const unsigned d = threadIdx.x;
@@ -395,7 +396,7 @@ __global__ __launch_bounds__(NT) void k_reduce(const unsigned* __restrict__ keys
                                                const long long* __restrict__ n_dev, Ctl* ctl,
                                                int* ykey, float* yval, float* carry_val,
                                                int* carry_idx, unsigned long long* state, Ep epa,
-                                               int small_cap, Gate g) {
+                                               int small_cap, long long n_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
@@ -406,7 +407,7 @@ __global__ __launch_bounds__(NT) void k_reduce(const unsigned* __restrict__ keys
   __shared__ float s_fv[NW];
   __shared__ unsigned long long s_pre;
   const long long n = *n_dev;
-  if (n <= small_cap) return;
+  if (n <= small_cap || n > n_cap) return;
   const unsigned ntiles = (unsigned)((n + TILE - 1) / TILE);
   const unsigned t = blockIdx.x;
   if (t >= ntiles) return;
@@ -449,18 +450,32 @@ __global__ __launch_bounds__(NT) void k_reduce(const unsigned* __restrict__ keys
 }
 
 __global__ void k_carry_fixup(const float* __restrict__ carry_val, const int* __restrict__ carry_idx,
-                              const long long* __restrict__ n_dev, int tile, int small_cap,
-                              float* yval, Gate g) {
+                              const long long* __restrict__ n_dev, int tile, int small_cap, long long n_cap,
+                              float* yval, Ctl* ctl, long long* sig, Gate g) {
   if (gate_shut(g)) return;
   const long long n = *n_dev;
-  if (n <= small_cap) return;
+  if (n <= small_cap || n > n_cap) return;
   const long long ntiles = (n + tile - 1) / tile;
   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < ntiles;
        t += (long long)gridDim.x * blockDim.x) {
     int idx, h;
     float s;
     if (!carry_run<long long>(carry_val, carry_idx, nullptr, t, ntiles, idx, s, h)) continue;
-    yval[idx] += s;
+    __hip_atomic_store(yval + idx, yval[idx] + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (sig) {
+    // the results before this launch are visible to it; its own stores are
+    // device-coherent and acknowledged before the workgroup's arrival: the
+    // last one sends the count (as k_compact does)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned* arrived = &ctl->done[kSlotSort];
+      if (__hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+        __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *sig = ctl->ynnz;
+      }
+    }
   }
 }
 
@@ -489,12 +504,12 @@ static void launch_digit_pass(hipStream_t s, const SortBufs& b, const SortSet& i
   const int pgrid = std::min(tiles, 2048);  // count / scatter loop over their tiles
   const int sgrid = (int)std::max<long long>(1, (((long long)tiles << bits) + kDScanTile - 1) / kDScanTile);
   hipLaunchKernelGGL((k_digit_count<kSortNT, kSortIPT>), dim3(pgrid), dim3(kSortNT), 0, s, in.k, n_dev,
-                     shift, bits, b.dcount, small_cap, g);
+                     shift, bits, b.dcount, small_cap, n_cap, g);
   hipLaunchKernelGGL((k_digit_scan<kDScanNT, kDScanIPT>), dim3(sgrid), dim3(kDScanNT), 0, s, b.dcount,
-                     n_dev, kSortTile, bits, small_cap, b.dstate, ctl, e, g);
+                     n_dev, kSortTile, bits, small_cap, n_cap, b.dstate, ctl, e, g);
 #define SPMSPV_SCATTER(PAY)                                                                                  \
   hipLaunchKernelGGL((k_sort_scatter<kSortNT, kSortIPT, PAY>), dim3(pgrid), dim3(kSortNT), 0, s, in, out, n_dev, \
-                     shift, bits, b.dcount, small_cap, g)
+                     shift, bits, b.dcount, small_cap, n_cap, g)
   if (in.w) SPMSPV_SCATTER(2);
   else if (in.v) SPMSPV_SCATTER(1);
   else SPMSPV_SCATTER(0);
@@ -542,7 +557,7 @@ int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long lo
 }
 
 void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* ykey, float* yval,
-                        long long binlen_hint, long long n_cap, Ep ep, Gate g, int small_cap) {
+                        long long binlen_hint, long long n_cap, Ep ep, Gate g, int small_cap, long long* sig) {
   const long long* n_dev = &ctl->bin_len;
   const int passes = key_passes(m);
   const bool small_known = binlen_hint >= 0 && binlen_hint <= small_cap;
@@ -558,10 +573,10 @@ void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* 
   const Ep er{ep.v + 4u, ep.dev < 0 ? -1 : ep.dev + 4};
   hipLaunchKernelGGL((k_reduce<kRedNT, kRedIPT>), dim3(tiles_grid(binlen_hint, n_cap, kRedTile)),
                      dim3(kRedNT), 0, s, kf, vf, n_dev, ctl, ykey, yval, b.carry_val, b.carry_idx,
-                     b.red_state, er, small_cap, g);
+                     b.red_state, er, small_cap, n_cap, g);
   const int fgrid = std::min(2048, std::max(1, tiles_grid(binlen_hint, n_cap, kRedTile) / 256 + 1));
   hipLaunchKernelGGL(k_carry_fixup, dim3(fgrid), dim3(256), 0, s, b.carry_val, b.carry_idx, n_dev,
-                     kRedTile, small_cap, yval, g);
+                     kRedTile, small_cap, n_cap, yval, ctl, sig, g);
 }
 
 }  // namespace spmspv
