@@ -130,7 +130,8 @@ __device__ __forceinline__ RowTile row_tile(const int* __restrict__ split, int t
 // unconditional (clamped) so that a stage's loads issue back to back.
 // Rows that cross tiles leave their tail in carry_*[t] (row i1), which
 // k_row_fixup adds in tile order.
-template <int NT, int VT, int XIN, bool MASKED, bool HITS>
+// STREAM: columns and values are read past the caches (nontemporal).
+template <int NT, int VT, int XIN, bool MASKED, bool HITS, bool STREAM>
 __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_ptr,
                                                   const int* __restrict__ col,
                                                   const float* __restrict__ val,
@@ -175,8 +176,8 @@ __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_pt
     for (int i = 0; i < VT; ++i) {
       unsigned k = tid + i * NT;
       k = k < lim ? k : lim;
-      cN[i] = __builtin_nontemporal_load(ct + k);
-      vN[i] = __builtin_nontemporal_load(val + jb + k);
+      cN[i] = STREAM ? __builtin_nontemporal_load(ct + k) : ct[k];
+      vN[i] = STREAM ? __builtin_nontemporal_load(val + jb + k) : val[jb + k];
     }
   };
   auto gather = [&](int tt) {
@@ -361,11 +362,21 @@ void launch_row_merge(hipStream_t s, bool masked, bool hits, const int* row_ptr,
     launch_fill_f32(s, y, m, 0.f, g);
     return;
   }
+  // Columns and values of a matrix of at most 64 MB go through the caches (the
+  // 256 MB one keeps them for the next call); those of a larger one would
+  // push x out of them. Per call, cached against nontemporal, the same matrix
+  // each time / three in turn: banded 24 MB 14.5 / 15.7 us against 16.2 / 17.8,
+  // random 56 MB 46.6 / 50.6 against 51.2 / 55.5, R-MAT 30 MB 22.0 / 23.4 against
+  // 24.9 / 26.2; but R-MAT 124 MB 71 / 84.6 against 79 / 80.2 and random 169 MB
+  // 141 / 158 against 148 / 149.
+  const bool stream = (long long)nnz * 8 > (64ll << 20);
   // one resident wave of workgroups, each walking many tiles
 #define SPMSPV_ROW_MERGE(V, XI, MK, HT)                                                          \
   {                                                                                             \
-    const void* fn = (const void*)k_row_merge<kRowNT, V, XI, MK, HT>;                           \
-    hipLaunchKernelGGL((k_row_merge<kRowNT, V, XI, MK, HT>),                                    \
+    auto* kern = stream ? k_row_merge<kRowNT, V, XI, MK, HT, true>                              \
+                        : k_row_merge<kRowNT, V, XI, MK, HT, false>;                            \
+    const void* fn = (const void*)kern;                                                         \
+    hipLaunchKernelGGL(kern,                                                                    \
                        dim3(std::min(ntiles, resident_blocks(fn, kRowNT))), dim3(kRowNT), 0, s, \
                        row_ptr, col, val, x, m, nnz, split, ntiles, y, ybits, carry_val, \
                        carry_row, carry_hit, g);                                                \
