@@ -314,33 +314,43 @@ static float* enc5_for_scatter(spmspv_handle_t h) {
 // Support encoding of x in the CSR5 copy's column order (x_enc itself when
 // the copy keeps the columns' order).
 static int need_enc_x(spmspv_handle_t h);
-static int need_enc_x5(spmspv_handle_t h, const float** out) {
+static int need_enc_x5(spmspv_handle_t h, const float** out, bool values_only) {
   if (!h->csr5.cperm) {
     *out = h->x_enc;
     return need_enc_x(h);
   }
-  if (h->enc5_valid) {
+  if (h->enc5_valid >= (values_only ? h->kEnc5Values : h->kEnc5Support)) {
     *out = h->x_enc5b[h->enc5_cur];
     return SPMSPV_SUCCESS;
   }
+  int holds = h->kEnc5Support;
   if (h->sparse_valid) {
     float* e = enc5_for_scatter(h);
     launch_scatter(h->stream, h->x_key, h->x_val, h->xnnz, nullptr, h->n, e, true, Gate{},
                    h->csr5.cperm);
   } else {
     int rc;
-    if ((rc = need_dense_x(h)) || (rc = need_bits(h))) return rc;
+    if ((rc = need_dense_x(h))) return rc;
+    if (values_only && !h->bits_valid) {
+      // no bit array (4.8 us of 104 at R-MAT s20); the vector type is the one
+      // that building it leaves
+      holds = h->kEnc5Values;
+      h->vec_type = SPMSPV_VEC_BITARRAY;
+    } else if ((rc = need_bits(h))) {
+      return rc;
+    }
     // every entry is written: take a buffer that is not clean, if any
     int cur = h->enc5_cur;
     if (h->enc5_clean[cur] && !h->enc5_clean[1 - cur]) cur = 1 - cur;
     h->enc5_cur = cur;
     h->enc5_clean[cur] = false;
-    launch_encode_x(h->stream, h->dense_x(), h->bits(), h->n, h->x_enc5b[cur], h->csr5.cperm);
+    launch_encode_x(h->stream, h->dense_x(), holds == h->kEnc5Values ? nullptr : h->bits(), h->n, h->x_enc5b[cur],
+                    h->csr5.cperm);
   }
   *out = h->x_enc5b[h->enc5_cur];
   int rc = check_launch(h, "encode x (CSR5 order)");
   if (rc) return rc;
-  h->enc5_valid = true;
+  h->enc5_valid = holds;
   return SPMSPV_SUCCESS;
 }
 
@@ -649,7 +659,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
         if (masked || hits || h->csr5.cperm) {
           // the support encoding in the copy's column order (also serves the
           // plain product: +0.0 outside the support)
-          if ((rc = need_enc_x5(h, &xin))) return rc;
+          if ((rc = need_enc_x5(h, &xin, !masked && !hits))) return rc;
         } else {
           if ((rc = need_dense_x(h))) return rc;
           xin = h->dense_x();
@@ -1432,7 +1442,7 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
     const bool order5 = row && h->spmv_type == 1 && h->csr5_ready && h->csr5.cperm &&
                         (guess == SPMSPV_K_ROW_LB || guess == SPMSPV_K_SPMV_LB);
     float* enc = nullptr;
-    if (row && !(order5 ? h->enc5_valid : h->enc_valid)) {
+    if (row && !(order5 ? h->enc5_valid == h->kEnc5Support : h->enc_valid)) {
       if (order5) {
         enc = enc5_for_scatter(h);
       } else {
@@ -1445,7 +1455,8 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
                        sel, enc, order5 ? h->csr5.cperm : nullptr);
     h->launches++;
     if ((rc = check_launch(h, "selector"))) return rc;
-    if (enc) (order5 ? h->enc5_valid : h->enc_valid) = true;
+    if (enc && order5) h->enc5_valid = h->kEnc5Support;
+    else if (enc) h->enc_valid = true;
   } else if ((rc = run_prep(h, true, &sel))) {
     return rc;
   }

@@ -1345,9 +1345,12 @@ __global__ void k_encode_x(const float* __restrict__ x, const unsigned* __restri
                            float* __restrict__ enc, const int* __restrict__ perm) {
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n;
        c += (long long)gridDim.x * blockDim.x) {
-    const bool in = (bits[c >> 5] >> (c & 31)) & 1u;
-    const float v = x[c];
-    enc[perm ? perm[c] : c] = in ? (v == 0.f ? -0.f : v) : 0.f;
+    float v = x[c];
+    if (bits) {
+      const bool in = (bits[c >> 5] >> (c & 31)) & 1u;
+      v = in ? (v == 0.f ? -0.f : v) : 0.f;
+    }
+    enc[perm ? perm[c] : c] = v;
   }
 }
 void launch_encode_x(hipStream_t s, const float* x, const unsigned* bits, int n, float* enc,

@@ -45,7 +45,11 @@ struct spmspv_handle_s {
   bool bits_valid = false;    // bit array holds the current x's support
   bool prep_valid = false;    // ptr/xbeg/split/bin_len computed for the current x
   bool enc_valid = false;     // x_enc holds the support encoding of the current x
-  bool enc5_valid = false;    // x_enc5b[enc5_cur] holds it in the CSR5 column order
+  // what x_enc5b[enc5_cur] holds of the current x, in the CSR5 column order:
+  // 0 nothing, kEnc5Values its values (all that the plain product needs),
+  // kEnc5Support the support encoding
+  int enc5_valid = 0;
+  static constexpr int kEnc5Values = 1, kEnc5Support = 2;
   long long binlen_host = -1; // bin_len read back for the current x (or -1)
   int spmv_type = 0;          // 0 merge (Hola role), 1 CSR5
   int sigma = -1;

@@ -176,8 +176,8 @@ void launch_fill_i32(hipStream_t s, int* p, long long n, int v);
 // With perm, entry k lands at dense[perm[k]].
 void launch_scatter(hipStream_t s, const int* key, const float* val, int nnz, const int* nnz_dev,
                     int len, float* dense, bool encode = false, Gate g = {}, const int* perm = nullptr);
-// enc[c] = bit c of bits ? (x[c] == 0 ? -0.0 : x[c]) : +0.0 (at enc[perm[c]]
-// with perm)
+// enc[c] = bit c of bits ? (x[c] == 0 ? -0.0 : x[c]) : +0.0, or x[c] without
+// bits (at enc[perm[c]] with perm)
 void launch_encode_x(hipStream_t s, const float* x, const unsigned* bits, int n, float* enc,
                      const int* perm = nullptr);
 void launch_set_bits(hipStream_t s, const int* key, int nnz, const int* nnz_dev, int len,
