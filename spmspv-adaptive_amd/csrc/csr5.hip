@@ -25,6 +25,7 @@
 // is a copy of the first x entries (the densest columns), made by each block
 // at its start: one block per CU then serves most gathers from LDS.
 #include <algorithm>
+#include <climits>
 
 #include "handle.hpp"
 #include "ranking.hpp"
@@ -411,13 +412,29 @@ __global__ void k_csr5_fixup(const float* __restrict__ carry_val, const int* __r
   }
 }
 
-// dense y from the non-empty-row results: y[r] = y_ne[rank[r]] or 0
-__global__ void k_csr5_expand(const int* __restrict__ row_ptr, const int* __restrict__ rank, int m,
-                              const float* __restrict__ y_ne, float* __restrict__ y, Gate g) {
+// dense y from the non-empty-row results: y[r] = y_ne[rank[r]] or 0, the rows
+// that run through several tiles with their tail parts added in tile order
+// (by the first fix_blocks workgroups, the others leave those rows alone; one
+// launch where a fix-up in front of this one cost 5 us)
+__global__ void k_csr5_expand(const int* __restrict__ row_ptr, const int* __restrict__ rank,
+                              const int* __restrict__ rows_ne, int m, int T, const float* __restrict__ y_ne,
+                              const float* __restrict__ carry_val, const int* __restrict__ carry_row, int ntiles,
+                              int fix_blocks, float* __restrict__ y, Gate g) {
   if (gate_shut(g)) return;
-  for (long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x; r < m;
-       r += (long long)gridDim.x * blockDim.x)
-    y[r] = row_ptr[r + 1] > row_ptr[r] ? y_ne[rank[r]] : 0.f;
+  if ((int)blockIdx.x < fix_blocks) {
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < ntiles; t += fix_blocks * blockDim.x) {
+      int k, h;
+      float s;
+      if (carry_run<int>(carry_val, carry_row, nullptr, t, ntiles, k, s, h)) y[rows_ne[k]] = y_ne[k] + s;
+    }
+    return;
+  }
+  for (long long r = (long long)(blockIdx.x - fix_blocks) * blockDim.x + threadIdx.x; r < m;
+       r += (long long)(gridDim.x - fix_blocks) * blockDim.x) {
+    const int b = row_ptr[r], e = row_ptr[r + 1];
+    const float v = e > b ? y_ne[rank[r]] : 0.f;
+    if (e <= b || b / T == (e - 1) / T) y[r] = v;
+  }
 }
 
 }  // namespace
@@ -883,11 +900,20 @@ void launch_csr5(hipStream_t s, const Csr5& c, bool masked, bool hits, const flo
 #undef SPMSPV_CSR5_H
 #undef SPMSPV_CSR5
   if (ev_end) (void)hipEventRecord(ev_end, s);
-  hipLaunchKernelGGL(k_csr5_fixup, dim3(std::min(1024, (c.ntiles + 255) / 256)), dim3(256), 0, s,
-                     c.carry_val, c.carry_row, c.carry_hit, c.ntiles, yk, hits ? marks : nullptr, g);
-  if (compressed && y_dense_rows)
-    hipLaunchKernelGGL(k_csr5_expand, dim3(std::min(8192, (m + 255) / 256)), dim3(256), 0, s, c.row_ptr,
-                       c.rank, m, c.y_ne, y, g);
+  const int fix = std::min(1024, (c.ntiles + 255) / 256);
+  const bool expand = compressed && y_dense_rows;
+  // with hits, the compaction reads the fixed non-empty-row results
+  const bool fused = expand && !hits;
+  if (!fused)
+    hipLaunchKernelGGL(k_csr5_fixup, dim3(fix), dim3(256), 0, s, c.carry_val, c.carry_row, c.carry_hit, c.ntiles, yk,
+                       hits ? marks : nullptr, g);
+  if (expand) {
+    const int fix_blocks = fused ? fix : 0;
+    // already fixed: no row is left out
+    const int T = fused ? kWave * c.S : INT_MAX;
+    hipLaunchKernelGGL(k_csr5_expand, dim3(fix_blocks + std::min(8192, (m + 255) / 256)), dim3(256), 0, s, c.row_ptr,
+                       c.rank, c.rows_ne, m, T, c.y_ne, c.carry_val, c.carry_row, c.ntiles, fix_blocks, y, g);
+  }
 }
 
 }  // namespace spmspv

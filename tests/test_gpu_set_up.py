@@ -57,3 +57,10 @@ def test_formats_of_row_lengths(gpu, shape):
             cnt = M.A.run(slot, y_key=yk, y_val=yv)
             np.testing.assert_array_equal(yk.to_host(cnt), ek, err_msg=f"sigma {sigma} slot {slot}")
             assert np.all(np.abs(yv.to_host(cnt).astype(np.float64) - ev) <= 1e-5 * eb + 1e-30)
+        # a dense y, every row written (rows through several tiles, empty rows)
+        yd = sa.DeviceArray.from_host(np.full(m, np.nan, np.float32), np.float32)
+        M.A.set_sparse_x(dk, dv, n)
+        M.A.run(sa.K_SPMV_LB, y_dense=yd, want_nnz=False)
+        ref, bound = np.zeros(m), np.zeros(m)
+        ref[ek], bound[ek] = ev, eb
+        assert np.all(np.abs(yd.to_host() - ref) <= 1e-5 * bound + 1e-30), f"sigma {sigma} dense"
