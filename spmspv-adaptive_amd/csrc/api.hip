@@ -135,7 +135,7 @@ static size_t carve(spmspv_handle_t h, char* base) {
   long long* selp = c.take<long long>(5 * kSelMaxGrid);
   long long* psamp = c.take<long long>(2 * (kSampleKeys / kPrepNT));
   BinWs bws;
-  bws.cursor = c.take<unsigned>((size_t)kBinMax * kBinCurStride);
+  bws.cursor = c.take<unsigned long long>((size_t)kBinMax / 2 * kBinCurStride);
   bws.base = c.take<int>(kBinMax + 1);
   bws.start = c.take<int>(kBinMax + 1);
   bws.tbl = c.take<int>(kBinTbl);
@@ -634,7 +634,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
                     h->bin_nbins, h->sb.keyB, h->sb.valB, h->acc, h->marks, lb_tiles_hint(h), h->binlen_host,
                     h->nnz, h->gate);
       launch_compact(s, nullptr, h->marks, m, h->acc, 1, ok, ov, h->scan_state, h->ctl, next_ep(h, 1), nullptr,
-                     h->gate, y_dense ? nullptr : count_sig(), h->bin_ws.cursor, h->bin_nbins);
+                     h->gate, y_dense ? nullptr : count_sig(), h->bin_ws.cursor, (h->bin_nbins + 1) / 2);
       h->launches += 3;
       if (y_dense) {
         launch_fill_f32(s, y_dense, m, 0.f, h->gate);

@@ -6,9 +6,9 @@
 // variant truncates values to int (:684). Here the buckets are row bins,
 // ranges of consecutive rows holding about equal numbers of the matrix's
 // nonzeros and at most 2^12 rows (one bin's sums fit a 48 KB LDS window,
-// two accumulate workgroups per CU). The layout is fixed per matrix and bin count (BinLayout, built
-// on the host from the row pointer): a bin never receives more products
-// than its rows have nonzeros, so bin b owns the product slots [base[b],
+// two accumulate workgroups per CU). The layout is fixed per matrix and bin
+// count (BinLayout, built on the host from the row pointer): a bin never
+// receives more products than its rows have nonzeros, so bin b owns the product slots [base[b],
 // base[b+1]) with base[b] = nonzeros in the rows before it, and no per-call
 // count is needed; equal nonzero counts keep the bins' product counts
 // level on a power-law matrix, where equal row ranges put a tenth of them
@@ -17,12 +17,13 @@
 //      split, kBinS of its tiles at a time), one per workgroup round, form
 //      every product (row, a*x), find its bin (a table of row blocks, then a
 //      search among the bins that start inside the row's block) and rank it
-//      there in LDS; the round reserves each bin's slots with one global
-//      atomic on the bin's cursor (one cursor per 128-byte line), places its
-//      products bin by bin in LDS and writes them out in that order;
+//      there in LDS; the round reserves the slots of each pair of bins with
+//      one global 64-bit atomic on their cursors (one pair per 128-byte
+//      line), places its products bin by bin in LDS and writes them out in
+//      that order;
 //   2. k_bin_accum: every workgroup reads the cursors (products per bin) and
 //      plans the chunks itself: a bin is cut into chunks of kBinChunk
-//      products (one round of registers), so a bin that an uneven x fills
+//      products (a few rounds of registers), so a bin that an uneven x fills
 //      far beyond its share still spreads over workgroups; one chunk per
 //      workgroup. Each chunk is summed per row in an LDS window over its
 //      bin's rows, in 64-bit fixed point scaled to the row's largest
@@ -49,14 +50,26 @@ namespace {
 
 // The scatter: 1,024-thread workgroups whose merge-path tile is kBinS of
 // the prep's tiles (one latency chain for 7,168 merged positions), one
-// such tile per round. Each round reserves its slots with one device-scope
-// atomic per bin it fills (about 17 G/s on the chip, one address taking
-// them in turn at about 16 ns).
+// such tile per round. Each round reserves its slots with device-scope
+// atomics (about 17 G/s on the chip, one address taking them in turn at
+// about 16 ns), one for each pair of bins of which it fills at least one,
+// and places its products in LDS while they are on their way. R-MAT scale
+// 20, x 10 % dense (3 M products, 429 rounds, 617 bins; a workgroup's two
+// rounds: 16 k cycles merge, 24 k loads and ranks, 34 k reservation, 5 k
+// placing, 11 k writing): 47.4 us with one atomic per bin, 40.5 per pair,
+// 38.4 with the placing before the wait. Two workgroups per CU (64
+// registers, 57 KB of LDS) took 49.0, rounds of equal size 40.7 against
+// 40.5.
 constexpr int kScatNT = 1024, kBinS = 4, kScatGrid = 2048;
 static_assert(kScatNT * kLbVT == kBinS * kLbTile, "the scatter's tile is kBinS prep tiles");
 static_assert(kBinS * kLbTile < 65536 && kBinMax < 65535, "bin and rank share a word");
-constexpr int kAccNT = 1024;        // accumulate workgroup
-constexpr int kAccPPT = 16;         // products per thread per sub-round
+// The accumulate: rounds of kAccNT * kAccPPT products. An average bin (5 k
+// products at the size above) leaves few lanes idle in the last of them,
+// and two workgroups fit a CU by registers as by LDS. There: 23.9 us with
+// one round of 1,024 x 16 per chunk, 24.7 for 512 x 16, 27.1 for 256 x 16,
+// 22.6 for 1,024 x 8, 21.8 for 512 x 8.
+constexpr int kAccNT = 512;         // accumulate workgroup
+constexpr int kAccPPT = 8;          // products per thread and round
 constexpr int kAccGrid = 2048;      // accumulate workgroups at most
 constexpr int kFewRows = 16;        // bins of at most this many rows sum in registers
 constexpr int kMaxDevices = 64;     // devices whose kernel attributes are tracked
@@ -178,7 +191,7 @@ __global__ __launch_bounds__(NT) void k_bin_scatter(const int* __restrict__ ptr,
                                                     unsigned* __restrict__ okey, float* __restrict__ oval, Gate g) {
   if (gate_shut(g)) return;
   constexpr int T = NT * VT;
-  constexpr int BPT = (kBinMax + 1 + NT - 1) / NT;
+  constexpr int PPT = (kBinMax / 2 + NT) / NT;  // pairs of bins per thread at most
   __shared__ int s_ptr[T + 2];
   __shared__ int s_beg[T + 2];
   __shared__ unsigned short s_seg[T];
@@ -191,6 +204,7 @@ __global__ __launch_bounds__(NT) void k_bin_scatter(const int* __restrict__ ptr,
   unsigned* s_base = s_c + nbins + 1;
   for (int b = threadIdx.x; b <= nbins; b += NT) s_start[b] = ws.start[b];
   for (int b = threadIdx.x; b < ntbl; b += NT) s_tbl[b] = ws.tbl[b];
+  const int ppt = (nbins / 2 + NT) / NT;  // spread over the workgroup's threads
   const long long ntiles = ctl->n_tiles;
   const long long nbig = (ntiles + kBinS - 1) / kBinS;
   const long long W = (long long)xnnz + ctl->bin_len;
@@ -221,24 +235,32 @@ __global__ __launch_bounds__(NT) void k_bin_scatter(const int* __restrict__ ptr,
       }
     }
     __syncthreads();
-    // reserve each bin's slots, and the bins' offsets in the round
+    // reserve each bin's slots, and the bins' offsets in the round; the
+    // products are placed while the atomics are on their way
+    unsigned c[PPT][2];
+    unsigned long long at[PPT];
     {
-      unsigned c[BPT];
       int sum = 0;
 #pragma unroll
-      for (int j = 0; j < BPT; ++j) {
-        const int b = threadIdx.x * BPT + j;
-        c[j] = b < nbins ? s_c[b] : 0u;
-        sum += (int)c[j];
-        if (c[j]) s_base[b] = (unsigned)ws.base[b] + atomicAdd(ws.cursor + (long long)b * kBinCurStride, c[j]);
+      for (int j = 0; j < PPT; ++j) {
+        const int b = 2 * ((int)threadIdx.x * ppt + j);
+        c[j][0] = j < ppt && b < nbins ? s_c[b] : 0u;
+        c[j][1] = j < ppt && b + 1 < nbins ? s_c[b + 1] : 0u;
+        sum += (int)(c[j][0] + c[j][1]);
+        if (c[j][0] | c[j][1]) {
+          // a bin's count stays below 2^31, so the halves do not carry
+          at[j] = atomicAdd(ws.cursor + (long long)(b / 2) * kBinCurStride,
+                            c[j][0] | ((unsigned long long)c[j][1] << 32));
+        }
       }
       int tot;
       unsigned pre = (unsigned)block_excl_sum<NT, int>(sum, s_w, &tot);
 #pragma unroll
-      for (int j = 0; j < BPT; ++j) {
-        const int b = threadIdx.x * BPT + j;
-        if (b <= nbins) s_c[b] = pre;  // every thread read its counts before the scan's barriers
-        pre += c[j];
+      for (int j = 0; j < PPT; ++j) {  // every thread read its counts before the scan's barriers
+        const int b = 2 * ((int)threadIdx.x * ppt + j);
+        if (j < ppt && b <= nbins) s_c[b] = pre;
+        if (j < ppt && b + 1 <= nbins) s_c[b + 1] = pre + c[j][0];
+        pre += c[j][0] + c[j][1];
       }
     }
     __syncthreads();
@@ -253,6 +275,12 @@ __global__ __launch_bounds__(NT) void k_bin_scatter(const int* __restrict__ ptr,
         s_val[q] = val[k];
         s_seg[q] = (unsigned short)b;
       }
+    }
+#pragma unroll
+    for (int j = 0; j < PPT; ++j) {
+      const int b = 2 * ((int)threadIdx.x * ppt + j);
+      if (c[j][0]) s_base[b] = (unsigned)ws.base[b] + (unsigned)at[j];
+      if (c[j][1]) s_base[b + 1] = (unsigned)ws.base[b + 1] + (unsigned)(at[j] >> 32);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < np; i += NT) {
@@ -273,8 +301,8 @@ __global__ __launch_bounds__(NT) void k_bin_accum(const unsigned* __restrict__ k
                                                   BinWs ws, int nbins, float* acc, unsigned char* marks, Gate g) {
   if (gate_shut(g)) return;
   constexpr int SUB = NT * PPT;
-  static_assert(SUB == kBinChunk, "a chunk is one round of registers");
-  constexpr int BPT = kBinMax / NT;
+  constexpr int SUBS = kBinChunk / SUB;
+  static_assert(SUB * SUBS == kBinChunk, "a chunk is whole rounds of registers");
   constexpr int NW = NT / kWave;
   extern __shared__ unsigned long long s_q[];
   const int R = ws.max_rows;
@@ -283,37 +311,25 @@ __global__ __launch_bounds__(NT) void k_bin_accum(const unsigned* __restrict__ k
   int* s_base = s_cnt + nbins;
   int* s_cst = s_base + nbins;
   __shared__ int s_i[NW];
-  __shared__ float s_few[NW][kFewRows];  // per-wave sums of a bin of few rows
-  __shared__ unsigned s_fewhit[NW];
+  __shared__ float s_few[SUBS * NW][kFewRows];  // per-wave sums of a bin of few rows
+  __shared__ unsigned s_fewhit[SUBS * NW];
   // the plan, the same in every workgroup: a bin is cut into chunks of
   // kBinChunk products (the last one shorter)
+  for (int b = threadIdx.x; b < nbins; b += NT) {
+    s_cnt[b] = (int)(unsigned)(ws.cursor[(long long)(b / 2) * kBinCurStride] >> (b % 2 * 32));
+    s_base[b] = ws.base[b];
+  }
+  __syncthreads();
   {
-    unsigned c[BPT];
-    int bb[BPT];
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-      const int b = threadIdx.x * BPT + j;
-      c[j] = b < nbins ? ws.cursor[(long long)b * kBinCurStride] : 0u;
-      bb[j] = b < nbins ? ws.base[b] : 0;
-    }
+    const int bpt = (nbins + NT - 1) / NT;
+    const int b0 = std::min(nbins, (int)threadIdx.x * bpt), b1 = std::min(nbins, b0 + bpt);
     int nsum = 0;
-    int nch[BPT];
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-      nch[j] = (int)((c[j] + kBinChunk - 1) / kBinChunk);
-      nsum += nch[j];
-    }
+    for (int b = b0; b < b1; ++b) nsum += (s_cnt[b] + kBinChunk - 1) / kBinChunk;
     int ntot;
     int npre = block_excl_sum<NT, int>(nsum, s_i, &ntot);
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-      const int b = threadIdx.x * BPT + j;
-      if (b < nbins) {
-        s_cnt[b] = (int)c[j];
-        s_base[b] = bb[j];
-        s_cst[b] = npre;
-      }
-      npre += nch[j];
+    for (int b = b0; b < b1; ++b) {
+      s_cst[b] = npre;
+      npre += (s_cnt[b] + kBinChunk - 1) / kBinChunk;
     }
     if (threadIdx.x == 0) s_cst[nbins] = ntot;
   }
@@ -339,53 +355,56 @@ __global__ __launch_bounds__(NT) void k_bin_accum(const unsigned* __restrict__ k
     const long long pe = std::min<long long>(p0 + kBinChunk, (long long)s_base[b] + s_cnt[b]);
     const unsigned rs = (unsigned)ws.start[b];
     const int nr = ws.start[b + 1] - (int)rs;
+    const int nsub = (int)((pe - p0 + SUB - 1) / SUB);
     unsigned kk[PPT];
     float vv[PPT];
+    const auto load = [&](long long ps) {
 #pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      const long long i = p0 + threadIdx.x + (long long)j * NT;
-      const long long ic = i < pe ? i : p0;
-      kk[j] = __builtin_nontemporal_load(key + ic);
-      vv[j] = __builtin_nontemporal_load(val + ic);
-    }
+      for (int j = 0; j < PPT; ++j) {
+        const long long i = ps + threadIdx.x + (long long)j * NT;
+        const long long ic = i < pe ? i : p0;
+        kk[j] = __builtin_nontemporal_load(key + ic);
+        vv[j] = __builtin_nontemporal_load(val + ic);
+      }
+    };
     if (nr <= kFewRows) {
       // a bin of few (hub) rows: the lanes of a wave would all add into the
       // same LDS words, so each thread sums per row in registers and the
-      // workgroup reduces the kFewRows sums
-      float part[kFewRows];
-      unsigned hit = 0u;
+      // workgroup reduces the sums of its waves and rounds
+      for (int u = 0; u < nsub; ++u) {
+        const long long ps = p0 + (long long)u * SUB;
+        load(ps);
+        float part[kFewRows];
+        unsigned hit = 0u;
 #pragma unroll
-      for (int q = 0; q < kFewRows; ++q) part[q] = 0.f;
+        for (int q = 0; q < kFewRows; ++q) part[q] = 0.f;
 #pragma unroll
-      for (int j = 0; j < PPT; ++j) {
-        if (p0 + threadIdx.x + (long long)j * NT < pe) {
-          const unsigned r = kk[j] - rs;
-          hit |= 1u << r;
+        for (int j = 0; j < PPT; ++j) {
+          if (ps + threadIdx.x + (long long)j * NT < pe) {
+            const unsigned r = kk[j] - rs;
+            hit |= 1u << r;
 #pragma unroll
-          for (int q = 0; q < kFewRows; ++q) part[q] += r == (unsigned)q ? vv[j] : 0.f;
+            for (int q = 0; q < kFewRows; ++q) part[q] += r == (unsigned)q ? vv[j] : 0.f;
+          }
         }
-      }
 #pragma unroll
-      for (int q = 0; q < kFewRows; ++q) part[q] = wave_sum(part[q]);
+        for (int q = 0; q < kFewRows; ++q) part[q] = wave_sum(part[q]);
 #pragma unroll
-      for (int o = kWave / 2; o > 0; o >>= 1) hit |= __shfl_xor(hit, o, kWave);
-      const int w = threadIdx.x / kWave;
-      if (lane() == 0) {
+        for (int o = kWave / 2; o > 0; o >>= 1) hit |= __shfl_xor(hit, o, kWave);
+        const int w = u * NW + threadIdx.x / kWave;
+        if (lane() == 0) {
 #pragma unroll
-        for (int q = 0; q < kFewRows; ++q) s_few[w][q] = part[q];
-        s_fewhit[w] = hit;
+          for (int q = 0; q < kFewRows; ++q) s_few[w][q] = part[q];
+          s_fewhit[w] = hit;
+        }
       }
       __syncthreads();
-      if ((int)threadIdx.x < nr) {
-        const int q = threadIdx.x;
-        float v = 0.f;
-        unsigned h = 0u;
-#pragma unroll
-        for (int k = 0; k < NW; ++k) {
-          v += s_few[k][q];
-          h |= s_fewhit[k];
-        }
-        if ((h >> q) & 1u) {
+      static_assert(SUBS * NW <= kWave, "a wave holds a row's partial sums");
+      for (int q = threadIdx.x / kWave; q < nr; q += NW) {  // one wave per row
+        const bool in = lane() < nsub * NW;
+        const float v = wave_sum(in ? s_few[lane()][q] : 0.f);
+        const bool h = __any(in && ((s_fewhit[lane()] >> q) & 1u));
+        if (h && lane() == 0) {
           if (owned) acc[rs + q] = v;  // the accumulator holds 0 there
           else atomic_add_f32(acc + rs + q, v);
           marks[rs + q] = 1;
@@ -395,23 +414,32 @@ __global__ __launch_bounds__(NT) void k_bin_accum(const unsigned* __restrict__ k
       continue;
     }
     // every row's largest exponent first; a chunk with an Inf or NaN
-    // product sums in FP32 instead (the window's sums read as floats)
+    // product sums in FP32 instead (the window's sums read as floats). The
+    // registers keep the last round of products for the sums.
     int special = 0;
+    for (int u = 0; u < nsub; ++u) {
+      const long long ps = p0 + (long long)u * SUB;
+      load(ps);
 #pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      if (p0 + threadIdx.x + (long long)j * NT < pe) {
-        const unsigned ef = prod_ef(vv[j]);
-        special |= ef == 0xFFu;
-        atomicMax(&s_e[kk[j] - rs], ef);
+      for (int j = 0; j < PPT; ++j) {
+        if (ps + threadIdx.x + (long long)j * NT < pe) {
+          const unsigned ef = prod_ef(vv[j]);
+          special |= ef == 0xFFu;
+          atomicMax(&s_e[kk[j] - rs], ef);
+        }
       }
     }
     special = __syncthreads_or(special);
+    for (int u = nsub - 1; u >= 0; --u) {
+      const long long ps = p0 + (long long)u * SUB;
+      if (u < nsub - 1) load(ps);
 #pragma unroll
-    for (int j = 0; j < PPT; ++j) {
-      if (p0 + threadIdx.x + (long long)j * NT < pe) {
-        const unsigned r = kk[j] - rs;
-        if (special) atomicAdd(reinterpret_cast<float*>(s_q + r), vv[j]);
-        else atomicAdd(s_q + r, (unsigned long long)prod_fixed(vv[j], s_e[r]));
+      for (int j = 0; j < PPT; ++j) {
+        if (ps + threadIdx.x + (long long)j * NT < pe) {
+          const unsigned r = kk[j] - rs;
+          if (special) atomicAdd(reinterpret_cast<float*>(s_q + r), vv[j]);
+          else atomicAdd(s_q + r, (unsigned long long)prod_fixed(vv[j], s_e[r]));
+        }
       }
     }
     __syncthreads();

@@ -159,12 +159,12 @@ void launch_tl_gather(hipStream_t s, int mode, const int* ptr, const int* xbeg, 
 // (keymap ascending keeps the keys sorted). With sig (may be host-mapped),
 // the result count is also written to *sig once every workgroup's stores
 // are visible, as launch_signal_int after this launch would.
-// clr (nullable): nclr words at a stride of kBinCurStride set to 0 (the
+// clr (nullable): nclr 64-bit words at a stride of kBinCurStride set to 0 (the
 // bucket slot's cursors, once its accumulate kernel has read them).
 void launch_compact(hipStream_t s, unsigned* bitmap, unsigned char* marks, int m, float* acc,
                     int reset_acc, int* ykey, float* yval, unsigned long long* state, Ctl* ctl,
                     Ep ep, const int* keymap = nullptr, Gate g = {}, long long* sig = nullptr,
-                    unsigned* clr = nullptr, int nclr = 0);
+                    unsigned long long* clr = nullptr, int nclr = 0);
 // bitmap of (v != 0) over a dense vector (whole words, no atomics)
 void launch_bitmap_from_dense(hipStream_t s, const float* v, int n, unsigned* bits);
 void launch_fill_f32(hipStream_t s, float* p, long long n, float v, Gate g = {});
@@ -256,9 +256,9 @@ int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long lo
 // than kBinMax bins would be needed). Per call the products are scattered
 // into their bins and summed per bin in LDS windows into acc (marks set);
 // the caller's compaction gives the sorted result and clears acc, marks
-// and the cursors (one per 128-byte line; its clr argument). Needs k_prep's
+// and the cursors (two bins' per 128-byte line; its clr argument). Needs k_prep's
 // scan and splits.
-constexpr int kBinRowBits = 12, kBinMax = 6144, kBinChunk = 16384, kBinCurStride = 32, kBinTbl = 2048;
+constexpr int kBinRowBits = 12, kBinMax = 6144, kBinChunk = 16384, kBinCurStride = 16, kBinTbl = 2048;
 struct BinLayout {
   std::vector<int> start;  // first row of each bin, then m
   std::vector<int> base;   // first product slot of each bin, then nnz
@@ -267,7 +267,7 @@ struct BinLayout {
   int max_rows = 1;        // rows of the largest bin
 };
 struct BinWs {
-  unsigned* cursor;  // kBinMax * kBinCurStride: products reserved per bin (word b * kBinCurStride)
+  unsigned long long* cursor;  // kBinMax / 2 * kBinCurStride: products reserved in bins 2i (low half) and 2i + 1
   int* base;         // kBinMax + 1
   int* start;        // kBinMax + 1
   int* tbl;          // kBinTbl
