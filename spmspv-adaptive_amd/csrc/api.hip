@@ -499,7 +499,8 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       if (on) h->gate = Gate{};
     }
   } gate_restore{h};
-  if (!h->gate.word && !y_dense && takes_small_path(h, kid)) {
+  bool gathered = h->x_gathered;
+  if (!gathered && !h->gate.word && !y_dense && takes_small_path(h, kid)) {
     if ((rc = need_csc(h))) return rc;
     if (h->count_to_host) mark_sig3();
     const bool wait = h->count_to_host;
@@ -507,7 +508,8 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
     const SelectorArgs fixed{nullptr, nullptr, 2, kid, wait ? h->sig_dev + 1 : nullptr, 0};
     launch_col_fused(s, h->csc_colptr, h->csc_row, h->csc_val, h->x_key, h->x_val, h->n, h->xnnz, m, h->ptr,
                      h->xbeg, h->split, h->ctl, fixed, y_key ? y_key : h->yk_tmp, y_val ? y_val : h->yv_tmp,
-                     h->count_to_host ? h->sig_dev + 3 : nullptr, h->fuse_cap, h->scan_state, next_ep(h, 1));
+                     h->count_to_host ? h->sig_dev + 3 : nullptr, h->fuse_cap, h->scan_state, next_ep(h, 1),
+                     wait ? h->acc : nullptr, h->marks);
     h->launches++;
     if ((rc = check_launch(h, "small-x column path"))) return rc;
     h->prep_valid = true;
@@ -520,6 +522,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
         return SPMSPV_SUCCESS;
       }
       h->binlen_host = sel_word_binlen(word);
+      gathered = sel_word_gathered(word);
     } else if (h->binlen_host >= 0) {
       return SPMSPV_SUCCESS;  // the products are known to fit: that launch finishes the call
     } else {
@@ -534,7 +537,9 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       if ((rc = need_csc(h)) || (rc = need_sparse_x(h))) return rc;
       float* acc = y_dense ? y_dense : h->acc;
       if (y_dense) launch_fill_f32(s, y_dense, m, 0.f, h->gate);
-      if (kid == SPMSPV_K_COL_NAIVE_ATOMIC) {
+      if (gathered) {
+        // the small-x launch did it
+      } else if (kid == SPMSPV_K_COL_NAIVE_ATOMIC) {
         launch_naive_col(s, 0, h->csc_colptr, h->csc_row, h->csc_val, h->x_key, h->x_val, nullptr,
                          h->n, h->xnnz, nullptr, h->team_col, acc, h->marks, nullptr, nullptr,
                          h->gate);
@@ -545,7 +550,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       }
       launch_compact(s, nullptr, h->marks, m, acc, y_dense ? 0 : 1, y_key, y_val, h->scan_state, h->ctl,
                      next_ep(h, 1), nullptr, h->gate, count_sig());
-      h->launches += 2;
+      h->launches += gathered ? 1 : 2;
       return check_launch(h, "column atomic kernel");
     }
     case SPMSPV_K_COL_NAIVE_SORT:
@@ -1430,7 +1435,8 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   if (fused) {
     launch_col_fused(h->stream, h->csc_colptr, h->csc_row, h->csc_val, h->x_key, h->x_val, h->n, h->xnnz, h->m,
                      h->ptr, h->xbeg, h->split, h->ctl, sel, d_y_key ? d_y_key : h->yk_tmp,
-                     d_y_val ? d_y_val : h->yv_tmp, nullptr, h->fuse_cap, h->scan_state, next_ep(h, 1));
+                     d_y_val ? d_y_val : h->yv_tmp, nullptr, h->fuse_cap, h->scan_state, next_ep(h, 1), h->acc,
+                     h->marks);
     h->launches++;
     if ((rc = check_launch(h, "small-x column path"))) return rc;
     h->prep_valid = true;
@@ -1460,12 +1466,20 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   } else if ((rc = run_prep(h, true, &sel))) {
     return rc;
   }
+  // the class's last gather was done by the small-x launch: only the
+  // compaction is queued
+  const bool spec_gathered = spec && fused && h->spec_gathered[cls] &&
+                             (guess == SPMSPV_K_COL_NAIVE_ATOMIC || guess == SPMSPV_K_COL_LB_ATOMIC);
   if (spec) {
     struct Ungate {
       spmspv_handle_t h;
-      ~Ungate() { h->gate = Gate{}; }
+      ~Ungate() {
+        h->gate = Gate{};
+        h->x_gathered = false;
+      }
     } ungate{h};
-    h->gate = Gate{&h->ctl->kernel_choice, guess};
+    h->x_gathered = spec_gathered;
+    h->gate = Gate{&h->ctl->kernel_choice, spec_gathered ? guess | kSelGathered : guess};
     h->spec_cap = h->nnz;
     if (h->spec_binlen[cls] > 0) h->spec_cap = std::min<long long>(h->nnz, 4 * h->spec_binlen[cls] + 65536);
     h->count_to_host = y_nnz != nullptr;
@@ -1485,7 +1499,11 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   const int kid = sel_word_choice(word);
   if (kid < 0 || kid > SPMSPV_K_COL_BUCKET)  // the eight classes or the bucket rule's slot
     return set_error(h, SPMSPV_DEVICE_ERROR, "selector returned no slot");
-  if (fused) h->spec_fused[cls] = sel_word_done(word);
+  const bool gathered = sel_word_gathered(word);
+  if (fused) {
+    h->spec_fused[cls] = sel_word_done(word);
+    if (!sel_word_done(word)) h->spec_gathered[cls] = gathered;
+  }
   h->prev_choice = kid;
   if (sel_word_done(word)) {
     // the single launch finished the call: its word carries y_nnz
@@ -1499,7 +1517,7 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   if (kernel_used) *kernel_used = kid;
   if (h->binlen_host >= 0) h->spec_binlen[cls] = h->binlen_host;
   const bool sorts = kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_SORT;
-  if (spec && kid == guess && !(sorts && h->binlen_host > h->spec_cap)) {
+  if (spec && kid == guess && gathered == spec_gathered && !(sorts && h->binlen_host > h->spec_cap)) {
     h->spec_hits++;
     // the gated tile kernel ran, and with it the clearing of the idle buffer
     if (clear_pending >= 0) h->enc5_clean[clear_pending] = true;
@@ -1511,13 +1529,16 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
     return SPMSPV_SUCCESS;
   }
   if (spec) h->spec_misses++;
-  if (spec && kid == guess && y_nnz) {
+  if (spec && kid == guess && sorts && y_nnz) {
     // more products than the queued sort covers: its launches left the result
     // alone, but the count of an earlier one is on its way to the host word
     long long v = 0;
     if ((rc = wait_signal(h, 3, &v))) return rc;
   }
-  return spmspv_run(h, kid, alpha, d_y_dense, d_y_key, d_y_val, y_nnz);
+  h->x_gathered = gathered;
+  rc = spmspv_run(h, kid, alpha, d_y_dense, d_y_key, d_y_val, y_nnz);
+  h->x_gathered = false;
+  return rc;
 }
 
 int spmspv_autotune_report(spmspv_handle_t h, int out[10]) {

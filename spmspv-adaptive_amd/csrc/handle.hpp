@@ -154,6 +154,8 @@ struct spmspv_handle_s {
   signed char spec_last[33] = {};
   int prev_choice = -1;        // slot of the last selector-dispatched call
   float switch_penalty = 0.f;  // switching-aware choice (0: off)
+  bool spec_gathered[33] = {};  // the last call of the size class was gathered there
+  bool x_gathered = false;      // the next atomic column slot's gather has been done (acc, marks)
   bool spec_fused[33] = {};  // the last call of the size class ended in the single-launch path
   bool small_x_path = true;  // column slots on a small x try the single-launch path first
   int fuse_cap = spmspv::kFuseCap;             // largest bin_len of that path (autotuned)

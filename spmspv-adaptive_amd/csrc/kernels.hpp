@@ -88,17 +88,26 @@ constexpr int kSelEstimated = 0x40;
 // single-launch small-x column path); the bin_len field holds y_nnz. Set
 // in ctl->kernel_choice too, where it shuts every gated launch.
 constexpr int kSelDone = 0x80;
+// Flag kSelGathered: the launch that selected an atomic column slot also did
+// its gather (the products are in acc, the rows in marks); the compaction is
+// left. Set in ctl->kernel_choice too: a launch gated on the slot alone
+// stays shut, a compaction gated on slot and flag runs.
+constexpr int kSelGathered = 0x20;
 __host__ __device__ inline long long sel_word(long long bin_len, int choice) {
   return (bin_len << 8) | (long long)(choice & 0xff);
 }
 __host__ __device__ inline long long sel_word_binlen(long long w) { return w >> 8; }
 __host__ __device__ inline int sel_word_choice(long long w) {
   const int c = (int)(w & 0xff);
-  return c == 0xff ? -1 : (c & 0x3f);
+  return c == 0xff ? -1 : (c & 0x1f);
 }
 __host__ __device__ inline bool sel_word_done(long long w) {
   const int c = (int)(w & 0xff);
   return c != 0xff && (c & kSelDone) != 0;
+}
+__host__ __device__ inline bool sel_word_gathered(long long w) {
+  const int c = (int)(w & 0xff);
+  return c != 0xff && (c & kSelGathered) != 0;
 }
 __host__ __device__ inline bool sel_word_estimated(long long w) {
   const int c = (int)(w & 0xff);
@@ -190,17 +199,20 @@ void launch_clear_keys(hipStream_t s, const int* key, int nnz, float* dense, uns
 // call that does not fit goes on with the usual launches (gated on
 // ctl->kernel_choice, which gets kSelDone when the launch finished the
 // call). In auto mode (sel.mode != 2) a call that fits is reported as
-// kFusedSlot, the sort-based slot whose result it computes. Returns false
-// (nothing launched) when xnnz or m is larger.
+// kFusedSlot, the sort-based slot whose result it computes. With acc set, a
+// call that does not fit and whose slot is an atomic one is gathered into acc
+// and marks (kSelGathered), up to kFuseGather products per workgroup. Returns
+// false (nothing launched) when xnnz or m is larger.
 constexpr int kFuseNT = 1024, kFuseKeys = 4096, kFuseCap = kFuseNT * 11;
 constexpr int kFuseRowsMax = 1 << 26;  // 512 workgroups of kFuseRows: two rounds of one per CU
 constexpr int kFusedSlot = 1;  // SPMSPV_K_COL_NAIVE_SORT
+constexpr int kFuseGather = 4096;
 // cap (<= kFuseCap): largest bin_len that takes the single launch (the
 // autotuner may lower it). state: a look-back word per workgroup.
 bool launch_col_fused(hipStream_t s, const int* colptr, const int* crow, const float* cval, const int* xkey,
                       const float* xval, int ncols, int xnnz, int m, int* ptr, int* xbeg, int* split, Ctl* ctl,
                       const SelectorArgs& sel, int* ykey, float* yval, long long* count_sig, int cap,
-                      unsigned long long* state, Ep ep);
+                      unsigned long long* state, Ep ep, float* acc = nullptr, unsigned char* marks = nullptr);
 
 // --- sort path -----------------------------------------------------------
 // Sorts (bkey, bval)[bin_len] by key (< m) with an LSD radix sort

@@ -21,7 +21,13 @@
 // it: no slot reads less than the products of x) and is reported as
 // kFusedSlot, the sort-based slot, whose result (rows in order, the same on
 // every run) it computes; one that does not fit runs the selector as k_prep
-// does. The workgroup that finishes last sets the done flag in
+// does, and where an atomic column slot is chosen, gathers its products into
+// acc and marks right away: every workgroup has the column bounds in LDS and
+// runs the selector in one wave while the others load their first products, so
+// only the compaction is left to launch. The gather as a launch of its own
+// (and the launch gap) took 11 us for 49,297 products of R-MAT scale 20 (1,049
+// keys, call 37.5 us -> 30.8; 115,997 products 48.8 -> 40.9; 15,999 products
+// of 65,536 rows 29.0 -> 28.1). The workgroup that finishes last sets the done flag in
 // ctl->kernel_choice (which shuts every gated launch queued behind), writes
 // the count to ctl->ynnz, then to *count_sig and the selector word (flagged
 // kSelDone, count in the bin_len field).
@@ -41,26 +47,39 @@ namespace {
 // holds
 constexpr int kFuseRowsMin = 8192, kFuseGrid = 32, kFuseRows = 131072;
 
+// Workgroups at least when the launch may gather: 32 of them took 36.3 us for
+// the 49,297 products above, 64 to 256 of them 32.4 to 32.9 us; 115,997
+// products 42.7, 43.9, 42.4 and 44.8 us with 64, 96, 128 and 256 of them (the
+// gather's loads still behind the selector). Up to kFuseGather products per
+// workgroup it is faster than the gather launch: 466 k products 51.2 -> 42.5,
+// 400 k of 3,000 keys 94.0 -> 81.7 us.
+constexpr int kGatherGrid = 128;
+constexpr int kNaiveAtomicSlot = 0, kLbAtomicSlot = 2;  // SPMSPV_K_COL_NAIVE_ATOMIC, SPMSPV_K_COL_LB_ATOMIC
+
 // One workgroup of 1,024 threads per CU (the sums of kFuseCap rows and the
 // bit array fill its LDS); KPT keys and IPT products per thread.
 template <int NT, int KPT, int IPT>
 __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr, const int* __restrict__ crow,
                                                   const float* __restrict__ cval, const int* __restrict__ xkey,
                                                   const float* __restrict__ xval, int ncols, int xnnz, int m,
-                                                  int rows, int* __restrict__ ptr, int* __restrict__ xbeg,
+                                                  int rows, int nranges, int* __restrict__ ptr, int* __restrict__ xbeg,
                                                   int* __restrict__ split, Ctl* ctl, SelectorArgs sel,
                                                   int* __restrict__ ykey, float* __restrict__ yval,
-                                                  long long* count_sig, int cap, unsigned long long* state, Ep ep) {
+                                                  long long* count_sig, int cap, unsigned long long* state, Ep ep,
+                                                  float* acc, unsigned char* marks) {
   constexpr int NW = NT / kWave, CAP = NT * IPT, KEYS = NT * KPT;
   static_assert(CAP < (1 << 14), "fixed-point sums of a row's products; 16-bit prefix counts");
   static_assert(KEYS < 65536, "16-bit x entries");
   constexpr int WORDS = kFuseRows / 32, WPT = WORDS / NT;
-  // the column scan and the product -> x entry map, then the sums; or the
-  // selector's weights
+  // the column scan and the product -> x entry map (or, when the products do
+  // not fit, the selector's weights), then the sums
   struct Scan {
-    int ptr[KEYS + 1];
+    int ptr[KEYS + 4];
     int beg[KEYS];
-    unsigned short seg[CAP];
+    union {
+      unsigned short seg[CAP];
+      float w[kNWeights];
+    };
   };
   struct Sums {
     unsigned long long q[CAP];
@@ -69,15 +88,15 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
   union Raw {
     Scan scan;
     Sums sums;
-    float w[kNWeights];
   };
   __shared__ __align__(16) Raw s;
   __shared__ unsigned s_bits[WORDS];
   __shared__ unsigned short s_pfx[WORDS];
   __shared__ long long s_l[NW];
-  __shared__ int s_i[NW];
+  __shared__ int s_i[NW], s_mn[NW];
   __shared__ unsigned long long s_pre;
   __shared__ MatFeat s_mf;
+  __shared__ Ctl s_ctl;  // the selector's outputs
   const bool first = blockIdx.x == 0;
   // the selector's weights and matrix features, loaded beside the column
   // scan (stored to LDS only when the products do not fit)
@@ -85,7 +104,7 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
   constexpr int kMF = sizeof(MatFeat) / sizeof(double);
   float wr[kWPT];
   double mfr = 0.0;
-  if (first && sel.mode != 2 && sel.mat) {
+  if ((first || acc) && sel.mode != 2 && sel.mat) {
     if (sel.weights) {
 #pragma unroll
       for (int i = 0; i < kWPT; ++i) {
@@ -122,12 +141,34 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
     }
     tsum += len[j];
   }
-  if (first) {
-    mx = block_max<NT, int>(mx, s_i);
-    mn = block_min<NT, int>(mn, s_i);
+  // sum, longest and shortest column over the workgroup with one barrier
+  long long bl = 0, run;
+  {
+    long long inc = tsum;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const long long u = __shfl_up(inc, o);
+      if (lane() >= o) inc += u;
+      mx = max(mx, __shfl_xor(mx, o));
+      mn = min(mn, __shfl_xor(mn, o));
+    }
+    const int w = threadIdx.x / kWave;
+    if (lane() == kWave - 1) {
+      s_l[w] = inc;
+      s_i[w] = mx;
+      s_mn[w] = mn;
+    }
+    __syncthreads();
+    run = inc - tsum;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) {
+      const long long u = s_l[k];
+      if (k < w) run += u;
+      bl += u;
+      mx = max(mx, s_i[k]);
+      mn = min(mn, s_mn[k]);
+    }
   }
-  long long bl;
-  long long run = block_excl_sum<NT, long long>(tsum, s_l, &bl);
 #pragma unroll
   for (int j = 0; j < KPT; ++j) {
     const int i = base + j;
@@ -164,33 +205,81 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
   }
   const bool fuse = bl <= CAP && bl <= cap && ykey != nullptr && yval != nullptr;
   if (!fuse) {
-    if (!first) return;
-    if (sel.mode == 2 || !sel.mat) {
-      // a fixed slot (or no selector): the gated launches behind run
-      if (threadIdx.x == 0) {
-        if (sel.mode == 2) ctl->kernel_choice = sel.fixed;
-        if (sel.stash) *sel.stash = sel_word(bl, sel.mode == 2 ? sel.fixed : -1);
-      }
-      return;
-    }
-    // the selector, as the last tile of k_prep runs it
-    __syncthreads();  // the scan's LDS is the weights'
-    if (sel.weights) {
+    const bool small = acc && bl <= (long long)gridDim.x * kFuseGather;
+    if (!first && !small) return;
+    const bool net = sel.mode != 2 && sel.mat;
+    __syncthreads();  // the scan is complete
+    if (net) {
+      if (sel.weights) {
 #pragma unroll
-      for (int i = 0; i < kWPT; ++i) {
-        const int idx = threadIdx.x + i * NT;
-        if (idx < kNWeights) s.w[wlds_index(idx)] = wr[i];
+        for (int i = 0; i < kWPT; ++i) {
+          const int idx = threadIdx.x + i * NT;
+          if (idx < kNWeights) s.scan.w[wlds_index(idx)] = wr[i];
+        }
       }
+      if (threadIdx.x < kMF) reinterpret_cast<double*>(&s_mf)[threadIdx.x] = mfr;
+      __syncthreads();
     }
-    if (threadIdx.x < kMF) reinterpret_cast<double*>(&s_mf)[threadIdx.x] = mfr;
-    __syncthreads();
-    SelectorArgs sl = sel;
-    if (sel.weights) sl.weights = s.w;
-    sl.mat = &s_mf;
-    select_in_wave(ctl, sl, (double)xnnz, (double)bl, (double)(xnnz > 0 ? mx : 0));
-    if (sel.stash && threadIdx.x == 0) *sel.stash = sel_word(bl, ctl->kernel_choice);
+    // Wave 0 runs the selector, as the last tile of k_prep does. The other
+    // waves take an equal share of the products, a few per thread and round;
+    // the first round is loaded beside the selector and dropped when another
+    // slot is chosen.
+    constexpr int GPT = 2, GNT = NT - kWave;
+    const int n = small ? (int)bl : 0, step = (int)gridDim.x * GNT;
+    int p0 = threadIdx.x < kWave ? n : (int)blockIdx.x * GNT + (int)threadIdx.x - kWave;
+    int r[GPT];
+    float v[GPT];
+    const auto load = [&]() {
+      int e[GPT];
+#pragma unroll
+      for (int j = 0; j < GPT; ++j) {
+        const int p = min(p0 + j * step, n - 1);
+        int lo = 0, hi = xnnz;  // ptr[lo] <= p < ptr[hi]
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (s.scan.ptr[mid] <= p) lo = mid;
+          else hi = mid;
+        }
+        e[j] = lo;
+        r[j] = s.scan.beg[lo] + (p - s.scan.ptr[lo]);
+      }
+#pragma unroll
+      for (int j = 0; j < GPT; ++j) {
+        v[j] = cval[r[j]] * xval[e[j]];
+        r[j] = crow[r[j]];
+      }
+    };
+    if (p0 < n) load();
+    int choice = sel.mode == 2 ? sel.fixed : -1;
+    if (net) {
+      SelectorArgs sl = sel;
+      if (sel.weights) sl.weights = s.scan.w;
+      sl.mat = &s_mf;
+      select_in_wave(&s_ctl, sl, (double)xnnz, (double)bl, (double)(xnnz > 0 ? mx : 0));
+      __syncthreads();
+      choice = s_ctl.kernel_choice;
+      if (first && threadIdx.x < kF) ctl->feat[threadIdx.x] = s_ctl.feat[threadIdx.x];
+    }
+    const bool gather = small && (choice == kNaiveAtomicSlot || choice == kLbAtomicSlot);
+    if (first && threadIdx.x == 0) {
+      if (choice >= 0) ctl->kernel_choice = choice | (gather ? kSelGathered : 0);
+      if (sel.stash) *sel.stash = sel_word(bl, gather ? choice | kSelGathered : choice);
+    }
+    if (!gather) return;
+    while (p0 < n) {
+#pragma unroll
+      for (int j = 0; j < GPT; ++j) {
+        if (p0 + j * step < n) {
+          atomic_add_f32(acc + r[j], v[j]);
+          marks[r[j]] = 1;
+        }
+      }
+      p0 += GPT * step;
+      if (p0 < n) load();
+    }
     return;
   }
+  if ((int)blockIdx.x >= nranges) return;  // only there for a gather
   __syncthreads();  // the scan is complete
   // products per thread for this call (<= IPT)
   const int ie = (int)((bl + NT - 1) / NT);
@@ -319,10 +408,10 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
   if (threadIdx.x == 0) {
     const unsigned long long count = (unsigned long long)(pre + tot);
     auto* word = reinterpret_cast<unsigned long long*>(&ctl->done[kSlotCount]);
-    const unsigned long long in = (1ull << 32) | (blockIdx.x == gridDim.x - 1 ? count : 0ull);
+    const unsigned long long in = (1ull << 32) | ((int)blockIdx.x == nranges - 1 ? count : 0ull);
     const unsigned long long now =
         __hip_atomic_fetch_add(word, in, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + in;
-    if ((unsigned)(now >> 32) == gridDim.x) {
+    if ((int)(now >> 32) == nranges) {
       __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const long long total = (long long)(unsigned)now;
       const int choice = sel.mode == 2 ? sel.fixed : kFusedSlot;
@@ -342,13 +431,13 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
 bool launch_col_fused(hipStream_t s, const int* colptr, const int* crow, const float* cval, const int* xkey,
                       const float* xval, int ncols, int xnnz, int m, int* ptr, int* xbeg, int* split, Ctl* ctl,
                       const SelectorArgs& sel, int* ykey, float* yval, long long* count_sig, int cap,
-                      unsigned long long* state, Ep ep) {
+                      unsigned long long* state, Ep ep, float* acc, unsigned char* marks) {
   if (xnnz > kFuseKeys || m > kFuseRowsMax) return false;
   const int grid = std::max(std::min(kFuseGrid, (m + kFuseRowsMin - 1) / kFuseRowsMin), (m + kFuseRows - 1) / kFuseRows);
-  const int rows = (m + grid - 1) / grid;
-  hipLaunchKernelGGL((k_col_fused<kFuseNT, kFuseKeys / kFuseNT, kFuseCap / kFuseNT>), dim3((m + rows - 1) / rows),
-                     dim3(kFuseNT), 0, s, colptr, crow, cval, xkey, xval, ncols, xnnz, m, rows, ptr, xbeg, split, ctl,
-                     sel, ykey, yval, count_sig, cap, state, ep);
+  const int rows = (m + grid - 1) / grid, ranges = (m + rows - 1) / rows;
+  hipLaunchKernelGGL((k_col_fused<kFuseNT, kFuseKeys / kFuseNT, kFuseCap / kFuseNT>), dim3(acc ? std::max(ranges, kGatherGrid) : ranges),
+                     dim3(kFuseNT), 0, s, colptr, crow, cval, xkey, xval, ncols, xnnz, m, rows, ranges, ptr, xbeg, split, ctl,
+                     sel, ykey, yval, count_sig, cap, state, ep, acc, marks);
   return true;
 }
 
