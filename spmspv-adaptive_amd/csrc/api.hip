@@ -112,6 +112,7 @@ static size_t carve(spmspv_handle_t h, char* base) {
   sb.valB = c.take<float>(nnz);
   const size_t dscan_tiles = sort_tiles * 256 / kDScanTile + 2;
   sb.dcount = c.take<unsigned>(sort_tiles * 256);
+  sb.dchunk = c.take<unsigned long long>((size_t)4 * kChunkRows * 64);
   sb.dstate = c.take<unsigned long long>(dscan_tiles);
   sb.red_state = c.take<unsigned long long>(red_tiles);
   sb.carry_val = c.take<float>(red_tiles);
@@ -528,6 +529,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
     } else {
       h->gate = Gate{&h->ctl->kernel_choice, kid};
       h->spec_cap = h->nnz;
+      h->spec_big = false;
       gate_restore.on = true;
     }
   }
@@ -592,7 +594,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       // 23 in the reduce at R-MAT s22, 1 %)
       const long long most = h->gate.word ? h->spec_cap : h->nnz;
       launch_sort_reduce(s, h->sb, m, h->ctl, ok, ov, hint, most, next_ep(h, 5), h->gate, h->small_sort_cap,
-                         hint > h->small_sort_cap && !y_dense ? count_sig() : nullptr);
+                         y_dense ? nullptr : count_sig(), h->gate.word && h->spec_big);
       h->launches += 6;
       if (y_dense) {
         launch_fill_f32(s, y_dense, m, 0.f, h->gate);
@@ -1470,6 +1472,7 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   // compaction is queued
   const bool spec_gathered = spec && fused && h->spec_gathered[cls] &&
                              (guess == SPMSPV_K_COL_NAIVE_ATOMIC || guess == SPMSPV_K_COL_LB_ATOMIC);
+  bool spec_sent = false;  // the slot's own launches send the count
   if (spec) {
     struct Ungate {
       spmspv_handle_t h;
@@ -1481,11 +1484,13 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
     h->x_gathered = spec_gathered;
     h->gate = Gate{&h->ctl->kernel_choice, spec_gathered ? guess | kSelGathered : guess};
     h->spec_cap = h->nnz;
-    if (h->spec_binlen[cls] > 0) h->spec_cap = std::min<long long>(h->nnz, 4 * h->spec_binlen[cls] + 65536);
+    if (h->spec_binlen[cls] > 0) h->spec_cap = std::min<long long>(h->nnz, 2 * h->spec_binlen[cls] + 65536);
+    h->spec_big = h->spec_binlen[cls] > 8 * h->small_sort_cap;
     h->count_to_host = y_nnz != nullptr;
     rc = run_kernel(h, guess, d_y_dense, d_y_key, d_y_val, y_nnz != nullptr);
     h->count_to_host = false;
     if (rc) return rc;
+    spec_sent = h->count_sent;
     if (y_nnz && !h->count_sent) {
       __atomic_store_n(h->sig + 3, kSigPending, __ATOMIC_RELEASE);
       launch_signal_int(h->stream, &h->ctl->ynnz, h->sig_dev + 3, h->gate);
@@ -1516,8 +1521,10 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
   h->spec_last[cls] = (signed char)(kid + 1);
   if (kernel_used) *kernel_used = kid;
   if (h->binlen_host >= 0) h->spec_binlen[cls] = h->binlen_host;
-  const bool sorts = kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_SORT;
-  if (spec && kid == guess && gathered == spec_gathered && !(sorts && h->binlen_host > h->spec_cap)) {
+  // a sort slot's queued launches may not cover this many (or this few) products
+  const bool uncovered = (kid == SPMSPV_K_COL_NAIVE_SORT || kid == SPMSPV_K_COL_LB_SORT) &&
+                         (h->binlen_host > h->spec_cap || (h->spec_big && h->binlen_host <= h->small_sort_cap));
+  if (spec && kid == guess && gathered == spec_gathered && !uncovered) {
     h->spec_hits++;
     // the gated tile kernel ran, and with it the clearing of the idle buffer
     if (clear_pending >= 0) h->enc5_clean[clear_pending] = true;
@@ -1529,9 +1536,9 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
     return SPMSPV_SUCCESS;
   }
   if (spec) h->spec_misses++;
-  if (spec && kid == guess && sorts && y_nnz) {
-    // more products than the queued sort covers: its launches left the result
-    // alone, but the count of an earlier one is on its way to the host word
+  if (spec && kid == guess && uncovered && y_nnz && !spec_sent) {
+    // the queued sort left the result alone, but the count of an earlier one is
+    // on its way to the host word
     long long v = 0;
     if ((rc = wait_signal(h, 3, &v))) return rc;
   }

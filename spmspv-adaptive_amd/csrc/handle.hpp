@@ -161,9 +161,11 @@ struct spmspv_handle_s {
   int fuse_cap = spmspv::kFuseCap;             // largest bin_len of that path (autotuned)
   int small_sort_cap = spmspv::kSmallSortCap;  // largest single-workgroup sort (autotuned)
   long long spec_hits = 0, spec_misses = 0;
-  // the sort slots' speculative launches cover spec_cap products: a few times
-  // what the last call of the size class had (an x with more is a wrong guess)
+  // the sort slots' speculative launches cover spec_cap products: twice what
+  // the last call of the size class had and some; with spec_big, none that the
+  // single-workgroup sort would take (an x outside is a wrong guess)
   long long spec_binlen[33] = {}, spec_cap = 0;
+  bool spec_big = false;
 
   float* dense_x() { return x_dense_user ? x_dense_user : x_dense_int; }
   unsigned* bits() { return bits_user ? bits_user : bits_int; }

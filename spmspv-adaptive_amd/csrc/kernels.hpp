@@ -18,6 +18,7 @@ constexpr int kPrepNT = 256, kPrepIPT = 8, kPrepTile = kPrepNT * kPrepIPT;
 constexpr int kLbNT = 256, kLbVT = 7, kLbTile = kLbNT * kLbVT;
 constexpr int kCmpNT = 256;  // bit-array words per compaction tile (8,192 rows, 8 per thread)
 constexpr int kSortNT = 256, kSortIPT = 12, kSortTile = kSortNT * kSortIPT;
+constexpr int kChunk = 16, kChunkRows = 100;  // tiles of a chunk of the digit counts, chunks at most
 constexpr int kDScanNT = 256, kDScanIPT = 8, kDScanTile = kDScanNT * kDScanIPT;
 constexpr int kRedNT = 256, kRedIPT = 7, kRedTile = kRedNT * kRedIPT;
 constexpr int kRowNT = 256, kRowVT = 7, kRowTile = kRowNT * kRowVT;
@@ -224,6 +225,7 @@ struct SortBufs {
   unsigned* keyB;
   float* valB;
   unsigned* dcount;     // 256 per sort tile: per-tile digit counts, then their scan
+  unsigned long long* dchunk;     // 4 * kChunkRows * 64: digit counts per kChunk tiles, 0 between sorts but for the last pass's
   unsigned long long* dstate;     // look-back words of the digit-count scan
   unsigned long long* red_state;  // per reduce tile
   float* carry_val;
@@ -238,12 +240,12 @@ struct SortSet {
 // n_hint: item count when the host knows it (exact grids), else -1 and the
 // grids cover n_cap; with more items than n_cap nothing is sorted. ep: first of the 5 epochs the sort + reduce use.
 // small_cap (<= kSmallSortCap): largest item count that takes the
-// single-workgroup path (the autotuner may lower it). sig (only with
-// binlen_hint > small_cap): the result count goes there once the results are
-// visible.
+// single-workgroup path (the autotuner may lower it); skip_small: nothing is
+// done for that many. sig: the result count goes there once the results are
+// visible (and nothing when nothing is sorted).
 void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* ykey, float* yval,
                         long long binlen_hint, long long n_cap, Ep ep, Gate g = {},
-                        int small_cap = kSmallSortCap, long long* sig = nullptr);
+                        int small_cap = kSmallSortCap, long long* sig = nullptr, bool skip_small = false);
 // Sorts in[*n_dev] by key < range, stable, its passes writing out0 and out1 in
 // turn (`in` may be out1, and is not written otherwise); returns which of the
 // two holds the result. With ep.dev >= 0 (captured graphs) the passes use

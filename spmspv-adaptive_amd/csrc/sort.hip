@@ -5,9 +5,10 @@
 // 1030-1152), written for wave64:
 //  * keys are ranked inside a tile with 8 wave ballots per key (peers with
 //    the same 8-bit digit) and per-wave digit counters in LDS (stable);
-//  * each pass counts digits per tile, scans the digit-major count array
-//    (one small look-back scan over 256 x tiles entries) and scatters, so no
-//    tile waits on a chain of earlier tiles;
+//  * each pass counts digits per tile, turns the counts into positions (the
+//    scatter's workgroups sum them; for many tiles one small look-back scan
+//    over 256 x tiles entries) and scatters, so no tile waits on a chain of
+//    earlier tiles;
 //  * tiles are re-ordered in LDS before the store so that runs of equal
 //    digits leave as contiguous, coalesced writes;
 //  * n <= one tile takes a single-workgroup path that sorts all passes in
@@ -119,11 +120,9 @@ __device__ __forceinline__ long long tile_reduce(const unsigned* s_k, const floa
   return gpre + htot;
 }
 
-// ------------------------------------------------------------- histogram
-// Digit counts of every pass into hist[pass][256] (zeroed by the caller's
-// preceding fill); each pass kernel scans its row of it.
 // ------------------------------------------------------------ one pass
-// A pass is three launches, with no look-back chain between tiles:
+// A pass is three launches (two where the counts are summed in the scatter),
+// with no look-back chain between tiles:
 //   k_digit_count  per-tile digit counts, digit-major: cnt[d * ntiles + t];
 //   k_digit_scan   exclusive scan of that array in place, so that
 //                  cnt[d * ntiles + t] becomes the global position of the
@@ -132,6 +131,25 @@ __device__ __forceinline__ long long tile_reduce(const unsigned* s_k, const floa
 // (With every tile resident at once, a per-digit decoupled look-back
 // spends most of the pass waiting for the prefix to crawl along the tile
 // chain; the scan of 256 x ntiles counts costs a few microseconds.)
+// Smaller sorts have no scan: the counts are 16 bits wide and tile-major,
+// cnt[t << bits | d], k_digit_count also adds them up per kChunk tiles
+// (chunk, a buffer for each pass: cleared by the next pass, or by the first
+// pass of the next sort), and every scatter workgroup sums the chunks and the
+// tiles of its own chunk itself while its keys are on their way. The
+// scan is 6 us and a launch gap per pass whatever the size; the sums cost what
+// is read for them, tiles * (chunks + half a chunk) rows. The whole slot (3
+// passes of 7 bits): 391 k products 93.9 -> 82.6 us, 1.53 M 114.9 -> 102.9,
+// 2.93 M 137.1 -> 128.7; (8 + 7 + 7): 0.81 M 111.0 -> 99.0, 3.02 M 152.5 ->
+// 142.3, 3.44 M (its 8-bit pass over the line) 166.5 -> 163.9. Nothing more was
+// gained above the line (5.6 M: 227.0 without it, 226.1 with the scan).
+constexpr long long kDirectReads = 20 << 20;
+constexpr int kChunkWords = kChunkRows * 64;  // 64-bit words (4 digits) of a pass's buffer
+__host__ __device__ inline bool counts_direct(long long ntiles, int bits) {
+  return ntiles <= kChunkRows * kChunk && (ntiles * (ntiles / kChunk + kChunk / 2)) << bits <= kDirectReads;
+}
+static_assert(kChunk * kSortTile < 65536, "16-bit digit counts of a chunk");
+// digits of a row of those counts (whole 8-byte words)
+__host__ __device__ inline int direct_row(int bits) { return bits < 2 ? 4 : 1 << bits; }
 
 // Keys of tile t in the wave-major layout of wave_rank.
 template <int NT, int IPT>
@@ -150,7 +168,8 @@ __device__ __forceinline__ void load_tile_keys(const unsigned* __restrict__ kin,
 template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__ kin,
                                                     const long long* __restrict__ n_dev, int shift, int bits,
-                                                    unsigned* __restrict__ cnt, int small_cap,
+                                                    unsigned* __restrict__ cnt,
+                                                    unsigned long long* __restrict__ chunk, int pass, int small_cap,
                                                     long long n_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
@@ -162,6 +181,11 @@ __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__
   if (n <= small_cap || n > n_cap) return;
   const unsigned ntiles = (unsigned)((n + TILE - 1) / TILE);
   const int w = threadIdx.x / kWave;
+  if (chunk) {
+    const int first = pass == 0 ? 1 : pass - 1, last = pass == 0 ? 4 : pass;
+    for (int i = first * kChunkWords + blockIdx.x * NT + threadIdx.x; i < last * kChunkWords; i += gridDim.x * NT)
+      chunk[i] = 0ull;
+  }
   // tiles are independent: any grid covers them. Only counts are needed
   // here (no ranks): LDS atomics into a private histogram per wave. Lanes that
   // add to one LDS word take turns, so where many lanes hold the first lane's
@@ -190,7 +214,20 @@ __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__
     unsigned tot = 0;
 #pragma unroll
     for (int q = 0; q < NW; ++q) tot += s_cnt[q * 256 + threadIdx.x];
-    if (threadIdx.x <= mask) cnt[(size_t)threadIdx.x * ntiles + t] = tot;
+    if (chunk && counts_direct(ntiles, bits)) {
+      const int row = direct_row(bits);
+      if ((int)threadIdx.x < row) reinterpret_cast<unsigned short*>(cnt)[t * row + threadIdx.x] = (unsigned short)tot;
+      s_cnt[threadIdx.x] = tot;
+      __syncthreads();
+      if ((int)threadIdx.x < row / 4) {
+        unsigned long long four = 0ull;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) four |= (unsigned long long)s_cnt[threadIdx.x * 4 + k] << (16 * k);
+        if (four) atomicAdd(chunk + (size_t)pass * kChunkWords + t / kChunk * (row / 4) + threadIdx.x, four);
+      }
+    } else if (threadIdx.x <= mask) {
+      cnt[(size_t)threadIdx.x * ntiles + t] = tot;
+    }
     __syncthreads();
   }
 }
@@ -200,7 +237,7 @@ __global__ __launch_bounds__(NT) void k_digit_count(const unsigned* __restrict__
 template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
                                                    const long long* __restrict__ n_dev, int sort_tile,
-                                                   int bits, int small_cap, long long n_cap,
+                                                   int bits, bool chunks, int small_cap, long long n_cap,
                                                    unsigned long long* state, Ctl* ctl,
                                                    Ep epa, Gate g) {
   if (gate_shut(g)) return;
@@ -208,6 +245,7 @@ __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
   __shared__ unsigned s_t[NT / kWave];
   const long long n = *n_dev;
   if (n <= small_cap || n > n_cap) return;
+  if (chunks && counts_direct((n + sort_tile - 1) / sort_tile, bits)) return;
   const long long E = ((n + sort_tile - 1) / sort_tile) << bits;
   const unsigned nb = (unsigned)((E + NT * IPT - 1) / (NT * IPT));
   const unsigned t = blockIdx.x;
@@ -235,11 +273,82 @@ __global__ __launch_bounds__(NT) void k_digit_scan(unsigned* __restrict__ cnt,
   }
 }
 
-// PAY: payload words per item (0: keys only).
+// Global start of digit threadIdx.x in tile t from the 16-bit counts, by the
+// whole workgroup: 8-byte loads of 4 digits (16-byte ones take the registers
+// of a wave per SIMD), the rows (every chunk's, then those of the earlier
+// tiles of t's chunk) split over the groups of lanes that cover a row. s_a,
+// s_b: NW * 256 words each; the caller syncs before it uses them again.
+template <int NT>
+__device__ __forceinline__ unsigned direct_start(const unsigned* cnt, const unsigned long long* chunk, unsigned t,
+                                                 unsigned ntiles, int bits, unsigned* s_a, unsigned* s_b,
+                                                 unsigned* s_t) {
+  constexpr int NW = NT / kWave, U = 4;
+  const int row = direct_row(bits), lpr = row / 4;
+  const unsigned grp = NT / lpr;
+  const int c = threadIdx.x % lpr;
+  const unsigned mine = t / kChunk, nch = (ntiles + kChunk - 1) / kChunk, rows = nch + t % kChunk;
+  const uint2* pc = reinterpret_cast<const uint2*>(chunk) + c;
+  const uint2* pt = reinterpret_cast<const uint2*>(cnt) + (size_t)mine * kChunk * lpr + c;
+  unsigned before[4], all[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) before[k] = all[k] = 0u;
+  for (unsigned u0 = threadIdx.x / lpr; u0 < rows; u0 += grp * U) {
+    uint2 v[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const unsigned u = min(u0 + j * grp, rows - 1);
+      v[j] = *(u < nch ? pc + (size_t)u * lpr : pt + (size_t)(u - nch) * lpr);
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const unsigned u = u0 + j * grp;
+      const unsigned mb = u < mine || (u >= nch && u < rows) ? ~0u : 0u, ma = u < nch ? ~0u : 0u;
+      const unsigned w[2] = {v[j].x, v[j].y};
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        before[2 * k] += w[k] & mb & 0xFFFFu;
+        before[2 * k + 1] += (w[k] & mb) >> 16;
+        all[2 * k] += w[k] & ma & 0xFFFFu;
+        all[2 * k + 1] += (w[k] & ma) >> 16;
+      }
+    }
+  }
+  // the groups of a wave, then the waves
+  for (int o = lpr; o < kWave; o <<= 1) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      before[k] += __shfl_xor(before[k], o);
+      all[k] += __shfl_xor(all[k], o);
+    }
+  }
+  if (lane() < lpr) {
+    const int w = threadIdx.x / kWave;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      s_a[w * 256 + c * 4 + k] = before[k];
+      s_b[w * 256 + c * 4 + k] = all[k];
+    }
+  }
+  __syncthreads();
+  unsigned b = 0u, a = 0u;  // items of the digit before the tile, and in all tiles
+  if ((int)threadIdx.x < row) {
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      b += s_a[w * 256 + threadIdx.x];
+      a += s_b[w * 256 + threadIdx.x];
+    }
+  }
+  unsigned tot;
+  return block_excl_sum<NT, unsigned>(a, s_t, &tot) + b;
+}
+
+// PAY: payload words per item (0: keys only). Four waves per SIMD (three with
+// two payloads, as LDS allows): five spill the payloads (R-MAT scale 22, 1 %:
+// 105.5 -> 110.7 us).
 template <int NT, int IPT, int PAY>
-__global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, const long long* __restrict__ n_dev,
+__global__ __launch_bounds__(NT, PAY > 1 ? 3 : 4) void k_sort_scatter(SortSet in, SortSet out, const long long* __restrict__ n_dev,
                                                      int shift, int bits, const unsigned* __restrict__ pos0,
-                                                     int small_cap, long long n_cap, Gate g) {
+                                                     const unsigned long long* __restrict__ chunk, int small_cap, long long n_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
@@ -261,7 +370,8 @@ __global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, co
   for (unsigned t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const long long base = (long long)t * TILE;
     // this tile's global start of digit d, from the scan (issued with the keys)
-    const unsigned gb = pos0[(size_t)(d & mask) * ntiles + t];
+    const bool direct = chunk && counts_direct(ntiles, bits);
+    unsigned gb = direct ? 0u : pos0[(size_t)(d & mask) * ntiles + t];
     unsigned key[IPT], pv[IPT], pw[IPT];
     bool valid[IPT];
     int rank[IPT];
@@ -272,6 +382,10 @@ __global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, co
       const long long gi = base + (long long)w * kWave * IPT + j * kWave + lane();
       if (PAY > 0) pv[j] = in.v[valid[j] ? gi : n - 1];
       if (PAY > 1) pw[j] = in.w[valid[j] ? gi : n - 1];
+    }
+    if (direct) {
+      gb = direct_start<NT>(pos0, chunk, t, ntiles, bits, s_cnt, s_k, s_t);
+      __syncthreads();
     }
     wave_rank<IPT>(key, valid, shift, s_cnt + w * 256, rank, dig, IPT, bits);
     __syncthreads();
@@ -309,7 +423,7 @@ __global__ __launch_bounds__(NT) void k_sort_scatter(SortSet in, SortSet out, co
 template <int NT, int IPT, int PAY>
 __global__ __launch_bounds__(NT) void k_sort_small(SortSet in, const long long* __restrict__ n_dev, int passes,
                                                    int mode, Ctl* ctl, int* ykey, float* yval, SortSet out,
-                                                   int cap, Gate g) {
+                                                   int cap, long long* sig, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
@@ -386,6 +500,11 @@ __global__ __launch_bounds__(NT) void k_sort_small(SortSet in, const long long* 
   if (threadIdx.x == 0) {
     ctl->ynnz = (int)tot;
     ctl->sort_small = 1;
+  }
+  if (sig) {  // the result first, then its count
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) *sig = tot;
   }
 }
 
@@ -498,18 +617,19 @@ static int tiles_grid(long long n_hint, long long n_cap, int tile) {
 // the device-side count exit at once. small_cap: passes do nothing when
 // n <= small_cap (the single-workgroup path handled them).
 static void launch_digit_pass(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out, int shift,
-                              int bits, const long long* n_dev, Ctl* ctl, long long n_hint, long long n_cap,
-                              int small_cap, Ep e, Gate g) {
+                              int bits, int pass, bool chunks, const long long* n_dev, Ctl* ctl, long long n_hint,
+                              long long n_cap, int small_cap, Ep e, Gate g) {
   const int tiles = tiles_grid(n_hint, n_cap, kSortTile);
   const int pgrid = std::min(tiles, 2048);  // count / scatter loop over their tiles
   const int sgrid = (int)std::max<long long>(1, (((long long)tiles << bits) + kDScanTile - 1) / kDScanTile);
   hipLaunchKernelGGL((k_digit_count<kSortNT, kSortIPT>), dim3(pgrid), dim3(kSortNT), 0, s, in.k, n_dev,
-                     shift, bits, b.dcount, small_cap, n_cap, g);
-  hipLaunchKernelGGL((k_digit_scan<kDScanNT, kDScanIPT>), dim3(sgrid), dim3(kDScanNT), 0, s, b.dcount,
-                     n_dev, kSortTile, bits, small_cap, n_cap, b.dstate, ctl, e, g);
+                     shift, bits, b.dcount, chunks ? b.dchunk : nullptr, pass, small_cap, n_cap, g);
+  if (!chunks || !counts_direct(tiles, bits))
+    hipLaunchKernelGGL((k_digit_scan<kDScanNT, kDScanIPT>), dim3(sgrid), dim3(kDScanNT), 0, s, b.dcount,
+                       n_dev, kSortTile, bits, chunks, small_cap, n_cap, b.dstate, ctl, e, g);
 #define SPMSPV_SCATTER(PAY)                                                                                  \
   hipLaunchKernelGGL((k_sort_scatter<kSortNT, kSortIPT, PAY>), dim3(pgrid), dim3(kSortNT), 0, s, in, out, n_dev, \
-                     shift, bits, b.dcount, small_cap, n_cap, g)
+                     shift, bits, b.dcount, chunks ? b.dchunk + pass * kChunkWords : nullptr, small_cap, n_cap, g)
   if (in.w) SPMSPV_SCATTER(2);
   else if (in.v) SPMSPV_SCATTER(1);
   else SPMSPV_SCATTER(0);
@@ -517,12 +637,12 @@ static void launch_digit_pass(hipStream_t s, const SortBufs& b, const SortSet& i
 }
 
 // The digits of a key of key_bits(range) bits are as equal as they can be:
-// 20 bits are 7 + 7 + 6, not 8 + 8 + 4 (fewer ballots per item and counts per
+// 20 bits are 7 + 7 + 6, not 8 + 8 + 4, and 22 are 8 + 7 + 7 (fewer ballots per item and counts per
 // tile, longer runs of equal digits to store).
 int launch_radix_sets(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out0, const SortSet& out1,
                       int range, const long long* n_dev, Ctl* ctl, long long n_hint, long long n_cap,
                       bool skip_small, Ep ep, Gate g, int small_cap) {
-  const int total = key_bits(range), passes = key_passes(range), per = (total + passes - 1) / passes;
+  const int total = key_bits(range), passes = key_passes(range);
   const int last = (passes & 1) ? 0 : 1;
   const SortSet outs[2] = {out0, out1};
   const bool small_known = n_hint >= 0 && n_hint <= small_cap;
@@ -530,17 +650,17 @@ int launch_radix_sets(hipStream_t s, const SortBufs& b, const SortSet& in, const
   if (!big_known && !skip_small) {
 #define SPMSPV_SMALL(PAY)                                                                                \
   hipLaunchKernelGGL((k_sort_small<kSortNT, kSortIPT, PAY>), dim3(1), dim3(kSortNT), 0, s, in, n_dev, passes, 1, \
-                     ctl, nullptr, nullptr, outs[last], small_cap, g)
+                     ctl, nullptr, nullptr, outs[last], small_cap, nullptr, g)
     if (in.w) SPMSPV_SMALL(2);
     else if (in.v) SPMSPV_SMALL(1);
     else SPMSPV_SMALL(0);
 #undef SPMSPV_SMALL
   }
   if (small_known) return last;
-  for (int p = 0; p < passes; ++p) {
+  for (int p = 0, shift = 0, bits; p < passes; ++p, shift += bits) {
     const Ep e{ep.v + (unsigned)p, ep.dev < 0 ? -1 : ep.dev + p};
-    const int shift = p * per, bits = std::min(per, total - shift);
-    launch_digit_pass(s, b, p == 0 ? in : outs[(p - 1) & 1], outs[p & 1], shift, bits, n_dev, ctl, n_hint, n_cap,
+    bits = (total - shift + passes - p - 1) / (passes - p);
+    launch_digit_pass(s, b, p == 0 ? in : outs[(p - 1) & 1], outs[p & 1], shift, bits, p, passes > 1, n_dev, ctl, n_hint, n_cap,
                       small_cap, e, g);
   }
   return last;
@@ -557,14 +677,14 @@ int launch_radix_sort(hipStream_t s, const SortBufs& b, int range, const long lo
 }
 
 void launch_sort_reduce(hipStream_t s, const SortBufs& b, int m, Ctl* ctl, int* ykey, float* yval,
-                        long long binlen_hint, long long n_cap, Ep ep, Gate g, int small_cap, long long* sig) {
+                        long long binlen_hint, long long n_cap, Ep ep, Gate g, int small_cap, long long* sig,
+                        bool skip_small) {
   const long long* n_dev = &ctl->bin_len;
   const int passes = key_passes(m);
   const bool small_known = binlen_hint >= 0 && binlen_hint <= small_cap;
-  const bool big_known = binlen_hint > small_cap;
-  if (!big_known) {
+  if (binlen_hint <= small_cap && !skip_small) {
     hipLaunchKernelGGL((k_sort_small<kSortNT, kSortIPT, 1>), dim3(1), dim3(kSortNT), 0, s, set_a(b), n_dev, passes, 0,
-                       ctl, ykey, yval, SortSet{}, small_cap, g);
+                       ctl, ykey, yval, SortSet{}, small_cap, sig, g);
   }
   if (small_known) return;
   const int fb = launch_radix_sort(s, b, m, n_dev, ctl, binlen_hint, n_cap, true, ep, g, small_cap);
