@@ -66,6 +66,11 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
                                              int* __restrict__ xbeg, int* __restrict__ split,
                                              unsigned long long* state, int* tile_mm, Ctl* ctl,
                                              Ep ep, SelectorArgs sel, long long* samp) {
+  struct Red {
+    long long sum, ssum;
+    int mx, mn, smx;
+  };
+  __shared__ Red s_red[NT / kWave];
   __shared__ unsigned long long s_pre;
   __shared__ long long s_l[NT / kWave];
   __shared__ int s_i[NT / kWave];
@@ -182,13 +187,38 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
   // above are in, instead of after its look-back (the barrier below
   // publishes them)
   if (selects) stage();
-  mx = block_max<NT, int>(mx, s_i);
-  mn = block_min<NT, int>(mn, s_i);
-  long long ssum = 0;
-  int smx = 0;
-  if (my_samp) {
-    ssum = block_sum<NT, long long>((long long)slen, s_l);
-    smx = block_max<NT, int>(slen, s_i);
+  // sum, longest and shortest column, and the sample's sum and longest, over
+  // the workgroup with one barrier
+  long long bex, btot = 0, ssum = slen;
+  int smx = slen;
+  {
+    long long inc = tsum;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const long long u = __shfl_up(inc, o);
+      if (lane() >= o) inc += u;
+      mx = max(mx, __shfl_xor(mx, o));
+      mn = min(mn, __shfl_xor(mn, o));
+      if (my_samp) {
+        ssum += __shfl_xor(ssum, o);
+        smx = max(smx, __shfl_xor(smx, o));
+      }
+    }
+    const int w = threadIdx.x / kWave;
+    if (lane() == kWave - 1) s_red[w] = Red{inc, ssum, mx, mn, smx};
+    __syncthreads();
+    bex = inc - tsum;
+    ssum = 0;
+#pragma unroll
+    for (int q = 0; q < NT / kWave; ++q) {
+      const Red u = s_red[q];
+      if (q < w) bex += u.sum;
+      btot += u.sum;
+      ssum += u.ssum;
+      mx = max(mx, u.mx);
+      mn = min(mn, u.mn);
+      smx = max(smx, u.smx);
+    }
   }
   // a single tile (small x) needs neither the look-back nor the tile max/min
   const bool single = ntiles == 1;
@@ -204,8 +234,6 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  long long btot;
-  const long long bex = block_excl_sum<NT, long long>(tsum, s_l, &btot);
   const unsigned long long pre =
       single ? 0ull : tile_prefix(state, t, epoch, (unsigned long long)btot, &s_pre);
   long long run = (long long)pre + bex;
@@ -612,7 +640,7 @@ void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, i
 
 // ---------------------------------------------------------------- batch
 // Selector inputs and choice of every vector of a batch, a workgroup per tile
-// of kPrepTile keys: the workgroup of a vector that finishes last adds up the
+// of kBatchTile keys: the workgroup of a vector that finishes last adds up the
 // vector's tiles (exact bin_len, longest column; sampled inputs for a large
 // x, as everywhere) and runs the selector. One launch per vector took 12 us
 // for each of them.
@@ -752,7 +780,7 @@ __global__ __launch_bounds__(NT) void k_batch_scan(const int* __restrict__ colpt
 void launch_batch_select(hipStream_t s, const int* colptr, const int* xkey, int ncols, int ntiles, const int* tile_vec,
                          const BatchVec* vec, long long* tsum, int* tmax, unsigned* arrive, Ctl* ctls,
                          const SelectorArgs& sel, long long* stash) {
-  hipLaunchKernelGGL((k_batch_select<kPrepNT, kPrepIPT>), dim3(ntiles), dim3(kPrepNT), 0, s, colptr, xkey, ncols,
+  hipLaunchKernelGGL((k_batch_select<kPrepNT, kBatchIPT>), dim3(ntiles), dim3(kPrepNT), 0, s, colptr, xkey, ncols,
                      tile_vec, vec, tsum, tmax, arrive, ctls, sel, stash);
 }
 
@@ -760,7 +788,7 @@ void launch_batch_scan(hipStream_t s, const int* colptr, const int* xkey, int nc
                        const int* tile_vec, const BatchVec* vec, const long long* tsum, int key_base, int* ptr,
                        int* xbeg, int* split) {
   if (nlist > 0)
-    hipLaunchKernelGGL((k_batch_scan<kPrepNT, kPrepIPT>), dim3(nlist), dim3(kPrepNT), 0, s, colptr, xkey, ncols, list,
+    hipLaunchKernelGGL((k_batch_scan<kPrepNT, kBatchIPT>), dim3(nlist), dim3(kPrepNT), 0, s, colptr, xkey, ncols, list,
                        tile_vec, vec, tsum, key_base, ptr, xbeg, split);
 }
 

@@ -12,7 +12,14 @@
 namespace spmspv {
 
 // Tile geometry (one place, so the arena sizing in the handle agrees).
-constexpr int kPrepNT = 256, kPrepIPT = 8, kPrepTile = kPrepNT * kPrepIPT;
+// Tile of the column scan: a chain of round trips (keys, column bounds, look-
+// back), so the tiles are small while the look-back stays short. 105 k keys of
+// R-MAT scale 20: 15.1 us with 8 keys per thread, 12.8 with 4, 12.3 with 2; the
+// eight levels of a BFS on scale 22 (up to 10^6 keys) 125, 113 and 116 us.
+constexpr int kPrepNT = 256, kPrepIPT = 4, kPrepTile = kPrepNT * kPrepIPT;
+// The scans of many vectors in one launch fill the chip as they are (48 vectors
+// of R-MAT scale 20: 29 us with 8 keys per thread, 38 with 4).
+constexpr int kBatchIPT = 8, kBatchTile = kPrepNT * kBatchIPT;
 // odd items per thread: a lane walking VT consecutive LDS words then hits
 // a different bank than its neighbours (stride 7 is coprime with 32 banks)
 constexpr int kLbNT = 256, kLbVT = 7, kLbTile = kLbNT * kLbVT;
@@ -122,7 +129,7 @@ void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, i
                  int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp = nullptr);
 // The vectors of a batch: one launch selects for all of them, one scans all
 // that need it. Vector v has keys xkey[key0 .. key0 + xnnz), tiles
-// [tile0, tile0 + ntiles) of kPrepTile keys (at least one) and, once its
+// [tile0, tile0 + ntiles) of kBatchTile keys (at least one) and, once its
 // slot is known, splits from split0.
 struct BatchVec {
   int key0, xnnz, tile0, ntiles;
