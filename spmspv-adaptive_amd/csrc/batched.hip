@@ -68,7 +68,7 @@ struct Layout {
   }
 };
 
-size_t tiles_of(size_t keys) { return std::max<size_t>(1, (keys + kBatchTile - 1) / kBatchTile); }
+size_t tiles_of(size_t keys) { return std::max<size_t>(1, (keys + kWideTile - 1) / kWideTile); }
 
 int grow(spmspv_handle_t h, size_t bytes, size_t splits) {
   if (!h->batch) h->batch = new BatchState();
@@ -96,7 +96,7 @@ int grow(spmspv_handle_t h, size_t bytes, size_t splits) {
 
 namespace spmspv {
 int batch_alloc(spmspv_handle_t h) {
-  const size_t tiles = kBatchKeys / kBatchTile + kBatchVecs + 1;
+  const size_t tiles = kBatchKeys / kWideTile + kBatchVecs + 1;
   return grow(h, Layout(kBatchVecs, kBatchKeys, tiles).bytes + kBatchSplits * sizeof(int), 0);
 }
 

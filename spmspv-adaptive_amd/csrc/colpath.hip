@@ -628,19 +628,24 @@ void launch_select_feat(hipStream_t s, const int* colptr, const int* xkey, const
 
 void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, int xnnz,
                  const int* xnnz_dev, int* ptr, int* xbeg, int* split, unsigned long long* state,
-                 int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp) {
+                 int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp, bool wide) {
   // exact grid when the host knows xnnz, else the bound from ncols
   const long long cnt = xnnz_dev ? ncols : xnnz;
-  const int grid = (int)std::max<long long>(1, (cnt + kPrepTile - 1) / kPrepTile);
+  const int tile = wide ? kWideTile : kPrepTile;
+  const int grid = (int)std::max<long long>(1, (cnt + tile - 1) / tile);
   SelectorArgs a{};
   if (sel) a = *sel;
-  hipLaunchKernelGGL((k_prep<kPrepNT, kPrepIPT>), dim3(grid), dim3(kPrepNT), 0, s, colptr, xkey,
-                     ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp);
+  if (wide)
+    hipLaunchKernelGGL((k_prep<kPrepNT, kWideIPT>), dim3(grid), dim3(kPrepNT), 0, s, colptr, xkey,
+                       ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp);
+  else
+    hipLaunchKernelGGL((k_prep<kPrepNT, kPrepIPT>), dim3(grid), dim3(kPrepNT), 0, s, colptr, xkey,
+                       ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp);
 }
 
 // ---------------------------------------------------------------- batch
 // Selector inputs and choice of every vector of a batch, a workgroup per tile
-// of kBatchTile keys: the workgroup of a vector that finishes last adds up the
+// of kWideTile keys: the workgroup of a vector that finishes last adds up the
 // vector's tiles (exact bin_len, longest column; sampled inputs for a large
 // x, as everywhere) and runs the selector. One launch per vector took 12 us
 // for each of them.
@@ -780,7 +785,7 @@ __global__ __launch_bounds__(NT) void k_batch_scan(const int* __restrict__ colpt
 void launch_batch_select(hipStream_t s, const int* colptr, const int* xkey, int ncols, int ntiles, const int* tile_vec,
                          const BatchVec* vec, long long* tsum, int* tmax, unsigned* arrive, Ctl* ctls,
                          const SelectorArgs& sel, long long* stash) {
-  hipLaunchKernelGGL((k_batch_select<kPrepNT, kBatchIPT>), dim3(ntiles), dim3(kPrepNT), 0, s, colptr, xkey, ncols,
+  hipLaunchKernelGGL((k_batch_select<kPrepNT, kWideIPT>), dim3(ntiles), dim3(kPrepNT), 0, s, colptr, xkey, ncols,
                      tile_vec, vec, tsum, tmax, arrive, ctls, sel, stash);
 }
 
@@ -788,7 +793,7 @@ void launch_batch_scan(hipStream_t s, const int* colptr, const int* xkey, int nc
                        const int* tile_vec, const BatchVec* vec, const long long* tsum, int key_base, int* ptr,
                        int* xbeg, int* split) {
   if (nlist > 0)
-    hipLaunchKernelGGL((k_batch_scan<kPrepNT, kBatchIPT>), dim3(nlist), dim3(kPrepNT), 0, s, colptr, xkey, ncols, list,
+    hipLaunchKernelGGL((k_batch_scan<kPrepNT, kWideIPT>), dim3(nlist), dim3(kPrepNT), 0, s, colptr, xkey, ncols, list,
                        tile_vec, vec, tsum, key_base, ptr, xbeg, split);
 }
 

@@ -17,9 +17,10 @@ namespace spmspv {
 // R-MAT scale 20: 15.1 us with 8 keys per thread, 12.8 with 4, 12.3 with 2; the
 // eight levels of a BFS on scale 22 (up to 10^6 keys) 125, 113 and 116 us.
 constexpr int kPrepNT = 256, kPrepIPT = 4, kPrepTile = kPrepNT * kPrepIPT;
-// The scans of many vectors in one launch fill the chip as they are (48 vectors
-// of R-MAT scale 20: 29 us with 8 keys per thread, 38 with 4).
-constexpr int kBatchIPT = 8, kBatchTile = kPrepNT * kBatchIPT;
+// The wide tile: the scans of many vectors in one launch, which fill the chip as
+// they are (48 vectors of R-MAT scale 20: 29 us with 8 keys per thread, 38 with
+// 4), and the no-allocation call, whose fixed scratch holds words per tile.
+constexpr int kWideIPT = 8, kWideTile = kPrepNT * kWideIPT;
 // odd items per thread: a lane walking VT consecutive LDS words then hits
 // a different bank than its neighbours (stride 7 is coprime with 32 banks)
 constexpr int kLbNT = 256, kLbVT = 7, kLbTile = kLbNT * kLbVT;
@@ -126,10 +127,11 @@ __host__ __device__ inline bool sel_word_estimated(long long w) {
 // overlaps the scan instead of following the last tile's look-back.
 void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, int xnnz,
                  const int* xnnz_dev, int* ptr, int* xbeg, int* split, unsigned long long* state,
-                 int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp = nullptr);
+                 int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp = nullptr,
+                 bool wide = false);
 // The vectors of a batch: one launch selects for all of them, one scans all
 // that need it. Vector v has keys xkey[key0 .. key0 + xnnz), tiles
-// [tile0, tile0 + ntiles) of kBatchTile keys (at least one) and, once its
+// [tile0, tile0 + ntiles) of kWideTile keys (at least one) and, once its
 // slot is known, splits from split0.
 struct BatchVec {
   int key0, xnnz, tile0, ntiles;

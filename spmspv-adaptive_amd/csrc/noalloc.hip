@@ -41,7 +41,7 @@ struct Layout {
 
 Layout layout(int m, int xnnz, long long nnz) {
   Layout L{};
-  const size_t prep_tiles = ((size_t)xnnz + kPrepTile - 1) / kPrepTile + 2;
+  const size_t prep_tiles = ((size_t)xnnz + kWideTile - 1) / kWideTile + 2;
   const size_t mwords = ((size_t)m + 31) / 32;
   const size_t cmp_tiles = (mwords + kCmpNT - 1) / kCmpNT + 2;
   const size_t lb_tiles = ((size_t)xnnz + (size_t)nnz + kLbTile - 1) / kLbTile + 2;
@@ -124,7 +124,7 @@ int spmspv_csc_spmspv_noalloc(int m, int n, long long nnz, const int* d_col_ptr,
   launch_fill_i32(s, reinterpret_cast<int*>(base), (long long)(L.zero_bytes / sizeof(int)), 0);
   // look-back words were just cleared, so fixed epochs never meet a stale word
   launch_prep(s, d_col_ptr, d_x_key, n, xnnz, nullptr, ptr, xbeg, split, state, tile_mm, ctl, nullptr,
-              Ep{1u, -1});
+              Ep{1u, -1}, nullptr, true);
   launch_lb_gather(s, 0, ptr, xbeg, d_x_val, split, d_row, d_val, ctl, xnnz, nullptr, acc, marks, nullptr,
                    nullptr, -1);
   launch_compact(s, nullptr, marks, m, acc, 1, d_y_key, d_y_val, state, ctl, Ep{2u, -1});
