@@ -1813,12 +1813,16 @@ int spmspv_autotune2(spmspv_handle_t h, int reps, int csr5, int* report) {
     h->small_sort_cap = cap > 0 ? cap : kSmallSortCap;
   }
   // The bin_len range of the bucket rule: on sub-vectors of x whose bin_len
-  // lies just under nnz / 4^k (k = 5..0), the bucket slot against the
-  // load-balanced column and row slots (2, 3, 5, 7), which the rule
-  // replaces; the range spans the sizes where it is more than 2 % faster
-  // than all four. Each end is then narrowed by two bisection steps
-  // (geometric) between the last size where the bucket slot loses and the
-  // first where it wins, and set three quarters of the way to the losing one.
+  // lies just under nnz / 4^k, the bucket slot against the load-balanced column
+  // and row slots (2, 3, 5, 7), which the rule replaces; the range spans the
+  // sizes where it is more than 2 % faster than all four. k goes from 5, or
+  // from the smallest size past the single launch, down to 0, and where the
+  // smallest size that x holds wins already the range starts at half of it
+  // (R-MAT s22, 128 M nonzeros: the bucket slot wins at 487 k products, the
+  // smallest found; at 31 k it takes 58 us and slot 2, gathered by the small-x
+  // launch, 33). Each end is then narrowed by two bisection steps (geometric)
+  // between the last size where the bucket slot loses and the first where it
+  // wins, and set three quarters of the way to the losing one.
   if (bucket_ok) {
     h->bucket_lo = 0;
     h->bucket_hi = -1;
@@ -1865,8 +1869,9 @@ int spmspv_autotune2(spmspv_handle_t h, int reps, int csr5, int* report) {
     };
     long long prev_lose = -1, lo = -1, hi = -1, first_win = -1, last_win = -1;
     bool done = false;
-    for (int k = 5; k >= 0 && !done; --k) {
+    for (int k = 12; k >= 0 && !done; --k) {
       const long long c = std::max<long long>(1, (long long)h->nnz >> (2 * k));
+      if (k > 5 && c <= kFuseCap) continue;  // the single launch's sizes
       int w;
       long long bl;
       if ((rc = wins(c, &w, &bl))) return rc;
@@ -1874,7 +1879,7 @@ int spmspv_autotune2(spmspv_handle_t h, int reps, int csr5, int* report) {
       if (w) {
         if (first_win < 0) {
           first_win = bl;
-          if (prev_lose < 0) lo = 1;
+          if (prev_lose < 0) lo = std::max<long long>(1, bl / 2);  // no smaller size is known
           else if ((rc = edge(prev_lose, bl, &lo))) return rc;
         }
         last_win = bl;
