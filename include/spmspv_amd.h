@@ -307,11 +307,13 @@ int spmspv_set_speculation(spmspv_handle_t h, int on);
  * so penalty = switching cost / (tau * t_best). 0 (the default) is off. */
 int spmspv_set_switch_penalty(spmspv_handle_t h, float penalty);
 /* No counterpart in the reference: on (1, the default) a column slot on an
- * x of at most 4,096 keys whose products fit one workgroup (11,264) runs
- * as one launch: scan, gather, LDS sort, reduce and the sorted output (the
- * sort-based slots' result); spmspv_run_auto then decides such calls by
- * this size rule before the network and reports slot 1. Off (0): every
- * slot always runs its own launches. Results are the same either way. */
+ * x of at most 4,096 keys and 11,264 products runs as one launch: scan,
+ * gather, row sums and the sorted output (the sort-based slots' result);
+ * spmspv_run_auto then decides such calls by this size rule before the
+ * network and reports slot 1. With more products the launch runs the
+ * network, and the gather too when an atomic column slot is chosen. Off
+ * (0): every slot always runs its own launches. Results are the same
+ * either way. */
 int spmspv_set_small_x_path(spmspv_handle_t h, int on);
 int spmspv_speculation_stats(spmspv_handle_t h, long long* hits, long long* misses);
 
