@@ -99,33 +99,6 @@ __global__ void k_bfs_init(int* levels, int n, unsigned* visited, unsigned* fb0,
   }
 }
 
-// The next level's frontier size and selector choice, tagged with the level
-// counter, into one host-coherent word (sig[0]), its selector features into
-// sig[1..8] first: the host polls one word per level instead of waiting for
-// the stream and three copies. Then opens that level: the counts of the
-// frontier it will fill and of its queue at 0, the level number and the
-// device epoch that its look-back kernels use (their launch arguments are
-// frozen inside a captured graph) advanced.
-__global__ void k_bfs_signal(int* cnt, int nxt, Ctl* ctl, long long* sig) {
-  // the feature words are acknowledged (each writer waits for its store)
-  // before the level word goes out; the host reads nothing else, so no L2
-  // write-back is needed
-  if (threadIdx.x < 16) {
-    reinterpret_cast<float*>(sig + 1)[threadIdx.x] = ctl->feat[threadIdx.x];
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const long long w = ((long long)(cnt[2] & 0xffffff) << 40) | ((long long)(ctl->kernel_choice & 0xff) << 32) |
-                        (long long)(unsigned)cnt[nxt];
-    __hip_atomic_store(sig, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    cnt[nxt ^ 1] = 0;
-    cnt[2] += 1;
-    cnt[3] = 0;
-    ctl->epoch += 16;
-  }
-}
-
 // K0: top-down, a team of 2^lg lanes per frontier vertex.
 __global__ __launch_bounds__(kBfsNT) void k_td_naive(const int* __restrict__ colptr,
                                                      const int* __restrict__ crow,
@@ -473,8 +446,7 @@ void enqueue_level(spmspv_handle_t h, hipStream_t s, int slot, int cur, int* lev
   hipLaunchKernelGGL(k_bfs_collect, dim3(std::min(kBfsGrid, (words + kBfsNT - 1) / kBfsNT)), dim3(kBfsNT), 0, s,
                      nbits, b->fbits[cur], h->n, b->cnt, cur, b->visited, levels, nf);
   launch_prep(s, h->csc_colptr, nf, h->n, 0, b->cnt + nxt, h->ptr, h->xbeg, h->split, h->scan_state,
-              h->tile_mm, h->ctl, &sel, Ep{0, 0}, h->prep_samp);
-  hipLaunchKernelGGL(k_bfs_signal, dim3(1), dim3(64), 0, s, b->cnt, nxt, h->ctl, h->sig_dev + kSigBfs);
+              h->tile_mm, h->ctl, &sel, Ep{0, 0}, h->prep_samp, false, LevelOpen{b->cnt, nxt, h->sig_dev + kSigBfs});
 }
 
 }  // namespace
@@ -583,12 +555,12 @@ static int bfs_run(spmspv_handle_t h, int src, int* d_levels, int policy, int us
   const auto t0 = std::chrono::steady_clock::now();
   hipLaunchKernelGGL(k_bfs_init, dim3(std::min(4096, (h->n + 255) / 256)), dim3(256), 0, s, d_levels,
                      h->n, b->visited, b->fbits[0], b->fbits[1], b->front[0], b->cnt, b->reached, src);
-  launch_prep(s, h->csc_colptr, b->front[0], h->n, 0, b->cnt, h->ptr, h->xbeg, h->split,
-              h->scan_state, h->tile_mm, h->ctl, &sel, next_ep(h, 1), h->prep_samp);
   // the level words: frontier size, choice and the level counter as tag
   long long* sw = h->sig + kSigBfs;
   __atomic_store_n(sw, kSigPending, __ATOMIC_RELEASE);
-  hipLaunchKernelGGL(k_bfs_signal, dim3(1), dim3(64), 0, s, b->cnt, 0, h->ctl, h->sig_dev + kSigBfs);
+  launch_prep(s, h->csc_colptr, b->front[0], h->n, 0, b->cnt, h->ptr, h->xbeg, h->split,
+              h->scan_state, h->tile_mm, h->ctl, &sel, next_ep(h, 1), h->prep_samp, false,
+              LevelOpen{b->cnt, 0, h->sig_dev + kSigBfs});
   hipError_t e = hipGetLastError();
   const bool trace = max_levels > 0 && level_ms && level_feat;
   // waits for the word of level `tag` (polling; the trace's events need the

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
                                              const int* __restrict__ xnnz_dev, int* __restrict__ ptr,
                                              int* __restrict__ xbeg, int* __restrict__ split,
                                              unsigned long long* state, int* tile_mm, Ctl* ctl,
-                                             Ep ep, SelectorArgs sel, long long* samp) {
+                                             Ep ep, SelectorArgs sel, long long* samp, LevelOpen open) {
   struct Red {
     long long sum, ssum;
     int mx, mn, smx;
@@ -117,6 +117,32 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
     sl.mat = &s_mf;
     select_in_wave(ctl, sl, (double)xn, (double)bl, (double)mxl);
   };
+  // A BFS level (after run_selector, by the selecting workgroup; the earlier
+  // tiles have read what this changes): the frontier's size and the choice,
+  // tagged with the level counter, into one host-coherent word (sig[0]), the
+  // features into sig[1..8] first, so that the host polls one word per level.
+  // Then the level opens: the counts of the frontier it will fill and of its
+  // queue at 0, the level number and the device epoch that its look-back
+  // kernels use (their launch arguments are frozen inside a captured graph)
+  // advanced. A launch of its own for this cost 4 us and a launch gap per
+  // level (BFS of R-MAT scale 22, eight levels: 465 -> 453 us).
+  auto open_level = [&](int size) {
+    if (!open.cnt || threadIdx.x >= kWave) return;
+    // the feature words are acknowledged before the level word goes out; the
+    // host reads nothing else, so no L2 write-back is needed
+    if (threadIdx.x < 16) reinterpret_cast<float*>(open.sig + 1)[threadIdx.x] = ctl->feat[threadIdx.x];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (threadIdx.x == 0) {
+      int* cnt = open.cnt;
+      const long long w = ((long long)(cnt[2] & 0xffffff) << 40) | ((long long)(ctl->kernel_choice & 0xff) << 32) |
+                          (long long)(unsigned)size;
+      __hip_atomic_store(open.sig, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      cnt[open.nxt ^ 1] = 0;
+      cnt[2] += 1;
+      cnt[3] = 0;
+      ctl->epoch += 16;
+    }
+  };
   if (ntiles == 0) {
     // empty x: block 0 alone writes the results
     if (t != 0) return;
@@ -133,6 +159,7 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
     __syncthreads();
     run_selector(0, 0, 0);
     if (sel.stash && threadIdx.x == 0) *sel.stash = sel_word(0, sel.mat ? ctl->kernel_choice : -1);
+    open_level(0);
     return;
   }
   if (t >= ntiles) return;
@@ -306,6 +333,7 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
   // the selector's choice was written by thread 0 (lane 0 of wave 0)
   if (sel.stash && threadIdx.x == 0)
     *sel.stash = sel_word((long long)pre + btot, sel.mat ? ctl->kernel_choice : -1);
+  open_level(xnnz);
 }
 
 // Features-only selector launch: bin_len and the largest and smallest
@@ -628,7 +656,7 @@ void launch_select_feat(hipStream_t s, const int* colptr, const int* xkey, const
 
 void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, int xnnz,
                  const int* xnnz_dev, int* ptr, int* xbeg, int* split, unsigned long long* state,
-                 int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp, bool wide) {
+                 int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp, bool wide, const LevelOpen& open) {
   // exact grid when the host knows xnnz, else the bound from ncols
   const long long cnt = xnnz_dev ? ncols : xnnz;
   const int tile = wide ? kWideTile : kPrepTile;
@@ -637,10 +665,10 @@ void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, i
   if (sel) a = *sel;
   if (wide)
     hipLaunchKernelGGL((k_prep<kPrepNT, kWideIPT>), dim3(grid), dim3(kPrepNT), 0, s, colptr, xkey,
-                       ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp);
+                       ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp, open);
   else
     hipLaunchKernelGGL((k_prep<kPrepNT, kPrepIPT>), dim3(grid), dim3(kPrepNT), 0, s, colptr, xkey,
-                       ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp);
+                       ncols, xnnz, xnnz_dev, ptr, xbeg, split, state, tile_mm, ctl, ep, a, samp, open);
 }
 
 // ---------------------------------------------------------------- batch

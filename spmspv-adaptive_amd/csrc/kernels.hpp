@@ -82,6 +82,13 @@ struct SelectorArgs {
   // (off by default: bin_hi < bin_lo)
   long long bin_lo = 0, bin_hi = -1;
 };
+// BFS (bfs.hip): the column scan of a frontier also sends the level's word and
+// opens the level: cnt the counters, nxt the frontier's index, sig the words.
+struct LevelOpen {
+  int* cnt = nullptr;
+  int nxt = 0;
+  long long* sig = nullptr;
+};
 __host__ __device__ inline int slot_family(int k) { return k < 4 ? 0 : (k < 6 ? 1 : 2); }
 // The selector's x inputs for a large x (xnnz > kSampleMin) come from
 // kSampleKeys evenly spaced keys (positions floor(i * xnnz / kSampleKeys)):
@@ -128,7 +135,7 @@ __host__ __device__ inline bool sel_word_estimated(long long w) {
 void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, int xnnz,
                  const int* xnnz_dev, int* ptr, int* xbeg, int* split, unsigned long long* state,
                  int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp = nullptr,
-                 bool wide = false);
+                 bool wide = false, const LevelOpen& open = {});
 // The vectors of a batch: one launch selects for all of them, one scans all
 // that need it. Vector v has keys xkey[key0 .. key0 + xnnz), tiles
 // [tile0, tile0 + ntiles) of kWideTile keys (at least one) and, once its
