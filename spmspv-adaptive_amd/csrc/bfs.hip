@@ -96,6 +96,7 @@ __global__ void k_bfs_init(int* levels, int n, unsigned* visited, unsigned* fb0,
     cnt[3] = 0;
     reached[0] = 0;
     reached[1] = 0;
+    reached[2] = 0;
   }
 }
 
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(kBfsNT) void k_bfs_collect(unsigned* nbits, unsigne
 // Graph500 edge count: sum of degrees over reached vertices.
 template <int NT>
 __global__ __launch_bounds__(NT) void k_reached(const int* __restrict__ levels, const int* __restrict__ colptr,
-                                                int n, unsigned long long* out) {
+                                                int n, unsigned long long* out, long long* sig) {
   __shared__ long long s_l[NT / kWave];
   long long c = 0, d = 0;
   for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
@@ -375,10 +376,7 @@ __global__ __launch_bounds__(NT) void k_reached(const int* __restrict__ levels, 
   }
   c = block_sum<NT, long long>(c, s_l);
   d = block_sum<NT, long long>(d, s_l);
-  if (threadIdx.x == 0) {
-    atomicAdd(out, (unsigned long long)c);
-    atomicAdd(out + 1, (unsigned long long)d);
-  }
+  if (threadIdx.x == 0) count_to_host((unsigned long long)c, (unsigned long long)d, out, sig);
 }
 
 int lg2(int t) {
@@ -633,16 +631,21 @@ static int bfs_run(spmspv_handle_t h, int src, int* d_levels, int policy, int us
     launch_fill_i32(s, reinterpret_cast<int*>(h->scan_state), (long long)h->scan_words * 2, 0);
     h->dev_levels = 0;
   }
+  unsigned long long red[2] = {0, 0};
+  rc = SPMSPV_SUCCESS;
+  if (!out_of_sequence && e == hipSuccess) {
+    __atomic_store_n(sw, kSigPending, __ATOMIC_RELEASE);
+    // 256 workgroups: three atomics each on one line
+    hipLaunchKernelGGL(k_reached<1024>, dim3(std::min(256, (h->n + 1023) / 1024)), dim3(1024), 0, s, d_levels,
+                       h->csc_colptr, h->n, b->reached, h->sig_dev + kSigBfs);
+    e = hipGetLastError();
+    if (e == hipSuccess) rc = wait_signal(h, kSigBfs, &word);
+    for (int k = 0; k < 2; ++k) red[k] = (unsigned long long)__atomic_load_n(sw + 1 + k, __ATOMIC_ACQUIRE);
+  }
   h->stream = saved;
   if (out_of_sequence) return set_error(h, SPMSPV_DEVICE_ERROR, "bfs: a level's word arrived out of sequence");
   if (e != hipSuccess) return set_error(h, SPMSPV_DEVICE_ERROR, std::string("bfs: ") + hipGetErrorString(e));
-  // 256 workgroups: two atomics each on one pair of words
-  hipLaunchKernelGGL(k_reached<1024>, dim3(std::min(256, (h->n + 1023) / 1024)), dim3(1024), 0, s, d_levels,
-                     h->csc_colptr, h->n, b->reached);
-  unsigned long long red[2] = {0, 0};
-  e = hipMemcpyAsync(red, b->reached, sizeof(red), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e != hipSuccess) return set_error(h, SPMSPV_DEVICE_ERROR, std::string("bfs: ") + hipGetErrorString(e));
+  if (rc) return rc;
   if (stats) {
     stats[0] = nlev - 1;             // levels with a nonempty frontier
     stats[1] = (double)red[1] / 2.0; // undirected edges in the reached component

@@ -47,7 +47,7 @@ struct MsState {
   int2* list[2] = {nullptr, nullptr};      // frontier work items (vertex, chunk), items_cap each
   int2* queue = nullptr;                   // items_cap: pull items (row, chunk); push: touched vertices
   unsigned long long* cnt = nullptr;       // two groups of kMsGroup words (kMsItems, ...), then
-                                           // [2 * kMsGroup] reached pairs, [+ 1] their edges
+                                           // [2 * kMsGroup] reached pairs, [+ 1] their edges, [+ 2] arrivals
 };
 
 namespace {
@@ -109,7 +109,7 @@ __global__ void k_ms_init(int n, int nsrc, unsigned long long* visit, unsigned l
     f1[v] = 0ull;
   }
   for (long long k = t; k < (long long)n * nsrc; k += stride) levels[k] = -1;
-  if (t < 2 * kMsGroup + 2) cnt[t] = 0ull;
+  if (t < 2 * kMsGroup + 3) cnt[t] = 0ull;
 }
 
 __device__ void ms_signal(const unsigned long long* c, int tag, long long* sig) {
@@ -373,7 +373,8 @@ __global__ void k_ms_clear(const int2* __restrict__ items, long long nitems, uns
 // Reached (vertex, source) pairs and the edges they span: sum over v of
 // popcount(visit[v]) and popcount(visit[v]) * deg(v).
 __global__ __launch_bounds__(kMsNT) void k_ms_reached(int n, const unsigned long long* __restrict__ visit,
-                                                      const int* __restrict__ colptr, unsigned long long* out) {
+                                                      const int* __restrict__ colptr, unsigned long long* out,
+                                                      long long* sig) {
   __shared__ long long s_l[kMsNT / kWave];
   long long c = 0, d = 0;
   for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (long long)gridDim.x * blockDim.x) {
@@ -383,10 +384,7 @@ __global__ __launch_bounds__(kMsNT) void k_ms_reached(int n, const unsigned long
   }
   c = block_sum<kMsNT, long long>(c, s_l);
   d = block_sum<kMsNT, long long>(d, s_l);
-  if (threadIdx.x == 0) {
-    atomicAdd(out, (unsigned long long)c);
-    atomicAdd(out + 1, (unsigned long long)d);
-  }
+  if (threadIdx.x == 0) count_to_host((unsigned long long)c, (unsigned long long)d, out, sig);
 }
 
 }  // namespace
@@ -446,7 +444,6 @@ int spmspv_bfs_multi(spmspv_handle_t h, int nsrc, const int* srcs, int* d_levels
   hipStream_t s = h->stream;
   const int n = h->n;
   const unsigned long long full = nsrc == 64 ? ~0ull : ((1ull << nsrc) - 1ull);
-  unsigned long long* hc = reinterpret_cast<unsigned long long*>(h->h_pin);
   const auto t0 = std::chrono::steady_clock::now();
   MsSrcs by_value{};
   std::copy(srcs, srcs + nsrc, by_value.v);
@@ -520,11 +517,14 @@ int spmspv_bfs_multi(spmspv_handle_t h, int nsrc, const int* srcs, int* d_levels
     ++levels_run;
   }
   const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-  // 256 workgroups: two atomics each on one pair of words
+  // 256 workgroups: three atomics each on one line
+  pending();
   hipLaunchKernelGGL(k_ms_reached, blocks(n, 256), dim3(kMsNT), 0, s, n, st->visit, h->csc_colptr,
-                     st->cnt + 2 * kMsGroup);
-  HIP_TRY(h, hipMemcpyAsync(hc, st->cnt + 2 * kMsGroup, 16, hipMemcpyDeviceToHost, s));
-  HIP_TRY(h, hipStreamSynchronize(s));
+                     st->cnt + 2 * kMsGroup, h->sig_dev + kSigMs);
+  HIP_TRY(h, hipGetLastError());
+  if ((rc = wait_signal(h, kSigMs, &word))) return rc;
+  unsigned long long hc[2];
+  for (int k = 0; k < 2; ++k) hc[k] = (unsigned long long)__atomic_load_n(sw + 1 + k, __ATOMIC_ACQUIRE);
   if (stats) {
     stats[0] = levels_run;              // levels with a nonempty frontier
     stats[1] = (double)hc[1] / 2.0;     // undirected edges summed over the sources' components
