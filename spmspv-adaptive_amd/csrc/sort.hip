@@ -342,20 +342,30 @@ __device__ __forceinline__ unsigned direct_start(const unsigned* cnt, const unsi
   return block_excl_sum<NT, unsigned>(a, s_t, &tot) + b;
 }
 
+// Sorts of many items with two payloads stream through HBM: twice the tile, so
+// that a run of equal digits fills its lines (15.9 M items of R-MAT scale 19,
+// 382 MB: 97 -> 86.5 us per pass; a copy would take 81). The second payload goes
+// through the first one's LDS, which leaves two workgroups per CU; 512 x 16 took
+// 88, 1,024 x 6 and x 8 105 us. Their counts do not fit 16 bits per 16 tiles, so
+// the positions come from the scan; smaller sorts are better off without it.
+constexpr int kWideNT = 512;
+constexpr long long kWideItems = 1 << 22;
+
 // PAY: payload words per item (0: keys only). Four waves per SIMD (three with
 // two payloads, as LDS allows): five spill the payloads (R-MAT scale 22, 1 %:
 // 105.5 -> 110.7 us).
 template <int NT, int IPT, int PAY>
-__global__ __launch_bounds__(NT, PAY > 1 ? 3 : 4) void k_sort_scatter(SortSet in, SortSet out, const long long* __restrict__ n_dev,
+__global__ __launch_bounds__(NT, NT == 256 && PAY > 1 ? 3 : 4) void k_sort_scatter(SortSet in, SortSet out, const long long* __restrict__ n_dev,
                                                      int shift, int bits, const unsigned* __restrict__ pos0,
                                                      const unsigned long long* __restrict__ chunk, int small_cap, long long n_cap, Gate g) {
   if (gate_shut(g)) return;
   constexpr int TILE = NT * IPT;
   constexpr int NW = NT / kWave;
-  static_assert(NT == 256, "one thread per digit");
+  constexpr bool WIDE = NT > 256;  // the second payload goes through the first one's LDS
+  static_assert(NT >= 256, "one thread per digit");
   __shared__ unsigned s_k[TILE];
   __shared__ unsigned s_v[PAY > 0 ? TILE : 1];
-  __shared__ unsigned s_w[PAY > 1 ? TILE : 1];
+  __shared__ unsigned s_w[PAY > 1 && !WIDE ? TILE : 1];
   __shared__ unsigned s_cnt[NW * 256];
   __shared__ unsigned s_dstart[256];
   __shared__ unsigned s_gbase[256];
@@ -383,16 +393,19 @@ __global__ __launch_bounds__(NT, PAY > 1 ? 3 : 4) void k_sort_scatter(SortSet in
       if (PAY > 0) pv[j] = in.v[valid[j] ? gi : n - 1];
       if (PAY > 1) pw[j] = in.w[valid[j] ? gi : n - 1];
     }
-    if (direct) {
-      gb = direct_start<NT>(pos0, chunk, t, ntiles, bits, s_cnt, s_k, s_t);
+    if (NT == 256 && direct) {
+      gb = direct_start<256>(pos0, chunk, t, ntiles, bits, s_cnt, s_k, s_t);
       __syncthreads();
     }
     wave_rank<IPT>(key, valid, shift, s_cnt + w * 256, rank, dig, IPT, bits);
     __syncthreads();
-    const unsigned tot = digit_wave_offsets<NW>(s_cnt);
+    const unsigned tot = NT == 256 || d < 256 ? digit_wave_offsets<NW>(s_cnt) : 0u;
     unsigned dtot;
-    s_dstart[d] = block_excl_sum<NT, unsigned>(tot, s_t, &dtot);
-    s_gbase[d] = gb;
+    const unsigned dst = block_excl_sum<NT, unsigned>(tot, s_t, &dtot);
+    if (NT == 256 || d < 256) {
+      s_dstart[d] = dst;
+      s_gbase[d] = gb;
+    }
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
@@ -400,7 +413,8 @@ __global__ __launch_bounds__(NT, PAY > 1 ? 3 : 4) void k_sort_scatter(SortSet in
         const unsigned p = s_dstart[dig[j]] + s_cnt[w * 256 + dig[j]] + rank[j];
         s_k[p] = key[j];
         if (PAY > 0) s_v[p] = pv[j];
-        if (PAY > 1) s_w[p] = pw[j];
+        if (PAY > 1 && !WIDE) s_w[p] = pw[j];
+        if (PAY > 1 && WIDE) rank[j] = (int)p;
       }
     }
     __syncthreads();
@@ -411,7 +425,18 @@ __global__ __launch_bounds__(NT, PAY > 1 ? 3 : 4) void k_sort_scatter(SortSet in
       const unsigned q = s_gbase[dd] + (i - s_dstart[dd]);
       out.k[q] = k;
       if (PAY > 0) out.v[q] = s_v[i];
-      if (PAY > 1) out.w[q] = s_w[i];
+      if (PAY > 1 && !WIDE) out.w[q] = s_w[i];
+    }
+    if (PAY > 1 && WIDE) {
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < IPT; ++j)
+        if (valid[j]) s_v[rank[j]] = pw[j];
+      __syncthreads();
+      for (int i = threadIdx.x; i < cnt; i += NT) {
+        const unsigned dd = (s_k[i] >> shift) & mask;
+        out.w[s_gbase[dd] + (i - s_dstart[dd])] = s_v[i];
+      }
     }
     __syncthreads();
   }
@@ -619,6 +644,18 @@ static int tiles_grid(long long n_hint, long long n_cap, int tile) {
 static void launch_digit_pass(hipStream_t s, const SortBufs& b, const SortSet& in, const SortSet& out, int shift,
                               int bits, int pass, bool chunks, const long long* n_dev, Ctl* ctl, long long n_hint,
                               long long n_cap, int small_cap, Ep e, Gate g) {
+  if (in.w && n_hint >= kWideItems) {
+    constexpr int tile = kWideNT * kSortIPT;
+    const int tiles = tiles_grid(n_hint, n_cap, tile), pgrid = std::min(tiles, 2048);
+    const int sgrid = (int)std::max<long long>(1, (((long long)tiles << bits) + kDScanTile - 1) / kDScanTile);
+    hipLaunchKernelGGL((k_digit_count<kSortNT, tile / kSortNT>), dim3(pgrid), dim3(kSortNT), 0, s, in.k, n_dev, shift,
+                       bits, b.dcount, nullptr, pass, small_cap, n_cap, g);
+    hipLaunchKernelGGL((k_digit_scan<kDScanNT, kDScanIPT>), dim3(sgrid), dim3(kDScanNT), 0, s, b.dcount, n_dev, tile,
+                       bits, false, small_cap, n_cap, b.dstate, ctl, e, g);
+    hipLaunchKernelGGL((k_sort_scatter<kWideNT, kSortIPT, 2>), dim3(pgrid), dim3(kWideNT), 0, s, in, out, n_dev, shift,
+                       bits, b.dcount, nullptr, small_cap, n_cap, g);
+    return;
+  }
   const int tiles = tiles_grid(n_hint, n_cap, kSortTile);
   const int pgrid = std::min(tiles, 2048);  // count / scatter loop over their tiles
   const int sgrid = (int)std::max<long long>(1, (((long long)tiles << bits) + kDScanTile - 1) / kDScanTile);
