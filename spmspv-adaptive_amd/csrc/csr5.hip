@@ -505,7 +505,7 @@ bool launch_column_order(hipStream_t s, const ColumnOrderArgs& a, const int* col
 // them to their places in the tiles. A longer row (it can only be the last one
 // of a window) is left to a sort of all such rows' items through memory.
 // Two stable sorts of every item through memory, by new column, then by row,
-// took 1,740 us at R-MAT s19 (15.9 M nonzeros), this 480 us: 330 in LDS, which
+// took 1,740 us at R-MAT s19 (15.9 M nonzeros), this 450 us: 302 in LDS, which
 // the ranking's ballots and LDS round trips bound, 150 for the 15 % of the
 // items in long rows. Two workgroups of 512 threads share a CU's LDS (10 bytes
 // per item and the counters) and overlap each other's barriers; one of 1,024

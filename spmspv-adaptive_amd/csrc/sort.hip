@@ -3,8 +3,9 @@
 // CSC sort kernels (thrust::sort_by_key + thrust::reduce_by_key,
 // la/include/spmspv/csc-spmspv/detail/device/csc_sort_spmspv.cuh:339-437,
 // 1030-1152), written for wave64:
-//  * keys are ranked inside a tile with 8 wave ballots per key (peers with
-//    the same 8-bit digit) and per-wave digit counters in LDS (stable);
+//  * keys are ranked inside a tile with a wave ballot per bit of the digit (at
+//    most 8; peers hold the same digit) and per-wave digit counters in LDS
+//    (stable);
 //  * each pass counts digits per tile, turns the counts into positions (the
 //    scatter's workgroups sum them; for many tiles one small look-back scan
 //    over 256 x tiles entries) and scatters, so no tile waits on a chain of
