@@ -38,6 +38,7 @@
 // HBM bytes per product: 8 read and 8 written (scatter) + 8 (accumulate),
 // against 44 and up for gather, radix passes and reduce.
 #include <algorithm>
+#include <climits>
 #include <mutex>
 #include <vector>
 
@@ -89,7 +90,7 @@ constexpr size_t accum_lds_bytes(int rows, int nbins) {
 template <int NT, int VT, int S>
 __device__ __forceinline__ int lb_tile(long long t, const int* __restrict__ ptr, const int* __restrict__ xbeg,
                                        const int* __restrict__ split, long long ntiles, int xnnz, long long W,
-                                       int* s_ptr, int* s_beg, unsigned short* s_seg, int (&idx)[VT],
+                                       int* s_pos, int* s_off, unsigned short* s_seg, int (&idx)[VT],
                                        int (&xi)[VT]) {
   constexpr int T = NT * VT;
   static_assert(T == S * kLbTile, "a tile is S of the prep's tiles");
@@ -117,29 +118,35 @@ __device__ __forceinline__ int lb_tile(long long t, const int* __restrict__ ptr,
     for (int u = 0; u < SEGPT; ++u) {
       const int k = threadIdx.x + u * NT;
       if (k < nseg) {
-        s_ptr[k] = pv[u];
-        s_beg[k] = bv[u];
+        s_pos[k] = (int)((long long)sa + k + pv[u] - d0);
+        s_off[k] = bv[u] - pv[u];
       }
     }
   }
   __syncthreads();
-  long long D = d0 + (long long)threadIdx.x * VT;
-  if (D < d1) {
-    int lo = a0, hi = a1;
+  // positions in the tile are 32 bits wide, and a marker's place is read once
+  // when the walk comes to it, not with every product (scatter of 3 M products
+  // 39.1 -> 37.6 us)
+  const int len = (int)(d1 - d0), i0 = a0 - sa, i1 = a1 - sa;
+  int D = (int)threadIdx.x * VT;
+  if (D < len) {
+    int lo = i0, hi = i1;
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
-      if ((long long)mid + s_ptr[mid - sa] < D) lo = mid + 1;
+      if (s_pos[mid] < D) lo = mid + 1;
       else hi = mid;
     }
     int i = lo;
-    long long p = D - i;
+    int p = D - (i - i0);
+    int nxt = i < i1 ? s_pos[i] : INT_MAX;
 #pragma unroll
     for (int k = 0; k < VT; ++k) {
-      if (D >= d1) break;
-      if (i < a1 && (long long)i + s_ptr[i - sa] == D) {
+      if (len < T && D >= len) break;
+      if (D == nxt) {
         ++i;
+        nxt = i < i1 ? s_pos[i] : INT_MAX;
       } else {
-        s_seg[p - b0] = (unsigned short)(i - 1 - sa);
+        s_seg[p] = (unsigned short)(i - 1);
         ++p;
       }
       ++D;
@@ -152,7 +159,7 @@ __device__ __forceinline__ int lb_tile(long long t, const int* __restrict__ ptr,
     const int q0 = threadIdx.x + k * NT;
     const bool ok = q0 < np;
     const int sg = ok ? s_seg[q0] : 0;
-    idx[k] = ok ? s_beg[sg] + (int)(b0 + q0 - s_ptr[sg]) : 0;
+    idx[k] = ok ? s_off[sg] + (int)(b0 + q0) : 0;
     xi[k] = ok ? sa + sg : 0;
   }
   return np;
