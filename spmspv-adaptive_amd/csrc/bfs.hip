@@ -532,6 +532,8 @@ static int bfs_run(spmspv_handle_t h, int src, int* d_levels, int policy, int us
   if ((rc = ensure_arena(h)) || (rc = need_csc(h))) return rc;
   if ((rc = ensure_mat_features(h)) || (rc = bfs_alloc(h))) return rc;
   BfsState* b = h->bfs;
+  // the frontiers' column scans overwrite the one made for the current x
+  h->prep_valid = false;
   hipStream_t s = h->stream ? h->stream : b->own_stream;
   const int smode = policy >= 0 ? 2 : h->sel_mode, sfixed = policy >= 0 ? policy : h->sel_fixed;
   // the BFS levels' own weights when set (trained on BFS levels), else the

@@ -1,0 +1,54 @@
+"""Calls that follow one another on one handle without x being set again:
+what one call leaves behind must not change the next one's result. Index sets
+and counts exact, values within 1e-5 * sum|a_ij x_j| of the FP64 oracle."""
+import numpy as np
+import pytest
+
+import oracle
+import spmspv_amd as sa
+
+pytestmark = pytest.mark.gpu
+SCAN_SLOTS = [sa.K_COL_LB_ATOMIC, sa.K_COL_LB_SORT, sa.K_COL_BUCKET, sa.K_COL_TWO_LAYER_ATOMIC]
+
+
+class Graph:
+    """R-MAT on a handle, x of k keys, and the product's reference."""
+
+    def __init__(self, scale, k, seed=5, per=8):
+        self.n = n = 1 << scale
+        rp, col, val = sa.gen_rmat_csr(scale, per, seed=seed)
+        self.csr = rp, col, val
+        self.M = sa.Matrix(n, n, rp, col, val)
+        self.A = self.M.A
+        self.csc = oracle.csr_to_csc(n, n, rp, col, val)
+        self.yk, self.yv = sa.DeviceArray(n, np.int32), sa.DeviceArray(n, np.float32)
+        self.set_x(k, seed)
+
+    def set_x(self, k, seed):
+        self.key, self.val = sa.gen_sparse_vector(self.n, k, seed)
+        self.dk, self.dv = sa.DeviceArray.from_host(self.key, np.int32), sa.DeviceArray.from_host(self.val, np.float32)
+        self.A.set_sparse_x(self.dk, self.dv, k)
+        self.ref = oracle.spmspv_f64(self.n, *self.csc, self.key, self.val)
+
+    def check(self, cnt, tag):
+        ek, ev, eb = self.ref
+        np.testing.assert_array_equal(self.yk.to_host(cnt), ek, err_msg=tag)
+        assert np.all(np.abs(self.yv.to_host(cnt).astype(np.float64) - ev) <= 1e-5 * eb + 1e-30), tag
+
+    def run(self, slot, tag):
+        print(tag, "slot", slot, flush=True)
+        self.check(self.A.run(slot, y_key=self.yk, y_val=self.yv), f"{tag}, slot {slot}")
+
+
+@pytest.mark.parametrize("slot", SCAN_SLOTS)
+@pytest.mark.parametrize("graphs", [0, 1])
+def test_product_after_bfs(gpu, slot, graphs):
+    """The column scan of x is made again after a BFS has scanned its
+    frontiers into the same arrays."""
+    g = Graph(15, 9000)
+    lev = sa.DeviceArray(g.n, np.int32)
+    g.run(slot, "before")
+    for src in (0, 77):
+        g.A.bfs(src, lev, policy=2, use_graphs=graphs)
+        g.run(slot, f"after the BFS from {src}")
+        assert g.A.computeBinlen() == int(np.diff(g.csc[0])[g.key].sum())
