@@ -1463,6 +1463,9 @@ int spmspv_run_auto(spmspv_handle_t h, float alpha, float* d_y_dense, int* d_y_k
                        sel, enc, order5 ? h->csr5.cperm : nullptr);
     h->launches++;
     if ((rc = check_launch(h, "selector"))) return rc;
+    // a sampled launch leaves its estimate where an earlier scan of this x
+    // had left the exact size, which its readers need
+    h->prep_valid = false;
     if (enc && order5) h->enc5_valid = h->kEnc5Support;
     else if (enc) h->enc_valid = true;
   } else if ((rc = run_prep(h, true, &sel))) {

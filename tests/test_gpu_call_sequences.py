@@ -52,3 +52,20 @@ def test_product_after_bfs(gpu, slot, graphs):
         g.A.bfs(src, lev, policy=2, use_graphs=graphs)
         g.run(slot, f"after the BFS from {src}")
         assert g.A.computeBinlen() == int(np.diff(g.csc[0])[g.key].sum())
+
+
+@pytest.mark.parametrize("slot", SCAN_SLOTS)
+def test_product_after_sampled_selection(gpu, slot):
+    """A selection from a sample of a large x (more than 65,536 keys, a row
+    slot guessed from the call before) leaves no estimate in the place of the
+    exact size that an earlier scan of the same x left."""
+    g = Graph(17, 70000)
+    g.A.selector_mode(2, sa.K_ROW_LB)
+    g.check(g.A.run_auto(y_key=g.yk, y_val=g.yv)[0], "first, no guess yet")
+    g.set_x(80000, 6)
+    size = int(np.diff(g.csc[0])[g.key].sum())
+    g.run(slot, "scans x")
+    g.check(g.A.run_auto(y_key=g.yk, y_val=g.yv)[0], "selected from a sample")
+    g.run(slot, "after the selection")
+    g.check(g.A.run_auto(y_key=g.yk, y_val=g.yv)[0], "selected from a sample")
+    assert g.A.computeBinlen() == size
