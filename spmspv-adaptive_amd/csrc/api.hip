@@ -252,8 +252,10 @@ int ensure_mat_features(spmspv_handle_t h) {
   const int rows = h->csr_row ? h->m : h->n;
   const int cols = h->csr_row ? h->n : h->m;
   if (!rp) return set_error(h, SPMSPV_MAT_FORMAT_ERR, "no matrix input");
-  // degree histogram needs max degree + 1 <= cols + 1 slots
+  // degree histogram needs max degree + 1 <= cols + 1 slots; the column scan
+  // of x, if there is one, is made again
   int* hist = cols <= h->n ? h->ptr : h->yk_tmp;
+  h->prep_valid = false;
   launch_mat_features(h->stream, rp, rows, cols, h->nnz, hist, h->mat_partials, h->mat, h->ctl);
   rc = check_launch(h, "mat features");
   if (rc) return rc;

@@ -69,3 +69,19 @@ def test_product_after_sampled_selection(gpu, slot):
     g.run(slot, "after the selection")
     g.check(g.A.run_auto(y_key=g.yk, y_val=g.yv)[0], "selected from a sample")
     assert g.A.computeBinlen() == size
+
+
+@pytest.mark.parametrize("slot", SCAN_SLOTS)
+def test_product_after_matrix_features(gpu, slot):
+    """The matrix features, computed at their first use, need the array that
+    holds the column scan of x."""
+    g = Graph(13, 6000)
+    A = sa.SpmspvHandle(g.n, g.n, g.csr[1].size)
+    d = [sa.DeviceArray.from_host(a) for a in g.csr]
+    A.InputCSR(g.csr[1].size, *d)
+    A.ToCSC()
+    A.set_sparse_x(g.dk, g.dv, g.key.size)
+    g.A = A
+    g.run(slot, "scans x")
+    A.computeMatFeature()
+    g.run(slot, "after the features")
