@@ -373,7 +373,27 @@ static int need_enc_x(spmspv_handle_t h) {
   return check_launch(h, "encode x");
 }
 
+// The handle's stream is being captured into a graph by the caller (the null
+// stream cannot be).
+static bool capturing(spmspv_handle_t h) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (!h->stream) return false;
+  if (hipStreamIsCapturing(h->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusActive;
+}
+
 Ep next_ep(spmspv_handle_t h, unsigned k) {
+  // a replay of a captured call has the arguments of the capture: its epoch
+  // comes from the device (with the host's, a second replay would take the
+  // first one's look-back words for its own)
+  if (capturing(h)) {
+    launch_next_epoch(h->stream, h->ctl, {h->scan_state, h->sb.dstate, h->sb.red_state},
+                      {h->scan_words, h->sort_words, h->red_words});
+    return Ep{0, 0};
+  }
   // host epochs live in [1, 2^23); before they wrap, every look-back state
   // array is cleared so that no stale word can carry a reused epoch
   if (h->epoch_host + k >= (1u << 23) - 1) {
@@ -526,9 +546,11 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       }
       h->binlen_host = sel_word_binlen(word);
       gathered = sel_word_gathered(word);
-    } else if (h->binlen_host >= 0) {
+    } else if (h->binlen_host >= 0 && !capturing(h)) {
       return SPMSPV_SUCCESS;  // the products are known to fit: that launch finishes the call
     } else {
+      // (a captured call is replayed on what x holds then)
+      h->binlen_host = -1;
       h->gate = Gate{&h->ctl->kernel_choice, kid};
       h->spec_cap = h->nnz;
       h->spec_big = false;

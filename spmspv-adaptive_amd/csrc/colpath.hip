@@ -1350,6 +1350,27 @@ void launch_signal_int(hipStream_t s, const int* src, long long* dst, Gate g) {
   hipLaunchKernelGGL(k_signal_int, dim3(1), dim3(1), 0, s, src, dst, g);
 }
 
+// One workgroup. The look-back words are cleared every 2^22 epochs, long
+// before one could carry an epoch that comes again (the field holds 2^23).
+__global__ __launch_bounds__(1024) void k_next_epoch(Ctl* ctl, unsigned long long* a, size_t na, unsigned long long* b,
+                                                     size_t nb, unsigned long long* c, size_t nc) {
+  const unsigned e = ctl->epoch + 16u;
+  const bool clear = e - ctl->epoch_clear >= 1u << 22;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    ctl->epoch = e;
+    if (clear) ctl->epoch_clear = e;
+  }
+  if (!clear) return;
+  for (size_t i = threadIdx.x; i < na; i += blockDim.x) a[i] = 0ull;
+  for (size_t i = threadIdx.x; i < nb; i += blockDim.x) b[i] = 0ull;
+  for (size_t i = threadIdx.x; i < nc; i += blockDim.x) c[i] = 0ull;
+}
+void launch_next_epoch(hipStream_t s, Ctl* ctl, unsigned long long* const (&state)[3], const size_t (&words)[3]) {
+  hipLaunchKernelGGL(k_next_epoch, dim3(1), dim3(1024), 0, s, ctl, state[0], words[0], state[1], words[1], state[2],
+                     words[2]);
+}
+
 __global__ void k_bitmap_from_dense(const float* __restrict__ v, int n, unsigned* __restrict__ bits) {
   // one wave per 64 elements; element e -> bit e of words 2w, 2w+1
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -20,7 +20,7 @@ struct Ctl {
   unsigned int ticket[kSlots];
   unsigned int done[kSlots];
   unsigned int epoch;
-  unsigned int pad0;
+  unsigned int epoch_clear;  // epoch at which k_next_epoch last cleared the look-back words
   long long bin_len;   // sum of column lengths over x's support
   int max_len;         // max column length over x's support
   int min_len;         // min column length over x's support
@@ -247,8 +247,9 @@ __device__ __forceinline__ bool finish_persistent(Ctl* ctl, int slot, unsigned* 
 
 // Epoch of a look-back launch. Host-driven launches pass a fresh value per
 // launch (bit 23 clear); launches inside captured graphs, whose arguments
-// are frozen, take ctl->epoch + dev, which a small kernel at the start of
-// each captured sequence advances (bit 23 set). Stale states of earlier
+// are frozen, take ctl->epoch + dev (dev < 16), which a launch inside each
+// captured sequence advances (bit 23 set): a BFS level's column scan, or
+// k_next_epoch in a call that the caller captures. Stale states of earlier
 // launches then never match.
 struct Ep {
   unsigned v;

@@ -211,6 +211,8 @@ void launch_compact(hipStream_t s, unsigned* bitmap, unsigned char* marks, int m
 // bitmap of (v != 0) over a dense vector (whole words, no atomics)
 void launch_bitmap_from_dense(hipStream_t s, const float* v, int n, unsigned* bits);
 void launch_fill_f32(hipStream_t s, float* p, long long n, float v, Gate g = {});
+// ctl->epoch advanced, for the launches of a captured call (Ep{0, 0 .. 15})
+void launch_next_epoch(hipStream_t s, Ctl* ctl, unsigned long long* const (&state)[3], const size_t (&words)[3]);
 // *dst = *src once every earlier launch on s has finished (dst may be host-mapped)
 void launch_signal_int(hipStream_t s, const int* src, long long* dst, Gate g = {});
 void launch_fill_i32(hipStream_t s, int* p, long long n, int v);

@@ -85,3 +85,75 @@ def test_product_after_matrix_features(gpu, slot):
     g.run(slot, "scans x")
     A.computeMatFeature()
     g.run(slot, "after the features")
+
+
+class Captured:
+    """A handle's calls on a stream of their own, captured into a graph."""
+
+    def __init__(self, A):
+        import ctypes
+        self.ct, self.A = ctypes, A
+        sa.lib()
+        self.hip = ctypes.CDLL("libamdhip64.so.7")
+        self.stream, self.graph, self.exec = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+        assert self.hip.hipStreamCreateWithFlags(ctypes.byref(self.stream), 1) == 0  # non-blocking
+        assert sa.lib().spmspv_set_stream(A.h, self.stream) == 0
+
+    def capture(self, call):
+        c = self.ct
+        assert self.hip.hipStreamBeginCapture(self.stream, 1) == 0  # thread-local
+        call()
+        assert self.hip.hipStreamEndCapture(self.stream, c.byref(self.graph)) == 0
+        assert self.hip.hipGraphInstantiate(c.byref(self.exec), self.graph, None, None, c.c_size_t(0)) == 0
+
+    def replay(self):
+        assert self.hip.hipGraphLaunch(self.exec, self.stream) == 0
+        assert self.hip.hipStreamSynchronize(self.stream) == 0
+        out = np.empty(1, np.int32)
+        p = self.ct.c_void_p(sa.lib().spmspv_ynnz_device(self.A.h))
+        assert sa.lib().spmspv_memcpy_d2h(out.ctypes.data_as(self.ct.c_void_p), p, 4) == 0
+        return int(out[0])
+
+    def close(self):
+        assert sa.lib().spmspv_set_stream(self.A.h, None) == 0
+        if self.exec:
+            self.hip.hipGraphExecDestroy(self.exec)
+            self.hip.hipGraphDestroy(self.graph)
+        self.hip.hipStreamDestroy(self.stream)
+
+
+@pytest.mark.parametrize("known", [False, True])
+@pytest.mark.parametrize("slot", [0, 1, 2, 3, sa.K_COL_BUCKET])
+def test_captured_call_on_new_x(gpu, slot, known):
+    """A call without a count, captured once and replayed on other contents of
+    x's arrays, with eager calls between the replays: x that ends in the
+    single launch (16 row ranges here) and, for the slots that try it, x of
+    the same number of keys that does not (the heaviest columns)."""
+    k = 600 if slot < 4 else 20000
+    g = Graph(17, k)
+    order = np.argsort(-np.diff(g.csc[0]), kind="stable")
+    xs = [sa.gen_sparse_vector(g.n, k, 100 + i) for i in range(4)]
+    heavy = np.sort(order[:k]).astype(np.int32)
+    xs.insert(2, (heavy, np.random.default_rng(7).uniform(-1, 1, k).astype(np.float32)))
+    if slot < 4:
+        assert int(np.diff(g.csc[0])[heavy].sum()) > 11264 >= max(int(np.diff(g.csc[0])[x[0]].sum()) for x in xs if x[0] is not heavy)
+    g.set_x(k, 100)
+    g.run(slot, "eager")
+    cap = Captured(g.A)
+    g.A.set_sparse_x(g.dk, g.dv, k)
+    if known and slot < 4:
+        g.A.computeBinlen()
+    cap.capture(lambda: g.A.run(slot, y_key=g.yk, y_val=g.yv, want_nnz=False))
+    keep = g.dk, g.dv
+    for rep in range(2):
+        for i, (key, val) in enumerate(xs):
+            keep[0].upload(key)
+            keep[1].upload(val)
+            sa.synchronize()
+            g.ref = oracle.spmspv_f64(g.n, *g.csc, key, val)
+            print(f"slot {slot} replay {rep} {i}", flush=True)
+            g.check(cap.replay(), f"slot {slot} replay {rep} x {i}")
+            if i % 2:
+                g.set_x(k, 50 + i)
+                g.run(slot, "eager between replays")
+    cap.close()
