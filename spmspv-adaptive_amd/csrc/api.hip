@@ -965,6 +965,17 @@ int spmspv_dealloc_pre_buffer(spmspv_handle_t h) {
   (void)hipStreamSynchronize(h->stream);
   bfs_drop_graphs(h);
   if (h->arena) (void)hipFree(h->arena);
+  // what was derived from x lay in the arena; x itself is unset where it did
+  // (sparse from a dense x, without arrays of the caller)
+  if (h->arena && h->x_key == h->xk_int) {
+    h->x_key = nullptr;
+    h->x_val = nullptr;
+    h->sparse_valid = false;
+    if (h->x_dense_user && h->dense_valid) h->vec_type = SPMSPV_VEC_DENSE;
+  }
+  if (!h->x_dense_user) h->dense_valid = false;
+  if (!h->bits_user) h->bits_valid = false;
+  h->enc_valid = h->enc5_valid = false;
   h->arena = nullptr;
   h->reserved = false;
   h->row_ready = false;

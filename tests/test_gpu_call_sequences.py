@@ -157,3 +157,30 @@ def test_captured_call_on_new_x(gpu, slot, known):
                 g.set_x(k, 50 + i)
                 g.run(slot, "eager between replays")
     cap.close()
+
+
+@pytest.mark.parametrize("csr5", [0, 1])
+@pytest.mark.parametrize("slot", [sa.K_COL_LB_ATOMIC, sa.K_ROW_LB, sa.K_SPMV_NAIVE, sa.K_SPMV_LB])
+@pytest.mark.parametrize("x", ["sparse", "dense"])
+def test_product_after_buffers_were_given_back(gpu, slot, csr5, x):
+    """What the handle derived from x lies in its buffers: after they are
+    given back and reserved again it is made again, x being the caller's."""
+    g = Graph(13, 3000)
+    g.A.set_spmv_type(csr5)
+    if x == "dense":
+        d = np.zeros(g.n, np.float32)
+        d[g.key] = g.val
+        dx = sa.DeviceArray.from_host(d)
+        A = sa.SpmspvHandle(g.n, g.n, g.csr[1].size)  # no sparse arrays lent
+        m = [sa.DeviceArray.from_host(a) for a in g.csr]
+        A.InputCSR(g.csr[1].size, *m)
+        A.ToCSC()
+        A.set_spmv_type(csr5)
+        A.set_vector_type(sa.SPMSPV_VEC_DENSE)
+        A.set_x(dx)
+        g.A = A
+    for rep in range(3):
+        g.run(slot, f"{x} x, buffers reserved {rep} times again")
+        g.A.deallocPreBuffer()
+        if rep:
+            g.A.allocPreBuffer()
