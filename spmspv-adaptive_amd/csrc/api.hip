@@ -1175,6 +1175,7 @@ int spmspv_dense2sparse_outer(spmspv_handle_t h, int m, float* d_dense, int* ynn
   if (rc) return rc;
   // use the m-sized bitmap region when it fits, else the n-sized one
   unsigned* b = m <= h->m ? h->bitmap : h->bits_int;
+  if (b == h->bits_int && !h->bits_user) h->bits_valid = false;  // the compaction clears it
   launch_bitmap_from_dense(h->stream, d_dense, m, b);
   launch_compact(h->stream, b, nullptr, m, d_dense, 0, d_key, d_val, h->scan_state, h->ctl,
                  next_ep(h, 1));

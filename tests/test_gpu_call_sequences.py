@@ -184,3 +184,26 @@ def test_product_after_buffers_were_given_back(gpu, slot, csr5, x):
         g.A.deallocPreBuffer()
         if rep:
             g.A.allocPreBuffer()
+
+
+def test_product_after_outer_conversion(gpu):
+    """An outer conversion of a vector longer than the result takes the
+    handle's bit array of x as scratch: x's bits are made again."""
+    import scipy.sparse as sp
+    m, n = 500, 4000
+    R = sp.random(m, n, density=0.01, format="csr", random_state=3, dtype=np.float32)
+    R.sort_indices()
+    M = sa.Matrix(m, n, R.indptr.astype(np.int32), R.indices.astype(np.int32), R.data)
+    key, val = sa.gen_sparse_vector(n, 300, 9)
+    d = np.zeros(n, np.float32)
+    d[key] = val
+    dx, yk, yv = sa.DeviceArray.from_host(d), sa.DeviceArray(n, np.int32), sa.DeviceArray(n, np.float32)
+    ek, ev, eb = oracle.spmspv_f64(m, *oracle.csr_to_csc(m, n, M.h_row_ptr, M.h_col, M.h_val), key, val)
+    M.A.set_vector_type(sa.SPMSPV_VEC_DENSE)
+    M.A.set_x(dx)
+    for rep in range(2):
+        cnt = M.A.run(sa.K_ROW_NAIVE, y_key=yk, y_val=yv)
+        np.testing.assert_array_equal(yk.to_host(cnt), ek, err_msg=f"call {rep}")
+        assert np.all(np.abs(yv.to_host(cnt).astype(np.float64) - ev) <= 1e-5 * eb + 1e-30)
+        assert M.A.dense2sparse_outer(n, dx, yk, yv) == key.size
+        np.testing.assert_array_equal(yk.to_host(key.size), key)
