@@ -334,9 +334,9 @@ static int need_enc_x5(spmspv_handle_t h, const float** out, bool values_only) {
   } else {
     int rc;
     if ((rc = need_dense_x(h))) return rc;
-    if (values_only && !h->bits_valid) {
-      // no bit array (4.8 us of 104 at R-MAT s20); the vector type is the one
-      // that building it leaves
+    if (values_only && !h->bits_valid && !h->bits_user) {
+      // no bit array (4.8 us of 104 at R-MAT s20), unless the caller lent one,
+      // which is filled; the vector type is the one that building it leaves
       holds = h->kEnc5Values;
       h->vec_type = SPMSPV_VEC_BITARRAY;
     } else if ((rc = need_bits(h))) {

@@ -207,3 +207,27 @@ def test_product_after_outer_conversion(gpu):
         assert np.all(np.abs(yv.to_host(cnt).astype(np.float64) - ev) <= 1e-5 * eb + 1e-30)
         assert M.A.dense2sparse_outer(n, dx, yk, yv) == key.size
         np.testing.assert_array_equal(yk.to_host(key.size), key)
+
+
+@pytest.mark.parametrize("csr5", [0, 1])
+@pytest.mark.parametrize("slot", [sa.K_ROW_LB, sa.K_SPMV_NAIVE, sa.K_SPMV_LB])
+def test_lent_bit_array_is_filled(gpu, slot, csr5):
+    """A bit array lent with set_bitvector holds a dense x's support after the
+    products that fill it (the plain merge-path product reads none)."""
+    g = Graph(12, 1500)
+    A, n = g.A, g.n
+    A.set_spmv_type(csr5)
+    d = np.zeros(n, np.float32)
+    d[g.key] = g.val
+    d[g.val.size:g.val.size + 5] = -0.0
+    dx, yd = sa.DeviceArray.from_host(d), sa.DeviceArray(n, np.float32)
+    bits = sa.DeviceArray.from_host(np.full((n + 31) // 32, 0x5A5A5A5A, np.int32))
+    A.set_bitvector(bits, bits.count)
+    A.set_vector_type(sa.SPMSPV_VEC_DENSE)
+    A.set_x(dx)
+    if slot == sa.K_SPMV_LB and csr5:
+        A.run(slot, y_dense=yd, want_nnz=False)
+    else:
+        A.run(slot, y_key=g.yk, y_val=g.yv)
+    got = np.unpackbits(bits.to_host().view(np.uint8), bitorder="little")[:n]
+    np.testing.assert_array_equal(got, (d != 0).astype(np.uint8))
