@@ -35,4 +35,16 @@ __device__ __forceinline__ float fixed_value(long long sum, unsigned E) {
   return (float)ldexp((double)sum, (int)E - 172);
 }
 
+// A sum with an Inf or NaN among its terms, in any order: the kinds of its
+// terms (1: +Inf, 2: -Inf, 4: NaN, 0: finite) ORed, and its value from them.
+__device__ __forceinline__ unsigned special_kind(float v) {
+  const unsigned b = __float_as_uint(v);
+  if ((b & 0x7F800000u) != 0x7F800000u) return 0u;
+  return (b & 0x7FFFFFu) ? 4u : 1u << (b >> 31);
+}
+
+__device__ __forceinline__ float special_value(unsigned kinds) {
+  return __uint_as_float(kinds == 1u ? 0x7F800000u : kinds == 2u ? 0xFF800000u : 0x7FC00000u);
+}
+
 }  // namespace spmspv

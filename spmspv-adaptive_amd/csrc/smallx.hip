@@ -357,34 +357,34 @@ __global__ __launch_bounds__(NT) void k_col_fused(const int* __restrict__ colptr
     s.sums.e[u] = 0u;
   }
   __syncthreads();
-  // ---- exact row sums; with an Inf or NaN among the products, in FP32
+  // ---- exact row sums; a row with an Inf or NaN among its products (exponent
+  // 0xFF, known to all once the maxima are in) collects which of the two
+  // infinities and NaN it holds, which is all that its sum depends on
   int num[IPT];
-  int special = 0;
 #pragma unroll
   for (int j = 0; j < IPT; ++j) {
     num[j] = 0;
     if (mine[j]) {
       const int wd = row[j] >> 5;
       num[j] = s_pfx[wd] + __popc(s_bits[wd] & ((1u << (row[j] & 31)) - 1u));
-      const unsigned ef = prod_ef(val[j]);
-      special |= ef == 0xFFu;
-      atomicMax(&s.sums.e[num[j]], ef);
+      atomicMax(&s.sums.e[num[j]], prod_ef(val[j]));
     }
   }
-  special = __syncthreads_or(special);
+  __syncthreads();
 #pragma unroll
   for (int j = 0; j < IPT; ++j) {
     if (mine[j]) {
-      if (special) atomicAdd(reinterpret_cast<float*>(&s.sums.q[num[j]]), val[j]);
-      else atomicAdd(&s.sums.q[num[j]], (unsigned long long)prod_fixed(val[j], s.sums.e[num[j]]));
+      const unsigned E = s.sums.e[num[j]];
+      if (E == 0xFFu) atomicOr(&s.sums.q[num[j]], (unsigned long long)special_kind(val[j]));
+      else atomicAdd(&s.sums.q[num[j]], (unsigned long long)prod_fixed(val[j], E));
     }
   }
   __syncthreads();
   const long long pre = (long long)tile_prefix(state, blockIdx.x, epoch, (unsigned long long)tot, &s_pre);
   // ---- sorted output, device-coherent (visible once acknowledged)
   for (int u = threadIdx.x; u < tot; u += NT) {
-    const float v = special ? *reinterpret_cast<const float*>(&s.sums.q[u])
-                            : fixed_value((long long)s.sums.q[u], s.sums.e[u]);
+    const float v = s.sums.e[u] == 0xFFu ? special_value((unsigned)s.sums.q[u])
+                                         : fixed_value((long long)s.sums.q[u], s.sums.e[u]);
     __hip_atomic_store(yval + pre + u, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   {

@@ -231,3 +231,46 @@ def test_lent_bit_array_is_filled(gpu, slot, csr5):
         A.run(slot, y_key=g.yk, y_val=g.yv)
     got = np.unpackbits(bits.to_host().view(np.uint8), bitorder="little")[:n]
     np.testing.assert_array_equal(got, (d != 0).astype(np.uint8))
+
+
+@pytest.mark.parametrize("m", [256, 20011])
+@pytest.mark.parametrize("slot", [0, 1, 2, 3])
+def test_finite_rows_beside_special_ones(gpu, m, slot):
+    """Rows without an Inf or NaN among their products have the same bits in
+    every call, and the bits they have where the other rows' special entries
+    are finite; the other rows are Inf or NaN as the sum in any order is."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(m)
+    n, k, per = 4000, 650, 16
+    rows = np.concatenate([rng.choice(min(m, 400), per, replace=False) for _ in range(n)]) * (m // min(m, 400))
+    R = sp.csr_matrix((rng.uniform(-1, 1, n * per).astype(np.float32), (rows, np.repeat(np.arange(n), per))), shape=(m, n))
+    R.sort_indices()
+    M = sa.Matrix(m, n, R.indptr.astype(np.int32), R.indices.astype(np.int32), R.data)
+    cp, ri, cv = oracle.csr_to_csc(m, n, M.h_row_ptr, M.h_col, M.h_val)
+    key, val = sa.gen_sparse_vector(n, k, 3)
+    odd = val.copy()
+    odd[[5, 300]], odd[77], odd[400] = np.inf, -np.inf, np.nan
+    yk, yv = sa.DeviceArray(m, np.int32), sa.DeviceArray(m, np.float32)
+    dk = sa.DeviceArray.from_host(key, np.int32)
+
+    def product(v):
+        dv = sa.DeviceArray.from_host(v, np.float32)
+        M.A.set_sparse_x(dk, dv, k)
+        cnt = M.A.run(slot, y_key=yk, y_val=yv)
+        return yk.to_host(cnt), yv.to_host(cnt)
+
+    ek, plain = product(val)
+    dense = np.zeros(n)
+    dense[key] = odd
+    with np.errstate(invalid="ignore"):
+        want = np.zeros(m)
+        for c in key:
+            want[ri[cp[c]:cp[c + 1]]] += cv[cp[c]:cp[c + 1]].astype(np.float64) * dense[c]
+    want = want[ek]
+    finite = np.isfinite(want)
+    assert 40 < finite.sum() < ek.size
+    for rep in range(8):
+        gk, got = product(odd)
+        np.testing.assert_array_equal(gk, ek)
+        np.testing.assert_array_equal(got[finite].view(np.uint32), plain[finite].view(np.uint32), err_msg=f"call {rep}")
+        np.testing.assert_array_equal(got[~finite], want[~finite].astype(np.float32))
