@@ -274,3 +274,20 @@ def test_finite_rows_beside_special_ones(gpu, m, slot):
         np.testing.assert_array_equal(gk, ek)
         np.testing.assert_array_equal(got[finite].view(np.uint32), plain[finite].view(np.uint32), err_msg=f"call {rep}")
         np.testing.assert_array_equal(got[~finite], want[~finite].astype(np.float32))
+
+
+@pytest.mark.parametrize("policy", [2, 3, 5])
+def test_bfs_after_queued_products(gpu, policy):
+    """Products without a count are still running on the handle's (null) stream
+    when a BFS starts on its own one: both use the handle's buffers."""
+    g = Graph(18, 100000, per=16)
+    lev = sa.DeviceArray(g.n, np.int32)
+    ref, _ = oracle.bfs(g.n, g.csc[0], g.csc[1], 5)
+    for slot in (sa.K_COL_LB_ATOMIC, sa.K_COL_BUCKET):
+        cnt = g.A.run(slot, y_key=g.yk, y_val=g.yv)
+        for rep in range(20):
+            g.A.set_sparse_x(g.dk, g.dv, g.key.size)
+            g.A.run(slot, y_key=g.yk, y_val=g.yv, want_nnz=False)
+        g.A.bfs(5, lev, policy=policy)
+        np.testing.assert_array_equal(lev.to_host(), ref)
+        g.check(cnt, f"slot {slot} before the BFS")
