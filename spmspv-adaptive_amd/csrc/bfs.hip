@@ -9,13 +9,13 @@
 //          unvisited rows (naive team per vertex / merge-path balanced);
 //   K1/K3  top-down gather of all neighbours' row keys, in-house radix sort
 //          of the keys alone, then each distinct row marked;
-//   K4/K5/K7  bottom-up: each unvisited row scans its neighbours and stops at
-//          the first frontier member (on booleans the masked and unmasked
-//          load-balanced row products coincide, and a row's result is known
-//          at its first hit: the merge-path scan of every nonzero that K5/K7
-//          ran before took 420 us at a large level of R-MAT s22, this 60 to
-//          120 us; at a level of one or two vertices, where no row stops
-//          early, 660 us against 390);
+//   K4/K5/K7  by direction: where the frontier holds more than 1 / kTopDown of
+//          the edges, bottom-up: each unvisited row scans its neighbours and
+//          stops at the first frontier member (on booleans the masked and
+//          unmasked load-balanced row products coincide, and a row's result is
+//          known at its first hit: the merge-path scan of every nonzero that
+//          K5/K7 ran before took 420 us at a large level of R-MAT s22, this 60
+//          to 120 us). Below that few rows stop early and K2's kernels run;
 //   K6     naive row scan without early exit.
 // Every slot marks the rows it reaches in the next frontier's bit array;
 // one collect pass then takes the unvisited ones among them, writes their
@@ -35,6 +35,7 @@
 #include <hip/hip_runtime.h>
 
 #include <chrono>
+#include <cmath>
 #include <cstring>
 
 #include "handle.hpp"
@@ -66,6 +67,15 @@ constexpr int kBuTeam = 16;    // lanes per queued item in the bottom-up tail pa
 constexpr int kBuChunk = 256;  // neighbours per queued item
 constexpr int kBuUnroll = 4;   // neighbours a lane has in flight
 constexpr int kBuRows = 8;     // most rows per thread and queue append
+
+// The row slots' direction: top-down up to this part of the edges in the
+// frontier. A level in us, top-down / bottom-up / every nonzero by merge path
+// (frontier's edges of all): R-MAT s22 16 / 679 / 385 (1 of 128 M), 62 / 369 /
+// 470 (0.13 %), 94 / 335 / 493 (1.1 %), 414 / 151 / 511 (17 %); s20 37 / 217 /
+// 131 (0.2 %), 246 / 50 / 141 (33 %); s18 41 / 46 / 52 (0.33 %), 66 / 40 / 58
+// (7.8 %); uniform, 1 M vertices 103 / 179 / 145 (2.8 %), 246 / 117 / 157
+// (10.5 %); a 1,000 x 1,000 grid 17 / 27 / 34.
+constexpr int kTopDown = 32;
 
 // Marks row v in the next frontier unless it is visited or marked already
 // (visited is constant while a slot's kernels run).
@@ -428,7 +438,7 @@ void enqueue_level(spmspv_handle_t h, hipStream_t s, int slot, int cur, int* lev
       launch_row_naive(s, true, true, h->csr_row, h->csr_col, nullptr, nullptr, b->fbits[cur],
                        h->m, h->team_row, nullptr, nbits);
       break;
-    default:  // 4, 5, 7: bottom-up
+    default:  // 4, 5, 7 on a frontier of many edges: bottom-up
       if (h->nnz > 0) {
         // rows per thread and queue append: as many as leave every CU its workgroups
         const int rows = std::max(1, std::min(kBuRows, h->m / (kBfsNT * 1024)));
@@ -588,11 +598,15 @@ static int bfs_run(spmspv_handle_t h, int src, int* d_levels, int policy, int us
   };
   if (e == hipSuccess) e = level_word(0);
   int cur = 0, nlev = 1;
-  int slot_hist[8] = {0};
   while (e == hipSuccess && (int)(word & 0xffffffff) > 0) {
     int slot = policy >= 0 ? policy : (int)((word >> 32) & 0xff);
     if (slot < 0 || slot >= SPMSPV_NUM_SLOTS) slot = SPMSPV_K_COL_LB_ATOMIC;
-    slot_hist[slot]++;
+    // selector feature 12: log2 of the frontier's part of the edges
+    if (slot == SPMSPV_K_ROW_NAIVE || slot == SPMSPV_K_ROW_LB || slot == SPMSPV_K_SPMV_LB) {
+      float part;
+      __atomic_load(reinterpret_cast<float*>(sw + 1) + 12, &part, __ATOMIC_ACQUIRE);
+      if (part <= -std::log2((float)kTopDown)) slot = SPMSPV_K_COL_LB_ATOMIC;
+    }
     const int lev = nlev - 1;  // index of the level about to run
     if (trace && lev < max_levels) {
       std::memcpy(level_feat + 16 * lev, sw + 1, sizeof(float) * 16);

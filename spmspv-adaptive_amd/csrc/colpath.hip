@@ -130,7 +130,9 @@ __global__ __launch_bounds__(NT) void k_prep(const int* __restrict__ colptr,
     if (!open.cnt || threadIdx.x >= kWave) return;
     // the feature words are acknowledged before the level word goes out; the
     // host reads nothing else, so no L2 write-back is needed
-    if (threadIdx.x < 16) reinterpret_cast<float*>(open.sig + 1)[threadIdx.x] = ctl->feat[threadIdx.x];
+    if (threadIdx.x < 16)
+      __hip_atomic_store(reinterpret_cast<float*>(open.sig + 1) + threadIdx.x, ctl->feat[threadIdx.x],
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (threadIdx.x == 0) {
       int* cnt = open.cnt;
