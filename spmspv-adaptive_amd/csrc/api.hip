@@ -703,7 +703,7 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
         float* clr = h->csr5.cperm && xin == h->x_enc5b[h->enc5_cur] && !h->enc5_clean[idle]
                          ? h->x_enc5b[idle]
                          : nullptr;
-        launch_csr5(s, h->csr5, masked, hits, xin, nullptr, m, h->nnz, yout, yout != h->acc, h->marks,
+        launch_csr5(s, h->csr5, masked, hits, xin, m, h->nnz, yout, yout != h->acc, h->marks,
                     &vals, &kmap, &nk, h->time_main ? h->evk0 : nullptr,
                     h->time_main ? h->evk1 : nullptr, h->gate, clr);
         h->main_timed = h->time_main;

@@ -34,7 +34,6 @@ namespace spmspv {
 
 namespace {
 
-constexpr int kXPlain5 = 0, kXEnc5 = 1, kXBits5 = 2;
 // columns (after renumbering, the ones with the most nonzeros) whose x
 // entries the tile kernel keeps in LDS: all 160 KB of a CU's LDS, shared by
 // one block per CU that holds as many waves as the registers allow. At R-MAT
@@ -167,13 +166,13 @@ __global__ void k_csr5_transpose(const int* __restrict__ col, const float* __res
 // HOT > 0: the first `hot` (<= HOT) entries of x, the columns with the most
 // nonzeros once the columns are renumbered, are copied into LDS at kernel
 // start and gathered from there; the other lanes of a gather read global x.
-template <int S, int XIN, bool MASKED, bool HITS, int HOT>
+template <int S, bool MASKED, bool HITS, int HOT>
 __global__ __launch_bounds__(csr5_nt(S, HOT)) void k_csr5(const int* __restrict__ ccol,
                                               const float* __restrict__ cval,
                                               const unsigned* __restrict__ flags,
                                               const unsigned* __restrict__ tinfo,
                                               const float* __restrict__ x,
-                                              const unsigned* __restrict__ xbits, int nnz, int ntiles,
+                                              int nnz, int ntiles,
                                               float* __restrict__ y, unsigned char* __restrict__ marks,
                                               float* __restrict__ carry_val,
                                               int* __restrict__ carry_row,
@@ -219,8 +218,7 @@ __global__ __launch_bounds__(csr5_nt(S, HOT)) void k_csr5(const int* __restrict_
 
   int cN[S];  // stage 2: columns / values loading
   float vN[S];
-  float vG[S], xG[S];  // stage 1: values and gathered x (or bit words)
-  int cG[S];
+  float vG[S], xG[S];  // stage 1: values and gathered x
   // hot items: their product (masked) is formed as soon as LDS answers and
   // kept in vG; bit i of hG marks item i hot, bit i of bG its support bit
   unsigned hG = 0u, bG = 0u;
@@ -254,10 +252,7 @@ __global__ __launch_bounds__(csr5_nt(S, HOT)) void k_csr5(const int* __restrict_
     // loads are a tile old; the column loads issued beside them are waited
     // for by the gathers anyway)
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-      asm volatile("v_mov_b32 %0, %1" : "=v"(vG[i]) : "v"(vN[i]));
-      if (XIN == kXBits5) asm volatile("v_mov_b32 %0, %1" : "=v"(cG[i]) : "v"(cN[i]));
-    }
+    for (int i = 0; i < S; ++i) asm volatile("v_mov_b32 %0, %1" : "=v"(vG[i]) : "v"(vN[i]));
     unsigned hm = 0u;
     if (HOT > 0) {
 #pragma unroll
@@ -266,9 +261,7 @@ __global__ __launch_bounds__(csr5_nt(S, HOT)) void k_csr5(const int* __restrict_
     float xL[HOT > 0 ? S : 1];
 #pragma unroll
     for (int i = 0; i < S; ++i) {
-      if (XIN == kXBits5) {
-        xG[i] = __builtin_bit_cast(float, xbits[(unsigned)cN[i] >> 5]);
-      } else if (HOT > 0) {
+      if (HOT > 0) {
         // both reads unconditional: the hot lanes give the global read an
         // offset past the end of x (the buffer read returns 0 without a
         // memory access), the others read LDS word 0 (a broadcast)
@@ -346,19 +339,12 @@ __global__ __launch_bounds__(csr5_nt(S, HOT)) void k_csr5(const int* __restrict_
         ++j;
       }
       const bool ok = lanes * S + i < lim;
-      bool b;
-      float q;
-      if (XIN == kXBits5) {
-        b = (__builtin_bit_cast(unsigned, xG[i]) >> (cG[i] & 31)) & 1u;
-        q = b ? vG[i] : 0.f;
-      } else {
-        b = __builtin_bit_cast(unsigned, xG[i]) != 0u;
-        q = vG[i] * xG[i];
-        if (MASKED) q = b ? q : 0.f;
-        if (HOT > 0 && ((hh >> i) & 1u)) {  // a select, not a branch
-          b = (hb >> i) & 1u;
-          q = vG[i];
-        }
+      bool b = __builtin_bit_cast(unsigned, xG[i]) != 0u;
+      float q = vG[i] * xG[i];
+      if (MASKED) q = b ? q : 0.f;
+      if (HOT > 0 && ((hh >> i) & 1u)) {  // a select, not a branch
+        b = (hb >> i) & 1u;
+        q = vG[i];
       }
       s += ok ? q : 0.f;
       if (HITS) h |= (ok && b) ? 1 : 0;
@@ -850,7 +836,7 @@ hipError_t csr5_build(hipStream_t s, const int* row_ptr, const int* col, const f
 }
 
 void launch_csr5(hipStream_t s, const Csr5& c, bool masked, bool hits, const float* x,
-                 const unsigned* xbits, int m, int nnz, float* y, bool y_dense_rows,
+                 int m, int nnz, float* y, bool y_dense_rows,
                  unsigned char* marks, float** vals_out, const int** keymap_out, int* n_out,
                  hipEvent_t ev_begin, hipEvent_t ev_end, Gate g, float* clear) {
   const bool compressed = c.n_empty > 0;
@@ -867,25 +853,24 @@ void launch_csr5(hipStream_t s, const Csr5& c, bool masked, bool hits, const flo
   // the LDS copy holds the hot columns once they come first (column order),
   // or the whole of x when it fits
   const bool lds_hot = c.n >= 1 && (c.cperm != nullptr || c.n <= kCsr5Hot);
-#define SPMSPV_CSR5(SS, XI, MK, HT, HOTN)                                                        \
+#define SPMSPV_CSR5(SS, MK, HT, HOTN)                                                            \
   {                                                                                              \
-    const void* fn = (const void*)k_csr5<SS, XI, MK, HT, HOTN>;                                  \
+    const void* fn = (const void*)k_csr5<SS, MK, HT, HOTN>;                                  \
     constexpr int nt = csr5_nt(SS, HOTN), wpb = nt / kWave;                                      \
     const int waves = std::max(wpb, std::min(c.ntiles, resident_blocks(fn, nt) * wpb));          \
-    hipLaunchKernelGGL((k_csr5<SS, XI, MK, HT, HOTN>), dim3((waves + wpb - 1) / wpb), dim3(nt), 0, \
+    hipLaunchKernelGGL((k_csr5<SS, MK, HT, HOTN>), dim3((waves + wpb - 1) / wpb), dim3(nt), 0, \
                        s,                                                                        \
-                       c.ccol, c.cval, c.flags, c.tinfo, x, xbits, nnz, c.ntiles, yk, marks,     \
+                       c.ccol, c.cval, c.flags, c.tinfo, x, nnz, c.ntiles, yk, marks,            \
                        c.carry_val, c.carry_row, c.carry_hit, std::min(c.n, HOTN), c.n, clear, g); \
   }
-#define SPMSPV_CSR5_H(SS, XI, MK, HT)      \
-  if (lds_hot) SPMSPV_CSR5(SS, XI, MK, HT, kCsr5Hot) \
-  else SPMSPV_CSR5(SS, XI, MK, HT, 0)
-#define SPMSPV_CSR5_S(SS)                                          \
-  if (!x) SPMSPV_CSR5(SS, kXBits5, true, true, 0)                  \
-  else if (masked && hits) SPMSPV_CSR5_H(SS, kXEnc5, true, true)   \
-  else if (masked) SPMSPV_CSR5_H(SS, kXEnc5, true, false)          \
-  else if (hits) SPMSPV_CSR5_H(SS, kXEnc5, false, true)            \
-  else SPMSPV_CSR5_H(SS, kXPlain5, false, false)
+#define SPMSPV_CSR5_H(SS, MK, HT)                \
+  if (lds_hot) SPMSPV_CSR5(SS, MK, HT, kCsr5Hot) \
+  else SPMSPV_CSR5(SS, MK, HT, 0)
+#define SPMSPV_CSR5_S(SS)                               \
+  if (masked && hits) SPMSPV_CSR5_H(SS, true, true)     \
+  else if (masked) SPMSPV_CSR5_H(SS, true, false)       \
+  else if (hits) SPMSPV_CSR5_H(SS, false, true)         \
+  else SPMSPV_CSR5_H(SS, false, false)
   if (ev_begin) (void)hipEventRecord(ev_begin, s);
   if (c.S == 8) {
     SPMSPV_CSR5_S(8)

@@ -379,8 +379,8 @@ bool launch_column_order(hipStream_t s, const ColumnOrderArgs& a, const int* col
 hipError_t csr5_build(hipStream_t s, const int* row_ptr, const int* col, const float* val, int m,
                       int n, int nnz, int S, void* mem, int* h_pin, const ColumnOrderArgs* order,
                       Csr5* out);
-// Same gather modes as launch_row_merge (x == nullptr: bit array only, for
-// a copy without a column order). x is indexed by the copy's column order.
+// x as for launch_row_merge (the support encoding with masked or hits, else
+// plain), indexed by the copy's column order.
 // Without empty rows the results go to y (one mark byte per row with hits).
 // With empty rows they go to the non-empty-row space: vals_out = y_ne,
 // marks indexed by non-empty row, keymap_out = rows_ne (for the
@@ -390,7 +390,7 @@ hipError_t csr5_build(hipStream_t s, const int* row_ptr, const int* col, const f
 // clear (nullable, c.n floats, 16-byte aligned, not x) is set to +0.0 by the
 // tile kernel as it runs.
 void launch_csr5(hipStream_t s, const Csr5& c, bool masked, bool hits, const float* x,
-                 const unsigned* xbits, int m, int nnz, float* y, bool y_dense_rows,
+                 int m, int nnz, float* y, bool y_dense_rows,
                  unsigned char* marks, float** vals_out, const int** keymap_out, int* n_out,
                  hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr, Gate g = {},
                  float* clear = nullptr);

@@ -92,8 +92,6 @@ __device__ __forceinline__ void seg_scan_row(bool f, float v, int h, float* cin,
   *tail_h = th;
 }
 
-constexpr int kXPlain = 0, kXEnc = 1;
-
 // One merge-path tile: rows i0..i1-1 end in it, nonzeros j0..j0+nj-1.
 struct RowTile {
   int i0, i1, nr, nj, j0;
@@ -121,17 +119,16 @@ __device__ __forceinline__ RowTile row_tile(const int* __restrict__ split, int t
 //             position of its last nonzero, every thread sums its VT
 //             consecutive products, and a block-wide segmented scan joins
 //             rows that cross threads.
-// XIN selects what is gathered per nonzero:
-//   kXPlain: x values (support not needed: SpMV with dense output),
-//   kXEnc  : the support-encoded x (+0.0 outside the support, a nonzero bit
-//            pattern inside it, an explicit zero stored as -0.0), so one
-//            gather yields both the value and the support bit.
+// x is gathered once per nonzero: with MASKED or HITS the support-encoded x
+// (+0.0 outside the support, a nonzero bit pattern inside it, an explicit zero
+// stored as -0.0), so that one gather yields both the value and the support
+// bit, else x's values.
 // Loads use a per-tile base pointer with 32-bit offsets and are
 // unconditional (clamped) so that a stage's loads issue back to back.
 // Rows that cross tiles leave their tail in carry_*[t] (row i1), which
 // k_row_fixup adds in tile order.
 // STREAM: columns and values are read past the caches (nontemporal).
-template <int NT, int VT, int XIN, bool MASKED, bool HITS, bool STREAM>
+template <int NT, int VT, bool MASKED, bool HITS, bool STREAM>
 __global__ __launch_bounds__(NT) void k_row_merge(const int* __restrict__ row_ptr,
                                                   const int* __restrict__ col,
                                                   const float* __restrict__ val,
@@ -371,10 +368,10 @@ void launch_row_merge(hipStream_t s, bool masked, bool hits, const int* row_ptr,
   // 141 / 158 against 148 / 149.
   const bool stream = (long long)nnz * 8 > (64ll << 20);
   // one resident wave of workgroups, each walking many tiles
-#define SPMSPV_ROW_MERGE(V, XI, MK, HT)                                                          \
+#define SPMSPV_ROW_MERGE(V, MK, HT)                                                              \
   {                                                                                             \
-    auto* kern = stream ? k_row_merge<kRowNT, V, XI, MK, HT, true>                              \
-                        : k_row_merge<kRowNT, V, XI, MK, HT, false>;                            \
+    auto* kern = stream ? k_row_merge<kRowNT, V, MK, HT, true>                                  \
+                        : k_row_merge<kRowNT, V, MK, HT, false>;                                \
     const void* fn = (const void*)kern;                                                         \
     hipLaunchKernelGGL(kern,                                                                    \
                        dim3(std::min(ntiles, resident_blocks(fn, kRowNT))), dim3(kRowNT), 0, s, \
@@ -382,10 +379,10 @@ void launch_row_merge(hipStream_t s, bool masked, bool hits, const int* row_ptr,
                        carry_row, carry_hit, g);                                                \
   }
 #define SPMSPV_ROW_MERGE_VT(V)                                   \
-  if (masked && hits) SPMSPV_ROW_MERGE(V, kXEnc, true, true) \
-  else if (masked) SPMSPV_ROW_MERGE(V, kXEnc, true, false)       \
-  else if (hits) SPMSPV_ROW_MERGE(V, kXEnc, false, true)         \
-  else SPMSPV_ROW_MERGE(V, kXPlain, false, false)
+  if (masked && hits) SPMSPV_ROW_MERGE(V, true, true)    \
+  else if (masked) SPMSPV_ROW_MERGE(V, true, false)      \
+  else if (hits) SPMSPV_ROW_MERGE(V, false, true)        \
+  else SPMSPV_ROW_MERGE(V, false, false)
   if (ev_begin) (void)hipEventRecord(ev_begin, s);
   if (vt == 5) {
     SPMSPV_ROW_MERGE_VT(5)
