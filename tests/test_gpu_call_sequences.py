@@ -291,3 +291,58 @@ def test_bfs_after_queued_products(gpu, policy):
         g.A.bfs(5, lev, policy=policy)
         np.testing.assert_array_equal(lev.to_host(), ref)
         g.check(cnt, f"slot {slot} before the BFS")
+
+
+@pytest.mark.parametrize("slot", [sa.K_COL_NAIVE_SORT, sa.K_COL_LB_SORT])
+@pytest.mark.parametrize("out", ["count", "no count", "dense"])
+def test_products_fall_below_the_guess(gpu, slot, out):
+    """A sort slot queued behind the selector after a call of more than 24,576
+    products leaves out the single-workgroup sort: an x of the same size class
+    with at most 3,072 products (none among them) is sorted by a second run."""
+    import ctypes
+    import scipy.sparse as sp
+    m, n, k = 30011, 40000, 9000
+    rng = np.random.default_rng(slot)
+    # 15,000 empty columns, 5,000 of one entry, 20,000 of thirty
+    per = np.repeat([0, 1, 30], [15000, 5000, 20000])
+    cols = np.repeat(np.arange(n), per)
+    R = sp.csr_matrix((np.ones(cols.size, np.float32), (rng.integers(0, m, cols.size), cols)), shape=(m, n))
+    R.sort_indices()
+    R.data = rng.uniform(0.1, 1, R.nnz).astype(np.float32)
+    M = sa.Matrix(m, n, R.indptr.astype(np.int32), R.indices.astype(np.int32), R.data)
+    csc = oracle.csr_to_csc(m, n, M.h_row_ptr, M.h_col, M.h_val)
+    yk, yv, yd = sa.DeviceArray(m, np.int32), sa.DeviceArray(m, np.float32), sa.DeviceArray(m, np.float32)
+    M.A.selector_mode(2, slot)
+    M.A.set_small_x_path(False)
+    last = None
+    for ones, thirties in [(0, k), (0, k), (0, 0), (0, k), (3000, 0), (3000, 0), (500, k - 500), (0, 0), (0, 0), (3071, 0), (0, k)]:
+        key = np.sort(np.concatenate([rng.choice(15000, k - ones - thirties, replace=False),
+                                      15000 + rng.choice(5000, ones, replace=False),
+                                      20000 + rng.choice(20000, thirties, replace=False)])).astype(np.int32)
+        val = rng.uniform(-1, 1, k).astype(np.float32)
+        dk, dv = sa.DeviceArray.from_host(key, np.int32), sa.DeviceArray.from_host(val, np.float32)
+        M.A.set_sparse_x(dk, dv, k)
+        products = int(np.diff(csc[0])[key].sum())
+        before = M.A.speculation_stats()[1]
+        if out == "no count":
+            used = ctypes.c_int(-1)
+            assert sa.lib().spmspv_run_auto(M.A.h, 1.0, None, yk.ptr, yv.ptr, None, ctypes.byref(used)) == 0
+            sa.synchronize()
+            c = np.empty(1, np.int32)
+            p = ctypes.c_void_p(sa.lib().spmspv_ynnz_device(M.A.h))
+            assert sa.lib().spmspv_memcpy_d2h(c.ctypes.data_as(ctypes.c_void_p), p, 4) == 0
+            cnt = int(c[0])
+        else:
+            cnt, _ = M.A.run_auto(y_dense=yd if out == "dense" else None, y_key=yk, y_val=yv)
+        missed = M.A.speculation_stats()[1] - before
+        if last is not None and last > 8 * 3072 and products <= 3072:
+            assert missed == 1, (last, products)
+        ek, ev, eb = oracle.spmspv_f64(m, *csc, key, val)
+        assert cnt == ek.size
+        np.testing.assert_array_equal(yk.to_host(cnt), ek)
+        assert np.all(np.abs(yv.to_host(cnt).astype(np.float64) - ev) <= 1e-5 * eb + 1e-30)
+        if out == "dense":
+            ref, bound = np.zeros(m), np.zeros(m)
+            ref[ek], bound[ek] = ev, eb
+            assert np.all(np.abs(yd.to_host() - ref) <= 1e-5 * bound + 1e-30)
+        last = products
