@@ -22,10 +22,10 @@
  *  - No allocation after spmspv_alloc_pre_buffer(): it reserves the arena,
  *    the CSR5 copy at its largest width, the BFS and PageRank buffers (square
  *    matrices)
- *    and the selector stash of a 4,096-vector batch. The exceptions are
+ *    and the workspace of a batch of 4,096 vectors. The exceptions are
  *    stated where they apply: spmspv_to_csc (handle-owned CSC, once per
  *    matrix), a spmspv_run_batched call of more than 4,096 vectors (grows
- *    the stash once), spmspv_flush_cache and spmspv_measure_ceilings
+ *    the workspace once), spmspv_flush_cache and spmspv_measure_ceilings
  *    (measurement helpers). Without
  *    alloc_pre_buffer, the first call that needs a buffer allocates it.
  *  - No host exit(); errors come back as SPMSPV_* codes and

@@ -585,8 +585,8 @@ int run_kernel(spmspv_handle_t h, int kid, float* y_dense, int* y_key, float* y_
       const bool lb = kid == SPMSPV_K_COL_LB_SORT;
       // the scan sends bin_len to the host, which waits for it with the gather
       // queued behind the scan (a copy and a stream wait after the gather
-      // left the device idle for a round trip)
-      const bool sent = !h->prep_valid && !h->gate.word;
+      // left the device idle for a round trip), unless the host has it
+      const bool sent = !h->prep_valid && !h->gate.word && h->binlen_host < 0;
       if (!h->prep_valid) {
         const SelectorArgs word{nullptr, nullptr, 0, 0, h->sig_dev + 1};
         if (sent) __atomic_store_n(h->sig + 1, kSigPending, __ATOMIC_RELEASE);
@@ -937,8 +937,8 @@ int spmspv_alloc_pre_buffer(spmspv_handle_t h) {
   int rc = ensure_arena(h);
   if (rc) return rc;
   // Everything a later call could allocate is reserved here: the CSR5 copy
-  // at its largest width, the BFS, multi-source BFS and PageRank buffers and a batch
-  // workspace of the usual size.
+  // at its largest width, the BFS, multi-source BFS and PageRank buffers and the
+  // workspace of a batch of up to 4,096 vectors.
   if (h->csr_row) {
     size_t most = 0;
     for (int S = 1; S <= 32; ++S) most = std::max(most, csr5_bytes(h->m, h->n, h->nnz, S));

@@ -3,9 +3,11 @@
 //   1. one launch selects for every vector (exact bin_len and choice per
 //      vector); one readback;
 //   2. one launch scans the columns of every vector whose slot reads the
-//      scan; then every vector's chosen pipeline is queued back to back with
+//      scan, of as many at a time as the workspace holds (a vector that does
+//      not fit alone is scanned in its own pipeline, as a single call is);
+//      then every vector's chosen pipeline is queued back to back with
 //      its bin_len already known (no readback inside), results at the
-//      caller's offsets. Each vector has its own control block and scan, so
+//      caller's offsets. Each vector has its own control block, so
 //      nothing is copied between two pipelines, and one launch at the end
 //      hands all the counts to d_ynnz;
 //   3. one final synchronisation.
@@ -19,21 +21,18 @@
 
 using namespace spmspv;
 
-// Workspace: the vectors' descriptors, control blocks, selector words and
-// tiles (sized by vectors and keys), with the scans' splits (known after the
-// selection) behind them where they fit, else in `split`. Grown when a batch
-// needs more, freed with the handle.
+// Workspace: the vectors' descriptors, control blocks and selector words, their
+// tiles, and the scans of one group of vectors. Reserved for kBatchVecs vectors
+// of any size, grown by a batch of more vectors, freed with the handle.
 struct BatchState {
   char* mem = nullptr;
   size_t bytes = 0;
-  int* split = nullptr;
-  size_t splits = 0;
 };
 
 namespace {
 
-constexpr int kBatchVecs = 4096;
-constexpr size_t kBatchKeys = 1 << 21, kBatchSplits = 1 << 18;
+// Places of a group's scans and splits: 48 vectors of R-MAT s20 hold 1.4 M keys.
+constexpr int kBatchVecs = 4096, kBatchKeys = 1 << 21, kBatchSplits = 1 << 18;
 
 __global__ void k_batch_counts(const Ctl* __restrict__ ctls, int nvec, int* __restrict__ ynnz) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -42,11 +41,11 @@ __global__ void k_batch_counts(const Ctl* __restrict__ ctls, int nvec, int* __re
 
 size_t up256(size_t v) { return (v + 255) & ~size_t(255); }
 
-// Device layout for nvec vectors of `keys` keys in `tiles` tiles; the control
-// blocks and arrival counts, which start at zero, come first.
+// Device layout for nvec vectors in `tiles` tiles, scanned in groups of `places`
+// places; the control blocks and arrival counts, which start at zero, come first.
 struct Layout {
-  size_t ctls, arrive, zeroed, stash, vec, tile_vec, list, tsum, tmax, ptr, xbeg, bytes;
-  Layout(size_t nvec, size_t keys, size_t tiles) {
+  size_t ctls, arrive, zeroed, stash, vec, tile_vec, list, tsum, tmax, ptr, xbeg, split, bytes;
+  Layout(size_t nvec, size_t tiles, size_t places) {
     size_t o = 0;
     auto take = [&](size_t b) {
       const size_t r = o;
@@ -62,33 +61,25 @@ struct Layout {
     list = take(tiles * sizeof(int));
     tsum = take(tiles * sizeof(long long));
     tmax = take(tiles * sizeof(int));
-    ptr = take((keys + nvec) * sizeof(int));
-    xbeg = take(keys * sizeof(int));
+    ptr = take(places * sizeof(int));
+    xbeg = take(places * sizeof(int));
+    split = take(kBatchSplits * sizeof(int));
     bytes = o;
   }
 };
 
 size_t tiles_of(size_t keys) { return std::max<size_t>(1, (keys + kWideTile - 1) / kWideTile); }
 
-int grow(spmspv_handle_t h, size_t bytes, size_t splits) {
+int grow(spmspv_handle_t h, size_t bytes) {
   if (!h->batch) h->batch = new BatchState();
   BatchState* b = h->batch;
-  if (b->bytes < bytes) {
-    HIP_TRY(h, hipStreamSynchronize(h->stream));
-    if (b->mem) HIP_TRY(h, hipFree(b->mem));
-    b->mem = nullptr;
-    b->bytes = 0;
-    HIP_TRY(h, hipMalloc((void**)&b->mem, bytes));
-    b->bytes = bytes;
-  }
-  if (b->splits < splits) {
-    HIP_TRY(h, hipStreamSynchronize(h->stream));
-    if (b->split) HIP_TRY(h, hipFree(b->split));
-    b->split = nullptr;
-    b->splits = 0;
-    HIP_TRY(h, hipMalloc((void**)&b->split, splits * sizeof(int)));
-    b->splits = splits;
-  }
+  if (b->bytes >= bytes) return SPMSPV_SUCCESS;
+  HIP_TRY(h, hipStreamSynchronize(h->stream));
+  if (b->mem) HIP_TRY(h, hipFree(b->mem));
+  b->mem = nullptr;
+  b->bytes = 0;
+  HIP_TRY(h, hipMalloc((void**)&b->mem, bytes));
+  b->bytes = bytes;
   return SPMSPV_SUCCESS;
 }
 
@@ -96,14 +87,14 @@ int grow(spmspv_handle_t h, size_t bytes, size_t splits) {
 
 namespace spmspv {
 int batch_alloc(spmspv_handle_t h) {
-  const size_t tiles = kBatchKeys / kWideTile + kBatchVecs + 1;
-  return grow(h, Layout(kBatchVecs, kBatchKeys, tiles).bytes + kBatchSplits * sizeof(int), 0);
+  // the vectors' offsets are ints: all their keys lie in 2^31
+  const size_t tiles = std::min(kBatchVecs * tiles_of((size_t)h->n), (size_t{1} << 31) / kWideTile + kBatchVecs);
+  return grow(h, Layout(kBatchVecs, tiles, kBatchKeys).bytes);
 }
 
 void batch_release(spmspv_handle_t h) {
   if (!h || !h->batch) return;
   if (h->batch->mem) (void)hipFree(h->batch->mem);
-  if (h->batch->split) (void)hipFree(h->batch->split);
   delete h->batch;
   h->batch = nullptr;
 }
@@ -138,8 +129,9 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
     tiles += tiles_of((size_t)xn);
   }
   const size_t keys = (size_t)(vptr[nvec] - vptr[0]);
-  const Layout at((size_t)nvec, keys, tiles);
-  if ((rc = grow(h, at.bytes, 0))) return rc;
+  const int places = (int)std::min<size_t>(kBatchKeys, keys + nvec);
+  const Layout at((size_t)nvec, tiles, places);
+  if ((rc = grow(h, at.bytes))) return rc;
   BatchState* b = h->batch;
   auto* ctls = reinterpret_cast<Ctl*>(b->mem + at.ctls);
   auto* stash = reinterpret_cast<long long*>(b->mem + at.stash);
@@ -149,6 +141,7 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
   auto* tsum = reinterpret_cast<long long*>(b->mem + at.tsum);
   auto* ptr = reinterpret_cast<int*>(b->mem + at.ptr);
   auto* xbeg = reinterpret_cast<int*>(b->mem + at.xbeg);
+  auto* split = reinterpret_cast<int*>(b->mem + at.split);
   std::vector<BatchVec> h_vec(nvec);
   std::vector<long long> st(nvec);
   std::vector<int> h_tile_vec(tiles), h_list(tiles);
@@ -157,7 +150,7 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
   for (int v = 0; v < nvec; ++v) {
     const int xn = vptr[v + 1] - vptr[v];
     const int nt = (int)tiles_of((size_t)xn);
-    h_vec[v] = BatchVec{vptr[v], xn, tile, nt, 0};
+    h_vec[v] = BatchVec{vptr[v], xn, tile, nt, 0, 0};
     std::fill_n(h_tile_vec.begin() + tile, nt, v);
     tile += nt;
   }
@@ -191,35 +184,33 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
     return r;
   };
   // 2. scans: of the vectors whose slot reads one (the small-x path makes its
-  // own; every column slot has room for its splits)
-  int nlist = 0;
-  long long splits = 0;
-  std::vector<char> scanned(nvec, 0);
+  // own), in groups that fit the workspace; a vector's group, -1: none
+  std::vector<int> group(nvec, -1), group_list{0};
+  int nlist = 0, place = 0, nsplit = 0;
   for (int v = 0; v < nvec; ++v) {
     const int kid = sel_word_choice(st[v]);
     if ((rc = set_x(v))) return rc;
-    h_vec[v].split0 = splits;
-    if (kid <= SPMSPV_K_COL_LB_SORT || needs_scan(kid))
-      splits += (h->xnnz + h->binlen_host) / kLbTile + 3;
-    if (needs_scan(kid) && !takes_small_path(h, kid)) {
-      scanned[v] = 1;
-      for (int t = 0; t < h_vec[v].ntiles; ++t) h_list[nlist++] = h_vec[v].tile0 + t;
+    if (!needs_scan(kid) || takes_small_path(h, kid)) continue;
+    const long long sp = (h->xnnz + h->binlen_host) / kLbTile + 3;
+    if (h->xnnz >= places || sp > kBatchSplits) continue;
+    if (place + h->xnnz + 1 > places || nsplit + sp > kBatchSplits) {
+      group_list.push_back(nlist);
+      place = nsplit = 0;
     }
+    h_vec[v].scan0 = place;
+    h_vec[v].split0 = nsplit;
+    place += h->xnnz + 1;
+    nsplit += (int)sp;
+    group[v] = (int)group_list.size() - 1;
+    for (int t = 0; t < h_vec[v].ntiles; ++t) h_list[nlist++] = h_vec[v].tile0 + t;
   }
-  int* split = reinterpret_cast<int*>(b->mem + at.bytes);
-  if (at.bytes + (size_t)splits * sizeof(int) > b->bytes) {
-    if ((rc = grow(h, 0, (size_t)splits))) return rc;
-    split = b->split;
-  }
+  group_list.push_back(nlist);
   if (nlist > 0) {
     HIP_TRY(h, hipMemcpyAsync(d_vec, h_vec.data(), nvec * sizeof(BatchVec), hipMemcpyHostToDevice, s));
     HIP_TRY(h, hipMemcpyAsync(d_list, h_list.data(), nlist * sizeof(int), hipMemcpyHostToDevice, s));
-    launch_batch_scan(s, h->csc_colptr, d_vkey, h->n, nlist, d_list, d_tile_vec, d_vec, tsum, vptr[0], ptr, xbeg,
-                      split);
-    h->launches++;
-    HIP_TRY(h, hipGetLastError());
   }
-  // queued pipelines, each on its own control block and scan
+  // queued pipelines, each on its own control block and scan; a group's scans
+  // come before its first vector, after the pipelines of the group before it
   {
     struct Restore {
       spmspv_handle_t h;
@@ -232,16 +223,26 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
         h->split = split;
         h->prep_valid = false;
       }
-    } restore{h, h->ctl, h->ptr, h->xbeg, h->split};
+    } own{h, h->ctl, h->ptr, h->xbeg, h->split};
+    int scanned = -1;
     for (int v = 0; v < nvec; ++v) {
       const int kid = sel_word_choice(st[v]);
       if (kernel_used) kernel_used[v] = kid;
+      if (group[v] > scanned) {
+        scanned = group[v];
+        const int l0 = group_list[scanned], l1 = group_list[scanned + 1];
+        launch_batch_scan(s, h->csc_colptr, d_vkey, h->n, l1 - l0, d_list + l0, d_tile_vec, d_vec, tsum, ptr, xbeg,
+                          split);
+        h->launches++;
+        HIP_TRY(h, hipGetLastError());
+      }
       if ((rc = set_x(v))) return rc;
+      const bool in = group[v] >= 0;
       h->ctl = ctls + v;
-      h->ptr = ptr + (vptr[v] - vptr[0]) + v;
-      h->xbeg = xbeg + (vptr[v] - vptr[0]);
-      h->split = split + h_vec[v].split0;
-      h->prep_valid = scanned[v] != 0;
+      h->ptr = in ? ptr + h_vec[v].scan0 : own.ptr;
+      h->xbeg = in ? xbeg + h_vec[v].scan0 : own.xbeg;
+      h->split = in ? split + h_vec[v].split0 : own.split;
+      h->prep_valid = in;
       if ((rc = run_kernel(h, kid, nullptr, d_ykey + yoff[v], d_yval + yoff[v], true))) return rc;
     }
     hipLaunchKernelGGL(k_batch_counts, dim3((nvec + 255) / 256), dim3(256), 0, s, ctls, nvec, d_ynnz);

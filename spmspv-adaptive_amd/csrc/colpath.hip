@@ -758,15 +758,15 @@ template <int NT, int IPT>
 __global__ __launch_bounds__(NT) void k_batch_scan(const int* __restrict__ colptr, const int* __restrict__ xkey,
                                                    int ncols, const int* __restrict__ list,
                                                    const int* __restrict__ tile_vec, const BatchVec* __restrict__ vec,
-                                                   const long long* __restrict__ tsum, int key_base,
+                                                   const long long* __restrict__ tsum,
                                                    int* __restrict__ ptr_all, int* __restrict__ xbeg_all,
                                                    int* __restrict__ split_all) {
   __shared__ long long s_l[NT / kWave];
   const int t = list[blockIdx.x], v = tile_vec[t];
   const BatchVec bv = vec[v];
   const int* __restrict__ keys = xkey + bv.key0;
-  int* __restrict__ ptr = ptr_all + (bv.key0 - key_base) + v;
-  int* __restrict__ xbeg = xbeg_all + (bv.key0 - key_base);
+  int* __restrict__ ptr = ptr_all + bv.scan0;
+  int* __restrict__ xbeg = xbeg_all + bv.scan0;
   int* __restrict__ split = split_all + bv.split0;
   const int base = (t - bv.tile0) * (NT * IPT) + (int)threadIdx.x * IPT;
   int c[IPT], beg[IPT], len[IPT];
@@ -820,11 +820,11 @@ void launch_batch_select(hipStream_t s, const int* colptr, const int* xkey, int 
 }
 
 void launch_batch_scan(hipStream_t s, const int* colptr, const int* xkey, int ncols, int nlist, const int* list,
-                       const int* tile_vec, const BatchVec* vec, const long long* tsum, int key_base, int* ptr,
-                       int* xbeg, int* split) {
+                       const int* tile_vec, const BatchVec* vec, const long long* tsum, int* ptr, int* xbeg,
+                       int* split) {
   if (nlist > 0)
     hipLaunchKernelGGL((k_batch_scan<kPrepNT, kWideIPT>), dim3(nlist), dim3(kPrepNT), 0, s, colptr, xkey, ncols, list,
-                       tile_vec, vec, tsum, key_base, ptr, xbeg, split);
+                       tile_vec, vec, tsum, ptr, xbeg, split);
 }
 
 // ------------------------------------------------------------- naive col

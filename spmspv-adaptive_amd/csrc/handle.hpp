@@ -204,8 +204,8 @@ void pr_release(spmspv_handle_t h);
 // Allocates / frees the multi-source BFS buffers (square matrices).
 int ms_alloc(spmspv_handle_t h);
 void ms_release(spmspv_handle_t h);
-// Allocates (for kBatchVecs vectors of at least kBatchKeys keys in all; a
-// larger batch grows it) / frees the workspace of run_batched.
+// Allocates (for kBatchVecs vectors of any size; a batch of more grows it) /
+// frees the workspace of run_batched.
 int batch_alloc(spmspv_handle_t h);
 void batch_release(spmspv_handle_t h);
 // Drops the captured BFS level graphs (they hold matrix and arena pointers).

@@ -153,13 +153,13 @@ void launch_prep(hipStream_t s, const int* colptr, const int* xkey, int ncols, i
                  const int* xnnz_dev, int* ptr, int* xbeg, int* split, unsigned long long* state,
                  int* tile_mm, Ctl* ctl, const SelectorArgs* sel, Ep ep, long long* samp = nullptr,
                  bool wide = false, const LevelOpen& open = {});
-// The vectors of a batch: one launch selects for all of them, one scans all
+// The vectors of a batch: one launch selects for all of them, one scans many
 // that need it. Vector v has keys xkey[key0 .. key0 + xnnz), tiles
 // [tile0, tile0 + ntiles) of kWideTile keys (at least one) and, once its
-// slot is known, splits from split0.
+// slot is known, its scan from scan0 (xnnz + 1 places) and splits from split0.
 struct BatchVec {
   int key0, xnnz, tile0, ntiles;
-  long long split0;
+  int scan0, split0;
 };
 // Per vector: ctls[v].{bin_len, max_len, xnnz, n_tiles} and the selector word
 // (exact bin_len and choice) in stash[v]. tile_vec[t]: vector of tile t;
@@ -167,11 +167,11 @@ struct BatchVec {
 void launch_batch_select(hipStream_t s, const int* colptr, const int* xkey, int ncols, int ntiles, const int* tile_vec,
                          const BatchVec* vec, long long* tsum, int* tmax, unsigned* arrive, Ctl* ctls,
                          const SelectorArgs& sel, long long* stash);
-// ptr (at key0 - key_base + v), xbeg (at key0 - key_base) and split (at split0) as
-// launch_prep, for the tiles listed: list[i] = tile.
+// ptr and xbeg (at scan0) and split (at split0) as launch_prep, for the tiles
+// listed: list[i] = tile.
 void launch_batch_scan(hipStream_t s, const int* colptr, const int* xkey, int ncols, int nlist, const int* list,
-                       const int* tile_vec, const BatchVec* vec, const long long* tsum, int key_base, int* ptr,
-                       int* xbeg, int* split);
+                       const int* tile_vec, const BatchVec* vec, const long long* tsum, int* ptr, int* xbeg,
+                       int* split);
 // Features-only selector: ctl->{bin_len, max_len, min_len, xnnz} of x and,
 // with sel.mat set, the selector's choice (and the selector word in
 // sel.stash). part: 5 * kSelMaxGrid partials. No column scan. With enc set
