@@ -312,8 +312,10 @@ int spmspv_set_switch_penalty(spmspv_handle_t h, float penalty);
  * spmspv_run_auto then decides such calls by this size rule before the
  * network and reports slot 1. With more products the launch runs the
  * network, and the gather too when an atomic column slot is chosen. Off
- * (0): every slot always runs its own launches. Results are the same
- * either way. */
+ * (0): every slot always runs its own launches. The rows and their count are
+ * the same either way; the values agree within FP32 rounding (on the
+ * single-launch path a row's sum is exact but for 2^-46 of its largest
+ * product, and the same in every call). */
 int spmspv_set_small_x_path(spmspv_handle_t h, int on);
 int spmspv_speculation_stats(spmspv_handle_t h, long long* hits, long long* misses);
 

@@ -22,16 +22,16 @@
 // levels and lists them, with one list append per workgroup round: device
 // atomics on one address take 16 ns each, and an append per wave in every
 // slot kernel had made those kernels wait for the counter. R-MAT s22, one
-// source: 1,440 -> 490 us.
+// source: 1,440 -> 450 us.
 // Levels are int32 and unique, so any order of claims gives the same
 // levels. The selector for level L+1 runs in the same stream right after
-// level L (features of the new frontier + MLP, one launch), and a last
-// one-wave kernel writes the next frontier's size and choice, tagged with
-// the level counter, into one host-coherent word that the host polls (no
-// stream wait, no copies); with graphs on, each (slot, parity) level
-// sequence is captured once as a hipGraph and replayed. Every kernel reads
-// the frontier size from device memory, which is what makes the capture
-// valid for any level.
+// level L (column scan and features of the new frontier + MLP, one launch),
+// whose selecting workgroup writes the frontier's features and then its size
+// and the choice, tagged with the level counter, into host-coherent words; the
+// host polls the last one (no stream wait, no copies); with graphs on, each
+// (slot, parity) level sequence is captured once as a hipGraph and replayed.
+// Every kernel reads the frontier size from device memory, which is what makes
+// the capture valid for any level.
 #include <hip/hip_runtime.h>
 
 #include <chrono>
@@ -396,8 +396,8 @@ int lg2(int t) {
 }
 
 // Enqueues one level on stream s: the slot's kernels on frontier `cur`, the
-// collect pass, the selector on the new frontier, and the word with
-// (new frontier size, next slot) for the host.
+// collect pass, and the column scan of the new frontier with the selector and
+// the host's words.
 void enqueue_level(spmspv_handle_t h, hipStream_t s, int slot, int cur, int* levels,
                    const SelectorArgs& sel) {
   BfsState* b = h->bfs;

@@ -10,8 +10,8 @@ namespace spmspv {
 // integer q = m * 2^(ef - E + 22) (rounded to nearest when the shift is to
 // the right), where E is the largest ef among the products of r that
 // are summed together: |q| < 2^46, so at most 2^14 of them sum exactly in 64
-// bits, in any order, and the row's value is the sum times 2^(E - 172),
-// rounded once to FP32. Each product's error is at most 2^-46 of the row's
+// bits, in any order, and the row's value is the sum times 2^(E - 172), rounded
+// to FP64 and from there to FP32. Each product's error is at most 2^-46 of the row's
 // largest |product|. Integer LDS atomics (max for E, add for the sum) run
 // about 15 times faster on gfx950 than FP32 LDS atomic adds.
 __device__ __forceinline__ unsigned prod_ef(float v) {

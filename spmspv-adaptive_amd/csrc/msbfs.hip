@@ -96,9 +96,7 @@ __device__ __forceinline__ void write_levels(int v, unsigned long long nw, int n
 // frontier of vertices without neighbours is not empty).
 __device__ __forceinline__ int ms_chunks(int deg) { return max(1, (deg + kMsChunk - 1) / kMsChunk); }
 
-// Bits, levels and counters of the sources; the sources' work items are the
-// first frontier (a repeated source is listed once) and the sum of their
-// degrees gives the first level's direction.
+// No vertex visited or in a frontier, all levels -1, the counters at 0.
 __global__ void k_ms_init(int n, int nsrc, unsigned long long* visit, unsigned long long* f0,
                           unsigned long long* f1, int* levels, unsigned long long* cnt) {
   const long long stride = (long long)gridDim.x * blockDim.x;
@@ -120,6 +118,9 @@ __device__ void ms_signal(const unsigned long long* c, int tag, long long* sig) 
                      __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Bits and levels of the sources; their work items are the first frontier (a
+// repeated source is listed once) and the sum of their degrees gives the first
+// level's direction.
 __global__ __launch_bounds__(kWave) void k_ms_sources(int nsrc, MsSrcs srcs, const int* __restrict__ colptr,
                                                       unsigned long long* visit, unsigned long long* f0,
                                                       int* levels, int2* list, long long* sig) {
