@@ -143,7 +143,9 @@ int spmspv_set_sparse_x_dense_x(spmspv_handle_t h, int* d_key, float* d_val, flo
 /* ---- vector format conversions (spmspv.h:1121-1390, 1880-1998) ---------- */
 int spmspv_sparse2dense(spmspv_handle_t h);     /* sparse2dense    :1239-1268 */
 int spmspv_sparse2bitarray(spmspv_handle_t h);  /* sparse2bitarray :1270-1307 */
-int spmspv_dense2sparse(spmspv_handle_t h);     /* dense2sparse    :1176-1223 */
+/* dense2sparse (:1176-1223) writes the arrays lent with set_sparse_x where they
+ * hold that many entries (as many as were lent), else the handle's own. */
+int spmspv_dense2sparse(spmspv_handle_t h);
 int spmspv_dense2bitarray(spmspv_handle_t h);   /* dense2bitarray  :1371-1389 */
 int spmspv_bitarray2sparse(spmspv_handle_t h);  /* bitarray2sparse :1310-1352 */
 /* dense2sparse_outer, spmspv.h:1950-1998 (keeps entries != 0; *ynnz set). */

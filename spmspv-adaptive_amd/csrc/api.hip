@@ -201,6 +201,17 @@ int ensure_arena(spmspv_handle_t h) {
   return SPMSPV_SUCCESS;
 }
 
+void unset_x(spmspv_handle_t h) {
+  h->x_key = nullptr;
+  h->x_val = nullptr;
+  h->sparse_valid = h->dense_valid = h->bits_valid = false;
+  h->enc_valid = h->enc5_valid = false;
+  h->prep_valid = false;
+  h->binlen_host = -1;
+  h->vec_type = -1;
+  h->xnnz = 0;
+}
+
 int ensure_row_tiles(spmspv_handle_t h) {
   if (h->row_ready) return SPMSPV_SUCCESS;
   if (!h->csr_row) return set_error(h, SPMSPV_MAT_FORMAT_ERR, "row kernels need CSR input");
@@ -1039,6 +1050,7 @@ int spmspv_set_sparse_x(spmspv_handle_t h, int* key, float* val, int xnnz) {
   if (xnnz > 0 && (!key || !val)) return set_error(h, SPMSPV_INVALID_ARGUMENT, "null x arrays");
   h->x_key = key;
   h->x_val = val;
+  h->x_cap = xnnz;
   h->xnnz = xnnz;
   h->vec_type = SPMSPV_VEC_SPARSE;
   h->sparse_valid = true;
@@ -1127,14 +1139,15 @@ int spmspv_dense2bitarray(spmspv_handle_t h) {
 }
 
 int spmspv_dense2sparse(spmspv_handle_t h) {
-  // keeps entries != 0 (spmspv.h:1176-1223); writes the handle's own key/val
-  // buffers unless the caller set sparse buffers with set_sparse_x
+  // keeps entries != 0 (spmspv.h:1176-1223), in the handle's own key/val
+  // buffers, or in the arrays that the caller lent with set_sparse_x where they
+  // hold that many
   if (!h) return set_error(nullptr, SPMSPV_INVALID_ARGUMENT, "null handle");
   if (!h->dense_valid) return set_error(h, SPMSPV_VEC_FORMAT_ERR, "dense2sparse: no dense x");
   int rc = ensure_arena(h);
   if (rc) return rc;
-  int* k = h->x_key ? h->x_key : h->xk_int;
-  float* v = h->x_val ? h->x_val : h->xv_int;
+  int* k = h->xk_int;
+  float* v = h->xv_int;
   // the handle's own bit array as scratch (the compaction clears it): a
   // bit array the caller lent with set_bitvector keeps its contents
   unsigned* b = h->bits_int;
@@ -1148,6 +1161,14 @@ int spmspv_dense2sparse(spmspv_handle_t h) {
   int cnt = 0;
   rc = readback_ynnz(h, &cnt);
   if (rc) return rc;
+  if (h->x_key && h->x_val && h->x_key != k && cnt <= h->x_cap) {
+    if (cnt > 0) {
+      HIP_TRY(h, hipMemcpyAsync(h->x_key, k, sizeof(int) * (size_t)cnt, hipMemcpyDeviceToDevice, h->stream));
+      HIP_TRY(h, hipMemcpyAsync(h->x_val, v, sizeof(float) * (size_t)cnt, hipMemcpyDeviceToDevice, h->stream));
+    }
+    k = h->x_key;
+    v = h->x_val;
+  }
   h->x_key = k;
   h->x_val = v;
   h->xnnz = cnt;

@@ -183,6 +183,10 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
     h->binlen_host = sel_word_binlen(st[v]);
     return r;
   };
+  struct Unset {
+    spmspv_handle_t h;
+    ~Unset() { unset_x(h); }
+  } unset{h};
   // 2. scans: of the vectors whose slot reads one (the small-x path makes its
   // own), in groups that fit the workspace; a vector's group, -1: none
   std::vector<int> group(nvec, -1), group_list{0};
@@ -250,14 +254,6 @@ int spmspv_run_batched(spmspv_handle_t h, int nvec, const int* d_vptr, const int
   }
   // 3. the batch is complete when this returns; x is left unset
   HIP_TRY(h, hipStreamSynchronize(s));
-  h->sparse_valid = false;
-  h->dense_valid = false;
-  h->bits_valid = false;
-  h->enc_valid = h->enc5_valid = false;
-  h->prep_valid = false;
-  h->binlen_host = -1;
-  h->vec_type = -1;
-  h->xnnz = 0;
   return SPMSPV_SUCCESS;
 }
 

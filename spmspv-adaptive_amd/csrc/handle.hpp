@@ -36,6 +36,7 @@ struct spmspv_handle_s {
   int* x_key = nullptr;
   float* x_val = nullptr;
   int xnnz = 0;
+  int x_cap = 0;  // entries that x_key / x_val were lent with
   float* x_dense_user = nullptr;
   unsigned* bits_user = nullptr;
   int num_ints_user = 0;
@@ -223,6 +224,8 @@ int wait_signal(spmspv_handle_t h, int idx, long long* out);
 Ep next_ep(spmspv_handle_t h, unsigned k);
 // Reads bin_len of the current x back to the host (one synchronisation).
 int ensure_binlen_host(spmspv_handle_t h);
+// Leaves no x set (after a driver's own x, which the handle must not touch again).
+void unset_x(spmspv_handle_t h);
 // Builds the bucket slot's bin layout for the current matrix and bucket_bits.
 int ensure_bin_layout(spmspv_handle_t h);
 }  // namespace spmspv

@@ -263,6 +263,7 @@ int spmspv_pagerank(spmspv_handle_t h, float damping, float eps, int max_iter, i
     ~Restore() {
       h->sel_mode = mode;
       h->sel_fixed = fixed;
+      unset_x(h);  // x was the driver's own buffer
     }
   } restore{h, saved_mode, saved_fixed};
   const auto t0 = std::chrono::steady_clock::now();
@@ -296,13 +297,6 @@ int spmspv_pagerank(spmspv_handle_t h, float damping, float eps, int max_iter, i
   hipLaunchKernelGGL(k_pr_finish, dim3(grid_of(n)), dim3(256), 0, s, n, d_rank, st->r);
   HIP_TRY(h, hipGetLastError());
   HIP_TRY(h, hipStreamSynchronize(s));
-  // x was the driver's own buffer: leave none set
-  h->sparse_valid = h->dense_valid = h->bits_valid = false;
-  h->enc_valid = h->enc5_valid = false;
-  h->prep_valid = false;
-  h->binlen_host = -1;
-  h->vec_type = -1;
-  h->xnnz = 0;
   if (stats) {
     stats[0] = it;
     stats[1] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

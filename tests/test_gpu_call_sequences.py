@@ -346,3 +346,55 @@ def test_products_fall_below_the_guess(gpu, slot, out):
             ref[ek], bound[ek] = ev, eb
             assert np.all(np.abs(yd.to_host() - ref) <= 1e-5 * bound + 1e-30)
         last = products
+
+
+def test_lent_sparse_arrays_keep_their_size(gpu):
+    """A dense x that a column slot turns into a sparse one is written into
+    the caller's arrays where it fits the entries that were lent, else into the
+    handle's own; arrays lent to a batch are never written."""
+    n = 1 << 12
+    rp, col, val = sa.gen_rmat_csr(12, 8, seed=2)
+    M = sa.Matrix(n, n, rp, col, val)
+    csc = oracle.csr_to_csc(n, n, rp, col, val)
+    yk, yv = sa.DeviceArray(n, np.int32), sa.DeviceArray(n, np.float32)
+    # room for all of x, of which ten entries are lent
+    key, xv = np.full(n, -7, np.int32), np.full(n, 9.0, np.float32)
+    key[:10], xv[:10] = np.arange(10) * 300, 1.0
+    dk, dv = sa.DeviceArray.from_host(key), sa.DeviceArray.from_host(xv)
+
+    def product(x, tag):
+        dx = sa.DeviceArray.from_host(x)
+        M.A.set_vector_type(sa.SPMSPV_VEC_DENSE)
+        M.A.set_x(dx)
+        cnt = M.A.run(sa.K_COL_LB_ATOMIC, y_key=yk, y_val=yv)
+        nz = np.nonzero(x)[0].astype(np.int32)
+        ek, ev, eb = oracle.spmspv_f64(n, *csc, nz, x[nz])
+        np.testing.assert_array_equal(yk.to_host(cnt), ek, err_msg=tag)
+        assert np.all(np.abs(yv.to_host(cnt).astype(np.float64) - ev) <= 1e-5 * eb + 1e-30), tag
+        return nz
+
+    rng = np.random.default_rng(1)
+    large, small = np.zeros(n, np.float32), np.zeros(n, np.float32)
+    large[rng.choice(n, 2000, replace=False)] = rng.uniform(0.5, 1, 2000)
+    small[rng.choice(n, 10, replace=False)] = rng.uniform(0.5, 1, 10)
+    M.A.set_sparse_x(dk, dv, 10)
+    product(large, "past the lent entries")
+    np.testing.assert_array_equal(dk.to_host(), key)
+    np.testing.assert_array_equal(dv.to_host(), xv)
+    M.A.set_sparse_x(dk, dv, 10)
+    nz = product(small, "as many as were lent")
+    np.testing.assert_array_equal(dk.to_host(10), nz)
+    np.testing.assert_array_equal(dv.to_host(10), small[nz])
+    np.testing.assert_array_equal(dk.to_host()[10:], key[10:])
+    # a batch whose last vector has ten entries
+    dk.upload(key)
+    dv.upload(xv)
+    vptr, yoff = sa.DeviceArray.from_host(np.array([0, 10], np.int32)), sa.DeviceArray.from_host(np.array([0, n], np.int64))
+    M.A.run_batched(vptr, dk, dv, yoff, yk, yv, sa.DeviceArray(1, np.int32))
+    for x, tag in ((small, "after a batch"), (large, "after a batch, large")):
+        product(x, tag)
+        np.testing.assert_array_equal(dk.to_host(), key)
+        np.testing.assert_array_equal(dv.to_host(), xv)
+    rank = sa.DeviceArray(n, np.float32)
+    M.A.pagerank(rank)
+    product(large, "after PageRank")
