@@ -349,12 +349,13 @@ __device__ __forceinline__ unsigned direct_start(const unsigned* cnt, const unsi
 // through the first one's LDS, which leaves two workgroups per CU; 512 x 16 took
 // 88, 1,024 x 6 and x 8 105 us. Their counts do not fit 16 bits per 16 tiles, so
 // the positions come from the scan. ToCSC with the narrow / wide tile, us:
-// R-MAT 0.88 M nonzeros 59 / 75, 1.82 M 73 / 87, 3.73 M 131 / 144, 5.34 M 169 /
-// 176, 7.61 M 211 / 211, 15.5 M 432 / 408; even columns 2.10 M 89 / 109, 4.19 M
-// 137 / 145, 6.29 M 176 / 175, 8.39 M 219 / 223, 12.6 M 346 / 330, 16.8 M 504 /
-// 442.
+// R-MAT 0.88 M nonzeros 59 / 75, 1.82 M 73 / 87, 4.41 M 158 / 166, 5.34 M 182 /
+// 186, 6.26 M 198 / 198, 7.61 M 218 / 218, 15.5 M 432 / 408; even columns 2.10 M
+// 89 / 109, 4.88 M 162 / 165, 5.88 M 180 / 180, 6.88 M 195 / 200, 8.39 M 219 /
+// 223, 12.6 M 346 / 330, 16.8 M 504 / 442; banded 4.46 M 153 / 158, 6.29 M 206 /
+// 203, 7.34 M 229 / 225.
 constexpr int kWideNT = 512;
-constexpr long long kWideItems = 1 << 23;
+constexpr long long kWideItems = 6 << 20;
 
 // PAY: payload words per item (0: keys only). Four waves per SIMD (three with
 // two payloads, as LDS allows): five spill the payloads (R-MAT scale 22, 1 %:

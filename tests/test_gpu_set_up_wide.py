@@ -1,5 +1,5 @@
 """The CSC of a matrix around the size from which its sort runs in wide tiles
-(2^23 nonzeros, tiles of 6,144), with columns of one entry and columns of many:
+(6 * 2^20 nonzeros, tiles of 6,144), with columns of one entry and columns of many:
 products through the CSC against the FP64 oracle."""
 import numpy as np
 import pytest
@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("extra", [-1, 0, 1, 6143, 6145])
 @pytest.mark.parametrize("n", [900, 70001])
 def test_csc_around_the_wide_tiles(gpu, n, extra):
-    nnz, per = (1 << 23) + extra, 16
+    nnz, per = (6 << 20) + extra, 16
     m = nnz // per + 700
     lens = np.zeros(m, np.int64)
     lens[: nnz // per] = per
