@@ -340,8 +340,9 @@ int spmspv_mlp_forward(const float* params, const float* X, int B, float* logits
  * la/test/test_application.cu:207-261; this is the loop it lacked) ------- */
 /* Level-synchronous BFS over the CSC pattern from `src`. d_levels[n]
  * receives int32 levels (-1 unreached). policy: -1 = learned per-level
- * selection, 0..7 = fixed slot. Levels are captured as hipGraphs when
- * use_graphs != 0. stats (nullable) gets {levels, edges_traversed,
+ * selection, 0..7 = fixed slot; slots 4, 5 and 7 step bottom-up where the
+ * frontier holds more than 1/32 of the edges, else as slot 2. Levels are
+ * captured as hipGraphs when use_graphs != 0. stats (nullable) gets {levels, edges_traversed,
  * seconds, reached}. */
 int spmspv_bfs(spmspv_handle_t h, int src, int* d_levels, int policy, int use_graphs,
                double stats[4]);
